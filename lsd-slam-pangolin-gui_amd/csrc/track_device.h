@@ -141,10 +141,63 @@ __device__ inline float fsqrt(float x) {
   else return __builtin_amdgcn_sqrtf(x);
 }
 
+// The FP32 point math divides about ten times by six values.  A / operator is
+// a scaled sequence of ten instructions each time; where the operands are far
+// from the ends of the exponent range the scaling is not needed and one
+// correctly rounded reciprocal serves every division by the same value.
+//
+// recip_rn: v_rcp_f32 is within 1 ulp; one Newton step in fma arithmetic gives
+// 1 / b correctly rounded (checked for every significand).
+// div_rn: a / b from y = RN(1 / b).  q0 = RN(a y) is within two ulps; the
+// remainder a - b q0 is exact up to 2^-24 of itself, so q1 is within one ulp
+// of a / b, its remainder is exact, and the last fma rounds correctly
+// (Markstein 1990: a faithful quotient, an exact remainder and RN(1 / b)).
+// sqrt_rn: v_sqrt_f32 is within 1 ulp; s is moved to a neighbour when
+// s (s - ulp) >= x or s (s + ulp) < x.
+// All three need operands and results well inside the normal range, which
+// exp_in / num_ok test on the wave before they are used.
+// The evaluation is bound by VALU issue: about 120 of an FP32 point's 560
+// instructions were the scaled sequences, of which 45 remain (64 alignments of
+// 640x480 in one plan: 562 -> 534 us).
+struct RecipRN {
+  float b, y;
+};
+__device__ inline RecipRN recip_rn(float b) {
+  const float y0 = __builtin_amdgcn_rcpf(b);
+  return {b, __builtin_fmaf(__builtin_fmaf(-b, y0, 1.0f), y0, y0)};
+}
+__device__ inline float div_rn(float a, const RecipRN& r) {
+  const float q0 = a * r.y;
+  const float q1 = __builtin_fmaf(__builtin_fmaf(-r.b, q0, a), r.y, q0);
+  return __builtin_fmaf(__builtin_fmaf(-r.b, q1, a), r.y, q1);
+}
+__device__ inline float sqrt_rn(float x) {
+  const float s = __builtin_amdgcn_sqrtf(x);
+  const float lo = __uint_as_float(__float_as_uint(s) - 1u), hi = __uint_as_float(__float_as_uint(s) + 1u);
+  float o = __builtin_fmaf(-lo, s, x) <= 0.0f ? lo : s;
+  return __builtin_fmaf(-hi, s, x) > 0.0f ? hi : o;
+}
+// |x| in [2^-E, 2^E]: one shift-and-add and an unsigned compare (the sign
+// shifts out; zero, infinities and NaN fail).
+template <int E>
+__device__ inline unsigned exp_key(float x) {
+  return (__float_as_uint(x) << 1) - ((127u - E) << 24);
+}
+template <int E>
+__device__ inline bool exp_in(float x) {
+  return exp_key<E>(x) <= (2u * E) << 24;
+}
+// x is zero or at least 2^-90 in magnitude: the remainders of its division
+// stay normal numbers.
+__device__ inline unsigned num_key(float x) { return (__float_as_uint(x) << 1) - (37u << 24); }
+__device__ inline bool num_ok(unsigned key) { return key <= 0u - (37u << 24); }
+
 // Projection of one reference point into the frame (the warp every tracker
 // evaluation starts with).
 struct Proj {
   float Wx, Wy, Wz, u, v;
+  float rz;   // FP32, fast: RN(1 / Wz)
+  bool fast;  // FP32: the wave's Wz and p.z allow the unscaled divisions
   bool in;
 };
 
@@ -155,17 +208,31 @@ __device__ inline Proj project(const float4& p, const Xf& x, const LevelGeom& g)
   o.Wx = x.R[0] * p.x + x.R[1] * p.y + x.R[2] * p.z + x.t[0];
   o.Wy = x.R[3] * p.x + x.R[4] * p.y + x.R[5] * p.z + x.t[1];
   o.Wz = x.R[6] * p.x + x.R[7] * p.y + x.R[8] * p.z + x.t[2];
-  o.u = fdiv<PREC>(o.Wx, o.Wz) * g.fx + g.cx;
-  o.v = fdiv<PREC>(o.Wy, o.Wz) * g.fy + g.cy;
+  o.fast = false;
+  o.rz = 0.0f;
+  if constexpr (PREC == LSDG_FP32) {
+    // depths within [2^-20, 2^20] (any unit a map is kept in): every
+    // denominator below stays within [2^-60, 2^60]
+    o.fast = __all(max(exp_key<20>(o.Wz), exp_key<20>(p.z)) <= 40u << 24);
+    if (__builtin_expect(o.fast, 1)) {
+      const RecipRN r = recip_rn(o.Wz);
+      o.rz = r.y;
+      o.u = div_rn(o.Wx, r) * g.fx + g.cx;
+      o.v = div_rn(o.Wy, r) * g.fy + g.cy;
+    } else {
+      o.u = (o.Wx / o.Wz) * g.fx + g.cx;
+      o.v = (o.Wy / o.Wz) * g.fy + g.cy;
+    }
+  } else {
+    o.u = fdiv<PREC>(o.Wx, o.Wz) * g.fx + g.cx;
+    o.v = fdiv<PREC>(o.Wy, o.Wz) * g.fy + g.cy;
+  }
   o.in = o.u > 1.0f && o.v > 1.0f && o.u < wlim && o.v < hlim;
   return o;
 }
 
 // -v = dr/dxi of the photometric residual (SE3Tracker::calculateWarpUpdate).
-template <int PREC>
-__device__ inline void jac6(float px, float py, float pz, float gx, float gy, float* v) {
-  float z = frcp<PREC>(pz);
-  float z_sqr = frcp<PREC>(pz * pz);
+__device__ inline void jac6(float px, float py, float z, float z_sqr, float gx, float gy, float* v) {
   v[0] = z * gx;
   v[1] = z * gy;
   v[2] = (-px * z_sqr) * gx + (-py * z_sqr) * gy;
@@ -173,6 +240,73 @@ __device__ inline void jac6(float px, float py, float pz, float gx, float gy, fl
   v[4] = (1.0f + px * px * z_sqr) * gx + (px * py * z_sqr) * gy;
   v[5] = (-py * z) * gx + (px * z) * gy;
 }
+
+// The quotients every point needs of its depth before and after the warp:
+// z = 1 / Wz, z_sqr = 1 / Wz^2, dc = p.z / Wz, and of the denominator
+// Wz^2 / p.z the derivatives g0, g1 of the projection (and with G2 g2, of
+// 1 / Wz) by the point's inverse depth.
+struct PointGeom {
+  float z, z_sqr, dc, g0, g1, g2;
+};
+template <int PREC, bool G2>
+__device__ inline PointGeom point_geom(float pz, const Proj& w, const Xf& x) {
+  const float n0 = x.t[0] * w.Wz - x.t[2] * w.Wx;
+  const float n1 = x.t[1] * w.Wz - x.t[2] * w.Wy;
+  const float n2 = G2 ? w.Wz - x.t[2] : 0.0f;
+  PointGeom o;
+  o.g2 = 0.0f;
+  if constexpr (PREC == LSDG_FP32) {
+    unsigned nk = max(num_key(n0), num_key(n1));
+    if (G2) nk = max(nk, num_key(n2));
+    if (__builtin_expect(w.fast && __all(num_ok(nk)), 1)) {
+      o.z = w.rz;
+      o.z_sqr = recip_rn(w.Wz * w.Wz).y;
+      o.dc = div_rn(pz, RecipRN{w.Wz, w.rz});
+      const RecipRN den = recip_rn(w.Wz * w.Wz * recip_rn(pz).y);
+      o.g0 = div_rn(n0, den);
+      o.g1 = div_rn(n1, den);
+      if (G2) o.g2 = div_rn(n2, den);
+      return o;
+    }
+  }
+  const float d = frcp<PREC>(pz);
+  o.z = frcp<PREC>(w.Wz);
+  o.z_sqr = frcp<PREC>(w.Wz * w.Wz);
+  o.dc = fdiv<PREC>(pz, w.Wz);
+  o.g0 = fdiv<PREC>(n0, w.Wz * w.Wz * d);
+  o.g1 = fdiv<PREC>(n1, w.Wz * w.Wz * d);
+  if (G2) o.g2 = fdiv<PREC>(n2, w.Wz * w.Wz * d);
+  return o;
+}
+
+// w = 1 / D and sqrt(w) of a variance D.
+template <int PREC>
+__device__ inline void weight_of(float D, float& w, float& sq) {
+  if constexpr (PREC == LSDG_FP32) {
+    if (__builtin_expect(__all(exp_in<60>(D)), 1)) {
+      w = recip_rn(D).y;
+      sq = sqrt_rn(w);
+      return;
+    }
+  }
+  w = frcp<PREC>(D);
+  sq = fsqrt<PREC>(w);
+}
+
+// The Huber weight min(1, k / e) of a normalised residual e >= 0.
+template <int PREC>
+__device__ inline float huber_weight(float e, float k) {
+  if (e < k) return 1.0f;
+  if constexpr (PREC == LSDG_FP32) {
+    if (__builtin_expect(__all(exp_in<60>(e) && exp_in<60>(k)), 1)) return fabsf(div_rn(k, recip_rn(e)));
+  }
+  return fabsf(fdiv<PREC>(k, e));
+}
+
+// a / b < 1 for a >= 0 without the division: for floats a < b the quotient is
+// at most pred(b) / b <= 1 - 2^-24, a float, and rounds to no more than that;
+// with b < 0 it is negative (or -0).
+__device__ inline bool ratio_below_one(float a, float b) { return a < b || (b < 0.0f && a == a); }
 
 // Per-thread accumulators of the per-point FP32 terms.
 //  ACC_F64:   each FP32 term is widened and summed in FP64 (the parity mode:
@@ -371,7 +505,7 @@ template <int PREC, class ACC>
 __device__ inline void se3_finish(const float4& p, float pvar, int pidx, const Proj& w, const TapRaw<PREC>& t,
                                   const Xf& x, const LevelGeom& g, const TrackKParams& kp,
                                   uint8_t* __restrict__ isGood, ACC& acc) {
-  const float Wx = w.Wx, Wy = w.Wy, Wz = w.Wz;
+  const float Wx = w.Wx, Wy = w.Wy;
   if (!w.in) {
     if (isGood) isGood[pidx] = 0;
     return;
@@ -388,10 +522,10 @@ __device__ inline void se3_finish(const float4& p, float pvar, int pidx, const P
     acc.add(S3_SY, c2 * wgt);
     acc.add(S3_SW, wgt);
   }
-  bool good = fdiv<PREC>(r * r, kp.max_diff_constant + kp.max_diff_grad_mult * (ri.gx * ri.gx + ri.gy * ri.gy)) < 1.0f;
+  bool good = ratio_below_one(r * r, kp.max_diff_constant + kp.max_diff_grad_mult * (ri.gx * ri.gx + ri.gy * ri.gy));
   if (isGood) isGood[pidx] = good ? 1 : 0;
   float gx = g.fx * ri.gx, gy = g.fy * ri.gy;
-  float d = frcp<PREC>(p.z);
+  const PointGeom q = point_geom<PREC, false>(p.z, w, x);
   if (good) {
     acc.add(S3_RESUNW, r * r);
     acc.add(S3_SIGNED, r);
@@ -399,21 +533,19 @@ __device__ inline void se3_finish(const float4& p, float pvar, int pidx, const P
   } else {
     acc.add(S3_BAD, 1.0f);
   }
-  float dc = fdiv<PREC>(p.z, Wz);
-  acc.add(S3_USAGE, dc < 1.0f ? dc : 1.0f);
+  acc.add(S3_USAGE, q.dc < 1.0f ? q.dc : 1.0f);
   acc.add(S3_WARPED, 1.0f);
   // calcWeightsAndResidual
   float s = kp.var_weight * pvar;
-  float g0 = fdiv<PREC>(x.t[0] * Wz - x.t[2] * Wx, Wz * Wz * d);
-  float g1 = fdiv<PREC>(x.t[1] * Wz - x.t[2] * Wy, Wz * Wz * d);
-  float drpdd = gx * g0 + gy * g1;
-  float w_p = frcp<PREC>(kp.noise2 + s * drpdd * drpdd);
-  float wr = fabsf(r * fsqrt<PREC>(w_p));
-  float wh = fabsf(wr < kp.huber ? 1.0f : fdiv<PREC>(kp.huber, wr));
+  float drpdd = gx * q.g0 + gy * q.g1;
+  float w_p, sq_p;
+  weight_of<PREC>(kp.noise2 + s * drpdd * drpdd, w_p, sq_p);
+  float wr = fabsf(r * sq_p);
+  float wh = huber_weight<PREC>(wr, kp.huber);
   float W = wh * w_p;
   // calculateWarpUpdate
   float jv[6];
-  jac6<PREC>(Wx, Wy, Wz, gx, gy, jv);
+  jac6(Wx, Wy, q.z, q.z_sqr, gx, gy, jv);
   int k = 0;
 #pragma unroll
   for (int a = 0; a < 6; ++a)
@@ -468,7 +600,7 @@ __device__ inline void sim3_finish(const float4& p, float pvar, float2 rg, const
                                    float fidR, float varF, const Xf& x, const LevelGeom& g, const TrackKParams& kp,
                                    ACC& acc) {
   if (!w.in) return;
-  const float Wx = w.Wx, Wy = w.Wy, Wz = w.Wz;
+  const float Wx = w.Wx, Wy = w.Wy;
   Taps ri = blend_taps<PREC>(t);
   float gx, gy;
   if (kp.use_esm) {
@@ -491,32 +623,28 @@ __device__ inline void sim3_finish(const float4& p, float pvar, float2 rg, const
     acc.add(SM_SY, c2 * wgt);
     acc.add(SM_SW, wgt);
   }
-  float refId = frcp<PREC>(Wz);
-  float d = frcp<PREC>(p.z);
+  const PointGeom q = point_geom<PREC, true>(p.z, w, x);
   float rd, vard;
   if (varF > 0.0f) {
-    rd = refId - fidR;
+    rd = q.z - fidR;
     vard = varF;
   } else {
     rd = -1.0f;
     vard = -1.0f;
   }
-  float dc = fdiv<PREC>(p.z, Wz);
-  acc.add(SM_USAGE, dc < 1.0f ? dc : 1.0f);
+  acc.add(SM_USAGE, q.dc < 1.0f ? q.dc : 1.0f);
   acc.add(SM_WARPED, 1.0f);
   // calcSim3WeightsAndResidual
   float s = kp.var_weight * pvar;
   float sv = kp.var_weight * vard;
-  float g0 = fdiv<PREC>(x.t[0] * Wz - x.t[2] * Wx, Wz * Wz * d);
-  float g1 = fdiv<PREC>(x.t[1] * Wz - x.t[2] * Wy, Wz * Wz * d);
-  float g2 = fdiv<PREC>(Wz - x.t[2], Wz * Wz * d);
-  float drpdd = gx * g0 + gy * g1;
-  float w_p = frcp<PREC>(kp.noise2 + s * drpdd * drpdd);
-  float w_d = frcp<PREC>(sv + g2 * g2 * s);
-  float wrd = fabsf(rd * fsqrt<PREC>(w_d));
-  float wrp = fabsf(rp * fsqrt<PREC>(w_p));
+  float drpdd = gx * q.g0 + gy * q.g1;
+  float w_p, w_d, sq_p, sq_d;
+  weight_of<PREC>(kp.noise2 + s * drpdd * drpdd, w_p, sq_p);
+  weight_of<PREC>(sv + q.g2 * q.g2 * s, w_d, sq_d);
+  float wrd = fabsf(rd * sq_d);
+  float wrp = fabsf(rp * sq_p);
   float wabs = sv > 0.0f ? wrd + wrp : wrp;
-  float wh = fabsf(wabs < kp.huber ? 1.0f : fdiv<PREC>(kp.huber, wabs));
+  float wh = huber_weight<PREC>(wabs, kp.huber);
   if (sv > 0.0f) {
     acc.add(SM_RESD, wh * w_d * rd * rd);
     acc.add(SM_NTD, 1.0f);
@@ -527,10 +655,8 @@ __device__ inline void sim3_finish(const float4& p, float pvar, float2 rg, const
   // calcSim3LGS: LGS6 over (v, w) and LGS4 over (v3, w1, w2, sigma), merged
   // into the 7x7 upper triangle at rows / columns {2, 3, 4, 6}.
   float jv[6];
-  jac6<PREC>(Wx, Wy, Wz, gx, gy, jv);
-  float z = frcp<PREC>(Wz);
-  float z_sqr = frcp<PREC>(Wz * Wz);
-  float v4[4] = {z_sqr, z_sqr * Wy, -z_sqr * Wx, z};
+  jac6(Wx, Wy, q.z, q.z_sqr, gx, gy, jv);
+  float v4[4] = {q.z_sqr, q.z_sqr * Wy, -q.z_sqr * Wx, q.z};
 #pragma unroll
   for (int a = 0; a < 6; ++a)
 #pragma unroll
@@ -596,34 +722,32 @@ __device__ inline void sim3_points(const PointsLevel& pts, int i, int stride, in
 template <int PREC, class ACC>
 __device__ inline void adjoint_point(const PointsLevel& pts, int i, const void* __restrict__ img, const LevelGeom& g,
                                      const Xf& x, const TrackKParams& kp, float* __restrict__ grad_d, ACC& acc) {
-  const float wlim = (float)(g.w - 2), hlim = (float)(g.h - 2);
-  float4 p = pts.posI[i];
-  float Wx = x.R[0] * p.x + x.R[1] * p.y + x.R[2] * p.z + x.t[0];
-  float Wy = x.R[3] * p.x + x.R[4] * p.y + x.R[5] * p.z + x.t[1];
-  float Wz = x.R[6] * p.x + x.R[7] * p.y + x.R[8] * p.z + x.t[2];
-  float u = (Wx / Wz) * g.fx + g.cx;
-  float v = (Wy / Wz) * g.fy + g.cy;
-  if (!(u > 1.0f && v > 1.0f && u < wlim && v < hlim)) {
+  // correctly rounded divisions at every storage precision
+  const float4 p = pts.posI[i];
+  const float pvar = pts.var[i];
+  const Proj w = project<LSDG_FP32>(p, x, g);
+  if (!w.in) {
     grad_d[i] = 0.0f;
     return;
   }
-  Taps ri = interp3<PREC>(img, u, v, g.w);
+  Taps ri = interp3<PREC>(img, w.u, w.v, g.w);
   float r = p.w - ri.I;
   float gx = g.fx * ri.gx, gy = g.fy * ri.gy;
-  float d = 1.0f / p.z;
-  float s = kp.var_weight * pts.var[i];
-  float g0 = (x.t[0] * Wz - x.t[2] * Wx) / (Wz * Wz * d);
-  float g1 = (x.t[1] * Wz - x.t[2] * Wy) / (Wz * Wz * d);
-  float drpdd = gx * g0 + gy * g1;
-  float w_p = 1.0f / (kp.noise2 + s * drpdd * drpdd);
-  float e = fabsf(r * sqrtf(w_p));
+  const PointGeom q = point_geom<LSDG_FP32, false>(p.z, w, x);
+  float s = kp.var_weight * pvar;
+  float drpdd = gx * q.g0 + gy * q.g1;
+  float w_p, sq_p;
+  weight_of<LSDG_FP32>(kp.noise2 + s * drpdd * drpdd, w_p, sq_p);
+  float e = fabsf(r * sq_p);
   float k = kp.huber;
-  float wh = e < k ? 1.0f : k / e;
+  float wh = huber_weight<LSDG_FP32>(e, k);
+  if (k < 0.0f) wh = -wh;  // the plain quotient k / e keeps the sign of k
   acc.add(6, e < k ? 0.5f * e * e : k * e - 0.5f * k * k);
   acc.add(7, 1.0f);
   float Wr = wh * w_p * r;
   float jv[6];
-  jac6<PREC>(Wx, Wy, Wz, gx, gy, jv);
+  if constexpr (PREC == LSDG_FP32) jac6(w.Wx, w.Wy, q.z, q.z_sqr, gx, gy, jv);
+  else jac6(w.Wx, w.Wy, frcp<PREC>(w.Wz), frcp<PREC>(w.Wz * w.Wz), gx, gy, jv);
 #pragma unroll
   for (int a = 0; a < 6; ++a) acc.add(a, -(Wr * jv[a]));
   grad_d[i] = -Wr * drpdd;
@@ -645,59 +769,55 @@ __device__ inline void adjoint_point_sim3(const PointsLevel& pts, int i, const v
                                           const LevelGeom& g, const Xf& x, const TrackKParams& kp,
                                           float* __restrict__ grad_d, ACC& acc) {
   const float4 p = pts.posI[i];
+  const float pvar = pts.var[i];
   const Proj w = project<PREC>(p, x, g);
   if (!w.in) {
     grad_d[i] = 0.0f;
     return;
   }
-  const float Wx = w.Wx, Wy = w.Wy, Wz = w.Wz;
+  const float Wx = w.Wx, Wy = w.Wy;
   Taps ri = interp3<PREC>(img, w.u, w.v, g.w);
   const int ir = (int)(w.u + 0.5f) + g.w * (int)(w.v + 0.5f);
   const float varF = fvar[ir], fidR = fid[ir];
   float gx = g.fx * ri.gx, gy = g.fy * ri.gy;
   float rp = (kp.aff_a * p.w + kp.aff_b) - ri.I;
-  float refId = frcp<PREC>(Wz);
-  float d = frcp<PREC>(p.z);
+  const PointGeom q = point_geom<PREC, true>(p.z, w, x);
   float rd, vard;
   if (varF > 0.0f) {
-    rd = refId - fidR;
+    rd = q.z - fidR;
     vard = varF;
   } else {
     rd = -1.0f;
     vard = -1.0f;
   }
-  float s = kp.var_weight * pts.var[i];
+  float s = kp.var_weight * pvar;
   float sv = kp.var_weight * vard;
-  float g0 = fdiv<PREC>(x.t[0] * Wz - x.t[2] * Wx, Wz * Wz * d);
-  float g1 = fdiv<PREC>(x.t[1] * Wz - x.t[2] * Wy, Wz * Wz * d);
-  float g2 = fdiv<PREC>(Wz - x.t[2], Wz * Wz * d);
-  float drpdd = gx * g0 + gy * g1;
-  float w_p = frcp<PREC>(kp.noise2 + s * drpdd * drpdd);
-  float w_d = frcp<PREC>(sv + g2 * g2 * s);
-  float wrd = fabsf(rd * fsqrt<PREC>(w_d));
-  float wrp = fabsf(rp * fsqrt<PREC>(w_p));
+  float drpdd = gx * q.g0 + gy * q.g1;
+  float w_p, w_d, sq_p, sq_d;
+  weight_of<PREC>(kp.noise2 + s * drpdd * drpdd, w_p, sq_p);
+  weight_of<PREC>(sv + q.g2 * q.g2 * s, w_d, sq_d);
+  float wrd = fabsf(rd * sq_d);
+  float wrp = fabsf(rp * sq_p);
   float wabs = sv > 0.0f ? wrd + wrp : wrp;
-  float wh = fabsf(wabs < kp.huber ? 1.0f : fdiv<PREC>(kp.huber, wabs));
+  float wh = huber_weight<PREC>(wabs, kp.huber);
   float wp = wh * w_p;
   float wd = sv > 0.0f ? wh * w_d : 0.0f;
   acc.add(AS_EP, wp * rp * rp);
   if (sv > 0.0f) acc.add(AS_ED, wh * w_d * rd * rd);
   acc.add(AS_COUNT, 1.0f);
   float jv[6];
-  jac6<PREC>(Wx, Wy, Wz, gx, gy, jv);
+  jac6(Wx, Wy, q.z, q.z_sqr, gx, gy, jv);
   float rpW = rp * wp;
 #pragma unroll
   for (int a = 0; a < 6; ++a) acc.add(AS_G + a, -(jv[a] * rpW));
   float gd = -rpW * drpdd;
   if (wd != 0.0f) {
-    float z = frcp<PREC>(Wz);
-    float z_sqr = frcp<PREC>(Wz * Wz);
-    float v4[4] = {z_sqr, z_sqr * Wy, -z_sqr * Wx, z};
+    float v4[4] = {q.z_sqr, q.z_sqr * Wy, -q.z_sqr * Wx, q.z};
     const int remap[4] = {2, 3, 4, 6};
     float rdW = rd * wd;
 #pragma unroll
     for (int a = 0; a < 4; ++a) acc.add(AS_G + remap[a], -(v4[a] * rdW));
-    gd = gd + rdW * g2;
+    gd = gd + rdW * q.g2;
   }
   grad_d[i] = gd;
 }
