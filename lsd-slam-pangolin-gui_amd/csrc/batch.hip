@@ -20,7 +20,7 @@
 // and exp(d) * T, and writes the pose the job's next evaluation uses.  The
 // kernel boundary between the two orders the partial sums, so no block waits
 // on or fences for another.  A hipGraph replays K such steps.
-#include "batch_internal.h"
+#include "lm_device.h"
 #include "track_device.h"
 
 namespace lsdg {
@@ -32,319 +32,6 @@ constexpr int BATCH_WAVES = BATCH_BS / 64;
 #endif
 constexpr int BATCH_U = LSDG_BATCH_U;  // points per thread with loads in flight together
 constexpr int BATCH_SOLVE_BS = 256;
-
-// f^n by repeated multiplication (exact for the default factor 2).
-__host__ __device__ inline float pow_int(float f, int n) {
-  float r = 1.0f;
-  for (int i = 0; i < n; ++i) r *= f;
-  return r;
-}
-
-// ------------------------------------------------------------ LM steps
-__device__ inline void set_eval_pose(JobState& s, const Pose& T, bool sim3) {
-  pose_rt_f(T, sim3, s.xf.R, s.xf.t);
-  if (sim3) pose_roll_f(T, s.roll);
-}
-
-// The LM step runs on the 64 lanes of the block's first wave: its scalar
-// control flow is uniform over the wave (every lane computes the same values
-// from the same LDS state and writes the same values back), and the
-// independent divisions and trigonometric calls of the solve are spread over
-// the lanes.  `sc` is LM_SCRATCH doubles of LDS.
-constexpr int LM_SCRATCH = 64;
-
-__device__ inline int lm_lane() { return (int)(threadIdx.x & 63); }
-
-// Orders the wave's LDS writes before its later LDS reads.
-__device__ inline void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// remaining may be null: blocks that repeat another block's LM step (the
-// cooperative kernel) leave the count to that block.
-__device__ inline void finish_job(JobState& s, int status, int* ntNext, int* remaining) {
-  s.status = status;
-  *ntNext = 0;
-  if (remaining && lm_lane() == 0) atomicSub(remaining, 1);
-}
-
-// se3_exp (lsdg_lie.h) with sin and cos of theta / 2 (lane 0) and theta
-// (lane 1) evaluated at once, one sincos per lane.
-__device__ inline Pose se3_exp_wave(const double* __restrict__ xi, double* __restrict__ sc) {
-  const double* w = xi + 3;
-  const double th2 = w[0] * w[0] + w[1] * w[1] + w[2] * w[2];
-  const double th = sqrt(th2);
-  if (th >= 1e-10) {
-    const int lane = lm_lane();
-    if (lane < 2) {
-      double sv, cv;
-      sincos(lane == 0 ? 0.5 * th : th, &sv, &cv);
-      sc[lane] = sv;
-      sc[2 + lane] = cv;
-    }
-    wave_sync();
-  }
-  Pose r;
-  double k, c;
-  if (th < 1e-10) {
-    k = 0.5 - th2 / 48.0;
-    c = 1.0 - th2 / 8.0;
-  } else {
-    k = sc[0] / th;
-    c = sc[2];
-  }
-  r.q[0] = k * w[0]; r.q[1] = k * w[1]; r.q[2] = k * w[2]; r.q[3] = c;
-  quat_normalize(r.q);
-  double bb, cc;
-  if (th < 1e-5) {
-    bb = 0.5 - th2 / 24.0;
-    cc = 1.0 / 6.0 - th2 / 120.0;
-  } else {
-    bb = (1.0 - sc[3]) / th2;
-    cc = (th - sc[1]) / (th2 * th);
-  }
-  apply_abc(1.0, bb, cc, w, xi, r.t);
-  r.s = 1.0;
-  return r;
-}
-
-// Solve (A diag*(1+lambda)) inc = b from the stored LGS and propose Tn = exp(inc) T.
-// Returns false when a Sim3 step diverges (|inc|^2 not in [0, 1)).
-template <int KIND>
-__device__ inline bool solve_and_propose(JobState& __restrict__ s, double* __restrict__ sc) {
-  constexpr int N = KIND == LSDG_JOB_SIM3 ? 7 : 6;
-  constexpr int NA = N * (N + 1) / 2;
-  double A[N * N], b[N], inc[N];
-  const double n = s.lgsN;
-  // the normalisation's NA + N divisions, one per lane
-  {
-    const int lane = lm_lane();
-    if (lane < NA) sc[lane] = s.lgsA[lane] / n;
-    else if (lane < NA + N) sc[lane] = -s.lgsB[lane - NA] / n;
-    wave_sync();
-  }
-  int k = 0;
-  for (int a = 0; a < N; ++a)
-    for (int c = a; c < N; ++c) {
-      double v = sc[k++];
-      A[N * a + c] = v;
-      A[N * c + a] = v;
-    }
-  for (int a = 0; a < N; ++a) b[a] = sc[NA + a];
-  wave_sync();
-  for (int a = 0; a < N; ++a) A[(N + 1) * a] *= 1.0 + (double)s.lambda;
-  ldlt_solve<N>(A, b, inc);
-  s.incTry++;
-  double dd = 0;
-  for (int a = 0; a < N; ++a) {
-    s.inc[a] = inc[a];
-    dd += inc[a] * inc[a];
-  }
-  s.incSq = dd;
-  if (KIND == LSDG_JOB_SIM3) {
-    if (!(dd >= 0 && dd < 1)) return false;
-    s.Tn = pose_mul(sim3_exp(inc), s.T);
-  } else {
-    s.Tn = pose_mul(se3_exp_wave(inc, sc), s.T);
-  }
-  s.phase = 1;
-  set_eval_pose(s, s.Tn, KIND == LSDG_JOB_SIM3);
-  return true;
-}
-
-// Keeps the evaluation's unnormalised LGS (SE3: 6x6 upper triangle from the
-// 7-stride sums; Sim3: 7x7) as the accepted pose's normal equations.
-template <int KIND>
-__device__ inline void store_lgs(JobState& __restrict__ s, const double* __restrict__ S) {
-  if (KIND == LSDG_JOB_SIM3) {
-    for (int k = 0; k < 28; ++k) s.lgsA[k] = S[SM_A + k];
-    for (int a = 0; a < 7; ++a) s.lgsB[a] = S[SM_B + a];
-    s.lgsN = 2.0 * S[SM_WARPED];
-  } else {
-    for (int k = 0; k < 21; ++k) s.lgsA[k] = S[S3_A + k];
-    for (int a = 0; a < 6; ++a) s.lgsB[a] = S[S3_B + a];
-    s.lgsN = S[S3_WARPED];
-  }
-}
-
-template <int KIND>
-__device__ inline void begin_level(JobState& s, const JobDesc& jd, const lsdg_params& P, int lvl, int* ntNext,
-                                   int* remaining) {
-  if (KIND == LSDG_JOB_SIM3) {
-    while (lvl >= jd.finalLevel && P.max_its_per_lvl[lvl] == 0) lvl--;
-  }
-  if (lvl < jd.finalLevel) {
-    if (KIND == LSDG_JOB_SIM3 && !s.upToDate) {
-      // a final evaluation at the accepted pose for the information matrix
-      s.level = jd.finalLevel;
-      s.phase = 2;
-      set_eval_pose(s, s.T, true);
-      *ntNext = jd.lv[s.level].ntiles;
-      return;
-    }
-    if (KIND == LSDG_JOB_SIM3 && s.T.s <= 0) {
-      finish_job(s, 2, ntNext, remaining);
-      return;
-    }
-    finish_job(s, 1, ntNext, remaining);
-    return;
-  }
-  s.level = lvl;
-  s.phase = 0;
-  set_eval_pose(s, s.T, KIND == LSDG_JOB_SIM3);
-  *ntNext = jd.lv[lvl].ntiles;
-}
-
-// One LM step of an SE3 job, after the evaluation whose sums are S.
-__device__ void lm_step_se3(JobState& __restrict__ s, const JobDesc& __restrict__ jd, const double* __restrict__ S,
-                            const lsdg_params& P, int* ntNext, int* remaining, double* __restrict__ sc) {
-  const int lvl = s.level;
-  const JobLevel& L = jd.lv[lvl];
-  s.evals++;
-  s.evalsAt[lvl]++;
-  s.good = S[S3_GOOD];
-  s.bad = S[S3_BAD];
-  s.meanRes = S[S3_SIGNED] / S[S3_GOOD];
-  s.usage = S[S3_USAGE] / (double)L.pts.n;
-  // the affine iterate is read only when the affine brightness is estimated
-  if (P.use_affine_lightning_estimation) {
-    const double sxx = S[S3_SXX], syy = S[S3_SYY], sx = S[S3_SX], sy = S[S3_SY], sw = S[S3_SW];
-    s.affAIt = (float)sqrt((syy - sy * sy / sw) / (sxx - sx * sx / sw));
-    s.affBIt = (float)((sy - (double)s.affAIt * sx) / sw);
-  }
-  const float lim = P.min_goodperall_pixel_absmin * (float)(L.g.w * L.g.h);
-  if ((float)S[S3_WARPED] < lim) {
-    finish_job(s, 2, ntNext, remaining);
-    return;
-  }
-  const double err = S[S3_ERR] / S[S3_WARPED];
-  s.numRes[lvl]++;
-  if (s.phase == 0) {
-    if (P.use_affine_lightning_estimation) { s.affA = s.affAIt; s.affB = s.affBIt; }
-    s.lastErr = err;
-    s.lambda = P.lambda_initial[lvl];
-    s.iteration = 0;
-    if (P.max_its_per_lvl[lvl] <= 0) {
-      begin_level<LSDG_JOB_SE3>(s, jd, P, lvl - 1, ntNext, remaining);
-      return;
-    }
-    store_lgs<LSDG_JOB_SE3>(s, S);
-    s.numWarp[lvl]++;
-    s.incTry = 0;
-    solve_and_propose<LSDG_JOB_SE3>(s, sc);
-    *ntNext = L.ntiles;
-    return;
-  }
-  if (err < s.lastErr) {
-    s.T = s.Tn;
-    if (P.use_affine_lightning_estimation) { s.affA = s.affAIt; s.affB = s.affBIt; }
-    bool conv = err / s.lastErr > (double)P.convergence_eps[lvl];
-    s.lastResidual = s.lastErr = err;
-    s.lambda = s.lambda <= 0.2f ? 0.0f : s.lambda * P.lambda_success_fac[lvl];
-    s.iteration++;
-    if (conv || s.iteration >= P.max_its_per_lvl[lvl]) {
-      begin_level<LSDG_JOB_SE3>(s, jd, P, lvl - 1, ntNext, remaining);
-      return;
-    }
-    store_lgs<LSDG_JOB_SE3>(s, S);
-    s.numWarp[lvl]++;
-    s.incTry = 0;
-    solve_and_propose<LSDG_JOB_SE3>(s, sc);
-    *ntNext = L.ntiles;
-    return;
-  }
-  if (!(s.incSq > (double)P.step_size_min[lvl])) {
-    begin_level<LSDG_JOB_SE3>(s, jd, P, lvl - 1, ntNext, remaining);
-    return;
-  }
-  s.lambda = s.lambda == 0.0f ? 0.2f : s.lambda * pow_int(P.lambda_fail_fac[lvl], s.incTry);
-  solve_and_propose<LSDG_JOB_SE3>(s, sc);
-  *ntNext = L.ntiles;
-}
-
-__device__ inline void sim3_res(const double* S, double* r) {
-  // r = {sumResD, sumResP, numTermsD, numTermsP, meanD, meanP, mean}
-  r[0] = S[SM_RESD];
-  r[1] = S[SM_RESP];
-  r[2] = S[SM_NTD];
-  r[3] = S[SM_WARPED];
-  r[6] = (S[SM_RESD] + S[SM_RESP]) / (S[SM_NTD] + S[SM_WARPED]);
-  r[4] = S[SM_RESD] / S[SM_NTD];
-  r[5] = S[SM_RESP] / S[SM_WARPED];
-}
-
-// One LM step of a Sim3 job.
-__device__ void lm_step_sim3(JobState& __restrict__ s, const JobDesc& __restrict__ jd, const double* __restrict__ S,
-                             const lsdg_params& P, int* ntNext, int* remaining, double* __restrict__ sc) {
-  const int lvl = s.level;
-  const JobLevel& L = jd.lv[lvl];
-  s.evals++;
-  s.evalsAt[lvl]++;
-  s.usage = S[SM_USAGE] / (double)L.pts.n;
-  if (s.phase == 2) {
-    // final evaluation for lastSim3Hessian
-    sim3_res(S, s.finalRes);
-    store_lgs<LSDG_JOB_SIM3>(s, S);
-    s.upToDate = 1;
-    finish_job(s, s.T.s <= 0 ? 2 : 1, ntNext, remaining);
-    return;
-  }
-  const float lim = 0.5f * P.min_goodperall_pixel_absmin * (float)(L.g.w * L.g.h);
-  if ((float)S[SM_WARPED] < lim || S[SM_WARPED] < 10) {
-    finish_job(s, 2, ntNext, remaining);
-    return;
-  }
-  double res[7];
-  sim3_res(S, res);
-  s.numRes[lvl]++;
-  if (s.phase == 0) {
-    for (int k = 0; k < 7; ++k) s.lastRes[k] = res[k];
-    s.lambda = P.lambda_initial[lvl];
-    s.upToDate = 0;
-    s.iteration = 0;
-    store_lgs<LSDG_JOB_SIM3>(s, S);
-    s.upToDate = 1;
-    s.numWarp[lvl]++;
-    s.incTry = 0;
-    if (!solve_and_propose<LSDG_JOB_SIM3>(s, sc)) {
-      for (int k = 0; k < 28; ++k) s.lgsA[k] = 0.0;
-      finish_job(s, 2, ntNext, remaining);
-      return;
-    }
-    *ntNext = L.ntiles;
-    return;
-  }
-  if (res[6] < s.lastRes[6]) {
-    s.T = s.Tn;
-    s.upToDate = 0;
-    bool conv = res[6] / s.lastRes[6] > (double)P.convergence_eps[lvl];
-    for (int k = 0; k < 7; ++k) s.finalRes[k] = s.lastRes[k] = res[k];
-    s.lambda = s.lambda <= 0.2f ? 0.0f : s.lambda * P.lambda_success_fac[lvl];
-    s.iteration++;
-    if (conv || s.iteration >= P.max_its_per_lvl[lvl]) {
-      begin_level<LSDG_JOB_SIM3>(s, jd, P, lvl - 1, ntNext, remaining);
-      return;
-    }
-    store_lgs<LSDG_JOB_SIM3>(s, S);
-    s.upToDate = 1;
-    s.numWarp[lvl]++;
-    s.incTry = 0;
-  } else {
-    if (!(s.incSq > (double)P.step_size_min[lvl])) {
-      begin_level<LSDG_JOB_SIM3>(s, jd, P, lvl - 1, ntNext, remaining);
-      return;
-    }
-    s.lambda = s.lambda == 0.0f ? 0.2f : s.lambda * pow_int(P.lambda_fail_fac[lvl], s.incTry);
-  }
-  if (!solve_and_propose<LSDG_JOB_SIM3>(s, sc)) {
-    for (int k = 0; k < 28; ++k) s.lgsA[k] = 0.0;
-    finish_job(s, 2, ntNext, remaining);
-    return;
-  }
-  *ntNext = L.ntiles;
-}
 
 // ------------------------------------------------------------- kernels
 // Start state of every job: T = (frameToRef_init)^-1, first level, counters
@@ -366,15 +53,9 @@ __global__ __launch_bounds__(256) void k_batch_init(BatchArgs a) {
   if (clearRows && a.coopRows)
     for (size_t i = threadIdx.x; i < a.coopWords; i += blockDim.x) a.coopRows[i] = 0ull;
   for (int j = threadIdx.x; j < a.njobs; j += blockDim.x) {
-    const JobDesc& jd = a.jobs[j];
-    JobState s = {};
-    s.T = pose_inv(jd.init);
-    if (jd.kind == LSDG_JOB_SE3) s.T.s = 1.0;
-    s.affA = 1.0f;
-    s.affB = 0.0f;
-    int nt = 0, dummy = 0;
-    if (jd.kind == LSDG_JOB_SIM3) begin_level<LSDG_JOB_SIM3>(s, jd, a.P, jd.startLevel, &nt, &dummy);
-    else begin_level<LSDG_JOB_SE3>(s, jd, a.P, jd.startLevel, &nt, &dummy);
+    JobState s;
+    int nt = 0;
+    lm_begin(s, a.jobs[j], a.P, &nt, nullptr);
     a.st[j] = s;
     a.ntiles[j] = nt;  // parity 0
     a.ntiles[a.njobs + j] = 0;
@@ -458,16 +139,6 @@ __global__ __launch_bounds__(BATCH_BS) void k_batch_eval(BatchArgs a, int parity
   }
 }
 
-// Copies a trivially copyable object between global memory and LDS with the
-// whole block (32-bit words).
-template <class T>
-__device__ inline void block_copy(T* dst, const T* src, int nthreads) {
-  static_assert(sizeof(T) % 4 == 0, "copied as 32-bit words");
-  const uint32_t* s = reinterpret_cast<const uint32_t*>(src);
-  uint32_t* d = reinterpret_cast<uint32_t*>(dst);
-  for (int w = threadIdx.x; w < (int)(sizeof(T) / 4); w += nthreads) d[w] = s[w];
-}
-
 // Merge and LM step of one LM iteration: one block per job.  Wave w sums the
 // job's tile rows w, w + 4, ... (row order within a wave), the four wave sums
 // are added in wave order, and lane 0 runs the LM step on the job's
@@ -483,7 +154,6 @@ __global__ __launch_bounds__(BATCH_SOLVE_BS) void k_batch_solve(BatchArgs a, int
   __shared__ JobState sst;
   __shared__ JobDesc sjd;
   __shared__ int next;
-  __shared__ double lmsc[LM_SCRATCH];
   const int j = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int nj = a.njobs;
   const int n = a.ntiles[parity * nj + j];
@@ -518,8 +188,8 @@ __global__ __launch_bounds__(BATCH_SOLVE_BS) void k_batch_solve(BatchArgs a, int
   __syncthreads();
   if (tid < 64) {
     int nx = 0;
-    if (KIND == LSDG_JOB_SIM3) lm_step_sim3(sst, sjd, S, a.P, &nx, a.remaining, lmsc);
-    else lm_step_se3(sst, sjd, S, a.P, &nx, a.remaining, lmsc);
+    if (KIND == LSDG_JOB_SIM3) lm_step_sim3(sst, sjd, S, a.P, &nx, a.remaining);
+    else lm_step_se3(sst, sjd, S, a.P, &nx, a.remaining);
     if (tid == 0) next = nx;
   }
   __syncthreads();
@@ -544,7 +214,6 @@ __global__ __launch_bounds__(BATCH_JOB_BS) void k_batch_job(BatchArgs a) {
   __shared__ JobDesc jd;
   __shared__ double sh[WAVES][NS];
   __shared__ double S[NS];
-  __shared__ double lmsc[LM_SCRATCH];
   const int j = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   block_copy(&s, a.st + j, BATCH_JOB_BS);
   block_copy(&jd, a.jobs + j, BATCH_JOB_BS);
@@ -576,8 +245,8 @@ __global__ __launch_bounds__(BATCH_JOB_BS) void k_batch_job(BatchArgs a) {
     __syncthreads();
     if (tid < 64) {
       int next = 0;
-      if (KIND == LSDG_JOB_SIM3) lm_step_sim3(s, jd, S, a.P, &next, a.remaining, lmsc);
-      else lm_step_se3(s, jd, S, a.P, &next, a.remaining, lmsc);
+      if (KIND == LSDG_JOB_SIM3) lm_step_sim3(s, jd, S, a.P, &next, a.remaining);
+      else lm_step_se3(s, jd, S, a.P, &next, a.remaining);
     }
     __syncthreads();
   }
@@ -613,7 +282,6 @@ __global__ __launch_bounds__(COOP_BS) void k_batch_coop(BatchArgs a) {
   __shared__ JobDesc jd;
   __shared__ double sh[WAVES][NS];
   __shared__ double S[NS];
-  __shared__ double lmsc[LM_SCRATCH];
   __shared__ int arrived;
   const int K = a.coopK;
   // Blocks are dispatched round-robin over the device's XCDs.  With
@@ -720,8 +388,8 @@ __global__ __launch_bounds__(COOP_BS) void k_batch_coop(BatchArgs a) {
     __syncthreads();
     if (tid < 64) {
       int next = 0;
-      if (KIND == LSDG_JOB_SIM3) lm_step_sim3(s, jd, S, a.P, &next, remaining, lmsc);
-      else lm_step_se3(s, jd, S, a.P, &next, remaining, lmsc);
+      if (KIND == LSDG_JOB_SIM3) lm_step_sim3(s, jd, S, a.P, &next, remaining);
+      else lm_step_se3(s, jd, S, a.P, &next, remaining);
     }
     __syncthreads();
   }

@@ -41,14 +41,14 @@ struct JobState {
   Pose T, Tn;        // accepted referenceToFrame, trial
   Xf xf;             // pose of the next evaluation, FP32
   float roll[4];     // its ESM roll (Sim3)
-  double inc[7];
   double incSq;
-  double lgsA[28], lgsB[7], lgsN;  // unnormalised LGS of the accepted pose
+  double lgsA[28], lgsB[7];        // unnormalised LGS of the accepted pose
   double lastErr, lastResidual;    // SE3
-  double lastRes[7], finalRes[7];  // Sim3 (sumResD, sumResP, numTermsD, numTermsP, meanD, meanP, mean)
-  double good, bad, meanRes, usage;
+  double lastRes[7], finalRes[7];  // Sim3 (sumResD, sumResP, numTermsD, numTermsP, set, 0, mean)
+  double good, bad, signedRes, usageSum;  // sums of the last evaluation, over usageN points
+  int usageN;
   float lambda, affA, affB, affAIt, affBIt;
-  int status;        // 0 running, 1 done, 2 diverged
+  int status;        // 0 running, 1 done, 2 diverged, 3 done with a scale <= 0 (Sim3: diverged)
   int level, phase, iteration, incTry, upToDate, evals;
   int numRes[PYR], numWarp[PYR];
   int evalsAt[PYR];  // evaluations run per level (every step the job was active)
@@ -76,6 +76,11 @@ struct BatchArgs {
   lsdg_params P;
   TrackKParams kp;
 };
+
+// Result fields both paths derive from a finished control block.
+inline double job_usage(const JobState& s) { return s.evals ? s.usageSum / (double)s.usageN : 0.0; }
+inline double job_mean_d(const JobState& s) { return s.finalRes[4] != 0.0 ? s.finalRes[0] / s.finalRes[2] : 0.0; }
+inline double job_mean_p(const JobState& s) { return s.finalRes[4] != 0.0 ? s.finalRes[1] / s.finalRes[3] : 0.0; }
 
 hipError_t launch_batch_init(const BatchArgs& a, hipStream_t s);
 // Cooperative whole-LM kernel (a.coopK blocks of `bs` threads per job, all

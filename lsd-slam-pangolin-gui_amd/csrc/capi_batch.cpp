@@ -497,11 +497,12 @@ static void fill_result(lsdg_batch b, int j, const JobState& s, lsdg_job_result*
     st.num_residual_calls[l] = s.numRes[l];
     st.num_warp_update_calls[l] = s.numWarp[l];
   }
-  st.point_usage = (float)s.usage;
+  const double usage = job_usage(s);
+  st.point_usage = (float)usage;
   st.affine_a = s.affA;
   st.affine_b = s.affB;
   Pose I = pose_identity();
-  if (s.status == 2) {
+  if (s.status >= 2) {
     st.diverged = 1;
     st.tracking_was_good = 0;
     st.last_good_count = (int)s.good;
@@ -516,7 +517,7 @@ static void fill_result(lsdg_batch b, int j, const JobState& s, lsdg_job_result*
     res.s = 1.0;
     st.last_good_count = (int)s.good;
     st.last_bad_count = (int)s.bad;
-    st.last_mean_res = (float)s.meanRes;
+    st.last_mean_res = (float)(s.signedRes / s.good);
     st.last_residual = (float)s.lastResidual;
     lsdg_frame f = J.frame;
     const int ml = b->ctx->P.se3_min_level;
@@ -525,14 +526,14 @@ static void fill_result(lsdg_batch b, int j, const JobState& s, lsdg_job_result*
     st.tracking_was_good = good ? 1 : 0;
     // the frame fields SE3Tracker::trackFrame writes
     if (good) J.ref->kf->numFramesTrackedOnThis++;
-    f->initialTrackedResidual = (float)(s.lastResidual / s.usage);
+    f->initialTrackedResidual = (float)(s.lastResidual / usage);
     f->thisToParent = res;
     f->parent = J.ref->kf;
     f->parentId = J.ref->kf->id;
   } else {
     st.last_residual = (float)s.finalRes[6];
-    st.last_depth_residual = (float)s.finalRes[4];
-    st.last_photometric_residual = (float)s.finalRes[5];
+    st.last_depth_residual = (float)job_mean_d(s);
+    st.last_photometric_residual = (float)job_mean_p(s);
     st.tracking_was_good = 1;
     int k = 0;
     for (int a = 0; a < 7; ++a)
