@@ -82,6 +82,27 @@ inline double job_usage(const JobState& s) { return s.evals ? s.usageSum / (doub
 inline double job_mean_d(const JobState& s) { return s.finalRes[4] != 0.0 ? s.finalRes[0] / s.finalRes[2] : 0.0; }
 inline double job_mean_p(const JobState& s) { return s.finalRes[4] != 0.0 ? s.finalRes[1] / s.finalRes[3] : 0.0; }
 
+// track_lm.hip: one alignment's whole LM loop in one launch, blocks
+// cooperating as in k_batch_coop.
+struct TrackLmArgs {
+  JobDesc jd;
+  lsdg_params P;
+  TrackKParams kp;
+  unsigned long long* rows;  // [2][blocks][NS][2] tagged words
+  JobState* out;             // the finished control block (host-mapped); status < 0: the blocks gave up
+  unsigned epochTag;         // tag of this launch in the upper 16 bits, never 0
+  int blocks;                // blocks of the launch
+  unsigned spinMax;          // polls of a wait before the blocks give up
+};
+constexpr unsigned TRACK_LM_SPIN_MAX = 1u << 14;  // polls of about a microsecond
+constexpr int TRACK_LM_MAX_BLOCKS = 64;
+constexpr size_t TRACK_LM_WORDS = (size_t)2 * TRACK_LM_MAX_BLOCKS * NS_MAX * 2;
+// Blocks of a launch for alignments whose largest level holds n points.
+int track_lm_blocks(lsdg_ctx c, int n);
+hipError_t launch_track_lm(const TrackLmArgs& a, int prec, int acc, hipStream_t s, const KTimer* t = nullptr);
+// Zeroes n tagged words (a fill kernel).
+hipError_t launch_track_lm_clear(unsigned long long* rows, size_t n, hipStream_t s);
+
 hipError_t launch_batch_init(const BatchArgs& a, hipStream_t s);
 // Cooperative whole-LM kernel (a.coopK blocks of `bs` threads per job, all
 // levels; bs is 256 or 512) and the number of its blocks the device holds at

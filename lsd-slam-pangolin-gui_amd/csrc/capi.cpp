@@ -5,11 +5,14 @@
 // and the 6x6 / 7x7 systems are solved in FP64 on the host.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <new>
 
+#include "batch_internal.h"
 #include "capi_common.h"
 
 using namespace lsdg;
@@ -123,10 +126,17 @@ extern "C" lsdg_status lsdg_ctx_create(int32_t device, const lsdg_params* params
       hipMalloc(&c->d_counter, 64) != hipSuccess || hipMemset(c->d_counter, 0, 64) != hipSuccess ||
       hipHostMalloc(&c->h_result, sizeof(double) * 64, hipHostMallocMapped) != hipSuccess ||
       hipHostGetDevicePointer((void**)&c->d_result, c->h_result, 0) != hipSuccess ||
+      hipMalloc(&c->d_track_rows, sizeof(unsigned long long) * TRACK_LM_WORDS) != hipSuccess ||
+      hipHostMalloc(&c->h_track, sizeof(JobState), hipHostMallocMapped) != hipSuccess ||
+      hipHostGetDevicePointer(&c->d_track, c->h_track, 0) != hipSuccess ||
       noalloc_scratch_init(device) != hipSuccess) {  // the allocation-free entry point's device array
     lsdg_ctx_destroy(c);
     return LSDG_EDEVICE;
   }
+  // polls of a one-launch alignment's waits before its blocks give up; a small
+  // value makes the launch-per-evaluation path run on purpose
+  c->track_spin_max = TRACK_LM_SPIN_MAX;
+  if (const char* e = std::getenv("LSDG_TRACK_SPIN_MAX")) c->track_spin_max = (unsigned)std::max(0, std::atoi(e));
   *out = c;
   return LSDG_OK;
 }
@@ -138,6 +148,8 @@ extern "C" lsdg_status lsdg_ctx_destroy(lsdg_ctx c) {
   if (c->d_partials) (void)hipFree(c->d_partials);
   if (c->d_counter) (void)hipFree(c->d_counter);
   if (c->h_result) (void)hipHostFree(c->h_result);
+  if (c->d_track_rows) (void)hipFree(c->d_track_rows);
+  if (c->h_track) (void)hipHostFree(c->h_track);
   if (c->d_export) (void)hipFree(c->d_export);
   if (c->d_adj) (void)hipFree(c->d_adj);
   if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -665,11 +677,82 @@ static void se3_pass_stats(const double* S, int N, Se3Out& o) {
   o.affBIt = (float)((sy - (double)o.affAIt * sx) / sw);
 }
 
-extern "C" lsdg_status lsdg_se3_track(lsdg_ctx c, lsdg_ref r, lsdg_frame f, const double init[7], double out[7],
-                                      lsdg_track_stats* stats) {
-  if (!c || !r || !f || !init || !out) return LSDG_EINVAL;
-  if (r->ctx != c || f->ctx != c) return fail(c, LSDG_EINVAL, "objects belong to another context");
-  if (f->w[0] != r->kf->w[0] || f->h[0] != r->kf->h[0]) return fail(c, LSDG_EINVAL, "frame / keyframe size mismatch");
+// ------------------------------------------------- one-launch alignments
+// Runs one alignment's LM loop in one launch (track_lm.hip).  *ran is false
+// when the blocks could not all run at once: nothing is written then, and the
+// caller takes the launch-per-evaluation path.
+static lsdg_status track_lm(lsdg_ctx c, lsdg_ref r, lsdg_frame f, int kind, const Pose& init, int startLevel,
+                            int finalLevel, uint8_t* mask, const JobState** out, bool* ran) {
+  TrackLmArgs a;
+  std::memset(&a, 0, sizeof a);
+  a.jd.kind = kind;
+  a.jd.startLevel = startLevel;
+  a.jd.finalLevel = finalLevel;
+  a.jd.init = init;
+  a.jd.isGood = mask;
+  int maxPoints = 0;
+  for (int l = finalLevel; l <= startLevel; ++l) {
+    lsdg_status st = ref_points(r, l);
+    if (st != LSDG_OK) return st;
+    JobLevel& L = a.jd.lv[l];
+    L.pts = r->lv[l];
+    L.img = f->precision == LSDG_FP32 ? (const void*)f->d_grad[l] : (const void*)f->d_gradh[l];
+    L.fid = f->d_idepth[l];
+    L.fvar = f->d_ivar[l];
+    L.g = LevelGeom{f->w[l], f->h[l], f->fx[l], f->fy[l], f->cx[l], f->cy[l]};
+    L.ntiles = 1;
+    maxPoints = std::max(maxPoints, L.pts.n);
+  }
+  lsdg_status st = frame_require(f, fd_track(f, finalLevel, startLevel));
+  if (st != LSDG_OK) return st;
+  a.P = c->P;
+  a.kp = track_kparams(c->P, kind == LSDG_JOB_SIM3);
+  a.kp.aff_stats = c->P.use_affine_lightning_estimation;
+  a.blocks = track_lm_blocks(c, maxPoints);
+  a.rows = c->d_track_rows;
+  a.spinMax = c->track_spin_max;
+  a.out = (JobState*)c->d_track;
+  // the launch's tag: never 0, and the rows are cleared whenever the counter
+  // wraps (and before the first launch), so no word of an earlier launch
+  // carries it
+  c->track_epoch = (c->track_epoch + 1) & 0xFFFFu;
+  if (c->track_epoch == 0) c->track_epoch = 1;
+  if (c->track_epoch == 1) CK(c, launch_track_lm_clear(c->d_track_rows, TRACK_LM_WORDS, c->stream));
+  a.epochTag = c->track_epoch << 16;
+  KTimer kt = prof_timer(c);
+  CK(c, launch_track_lm(a, f->precision, c->sums == LSDG_SUMS_KAHAN ? BATCH_ACC_KAHAN : BATCH_ACC_F64, c->stream, &kt));
+  CK(c, hipStreamSynchronize(c->stream));
+  const JobState* s = (const JobState*)c->h_track;
+  double bytes = 0.0;
+  for (int l = finalLevel; l <= startLevel; ++l)
+    bytes += s->evalsAt[l] * eval_bytes(a.jd.lv[l].pts.n, f, l, kind == LSDG_JOB_SIM3);
+  prof_timer_done(c, LSDG_KERNEL_EVAL, kt, bytes);
+  *out = s;
+  *ran = s->status >= 0;
+  return LSDG_OK;
+}
+
+// Fields both forms of the SE3 tracker write on success.
+static void se3_track_done(lsdg_ctx c, lsdg_ref r, lsdg_frame f, double good, double bad, double lastResidual,
+                           double usage, const Pose& T, lsdg_track_stats& st, double out[7]) {
+  st.last_residual = (float)lastResidual;
+  const int ml = c->P.se3_min_level;
+  const bool ok = good / (double)(f->w[ml] * f->h[ml]) > (double)c->P.min_goodperall_pixel &&
+                  good / (good + bad) > (double)c->P.min_goodpergoodbad_pixel;
+  st.tracking_was_good = ok ? 1 : 0;
+  if (ok) r->kf->numFramesTrackedOnThis++;
+  Pose res = pose_inv(T);
+  res.s = 1.0;
+  f->initialTrackedResidual = (float)(lastResidual / usage);
+  f->thisToParent = res;
+  f->parent = r->kf;
+  f->parentId = r->kf->id;
+  pose_to7(res, out);
+}
+
+// SE3Tracker::trackFrame with a launch and a host LM step per evaluation.
+static lsdg_status se3_track_steps(lsdg_ctx c, lsdg_ref r, lsdg_frame f, const double init[7], double out[7],
+                                   lsdg_track_stats* stats) {
   const lsdg_params& P = c->P;
   lsdg_track_stats st;
   std::memset(&st, 0, sizeof st);
@@ -759,22 +842,52 @@ extern "C" lsdg_status lsdg_se3_track(lsdg_ctx c, lsdg_ref r, lsdg_frame f, cons
     pose_to7(pose_identity(), out);
     return LSDG_DIVERGED;
   }
-  st.last_residual = (float)last_residual;
-  int ml = P.se3_min_level;
-  bool good = o.lastGoodCount / (double)(f->w[ml] * f->h[ml]) > (double)P.min_goodperall_pixel &&
-              o.lastGoodCount / (o.lastGoodCount + o.lastBadCount) > (double)P.min_goodpergoodbad_pixel;
-  st.tracking_was_good = good ? 1 : 0;
-  if (good) r->kf->numFramesTrackedOnThis++;
-  Pose res = pose_inv(T);
-  res.s = 1.0;
-  f->initialTrackedResidual = (float)(last_residual / o.pointUsage);
-  f->thisToParent = res;
-  f->parent = r->kf;
-  f->parentId = r->kf->id;
-  pose_to7(res, out);
+  se3_track_done(c, r, f, o.lastGoodCount, o.lastBadCount, last_residual, o.pointUsage, T, st, out);
   if (stats) *stats = st;
   return LSDG_OK;
 }
+
+extern "C" lsdg_status lsdg_se3_track(lsdg_ctx c, lsdg_ref r, lsdg_frame f, const double init[7], double out[7],
+                                      lsdg_track_stats* stats) {
+  if (!c || !r || !f || !init || !out) return LSDG_EINVAL;
+  if (r->ctx != c || f->ctx != c) return fail(c, LSDG_EINVAL, "objects belong to another context");
+  if (f->w[0] != r->kf->w[0] || f->h[0] != r->kf->h[0]) return fail(c, LSDG_EINVAL, "frame / keyframe size mismatch");
+  const lsdg_params& P = c->P;
+  uint8_t* mask = nullptr;
+  if (P.se3_min_level == 1) {  // refPixelWasGood is a level-1 mask
+    lsdg_status s0 = frame_ensure_was_good(f);
+    if (s0 != LSDG_OK) return s0;
+    mask = f->d_wasGood;
+  }
+  const JobState* s = nullptr;
+  bool ran = false;
+  lsdg_status s0 = track_lm(c, r, f, LSDG_JOB_SE3, pose_from7(init), P.se3_max_level - 1, P.se3_min_level, mask, &s, &ran);
+  if (s0 != LSDG_OK) return s0;
+  if (!ran) return se3_track_steps(c, r, f, init, out, stats);
+  lsdg_track_stats st;
+  std::memset(&st, 0, sizeof st);
+  for (int l = 0; l < PYR; ++l) {
+    st.num_residual_calls[l] = s->numRes[l];
+    st.num_warp_update_calls[l] = s->numWarp[l];
+  }
+  const double usage = job_usage(*s);
+  st.last_good_count = (int)s->good;
+  st.last_bad_count = (int)s->bad;
+  st.last_mean_res = (float)(s->signedRes / s->good);
+  st.point_usage = (float)usage;
+  st.affine_a = s->affA;
+  st.affine_b = s->affB;
+  if (s->status >= 2) {
+    st.diverged = 1;
+    if (stats) *stats = st;
+    pose_to7(pose_identity(), out);
+    return LSDG_DIVERGED;
+  }
+  se3_track_done(c, r, f, s->good, s->bad, s->lastResidual, usage, s->T, st, out);
+  if (stats) *stats = st;
+  return LSDG_OK;
+}
+
 
 static void fill_eval_se3(const double* S, lsdg_eval* o) {
   std::memset(o, 0, sizeof(*o));
@@ -879,14 +992,9 @@ static void unpack_A7(const double* S, double* A7, double* b7) {
   for (int a = 0; a < 7; ++a) b7[a] = S[SM_B + a];
 }
 
-extern "C" lsdg_status lsdg_sim3_track(lsdg_ctx c, lsdg_ref r, lsdg_frame f, const double init[8], int32_t startLevel,
-                                       int32_t finalLevel, double out[8], lsdg_track_stats* stats) {
-  if (!c || !r || !f || !init || !out) return LSDG_EINVAL;
-  if (r->ctx != c || f->ctx != c) return fail(c, LSDG_EINVAL, "objects belong to another context");
-  if (startLevel < 0 || startLevel >= PYR || finalLevel < 0 || finalLevel > startLevel)
-    return fail(c, LSDG_EINVAL, "level range");
-  if (f->w[0] != r->kf->w[0] || f->h[0] != r->kf->h[0]) return fail(c, LSDG_EINVAL, "frame / keyframe size mismatch");
-  if (!f->hasDepth) return fail(c, LSDG_ESTATE, "Sim3 tracking needs a frame with depth");
+// Sim3Tracker::trackFrameSim3 with a launch and a host LM step per evaluation.
+static lsdg_status sim3_track_steps(lsdg_ctx c, lsdg_ref r, lsdg_frame f, const double init[8], int32_t startLevel,
+                                    int32_t finalLevel, double out[8], lsdg_track_stats* stats) {
   const lsdg_params& P = c->P;
   lsdg_track_stats st;
   std::memset(&st, 0, sizeof st);
@@ -986,6 +1094,46 @@ extern "C" lsdg_status lsdg_sim3_track(lsdg_ctx c, lsdg_ref r, lsdg_frame f, con
   st.tracking_was_good = 1;
   Pose res = pose_inv(T);
   pose_to8(res, out);
+  if (stats) *stats = st;
+  return LSDG_OK;
+}
+
+extern "C" lsdg_status lsdg_sim3_track(lsdg_ctx c, lsdg_ref r, lsdg_frame f, const double init[8], int32_t startLevel,
+                                       int32_t finalLevel, double out[8], lsdg_track_stats* stats) {
+  if (!c || !r || !f || !init || !out) return LSDG_EINVAL;
+  if (r->ctx != c || f->ctx != c) return fail(c, LSDG_EINVAL, "objects belong to another context");
+  if (startLevel < 0 || startLevel >= PYR || finalLevel < 0 || finalLevel > startLevel)
+    return fail(c, LSDG_EINVAL, "level range");
+  if (f->w[0] != r->kf->w[0] || f->h[0] != r->kf->h[0]) return fail(c, LSDG_EINVAL, "frame / keyframe size mismatch");
+  if (!f->hasDepth) return fail(c, LSDG_ESTATE, "Sim3 tracking needs a frame with depth");
+  const JobState* s = nullptr;
+  bool ran = false;
+  lsdg_status s0 = track_lm(c, r, f, LSDG_JOB_SIM3, pose_from8(init), startLevel, finalLevel, nullptr, &s, &ran);
+  if (s0 != LSDG_OK) return s0;
+  if (!ran) return sim3_track_steps(c, r, f, init, startLevel, finalLevel, out, stats);
+  lsdg_track_stats st;
+  std::memset(&st, 0, sizeof st);
+  for (int l = 0; l < PYR; ++l) {
+    st.num_residual_calls[l] = s->numRes[l];
+    st.num_warp_update_calls[l] = s->numWarp[l];
+  }
+  if (s->status != 2) {  // finished every level: lastSim3Hessian
+    int k = 0;
+    for (int a = 0; a < 7; ++a)
+      for (int b = a; b < 7; ++b) st.hessian[7 * a + b] = st.hessian[7 * b + a] = s->lgsA[k++];
+  }
+  if (s->status >= 2) {
+    st.diverged = 1;
+    if (stats) *stats = st;
+    pose_to8(pose_identity(), out);
+    return LSDG_DIVERGED;
+  }
+  st.last_residual = (float)s->finalRes[6];
+  st.last_depth_residual = (float)job_mean_d(*s);
+  st.last_photometric_residual = (float)job_mean_p(*s);
+  st.point_usage = (float)job_usage(*s);
+  st.tracking_was_good = 1;
+  pose_to8(pose_inv(s->T), out);
   if (stats) *stats = st;
   return LSDG_OK;
 }

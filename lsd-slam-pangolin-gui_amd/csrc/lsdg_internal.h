@@ -243,6 +243,13 @@ struct lsdg_ctx_s {
   double* h_result = nullptr;  // pinned, host-mapped
   double* d_result = nullptr;  // device view of h_result
   int num_cus = 256;
+  // one-launch alignments (track_lm.hip): tagged rows, the launch counter that
+  // tags them, and the finished control block (pinned, host-mapped)
+  unsigned long long* d_track_rows = nullptr;
+  unsigned track_epoch = 0;
+  void* h_track = nullptr;
+  void* d_track = nullptr;
+  unsigned track_spin_max = 0;
   // per-kernel timing (lsdg_ctx_profile)
   struct ProfRec {
     int kind;

@@ -1,0 +1,176 @@
+// One alignment's whole Levenberg-Marquardt loop in one launch
+// (SE3Tracker::trackFrame, Sim3Tracker::trackFrameSim3): what lsdg_se3_track
+// and lsdg_sim3_track run.
+//
+// A launch per evaluation costs its kernel (about 11 us, of which the
+// evaluation itself is a third: the rest is the start of the launch, the
+// merge behind a completion counter and the result's way to the host) and
+// about as much again for the launch, the wait and the host's LM step: 22 us
+// for each of about 28 evaluations.  Here the blocks stay: every block
+// reduces its range of the level's points to an FP64 row, publishes it as
+// tagged words and reads the others' rows (k_batch_coop's exchange), and
+// repeats the same LM step on its own copy of the control block, so an
+// iteration is one evaluation, one exchange and one LM step.
+//
+// 320x240 camera image to pose: 764 -> 269 us; 640x480 through the
+// undistorter: 722 -> 306 us (the launch itself 203 us for 28 evaluations).
+//
+// Blocks: one point per thread of the largest level (the shortest
+// evaluation), at most TRACK_LM_MAX_BLOCKS.  On a small level every block
+// evaluates the whole level itself and nothing is exchanged.  The blocks must
+// be resident together.  They are when the device
+// has that many free slots (it holds several hundred); other work on it can
+// keep some of them out, so every wait is bounded, the blocks that waited in
+// vain stop, and the caller runs the alignment launch by launch instead.
+#include "lm_device.h"
+#include "track_device.h"
+
+namespace lsdg {
+
+#ifndef LSDG_TRACK_SOLO
+#define LSDG_TRACK_SOLO 1024
+#endif
+constexpr int TRACK_LM_BS = 256;
+constexpr int TRACK_LM_WAVES = TRACK_LM_BS / 64;
+// Levels of at most this many points are evaluated whole by every block: four
+// points per thread cost less than an exchange.
+constexpr int TRACK_LM_SOLO = LSDG_TRACK_SOLO;
+
+template <int KIND, int PREC, int ACC>
+__global__ __launch_bounds__(TRACK_LM_BS) void k_track_lm(TrackLmArgs a) {
+  constexpr int NS = KIND == LSDG_JOB_SIM3 ? NS_SIM3 : NS_SE3;
+  __shared__ JobState s;
+  __shared__ JobDesc jd;
+  __shared__ double sh[TRACK_LM_WAVES][NS];
+  __shared__ double S[NS];
+  __shared__ int failed;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, part = blockIdx.x;
+  block_copy(&jd, &a.jd, TRACK_LM_BS);
+  if (tid == 0) failed = 0;
+  __syncthreads();
+  if (tid < 64) {
+    int nt = 0;
+    lm_begin(s, jd, a.P, &nt, nullptr);
+  }
+  __syncthreads();
+  unsigned gen = 0;  // exchanges so far
+  for (int it = 0; it < BATCH_JOB_MAX_EVALS; ++it) {
+    // s is read after a barrier: the exit test is uniform over the block
+    if (s.status != 0) break;
+    const int lvl = s.level;
+    const JobLevel& L = jd.lv[lvl];
+    const int n = L.pts.n;
+    // every block takes part in every exchange: one that only read could be
+    // overtaken by the others' next rows
+    const int parts = a.blocks;
+    const bool split = parts > 1 && n > TRACK_LM_SOLO;
+    const int i0 = split ? (int)((long long)n * part / parts) : 0;
+    const int i1 = split ? (int)((long long)n * (part + 1) / parts) : n;
+    const Xf x = s.xf;
+    TrackKParams kp = a.kp;
+    kp.aff_a = s.affA;
+    kp.aff_b = s.affB;
+    Accum<ACC, NS> acc;
+    acc.zero();
+    if (KIND == LSDG_JOB_SIM3) {
+      kp.roll[0] = s.roll[0]; kp.roll[1] = s.roll[1]; kp.roll[2] = s.roll[2]; kp.roll[3] = s.roll[3];
+      sim3_points<PREC, EVAL_U>(L.pts, i0 + tid, TRACK_LM_BS, i1, L.img, L.fid, L.fvar, L.g, x, kp, acc);
+    } else {
+      uint8_t* mask = lvl == 1 ? jd.isGood : nullptr;
+      se3_points<PREC, EVAL_U>(L.pts, i0 + tid, TRACK_LM_BS, i1, L.img, L.g, x, kp, mask, acc);
+    }
+    const double wsum = acc.wave_slot();
+    if (lane < NS) sh[wave][lane] = wsum;
+    __syncthreads();
+    if (!split) {
+      if (tid < NS) S[tid] = Accum<ACC, NS>::merge_waves(&sh[0][tid], NS, TRACK_LM_WAVES);
+      __syncthreads();
+    } else {
+      unsigned long long* buf = a.rows + (size_t)(gen & 1) * a.blocks * NS * 2;
+      const unsigned tag = a.epochTag | (gen & 0xFFFFu);
+      if (tid < NS) {
+        const double v = Accum<ACC, NS>::merge_waves(&sh[0][tid], NS, TRACK_LM_WAVES);
+        const unsigned long long bits = (unsigned long long)__double_as_longlong(v);
+        unsigned long long* w = buf + ((size_t)part * NS + tid) * 2;
+        const unsigned long long t64 = (unsigned long long)tag << 32;
+        __hip_atomic_store(w, t64 | (bits & 0xFFFFFFFFull), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(w + 1, t64 | (bits >> 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      __syncthreads();  // sh is read above and written below
+      // each wave reads a quarter of the rows and adds them in part order
+      const int q0 = parts * wave / TRACK_LM_WAVES, q1 = parts * (wave + 1) / TRACK_LM_WAVES;
+      double v = 0.0;
+      for (unsigned spins = 0;; ++spins) {
+        bool mine = true;
+        double t = 0.0;
+        if (lane < NS) {
+#pragma unroll 4
+          for (int q = q0; q < q1; ++q) {
+            const unsigned long long* w = buf + ((size_t)q * NS + lane) * 2;
+            const unsigned long long lo = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const unsigned long long hi = __hip_atomic_load(w + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            mine = mine && (unsigned)(lo >> 32) == tag && (unsigned)(hi >> 32) == tag;
+            t += __longlong_as_double((long long)((hi << 32) | (lo & 0xFFFFFFFFull)));
+          }
+        }
+        if (__all(mine)) {
+          v = t;
+          break;
+        }
+        if (spins >= a.spinMax) {
+          if (lane == 0) failed = 1;
+          break;
+        }
+        __builtin_amdgcn_s_sleep(1);
+      }
+      if (lane < NS) sh[wave][lane] = v;
+      __syncthreads();
+      if (failed) break;  // uniform over the block
+      if (tid < NS) S[tid] = ((sh[0][tid] + sh[1][tid]) + sh[2][tid]) + sh[3][tid];
+      ++gen;
+      __syncthreads();
+    }
+    if (tid < 64) {
+      int next = 0;
+      if (KIND == LSDG_JOB_SIM3) lm_step_sim3(s, jd, S, a.P, &next, nullptr);
+      else lm_step_se3(s, jd, S, a.P, &next, nullptr);
+    }
+    __syncthreads();
+  }
+  if (part == 0) {
+    if (tid == 0 && failed) s.status = -1;
+    __syncthreads();
+    block_copy(a.out, &s, TRACK_LM_BS);
+  }
+}
+
+__global__ __launch_bounds__(256) void k_track_lm_clear(unsigned long long* rows, size_t n) {
+  for (size_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) rows[i] = 0ull;
+}
+
+int track_lm_blocks(lsdg_ctx c, int n) {
+  const int nb = (n + TRACK_LM_BS - 1) / TRACK_LM_BS;
+  return n <= TRACK_LM_SOLO ? 1 : std::min(nb, std::min(TRACK_LM_MAX_BLOCKS, c->num_cus));
+}
+
+template <int KIND, int PREC>
+static void (*track_kernel(int acc))(TrackLmArgs) {
+  return acc == BATCH_ACC_KAHAN ? k_track_lm<KIND, PREC, ACC_KAHAN> : k_track_lm<KIND, PREC, ACC_F64>;
+}
+
+hipError_t launch_track_lm(const TrackLmArgs& a, int prec, int acc, hipStream_t s, const KTimer* t) {
+  auto k = a.jd.kind == LSDG_JOB_SIM3 ? (prec == LSDG_FP16   ? track_kernel<LSDG_JOB_SIM3, LSDG_FP16>(acc)
+                                         : prec == LSDG_BF16 ? track_kernel<LSDG_JOB_SIM3, LSDG_BF16>(acc)
+                                                             : track_kernel<LSDG_JOB_SIM3, LSDG_FP32>(acc))
+                                      : (prec == LSDG_FP16   ? track_kernel<LSDG_JOB_SE3, LSDG_FP16>(acc)
+                                         : prec == LSDG_BF16 ? track_kernel<LSDG_JOB_SE3, LSDG_BF16>(acc)
+                                                             : track_kernel<LSDG_JOB_SE3, LSDG_FP32>(acc));
+  return launch_k(k, dim3(a.blocks), dim3(TRACK_LM_BS), s, t, a);
+}
+
+hipError_t launch_track_lm_clear(unsigned long long* rows, size_t n, hipStream_t s) {
+  k_track_lm_clear<<<dim3((unsigned)std::min<size_t>((n + 255) / 256, 256)), dim3(256), 0, s>>>(rows, n);
+  return hipGetLastError();
+}
+
+}  // namespace lsdg

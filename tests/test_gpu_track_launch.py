@@ -1,0 +1,95 @@
+"""The one-launch alignments: the same LM path as the launch-per-evaluation
+form they fall back to when their blocks cannot all run at once, over sizes
+with one block, a few and the most, and interleaved on several contexts."""
+import threading
+
+import numpy as np
+import pytest
+
+import lsdg
+import synth
+from helpers import twist
+
+pytestmark = pytest.mark.gpu
+
+
+def _steps_context(monkeypatch):
+    """A context whose one-launch alignments give up at the first wait."""
+    monkeypatch.setenv("LSDG_TRACK_SPIN_MAX", "0")
+    try:
+        return lsdg.Context(0)
+    finally:
+        monkeypatch.delenv("LSDG_TRACK_SPIN_MAX")
+
+
+def _pair(ctx, cam, seed, prec):
+    d = synth.sim3_instance(seed, cam=cam, max_trans=0.03, max_rot_deg=1.0, scale_range=(0.98, 1.02))
+    a = ctx.frame(0, cam, d["a_img"], prec)
+    a.set_depth(d["a_idepth"], d["a_var"])
+    b = ctx.frame(1, cam, d["b_img"], prec)
+    b.set_depth(d["b_idepth"], d["b_var"])
+    return a, b, ctx.ref(a)
+
+
+def _fields(st):
+    return [st.last_good_count, st.last_bad_count, st.diverged, st.tracking_was_good, *st.num_residual_calls,
+            *st.num_warp_update_calls]
+
+
+# 64x64: every level is small; 130x98: the split threshold; 322x242: ragged; 1282x962: the most blocks
+@pytest.mark.parametrize("w,h", [(64, 64), (130, 98), (322, 242), (1282, 962)])
+@pytest.mark.parametrize("prec", [lsdg.FP32, lsdg.FP16])
+def test_one_launch_equals_launch_per_evaluation(ctx, monkeypatch, w, h, prec):
+    cam = synth.camera(w, h)
+    other = _steps_context(monkeypatch)
+    for seed in (41, 42):
+        res = []
+        for c in (ctx, other):
+            a, b, ref = _pair(c, cam, seed, prec)
+            p, st, status = c.se3_track(ref, b, synth.IDENTITY7)
+            mask = b.read(lsdg.WHAT_REF_PIXEL_WAS_GOOD)
+            q, st3, status3 = c.sim3_track(ref, b, [*synth.IDENTITY7, 1.0], 4, 1)
+            res.append((p, st, status, mask, q, st3, status3))
+            for x in (ref, b, a):
+                x.destroy()
+        (p, st, status, mask, q, st3, status3), (p2, st2, status2, mask2, q2, st32, status32) = res
+        assert status == status2 and status3 == status32
+        assert _fields(st) == _fields(st2) and _fields(st3) == _fields(st32)
+        # FP64 sums and solves in another order: the FP32 path's terms are the
+        # same, so poses agree to the tests' usual 1e-9
+        assert twist(p, p2) <= 1e-9 and twist(q[:7], q2[:7]) <= 1e-9 and abs(q[7] - q2[7]) <= 1e-9
+        assert np.array_equal(mask, mask2)
+        for k in ("last_residual", "last_mean_res", "point_usage", "last_depth_residual", "last_photometric_residual"):
+            for u, v in ((st, st2), (st3, st32)):
+                assert np.isclose(getattr(u, k), getattr(v, k), rtol=1e-6, equal_nan=True), k
+        H, H2 = np.array(st3.hessian[:]), np.array(st32.hessian[:])
+        assert np.abs(H - H2).max() <= 1e-9 * max(np.abs(H2).max(), 1e-30)
+    other.close()
+
+
+def test_contexts_align_at_the_same_time():
+    """Six threads, each with its own context, aligning at once: every result
+    equals the single-threaded one."""
+    cam = synth.camera(640, 480)
+    out, errors = {}, []
+
+    def work(k):
+        try:
+            c = lsdg.Context(0)
+            a, b, ref = _pair(c, cam, 50, lsdg.FP32)
+            out[k] = [c.se3_track(ref, b, synth.IDENTITY7)[0] for _ in range(20)]
+            for x in (ref, b, a):
+                x.destroy()
+            c.close()
+        except Exception as e:  # reported below, in the test's own thread
+            errors.append(e)
+
+    work("alone")
+    ts = [threading.Thread(target=work, args=(k,)) for k in range(6)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not errors, errors
+    want = out["alone"][0]
+    assert all(twist(p, want) <= 1e-9 for v in out.values() for p in v)
