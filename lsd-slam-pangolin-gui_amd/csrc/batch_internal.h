@@ -52,6 +52,7 @@ struct JobState {
   int level, phase, iteration, incTry, upToDate, evals;
   int numRes[PYR], numWarp[PYR];
   int evalsAt[PYR];  // evaluations run per level (every step the job was active)
+  int npts[PYR];     // k_track_lm: the reference's points per level
 };
 
 struct BatchArgs {
@@ -89,6 +90,7 @@ struct TrackLmArgs {
   lsdg_params P;
   TrackKParams kp;
   unsigned long long* rows;  // [2][blocks][NS][2] tagged words
+  const int* counts;         // points per level of the reference (device memory)
   JobState* out;             // the finished control block (host-mapped); status < 0: the blocks gave up
   unsigned epochTag;         // tag of this launch in the upper 16 bits, never 0
   int blocks;                // blocks of the launch
@@ -97,8 +99,8 @@ struct TrackLmArgs {
 constexpr unsigned TRACK_LM_SPIN_MAX = 1u << 14;  // polls of about a microsecond
 constexpr int TRACK_LM_MAX_BLOCKS = 64;
 constexpr size_t TRACK_LM_WORDS = (size_t)2 * TRACK_LM_MAX_BLOCKS * NS_MAX * 2;
-// Blocks of a launch for alignments whose largest level holds n points.
-int track_lm_blocks(lsdg_ctx c, int n);
+// Blocks of a launch for alignments whose finest level has `pixels` pixels.
+int track_lm_blocks(lsdg_ctx c, int pixels);
 hipError_t launch_track_lm(const TrackLmArgs& a, int prec, int acc, hipStream_t s, const KTimer* t = nullptr);
 // Zeroes n tagged words (a fill kernel).
 hipError_t launch_track_lm_clear(unsigned long long* rows, size_t n, hipStream_t s);

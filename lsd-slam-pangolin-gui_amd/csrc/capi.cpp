@@ -519,6 +519,7 @@ extern "C" lsdg_status lsdg_ref_create(lsdg_ctx c, lsdg_frame kf, lsdg_ref* out)
   if (!r) return LSDG_ENOMEM;
   r->ctx = c;
   r->kf = kf;
+  for (PointsLevel& l : r->lv) l = PointsLevel{nullptr, nullptr, nullptr, nullptr, 0};
   *out = r;
   return LSDG_OK;
 }
@@ -528,23 +529,45 @@ extern "C" lsdg_status lsdg_ref_destroy(lsdg_ref r) {
   (void)hipStreamSynchronize(r->ctx->stream);
   for (int l = 0; l < PYR; ++l)
     if (r->d_pool[l]) (void)hipFree(r->d_pool[l]);
-  if (r->d_blockcounts) (void)hipFree(r->d_blockcounts);
+  if (r->d_counts) (void)hipFree(r->d_counts);
   delete r;
   return LSDG_OK;
 }
 
-lsdg_status lsdg::ref_points(lsdg_ref r, int level) {
+lsdg_status lsdg::ref_points_queue(lsdg_ref r, int lo, int hi) {
   lsdg_ctx c = r->ctx;
-  if (level < 0 || level >= PYR) return fail(c, LSDG_EINVAL, "level out of range");
+  if (lo < 0 || hi >= PYR || lo > hi) return fail(c, LSDG_EINVAL, "level out of range");
   if (!r->kf->hasDepth) return fail(c, LSDG_ESTATE, "keyframe has no depth");
   if (r->depthVersion != r->kf->depthVersion) {
     for (int l = 0; l < PYR; ++l) r->num[l] = -1;
+    r->pending = 0;
     r->depthVersion = r->kf->depthVersion;
   }
-  if (r->num[level] >= 0) return LSDG_OK;
-  lsdg_status st = frame_require(r->kf, fd_bit(FD_IMAGE, level) | fd_bit(FD_GRAD, level));
+  unsigned need = 0;
+  for (int l = lo; l <= hi; ++l)
+    if (r->num[l] < 0 && !(r->pending >> l & 1u)) need |= 1u << l;
+  if (!need) return LSDG_OK;
+  lsdg_status st = frame_require(r->kf, need << FD_IMAGE);
   if (st != LSDG_OK) return st;
-  CK(c, launch_point_cloud(r, level, c->stream));
+  CK(c, launch_point_clouds(r, need, c->stream));
+  r->pending |= need;
+  return LSDG_OK;
+}
+
+void lsdg::ref_points_known(lsdg_ref r, const int* counts) {
+  for (int l = 0; l < PYR; ++l)
+    if (r->pending >> l & 1u) r->num[l] = r->lv[l].n = counts[l];
+  r->pending = 0;
+}
+
+lsdg_status lsdg::ref_points(lsdg_ref r, int lo, int hi) {
+  lsdg_status st = ref_points_queue(r, lo, hi);
+  if (st != LSDG_OK || !r->pending) return st;
+  lsdg_ctx c = r->ctx;
+  int counts[PYR] = {0, 0, 0, 0, 0};
+  CK(c, hipMemcpyAsync(counts, r->d_counts, sizeof counts, hipMemcpyDeviceToHost, c->stream));
+  CK(c, hipStreamSynchronize(c->stream));
+  ref_points_known(r, counts);
   return LSDG_OK;
 }
 
@@ -690,10 +713,11 @@ static lsdg_status track_lm(lsdg_ctx c, lsdg_ref r, lsdg_frame f, int kind, cons
   a.jd.finalLevel = finalLevel;
   a.jd.init = init;
   a.jd.isGood = mask;
-  int maxPoints = 0;
+  // point clouds and pyramid levels are queued ahead of the launch, which
+  // reads the points' counts on the device
+  lsdg_status st = ref_points_queue(r, finalLevel, startLevel);
+  if (st != LSDG_OK) return st;
   for (int l = finalLevel; l <= startLevel; ++l) {
-    lsdg_status st = ref_points(r, l);
-    if (st != LSDG_OK) return st;
     JobLevel& L = a.jd.lv[l];
     L.pts = r->lv[l];
     L.img = f->precision == LSDG_FP32 ? (const void*)f->d_grad[l] : (const void*)f->d_gradh[l];
@@ -701,14 +725,14 @@ static lsdg_status track_lm(lsdg_ctx c, lsdg_ref r, lsdg_frame f, int kind, cons
     L.fvar = f->d_ivar[l];
     L.g = LevelGeom{f->w[l], f->h[l], f->fx[l], f->fy[l], f->cx[l], f->cy[l]};
     L.ntiles = 1;
-    maxPoints = std::max(maxPoints, L.pts.n);
   }
-  lsdg_status st = frame_require(f, fd_track(f, finalLevel, startLevel));
+  a.counts = r->d_counts;
+  st = frame_require(f, fd_track(f, finalLevel, startLevel));
   if (st != LSDG_OK) return st;
   a.P = c->P;
   a.kp = track_kparams(c->P, kind == LSDG_JOB_SIM3);
   a.kp.aff_stats = c->P.use_affine_lightning_estimation;
-  a.blocks = track_lm_blocks(c, maxPoints);
+  a.blocks = track_lm_blocks(c, f->w[finalLevel] * f->h[finalLevel]);
   a.rows = c->d_track_rows;
   a.spinMax = c->track_spin_max;
   a.out = (JobState*)c->d_track;
@@ -723,9 +747,10 @@ static lsdg_status track_lm(lsdg_ctx c, lsdg_ref r, lsdg_frame f, int kind, cons
   CK(c, launch_track_lm(a, f->precision, c->sums == LSDG_SUMS_KAHAN ? BATCH_ACC_KAHAN : BATCH_ACC_F64, c->stream, &kt));
   CK(c, hipStreamSynchronize(c->stream));
   const JobState* s = (const JobState*)c->h_track;
+  ref_points_known(r, s->npts);
   double bytes = 0.0;
   for (int l = finalLevel; l <= startLevel; ++l)
-    bytes += s->evalsAt[l] * eval_bytes(a.jd.lv[l].pts.n, f, l, kind == LSDG_JOB_SIM3);
+    bytes += s->evalsAt[l] * eval_bytes(r->lv[l].n, f, l, kind == LSDG_JOB_SIM3);
   prof_timer_done(c, LSDG_KERNEL_EVAL, kt, bytes);
   *out = s;
   *ran = s->status >= 0;

@@ -109,6 +109,11 @@ static lsdg_status build_job_table(lsdg_batch b) {
   const int tile = 256 * b->ppt;
   b->h_jobs.assign(b->n, JobDesc{});
   size_t slot = 0;
+  // queue every keyframe's point clouds before the first wait for a count
+  for (const lsdg_job& J : b->jobs) {
+    lsdg_status st = ref_points_queue(J.ref, J.final_level, J.start_level);
+    if (st != LSDG_OK) return st;
+  }
   for (int j = 0; j < b->n; ++j) {
     const lsdg_job& J = b->jobs[j];
     lsdg_ref r = J.ref;

@@ -22,7 +22,14 @@ unsigned fd_track(lsdg_frame f, int lo, int hi);
 // stage for the fd_bit data in `grads`).
 double pyramid_bytes(lsdg_frame f, bool images, unsigned grads);
 lsdg_status frame_ensure_was_good(lsdg_frame f);
-lsdg_status ref_points(lsdg_ref r, int level);
+// Point clouds of levels lo..hi of r: queued on the context stream if the
+// keyframe's depth moved on (r->lv[l].n may still be unknown), or with their
+// counts on the host.
+lsdg_status ref_points_queue(lsdg_ref r, int lo, int hi);
+lsdg_status ref_points(lsdg_ref r, int lo, int hi);
+inline lsdg_status ref_points(lsdg_ref r, int level) { return ref_points(r, level, level); }
+// Files counts read from r->d_counts for the levels still pending.
+void ref_points_known(lsdg_ref r, const int* counts);
 Xf pose_xf(const Pose& T, bool scaled);
 TrackKParams track_kparams(const lsdg_params& P, bool sim3);
 void esm_roll(const Pose& T, float* r4);

@@ -372,11 +372,13 @@ extern "C" lsdg_status lsdg_system_track(lsdg_system s, int32_t id, const uint8_
   const bool myCreate = s->createNewKeyFrame;
   // trackingReference->importFrame(currentKeyFrame) when the keyframe changed
   // (a depth change is picked up by the reference itself)
-  if (!s->ref || s->ref->kf != s->kf.get()) {
-    if (s->ref) lsdg_ref_destroy(s->ref);
-    s->ref = nullptr;
+  if (!s->ref) {
     st = lsdg_ref_create(s->ctx, s->kf.get(), &s->ref);
     if (st != LSDG_OK) return st;
+  } else if (s->ref->kf != s->kf.get()) {
+    // every keyframe has the system's size: the reference's storage stays
+    s->ref->kf = s->kf.get();
+    s->ref->depthVersion = -1;
   }
   double init[7], pose7[7];
   se3_of(pose_mul(pose_inv(s->kf->camToWorld), s->lastCamToWorld), init);

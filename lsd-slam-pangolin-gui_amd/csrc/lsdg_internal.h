@@ -310,8 +310,9 @@ struct lsdg_ref_s {
   int cap[lsdg::PYR] = {0, 0, 0, 0, 0};
   void* d_pool[lsdg::PYR] = {nullptr, nullptr, nullptr, nullptr, nullptr};
   lsdg::PointsLevel lv[lsdg::PYR];
-  int* d_blockcounts = nullptr;
-  int blockcounts_cap = 0;
+  // device: points of each level, then of each tile of the compaction
+  int* d_counts = nullptr;
+  unsigned pending = 0;  // levels (bit l) whose points are queued on the stream but whose num is not known yet
 };
 
 struct lsdg_depthmap_s {
@@ -369,7 +370,9 @@ hipError_t launch_ingest(lsdg_frame f, const uint8_t* d_src, int inW, const floa
 hipError_t launch_pyr_grads(lsdg_frame f, unsigned need, hipStream_t s);
 hipError_t launch_pyr_depth(lsdg_frame f, hipStream_t s);
 hipError_t launch_depth_normalize(float* idepth, float* ivar, int n, hipStream_t s);
-hipError_t launch_point_cloud(lsdg_ref r, int level, hipStream_t s);  // fills r->lv[level], r->num[level]
+// Queues the point clouds of the levels with a bit in `levels`: sets r->lv
+// (n left 0) and writes the counts to r->d_counts[level].
+hipError_t launch_point_clouds(lsdg_ref r, unsigned levels, hipStream_t s);
 size_t pyr_batch_bytes(int nf);
 void pyr_batch_tables(lsdg_frame const* fs, const unsigned* need, int nf, void* h, void* d, PyrBatch* out);
 hipError_t launch_pyr_batch(const PyrBatch& b, hipStream_t s);

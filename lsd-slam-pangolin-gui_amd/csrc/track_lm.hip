@@ -15,7 +15,7 @@
 // 320x240 camera image to pose: 764 -> 269 us; 640x480 through the
 // undistorter: 722 -> 306 us (the launch itself 203 us for 28 evaluations).
 //
-// Blocks: one point per thread of the largest level (the shortest
+// Blocks: about one point per thread of the largest level (the shortest
 // evaluation), at most TRACK_LM_MAX_BLOCKS.  On a small level every block
 // evaluates the whole level itself and nothing is exchanged.  The blocks must
 // be resident together.  They are when the device
@@ -49,8 +49,13 @@ __global__ __launch_bounds__(TRACK_LM_BS) void k_track_lm(TrackLmArgs a) {
   if (tid == 0) failed = 0;
   __syncthreads();
   if (tid < 64) {
+    // the counts of levels outside the job's are never read
+    if (tid < PYR) jd.lv[tid].pts.n = a.counts[tid];
+    wave_sync();
     int nt = 0;
     lm_begin(s, jd, a.P, &nt, nullptr);
+    wave_sync();
+    if (tid < PYR) s.npts[tid] = jd.lv[tid].pts.n;
   }
   __syncthreads();
   unsigned gen = 0;  // exchanges so far
@@ -148,9 +153,11 @@ __global__ __launch_bounds__(256) void k_track_lm_clear(unsigned long long* rows
   for (size_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) rows[i] = 0ull;
 }
 
-int track_lm_blocks(lsdg_ctx c, int n) {
-  const int nb = (n + TRACK_LM_BS - 1) / TRACK_LM_BS;
-  return n <= TRACK_LM_SOLO ? 1 : std::min(nb, std::min(TRACK_LM_MAX_BLOCKS, c->num_cus));
+int track_lm_blocks(lsdg_ctx c, int pixels) {
+  // a quarter of the pixels is what a semi-dense map holds; the size alone
+  // decides, so that an image's result does not depend on what the host knows
+  const int nb = (pixels / 4 + TRACK_LM_BS - 1) / TRACK_LM_BS;
+  return std::max(1, std::min(nb, std::min(TRACK_LM_MAX_BLOCKS, c->num_cus)));
 }
 
 template <int KIND, int PREC>
