@@ -153,6 +153,7 @@ __global__ __launch_bounds__(BATCH_SOLVE_BS) void k_batch_solve(BatchArgs a, int
   __shared__ double S[NS];
   __shared__ JobState sst;
   __shared__ JobDesc sjd;
+  __shared__ LmParams sP;
   __shared__ int next;
   const int j = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int nj = a.njobs;
@@ -165,6 +166,7 @@ __global__ __launch_bounds__(BATCH_SOLVE_BS) void k_batch_solve(BatchArgs a, int
   }
   block_copy(&sst, a.st + j, BATCH_SOLVE_BS);
   block_copy(&sjd, a.jobs + j, BATCH_SOLVE_BS);
+  block_copy(&sP, &a.P, BATCH_SOLVE_BS);
   if (lane < NS) {
     const double* rows = a.partials + (size_t)slotBase * NS + lane;
     double v = 0.0;
@@ -188,8 +190,8 @@ __global__ __launch_bounds__(BATCH_SOLVE_BS) void k_batch_solve(BatchArgs a, int
   __syncthreads();
   if (tid < 64) {
     int nx = 0;
-    if (KIND == LSDG_JOB_SIM3) lm_step_sim3(sst, sjd, S, a.P, &nx, a.remaining);
-    else lm_step_se3(sst, sjd, S, a.P, &nx, a.remaining);
+    if (KIND == LSDG_JOB_SIM3) lm_step_sim3(sst, sjd, S, sP, &nx, a.remaining);
+    else lm_step_se3(sst, sjd, S, sP, &nx, a.remaining);
     if (tid == 0) next = nx;
   }
   __syncthreads();
@@ -212,11 +214,13 @@ __global__ __launch_bounds__(BATCH_JOB_BS) void k_batch_job(BatchArgs a) {
   constexpr int WAVES = BATCH_JOB_BS / 64;
   __shared__ JobState s;
   __shared__ JobDesc jd;
+  __shared__ LmParams sP;
   __shared__ double sh[WAVES][NS];
   __shared__ double S[NS];
   const int j = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   block_copy(&s, a.st + j, BATCH_JOB_BS);
   block_copy(&jd, a.jobs + j, BATCH_JOB_BS);
+  block_copy(&sP, &a.P, BATCH_JOB_BS);
   __syncthreads();
   for (int it = 0; it < BATCH_JOB_MAX_EVALS; ++it) {
     // s and jd are read after a barrier: the exit test is uniform over the block
@@ -245,8 +249,8 @@ __global__ __launch_bounds__(BATCH_JOB_BS) void k_batch_job(BatchArgs a) {
     __syncthreads();
     if (tid < 64) {
       int next = 0;
-      if (KIND == LSDG_JOB_SIM3) lm_step_sim3(s, jd, S, a.P, &next, a.remaining);
-      else lm_step_se3(s, jd, S, a.P, &next, a.remaining);
+      if (KIND == LSDG_JOB_SIM3) lm_step_sim3(s, jd, S, sP, &next, a.remaining);
+      else lm_step_se3(s, jd, S, sP, &next, a.remaining);
     }
     __syncthreads();
   }
@@ -280,6 +284,7 @@ __global__ __launch_bounds__(COOP_BS) void k_batch_coop(BatchArgs a) {
   constexpr int WAVES = COOP_BS / 64;
   __shared__ JobState s;
   __shared__ JobDesc jd;
+  __shared__ LmParams sP;
   __shared__ double sh[WAVES][NS];
   __shared__ double S[NS];
   __shared__ int arrived;
@@ -303,6 +308,7 @@ __global__ __launch_bounds__(COOP_BS) void k_batch_coop(BatchArgs a) {
   const unsigned epochTag = (*a.epoch & 0xFFFFu) << 16;
   block_copy(&s, a.st + j, COOP_BS);
   block_copy(&jd, a.jobs + j, COOP_BS);
+  block_copy(&sP, &a.P, COOP_BS);
   __syncthreads();
   unsigned gen = 0;  // synchronised iterations of this job so far
   for (int it = 0; it < BATCH_JOB_MAX_EVALS; ++it) {
@@ -388,8 +394,8 @@ __global__ __launch_bounds__(COOP_BS) void k_batch_coop(BatchArgs a) {
     __syncthreads();
     if (tid < 64) {
       int next = 0;
-      if (KIND == LSDG_JOB_SIM3) lm_step_sim3(s, jd, S, a.P, &next, remaining);
-      else lm_step_se3(s, jd, S, a.P, &next, remaining);
+      if (KIND == LSDG_JOB_SIM3) lm_step_sim3(s, jd, S, sP, &next, remaining);
+      else lm_step_se3(s, jd, S, sP, &next, remaining);
     }
     __syncthreads();
   }

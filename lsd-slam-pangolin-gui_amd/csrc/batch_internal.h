@@ -42,7 +42,7 @@ struct JobState {
   Xf xf;             // pose of the next evaluation, FP32
   float roll[4];     // its ESM roll (Sim3)
   double incSq;
-  double lgsA[28], lgsB[7];        // unnormalised LGS of the accepted pose
+  double lgs[35];                  // unnormalised LGS of the accepted pose: upper triangle of A (21 / 28), then b
   double lastErr, lastResidual;    // SE3
   double lastRes[7], finalRes[7];  // Sim3 (sumResD, sumResP, numTermsD, numTermsP, set, 0, mean)
   double good, bad, signedRes, usageSum;  // sums of the last evaluation, over usageN points
@@ -54,6 +54,27 @@ struct JobState {
   int evalsAt[PYR];  // evaluations run per level (every step the job was active)
   int npts[PYR];     // k_track_lm: the reference's points per level
 };
+
+// What the LM step reads of lsdg_params, the comparisons' bounds in FP64.
+struct LmLevel {
+  double convergenceEps, stepSizeMin;
+  float lambdaInitial, lambdaSuccess, lambdaFail;
+  int maxIts;
+};
+struct LmParams {
+  LmLevel lv[PYR];
+  float lim;   // min_goodperall_pixel_absmin
+  int affine;  // use_affine_lightning_estimation
+};
+inline LmParams lm_params(const lsdg_params& P) {
+  LmParams q;
+  for (int l = 0; l < PYR; ++l)
+    q.lv[l] = LmLevel{(double)P.convergence_eps[l], (double)P.step_size_min[l], P.lambda_initial[l],
+                      P.lambda_success_fac[l], P.lambda_fail_fac[l], P.max_its_per_lvl[l]};
+  q.lim = P.min_goodperall_pixel_absmin;
+  q.affine = P.use_affine_lightning_estimation;
+  return q;
+}
 
 struct BatchArgs {
   const JobDesc* jobs;
@@ -73,8 +94,7 @@ struct BatchArgs {
   unsigned spinMax;   // k_batch_coop: polls of the row-exchange wait before the blocks give up
   int xcds;           // k_batch_coop: > 1: block b belongs to dispatch group b % xcds, which holds
                       // every block of jobs j with j % xcds == b % xcds (grid padded to a multiple)
-  int affineStats;    // accumulate the affine-brightness sums (only read when estimation is on)
-  lsdg_params P;
+  LmParams P;
   TrackKParams kp;
 };
 
@@ -87,7 +107,7 @@ inline double job_mean_p(const JobState& s) { return s.finalRes[4] != 0.0 ? s.fi
 // cooperating as in k_batch_coop.
 struct TrackLmArgs {
   JobDesc jd;
-  lsdg_params P;
+  LmParams P;
   TrackKParams kp;
   unsigned long long* rows;  // [2][blocks][NS][2] tagged words
   const int* counts;         // points per level of the reference (device memory)

@@ -729,7 +729,7 @@ static lsdg_status track_lm(lsdg_ctx c, lsdg_ref r, lsdg_frame f, int kind, cons
   a.counts = r->d_counts;
   st = frame_require(f, fd_track(f, finalLevel, startLevel));
   if (st != LSDG_OK) return st;
-  a.P = c->P;
+  a.P = lm_params(c->P);
   a.kp = track_kparams(c->P, kind == LSDG_JOB_SIM3);
   a.kp.aff_stats = c->P.use_affine_lightning_estimation;
   a.blocks = track_lm_blocks(c, f->w[finalLevel] * f->h[finalLevel]);
@@ -1145,7 +1145,7 @@ extern "C" lsdg_status lsdg_sim3_track(lsdg_ctx c, lsdg_ref r, lsdg_frame f, con
   if (s->status != 2) {  // finished every level: lastSim3Hessian
     int k = 0;
     for (int a = 0; a < 7; ++a)
-      for (int b = a; b < 7; ++b) st.hessian[7 * a + b] = st.hessian[7 * b + a] = s->lgsA[k++];
+      for (int b = a; b < 7; ++b) st.hessian[7 * a + b] = st.hessian[7 * b + a] = s->lgs[k++];
   }
   if (s->status >= 2) {
     st.diverged = 1;

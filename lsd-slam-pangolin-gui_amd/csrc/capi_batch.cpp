@@ -182,7 +182,7 @@ static BatchArgs batch_args(lsdg_batch b, int c) {
   a.coopK = b->coopK;
   a.soloMax = b->soloMax;
   a.spinMax = b->spinMax;
-  a.P = b->ctx->P;
+  a.P = lm_params(b->ctx->P);
   a.kp = track_kparams(b->ctx->P, b->kind == LSDG_JOB_SIM3);
   // the batched LM reads the affine sums only when it estimates the affine
   // brightness; the results report the estimate, not the sums
@@ -543,8 +543,8 @@ static void fill_result(lsdg_batch b, int j, const JobState& s, lsdg_job_result*
     int k = 0;
     for (int a = 0; a < 7; ++a)
       for (int cc = a; cc < 7; ++cc) {
-        st.hessian[7 * a + cc] = s.lgsA[k];
-        st.hessian[7 * cc + a] = s.lgsA[k];
+        st.hessian[7 * a + cc] = s.lgs[k];
+        st.hessian[7 * cc + a] = s.lgs[k];
         ++k;
       }
   }

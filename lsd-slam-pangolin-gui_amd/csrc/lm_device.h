@@ -12,10 +12,11 @@
 //   - exp of a step is its power series in th^2 up to |w| = 0.5 rad;
 //   - products of unit quaternions are renormalised with one Newton step;
 //   - the divisions by counts that only feed the result are left to the host.
+//   - the values a step's decision needs are read from LDS together.
 // All of it agrees with the host form to FP64 rounding.
-// 64 SE3 alignments of 640x480 in one plan: 534 -> 504 us; 24 of 752x478:
-// 408 -> 392 us; three stages of 16 Sim3 alignments of 640x480 (few points, so
-// the step weighs most): 2105 -> 1386 us.
+// 64 SE3 alignments of 640x480 in one plan: 534 -> 498 us; 24 of 752x478:
+// 408 -> 380 us; three stages of 16 Sim3 alignments of 640x480 (few points, so
+// the step weighs most): 2105 -> 1380 us.
 #pragma once
 #include "batch_internal.h"
 
@@ -188,27 +189,29 @@ __device__ inline void finish_job(JobState& s, int status, int* ntNext, int* rem
   if (remaining && lm_lane() == 0) atomicSub(remaining, 1);
 }
 
-// Solve (A diag*(1+lambda)) inc = b from the stored LGS and propose Tn = exp(inc) T.
-// Returns false when a Sim3 step diverges (|inc|^2 not in [0, 1)).
+// Solve (A diag*(1+lambda)) inc = b and propose Tn = exp(inc) T; lgs holds
+// the upper triangle of A, then b (an evaluation's sums, or the control
+// block's lgs).  Returns false when a Sim3 step diverges (|inc|^2 not in
+// [0, 1)).
 template <int KIND>
-__device__ inline bool solve_and_propose(JobState& __restrict__ s) {
+__device__ inline bool solve_and_propose(JobState& __restrict__ s, const double* __restrict__ lgs, const Pose& T,
+                                         float lambda) {
   constexpr int N = KIND == LSDG_JOB_SIM3 ? 7 : 6;
   constexpr int NA = N * (N + 1) / 2;
   double A[NA], b[N], inc[N];
 #pragma unroll
-  for (int k = 0; k < NA; ++k) A[k] = s.lgsA[k];
+  for (int k = 0; k < NA; ++k) A[k] = lgs[k];
 #pragma unroll
-  for (int a = 0; a < N; ++a) b[a] = -s.lgsB[a];
-  lm_solve<N>(A, b, 1.0 + (double)s.lambda, inc);
-  s.incTry++;
+  for (int a = 0; a < N; ++a) b[a] = -lgs[NA + a];
+  lm_solve<N>(A, b, 1.0 + (double)lambda, inc);
   double dd = 0;
   for (int a = 0; a < N; ++a) dd += inc[a] * inc[a];
   s.incSq = dd;
   if (KIND == LSDG_JOB_SIM3) {
     if (!(dd >= 0 && dd < 1)) return false;
-    s.Tn = lm_pose_mul(lm_sim3_exp(inc), s.T);
+    s.Tn = lm_pose_mul(lm_sim3_exp(inc), T);
   } else {
-    s.Tn = lm_pose_mul(lm_se3_exp(inc), s.T);
+    s.Tn = lm_pose_mul(lm_se3_exp(inc), T);
   }
   s.phase = 1;
   set_eval_pose(s, s.Tn, KIND == LSDG_JOB_SIM3);
@@ -219,19 +222,17 @@ __device__ inline bool solve_and_propose(JobState& __restrict__ s) {
 // accepted pose's normal equations.
 template <int KIND>
 __device__ inline void store_lgs(JobState& __restrict__ s, const double* __restrict__ S) {
-  constexpr int NA = KIND == LSDG_JOB_SIM3 ? 28 : 21, NB = KIND == LSDG_JOB_SIM3 ? 7 : 6;
+  constexpr int NL = KIND == LSDG_JOB_SIM3 ? 35 : 27;
   static_assert(SM_A == 0 && SM_B == 28 && S3_A == 0 && S3_B == 21, "b follows the triangle");
   const int lane = lm_lane();
-  if (lane < NA) s.lgsA[lane] = S[lane];
-  else if (lane < NA + NB) s.lgsB[lane - NA] = S[lane];
-  wave_sync();
+  if (lane < NL) s.lgs[lane] = S[lane];
 }
 
 template <int KIND>
-__device__ inline void begin_level(JobState& s, const JobDesc& jd, const lsdg_params& P, int lvl, int* ntNext,
+__device__ inline void begin_level(JobState& s, const JobDesc& jd, const LmParams& P, int lvl, int* ntNext,
                                    int* remaining) {
   if (KIND == LSDG_JOB_SIM3) {
-    while (lvl >= jd.finalLevel && P.max_its_per_lvl[lvl] == 0) lvl--;
+    while (lvl >= jd.finalLevel && P.lv[lvl].maxIts == 0) lvl--;
   }
   if (lvl < jd.finalLevel) {
     if (KIND == LSDG_JOB_SIM3 && !s.upToDate) {
@@ -255,12 +256,24 @@ __device__ inline void begin_level(JobState& s, const JobDesc& jd, const lsdg_pa
   *ntNext = jd.lv[lvl].ntiles;
 }
 
-// One LM step of an SE3 job, after the evaluation whose sums are S.  The
-// solve has one call site at the end.
+// One LM step of an SE3 job, after the evaluation whose sums are S.  Every
+// value the decision needs is read in one go at the top (an LDS round trip
+// each in the branches would be most of the step), and the accepted
+// evaluation's equations are solved from S itself, not from the copy kept for
+// later rejections.
 __device__ inline void lm_step_se3(JobState& __restrict__ s, const JobDesc& __restrict__ jd,
-                                   const double* __restrict__ S, const lsdg_params& P, int* ntNext, int* remaining) {
-  const int lvl = s.level;
+                                   const double* __restrict__ S, const LmParams& __restrict__ P, int* ntNext,
+                                   int* remaining) {
+  const int lvl = s.level, phase = s.phase, itStart = s.iteration;
   const JobLevel& L = jd.lv[lvl];
+  const double warped = S[S3_WARPED], sumErr = S[S3_ERR], lastErr = s.lastErr, incSq = s.incSq;
+  float lambda = s.lambda;
+  int incTry = s.incTry, iteration = itStart;
+  const LmLevel Q = P.lv[lvl];
+  const int affine = P.affine;
+  const float lim = P.lim * (float)(L.g.w * L.g.h);
+  Pose T = s.T;
+  const Pose Tn = s.Tn;
   s.evals++;
   s.evalsAt[lvl]++;
   s.good = S[S3_GOOD];
@@ -269,48 +282,51 @@ __device__ inline void lm_step_se3(JobState& __restrict__ s, const JobDesc& __re
   s.usageSum = S[S3_USAGE];
   s.usageN = L.pts.n;
   // the affine iterate is read only when the affine brightness is estimated
-  if (P.use_affine_lightning_estimation) {
+  if (affine) {
     const double sxx = S[S3_SXX], syy = S[S3_SYY], sx = S[S3_SX], sy = S[S3_SY], sw = S[S3_SW];
     s.affAIt = (float)sqrt((syy - sy * sy / sw) / (sxx - sx * sx / sw));
     s.affBIt = (float)((sy - (double)s.affAIt * sx) / sw);
   }
-  const float lim = P.min_goodperall_pixel_absmin * (float)(L.g.w * L.g.h);
-  if ((float)S[S3_WARPED] < lim) {
+  if ((float)warped < lim) {
     finish_job(s, 2, ntNext, remaining);
     return;
   }
-  const double err = S[S3_ERR] / S[S3_WARPED];
+  const double err = sumErr / warped;
   s.numRes[lvl]++;
-  bool next = false, keep = true;  // go to the next level; keep this evaluation's LGS
-  if (s.phase == 0) {
-    if (P.use_affine_lightning_estimation) { s.affA = s.affAIt; s.affB = s.affBIt; }
+  bool next = false, keep = true;  // go to the next level; this evaluation's LGS is the accepted pose's
+  if (phase == 0) {
+    if (affine) { s.affA = s.affAIt; s.affB = s.affBIt; }
     s.lastErr = err;
-    s.lambda = P.lambda_initial[lvl];
-    s.iteration = 0;
-    next = P.max_its_per_lvl[lvl] <= 0;
-  } else if (err < s.lastErr) {
-    s.T = s.Tn;
-    if (P.use_affine_lightning_estimation) { s.affA = s.affAIt; s.affB = s.affBIt; }
-    const bool conv = err / s.lastErr > (double)P.convergence_eps[lvl];
+    lambda = Q.lambdaInitial;
+    iteration = 0;
+    next = Q.maxIts <= 0;
+  } else if (err < lastErr) {
+    T = Tn;
+    s.T = Tn;
+    if (affine) { s.affA = s.affAIt; s.affB = s.affBIt; }
+    const bool conv = err / lastErr > Q.convergenceEps;
     s.lastResidual = s.lastErr = err;
-    s.lambda = s.lambda <= 0.2f ? 0.0f : s.lambda * P.lambda_success_fac[lvl];
-    s.iteration++;
-    next = conv || s.iteration >= P.max_its_per_lvl[lvl];
+    lambda = lambda <= 0.2f ? 0.0f : lambda * Q.lambdaSuccess;
+    iteration++;
+    next = conv || iteration >= Q.maxIts;
   } else {
-    next = !(s.incSq > (double)P.step_size_min[lvl]);
+    next = !(incSq > Q.stepSizeMin);
     keep = false;
-    if (!next) s.lambda = s.lambda == 0.0f ? 0.2f : s.lambda * pow_int(P.lambda_fail_fac[lvl], s.incTry);
+    if (!next) lambda = lambda == 0.0f ? 0.2f : lambda * pow_int(Q.lambdaFail, incTry);
   }
+  s.lambda = lambda;
+  s.iteration = iteration;
   if (next) {
     begin_level<LSDG_JOB_SE3>(s, jd, P, lvl - 1, ntNext, remaining);
     return;
   }
   if (keep) {
-    store_lgs<LSDG_JOB_SE3>(s, S);
     s.numWarp[lvl]++;
-    s.incTry = 0;
+    incTry = 0;
   }
-  solve_and_propose<LSDG_JOB_SE3>(s);
+  s.incTry = incTry + 1;
+  solve_and_propose<LSDG_JOB_SE3>(s, keep ? S : s.lgs, T, lambda);
+  if (keep) store_lgs<LSDG_JOB_SE3>(s, S);
   *ntNext = L.ntiles;
 }
 
@@ -326,63 +342,74 @@ __device__ inline void sim3_res(const double* S, double* r) {
   r[6] = (S[SM_RESD] + S[SM_RESP]) / (S[SM_NTD] + S[SM_WARPED]);
 }
 
-// One LM step of a Sim3 job.
+// One LM step of a Sim3 job (see lm_step_se3).
 __device__ inline void lm_step_sim3(JobState& __restrict__ s, const JobDesc& __restrict__ jd,
-                                    const double* __restrict__ S, const lsdg_params& P, int* ntNext, int* remaining) {
-  const int lvl = s.level;
+                                    const double* __restrict__ S, const LmParams& __restrict__ P, int* ntNext,
+                                    int* remaining) {
+  const int lvl = s.level, phase = s.phase;
   const JobLevel& L = jd.lv[lvl];
+  const double warped = S[SM_WARPED], incSq = s.incSq, lastMean = s.lastRes[6];
+  float lambda = s.lambda;
+  int incTry = s.incTry, iteration = s.iteration;
+  const LmLevel Q = P.lv[lvl];
+  const float lim = 0.5f * P.lim * (float)(L.g.w * L.g.h);
+  Pose T = s.T;
+  const Pose Tn = s.Tn;
   s.evals++;
   s.evalsAt[lvl]++;
   s.usageSum = S[SM_USAGE];
   s.usageN = L.pts.n;
-  if (s.phase == 2) {
+  if (phase == 2) {
     // final evaluation for lastSim3Hessian
     sim3_res(S, s.finalRes);
     store_lgs<LSDG_JOB_SIM3>(s, S);
     s.upToDate = 1;
-    finish_job(s, s.T.s <= 0 ? 3 : 1, ntNext, remaining);
+    finish_job(s, T.s <= 0 ? 3 : 1, ntNext, remaining);
     return;
   }
-  const float lim = 0.5f * P.min_goodperall_pixel_absmin * (float)(L.g.w * L.g.h);
-  if ((float)S[SM_WARPED] < lim || S[SM_WARPED] < 10) {
+  if ((float)warped < lim || warped < 10) {
     finish_job(s, 2, ntNext, remaining);
     return;
   }
   double res[7];
   sim3_res(S, res);
   s.numRes[lvl]++;
-  bool keep = true;  // keep this evaluation's LGS
-  if (s.phase == 0) {
+  bool next = false, keep = true;  // go to the next level; this evaluation's LGS is the accepted pose's
+  if (phase == 0) {
     for (int k = 0; k < 7; ++k) s.lastRes[k] = res[k];
-    s.lambda = P.lambda_initial[lvl];
-    s.iteration = 0;
-  } else if (res[6] < s.lastRes[6]) {
-    s.T = s.Tn;
+    lambda = Q.lambdaInitial;
+    iteration = 0;
+  } else if (res[6] < lastMean) {
+    T = Tn;
+    s.T = Tn;
     s.upToDate = 0;
-    const bool conv = res[6] / s.lastRes[6] > (double)P.convergence_eps[lvl];
+    const bool conv = res[6] / lastMean > Q.convergenceEps;
     for (int k = 0; k < 7; ++k) s.finalRes[k] = s.lastRes[k] = res[k];
-    s.lambda = s.lambda <= 0.2f ? 0.0f : s.lambda * P.lambda_success_fac[lvl];
-    s.iteration++;
-    if (conv || s.iteration >= P.max_its_per_lvl[lvl]) {
-      begin_level<LSDG_JOB_SIM3>(s, jd, P, lvl - 1, ntNext, remaining);
-      return;
-    }
+    lambda = lambda <= 0.2f ? 0.0f : lambda * Q.lambdaSuccess;
+    iteration++;
+    next = conv || iteration >= Q.maxIts;
   } else {
-    if (!(s.incSq > (double)P.step_size_min[lvl])) {
-      begin_level<LSDG_JOB_SIM3>(s, jd, P, lvl - 1, ntNext, remaining);
-      return;
-    }
-    s.lambda = s.lambda == 0.0f ? 0.2f : s.lambda * pow_int(P.lambda_fail_fac[lvl], s.incTry);
+    next = !(incSq > Q.stepSizeMin);
     keep = false;
+    if (!next) lambda = lambda == 0.0f ? 0.2f : lambda * pow_int(Q.lambdaFail, incTry);
+  }
+  s.lambda = lambda;
+  s.iteration = iteration;
+  if (next) {
+    begin_level<LSDG_JOB_SIM3>(s, jd, P, lvl - 1, ntNext, remaining);
+    return;
   }
   if (keep) {
-    store_lgs<LSDG_JOB_SIM3>(s, S);
     s.upToDate = 1;
     s.numWarp[lvl]++;
-    s.incTry = 0;
+    incTry = 0;
   }
-  if (!solve_and_propose<LSDG_JOB_SIM3>(s)) {
-    for (int k = 0; k < 28; ++k) s.lgsA[k] = 0.0;
+  s.incTry = incTry + 1;
+  const bool ok = solve_and_propose<LSDG_JOB_SIM3>(s, keep ? S : s.lgs, T, lambda);
+  if (keep) store_lgs<LSDG_JOB_SIM3>(s, S);
+  if (!ok) {
+    wave_sync();
+    for (int k = 0; k < 28; ++k) s.lgs[k] = 0.0;
     finish_job(s, 2, ntNext, remaining);
     return;
   }
@@ -390,7 +417,7 @@ __device__ inline void lm_step_sim3(JobState& __restrict__ s, const JobDesc& __r
 }
 
 // Start state of a job: T = (frameToRef_init)^-1, first level, counters zero.
-__device__ inline void lm_begin(JobState& s, const JobDesc& jd, const lsdg_params& P, int* ntNext, int* remaining) {
+__device__ inline void lm_begin(JobState& s, const JobDesc& jd, const LmParams& P, int* ntNext, int* remaining) {
   s = JobState{};
   s.T = pose_inv(jd.init);
   if (jd.kind == LSDG_JOB_SE3) s.T.s = 1.0;

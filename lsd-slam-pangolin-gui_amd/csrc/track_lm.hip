@@ -12,40 +12,43 @@
 // repeats the same LM step on its own copy of the control block, so an
 // iteration is one evaluation, one exchange and one LM step.
 //
-// 320x240 camera image to pose: 764 -> 269 us; 640x480 through the
-// undistorter: 722 -> 306 us (the launch itself 203 us for 28 evaluations).
+// 320x240 camera image to pose: 685 -> 228 us; 640x480 through the
+// undistorter: 635 -> 260 us (the launch itself about 170 us for 28
+// evaluations: 1.4-2 us of points, 2-2.5 us of exchange and 1.3 us of LM step
+// each).
 //
-// Blocks: about one point per thread of the largest level (the shortest
-// evaluation), at most TRACK_LM_MAX_BLOCKS.  On a small level every block
-// evaluates the whole level itself and nothing is exchanged.  The blocks must
-// be resident together.  They are when the device
+// Blocks: track_lm_blocks.  On a small level every block evaluates the whole
+// level itself and nothing is exchanged.  The blocks must be resident
+// together.  They are when the device
 // has that many free slots (it holds several hundred); other work on it can
 // keep some of them out, so every wait is bounded, the blocks that waited in
 // vain stop, and the caller runs the alignment launch by launch instead.
+#include <cmath>
+
 #include "lm_device.h"
 #include "track_device.h"
 
 namespace lsdg {
 
-#ifndef LSDG_TRACK_SOLO
-#define LSDG_TRACK_SOLO 1024
-#endif
 constexpr int TRACK_LM_BS = 256;
 constexpr int TRACK_LM_WAVES = TRACK_LM_BS / 64;
-// Levels of at most this many points are evaluated whole by every block: four
-// points per thread cost less than an exchange.
-constexpr int TRACK_LM_SOLO = LSDG_TRACK_SOLO;
+// Levels of at most this many points are evaluated whole by every block: two
+// points per thread cost less than an exchange (320x240: 162 us per alignment,
+// with 1024 points 169).
+constexpr int TRACK_LM_SOLO = 512;
 
 template <int KIND, int PREC, int ACC>
 __global__ __launch_bounds__(TRACK_LM_BS) void k_track_lm(TrackLmArgs a) {
   constexpr int NS = KIND == LSDG_JOB_SIM3 ? NS_SIM3 : NS_SE3;
   __shared__ JobState s;
   __shared__ JobDesc jd;
+  __shared__ LmParams sP;
   __shared__ double sh[TRACK_LM_WAVES][NS];
   __shared__ double S[NS];
   __shared__ int failed;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, part = blockIdx.x;
   block_copy(&jd, &a.jd, TRACK_LM_BS);
+  block_copy(&sP, &a.P, TRACK_LM_BS);
   if (tid == 0) failed = 0;
   __syncthreads();
   if (tid < 64) {
@@ -53,7 +56,7 @@ __global__ __launch_bounds__(TRACK_LM_BS) void k_track_lm(TrackLmArgs a) {
     if (tid < PYR) jd.lv[tid].pts.n = a.counts[tid];
     wave_sync();
     int nt = 0;
-    lm_begin(s, jd, a.P, &nt, nullptr);
+    lm_begin(s, jd, sP, &nt, nullptr);
     wave_sync();
     if (tid < PYR) s.npts[tid] = jd.lv[tid].pts.n;
   }
@@ -137,8 +140,8 @@ __global__ __launch_bounds__(TRACK_LM_BS) void k_track_lm(TrackLmArgs a) {
     }
     if (tid < 64) {
       int next = 0;
-      if (KIND == LSDG_JOB_SIM3) lm_step_sim3(s, jd, S, a.P, &next, nullptr);
-      else lm_step_se3(s, jd, S, a.P, &next, nullptr);
+      if (KIND == LSDG_JOB_SIM3) lm_step_sim3(s, jd, S, sP, &next, nullptr);
+      else lm_step_se3(s, jd, S, sP, &next, nullptr);
     }
     __syncthreads();
   }
@@ -154,10 +157,14 @@ __global__ __launch_bounds__(256) void k_track_lm_clear(unsigned long long* rows
 }
 
 int track_lm_blocks(lsdg_ctx c, int pixels) {
-  // a quarter of the pixels is what a semi-dense map holds; the size alone
-  // decides, so that an image's result does not depend on what the host knows
-  const int nb = (pixels / 4 + TRACK_LM_BS - 1) / TRACK_LM_BS;
-  return std::max(1, std::min(nb, std::min(TRACK_LM_MAX_BLOCKS, c->num_cus)));
+  // An evaluation shortens with the blocks, an exchange grows with them: the
+  // best number goes with the square root of the points.  Measured per
+  // alignment (FP32): 320x240 162 us with 16 blocks, 168 with 32, 187 with 64;
+  // 640x480 175, 171, 187; 1280x960 224, 179, 172; 1920x1080 (FP16) 292, 210,
+  // 189.  The size alone decides, so that an image's result does not depend on
+  // whether the host knows the count of points yet.
+  const int nb = ((int)(std::sqrt((double)pixels) / 9.0) + 4) / 8 * 8;
+  return std::max(1, std::min(std::max(nb, 8), std::min(TRACK_LM_MAX_BLOCKS, c->num_cus)));
 }
 
 template <int KIND, int PREC>
