@@ -243,6 +243,7 @@ lsdg_status lsdg::frame_alloc(lsdg_ctx c, int32_t id, const lsdg_camera* cam, in
     off[l][5] = take(n * 4);
   }
   size_t off_u8 = take((size_t)f->w[0] * f->h[0]);
+  size_t off_quad = take((size_t)f->w[0] * f->h[0] * 4);
   size_t off_wg = take((size_t)f->w[1] * f->h[1]);
   hipError_t e = hipMalloc(&f->d_pool, total);
   if (e != hipSuccess) {
@@ -259,6 +260,7 @@ lsdg_status lsdg::frame_alloc(lsdg_ctx c, int32_t id, const lsdg_camera* cam, in
     f->d_ivar[l] = (float*)(b + off[l][5]);
   }
   f->d_input_u8 = (uint8_t*)(b + off_u8);
+  f->d_quad = (uint32_t*)(b + off_quad);
   f->d_wasGood = (uint8_t*)(b + off_wg);
   *out = f;
   return LSDG_OK;
@@ -308,7 +310,7 @@ lsdg_status lsdg::frame_require(lsdg_frame f, unsigned need) {
   bool buildImages = (f->valid & images) != images && (miss & ~level0) != 0;
   unsigned grads = miss & derived;
   ProfMark pm = prof_begin(c, LSDG_KERNEL_PYRAMID);
-  if (buildImages) CK(c, launch_pyr_images(f, false, c->stream));
+  if (buildImages) CK(c, launch_pyr_images(f, c->stream));
   if (grads) CK(c, launch_pyr_grads(f, grads, c->stream));
   prof_end(c, pm, pyramid_bytes(f, buildImages, grads));
   f->valid |= (buildImages ? images : 0u) | grads;
@@ -363,7 +365,7 @@ extern "C" lsdg_status lsdg_frame_create_u8(lsdg_ctx c, int32_t id, const lsdg_c
   if (e == hipSuccess) {
     // the image stage converts level 0 and builds levels 1-4; the rest is built on first use
     ProfMark pm = prof_begin(c, LSDG_KERNEL_PYRAMID);
-    e = launch_pyr_images(f, true, c->stream);
+    e = launch_pyr_images_u8(f, c->stream);
     prof_end(c, pm, pyramid_bytes(f, true, 0));
     if (e == hipSuccess) {
       f->valid = fd_levels(FD_IMAGE, 0, PYR - 1);

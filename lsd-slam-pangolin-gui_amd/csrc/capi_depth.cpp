@@ -261,12 +261,16 @@ extern "C" lsdg_status lsdg_depth_update(lsdg_depthmap dm, const lsdg_frame* ref
   lsdg_status st = ensure_ref_storage(dm, n, (int)byId.size() + 1);
   if (st != LSDG_OK) return st;
   CK(c, hipStreamSynchronize(c->stream));  // staging buffers are free
+  // the packed images the search samples when every frame came in as 8-bit
+  bool q8 = kf->u8Level0;
+  for (int i = 0; i < n; ++i) q8 = q8 && refs[i]->u8Level0;
   for (int i = 0; i < n; ++i) {
     lsdg_frame f = refs[i];
     Pose refToKf = (f->parentId == kf->id) ? f->thisToParent : pose_mul(pose_inv(kf->camToWorld), f->camToWorld);
     StereoRef& r = dm->h_refs[i];
     prepare_stereo(dm->g, refToKf, r);
     r.img = f->d_image[0];
+    r.quad = q8 ? f->d_quad : nullptr;
     r.wasGood = (f->parentId == kf->id && f->wasGoodAllocated) ? f->d_wasGood : nullptr;
     r.initialTrackedResidual = f->initialTrackedResidual;
     r.id = f->id;

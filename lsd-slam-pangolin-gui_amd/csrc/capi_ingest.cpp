@@ -169,6 +169,7 @@ extern "C" lsdg_status lsdg_frame_ingest(lsdg_frame f, int32_t id, lsdg_undistor
     fresh.d_ivar[l] = f->d_ivar[l];
   }
   fresh.d_input_u8 = f->d_input_u8;
+  fresh.d_quad = f->d_quad;
   fresh.d_wasGood = f->d_wasGood;
   fresh.depthVersion = f->depthVersion + 1;
   *f = fresh;

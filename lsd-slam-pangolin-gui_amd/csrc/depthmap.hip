@@ -53,38 +53,82 @@ __device__ inline float2 dinterp42(const float4* __restrict__ g, float x, float 
   return make_float2(w11 * a.x + w01 * b.x + w10 * c.x + w00 * d.x, w11 * a.y + w01 * b.y + w10 * c.y + w00 * d.y);
 }
 
-// The four texels dinterp reads at (x, y), as two 8-byte loads; the index is
-// clamped to the image so that positions outside it (never blended) stay in
-// bounds, and is unchanged for every position dinterp may read.
-// The image pointer reaches the kernel through device memory (a reference
-// frame's descriptor), so it is cast to the global address space: generic
-// (flat) loads would make every wait drain all outstanding loads.
+// The images the epipolar search samples, in one of two forms.
+//
+// Float: the four texels dinterp reads at (x, y), as two 8-byte loads.
+//
+// Packed (Q8): an image that came in as 8-bit, with the four bytes of every
+// 2x2 neighbourhood in one word (pack_quad), so a sample is one 4-byte
+// load.  The lanes of a wave search different lines, so each load of a step
+// touches up to 64 cache lines: the search is bound by how many lines a CU's
+// L1 can serve, and one load of four bytes in the place of two of eight takes
+// half the lookups and leaves a line's pixels four times as likely to be
+// there.  The bytes convert to the floats the image level holds, so the
+// samples are the same bit for bit.  640x480, references at a random map
+// (lanes' lines scattered): 33.7 -> 18.7 us for the pass; a settled map
+// (neighbouring lines), bound by VALU issue, keeps its 16.4 us; searches up to
+// 100 px 31.6 -> 29 us.
+//
+// Indexes are clamped to the image so that positions outside it (never
+// blended) stay in bounds, and are unchanged for every position dinterp may
+// read.  The image pointers reach the kernel through device memory (a
+// reference frame's descriptor), so they are cast to the global address
+// space: generic (flat) loads would make every wait drain all outstanding
+// loads.
 typedef float Texel2 __attribute__((ext_vector_type(2), aligned(4)));
 typedef __attribute__((address_space(1))) const Texel2* GlobalTexel2;
+typedef __attribute__((address_space(1))) const uint32_t* GlobalWord;
 struct Quad {
   Texel2 t, b;  // (I(ix, iy), I(ix + 1, iy)), (I(ix, iy + 1), I(ix + 1, iy + 1))
 };
-__device__ inline Quad fetch_quad(const float* __restrict__ m, float x, float y, int w, int h) {
-  // the linear index, clamped to [0, w (h - 1) - 2]: unchanged for
-  // 0 <= ix <= w - 2, 0 <= iy <= h - 2 (every blended position; sizes are
-  // at most 16384, so the 24-bit product is exact there), and byte offsets
-  // in 32 bits (an image is far below 4 GiB)
+struct Quad8 {
+  uint32_t w;  // the same four, one byte each, I(ix, iy) lowest
+};
+template <bool Q8>
+struct TexImg {
+  using Q = Quad;
+  const float* p;
+};
+template <>
+struct TexImg<true> {
+  using Q = Quad8;
+  const uint32_t* p;
+};
+
+// The linear index, clamped to [0, w (h - 1) - 2]: unchanged for
+// 0 <= ix <= w - 2, 0 <= iy <= h - 2 (every blended position; sizes are at
+// most 16384, so the 24-bit product is exact there), and byte offsets in 32
+// bits (an image is far below 4 GiB).
+__device__ inline unsigned quad_index(float x, float y, int w, int h) {
   const unsigned lin = (unsigned)(int)x + __umul24((unsigned)(int)y, (unsigned)w);
-  const unsigned off = (unsigned)min(max((int)lin, 0), w * (h - 1) - 2);
-  const char* base = (const char*)m;
-  const unsigned top = off * 4u, bottom = top + (unsigned)w * 4u;
+  return (unsigned)min(max((int)lin, 0), w * (h - 1) - 2);
+}
+__device__ inline Quad fetch_quad(const TexImg<false>& m, float x, float y, int w, int h) {
+  const char* base = (const char*)m.p;
+  const unsigned top = quad_index(x, y, w, h) * 4u, bottom = top + (unsigned)w * 4u;
   Quad q;
   q.t = *(GlobalTexel2)(base + top);
   q.b = *(GlobalTexel2)(base + bottom);
   return q;
 }
+__device__ inline Quad8 fetch_quad(const TexImg<true>& m, float x, float y, int w, int h) {
+  return Quad8{*(GlobalWord)((const char*)m.p + quad_index(x, y, w, h) * 4u)};
+}
 // dinterp's bilinear blend of fetched texels (same expression and order).
-__device__ inline float blend_quad(const Quad& q, float x, float y) {
+__device__ inline float blend(float t0, float t1, float b0, float b1, float x, float y) {
   // truncf(x) == (float)(int)x over the int range
   float dx = x - truncf(x), dy = y - truncf(y);
   float dxdy = dx * dy;
-  return dxdy * q.b.y + (dy - dxdy) * q.b.x + (dx - dxdy) * q.t.y + (1.0f - dx - dy + dxdy) * q.t.x;
+  return dxdy * b1 + (dy - dxdy) * b0 + (dx - dxdy) * t1 + (1.0f - dx - dy + dxdy) * t0;
 }
+__device__ inline float blend_quad(const Quad& q, float x, float y) { return blend(q.t.x, q.t.y, q.b.x, q.b.y, x, y); }
+__device__ inline float blend_quad(const Quad8& q, float x, float y) {
+  return blend((float)(q.w & 0xffu), (float)((q.w >> 8) & 0xffu), (float)((q.w >> 16) & 0xffu), (float)(q.w >> 24), x, y);
+}
+// Takes the fetched value here, so that its load is not deferred past this
+// point.
+__device__ inline void hold(const Quad& q) { asm volatile("" ::"v"(q.t.x), "v"(q.t.y), "v"(q.b.x), "v"(q.b.y)); }
+__device__ inline void hold(const Quad8& q) { asm volatile("" ::"v"(q.w)); }
 
 // The quad fetch through a buffer resource over an image that is the same
 // for the whole wave.  The hardware's range check returns zeros for byte
@@ -95,16 +139,22 @@ struct TexBuf {
   __amdgpu_buffer_rsrc_t r;
   unsigned rowBytes;
 };
-__device__ inline TexBuf tex_buf(const float* img, int w, int h) {
+template <bool Q8>
+__device__ inline TexBuf tex_buf(const TexImg<Q8>& img, int w, int h) {
   // word 3 of the descriptor: 32-bit data format, as for any raw access
-  return TexBuf{__builtin_amdgcn_make_buffer_rsrc((void*)img, (short)0, w * h * 4, 0x00020000), (unsigned)w * 4u};
+  return TexBuf{__builtin_amdgcn_make_buffer_rsrc((void*)img.p, (short)0, w * h * 4, 0x00020000), (unsigned)w * 4u};
 }
-__device__ inline Quad fetch_quad(const TexBuf& b, float x, float y, int w) {
+template <bool Q8>
+__device__ inline typename TexImg<Q8>::Q fetch_quad_buf(const TexBuf& b, float x, float y, int w) {
   const unsigned top = ((unsigned)(int)x + __umul24((unsigned)(int)y, (unsigned)w)) * 4u;
-  Quad q;
-  q.t = __builtin_bit_cast(Texel2, __builtin_amdgcn_raw_buffer_load_b64(b.r, top, 0, 0));
-  q.b = __builtin_bit_cast(Texel2, __builtin_amdgcn_raw_buffer_load_b64(b.r, top + b.rowBytes, 0, 0));
-  return q;
+  if constexpr (Q8) {
+    return Quad8{__builtin_amdgcn_raw_buffer_load_b32(b.r, top, 0, 0)};
+  } else {
+    Quad q;
+    q.t = __builtin_bit_cast(Texel2, __builtin_amdgcn_raw_buffer_load_b64(b.r, top, 0, 0));
+    q.b = __builtin_bit_cast(Texel2, __builtin_amdgcn_raw_buffer_load_b64(b.r, top + b.rowBytes, 0, 0));
+    return q;
+  }
 }
 
 #ifndef LSDG_STEREO_AHEAD
@@ -158,11 +208,17 @@ __device__ inline Hyp make_hyp(float id, float var, int val) {
 }
 
 // ------------------------------------------------------------ stereo
+template <bool Q8>
 struct ObsCtx {
   DepthGeom g;
-  const float* kfImg;
+  TexImg<Q8> kf;
   const float4* kfGrad;
 };
+template <bool Q8>
+__device__ inline TexImg<Q8> ref_tex(const StereoRef& r) {
+  if constexpr (Q8) return TexImg<true>{r.quad};
+  else return TexImg<false>{r.img};
+}
 
 // gx, gy: the keyframe image's central differences at (x, y),
 // I(x+1, y) - I(x-1, y) and I(x, y+1) - I(x, y-1).
@@ -224,8 +280,8 @@ __device__ inline void walk(float& x, float& y, int& j, int to, float ix, float 
 // one round trip to memory, not N.  With bx set, (*bx, *by) receives
 // cp_{m0+N-4}: the position of the step whose newest sample is V_{m0+N-2}.
 // Fetches for m <= 1 are clamped to the image and not used.
-template <int N>
-__device__ inline void window_samples(const float* __restrict__ img, int w, int h, float ix, float iy, int m0,
+template <int N, class IMG>
+__device__ inline void window_samples(const IMG& img, int w, int h, float ix, float iy, int m0,
                                       float i_m2, float i_m1, float i_0, float i_p1, float* out, float& x, float& y,
                                       int& j, float* bx = nullptr, float* by = nullptr) {
   float sx[N], sy[N];
@@ -239,13 +295,13 @@ __device__ inline void window_samples(const float* __restrict__ img, int w, int 
       *by = y;
     }
   }
-  Quad q[N];
+  typename IMG::Q q[N];
 #pragma unroll
   for (int t = 0; t < N; ++t) q[t] = fetch_quad(img, sx[t], sy[t], w, h);
   // every fetch's value is taken here, so none is deferred into the
   // per-sample selects below (one wait for all N, not one per branch)
 #pragma unroll
-  for (int t = 0; t < N; ++t) asm volatile("" ::"v"(q[t].t.x), "v"(q[t].t.y), "v"(q[t].b.x), "v"(q[t].b.y));
+  for (int t = 0; t < N; ++t) hold(q[t]);
 #pragma unroll
   for (int t = 0; t < N; ++t) {
     const int m = m0 + t;
@@ -279,13 +335,13 @@ __device__ inline float stereo_dot(const float* a, const float* b) {
 // doLineStereo: the matching error (>= 0) or a code -1..-4.  With UNI the
 // reference image is the same for the whole wave and the search loop fetches
 // through a buffer resource.
-template <bool UNI>
-__device__ float line_stereo(const ObsCtx& o, const lsdg_params& P, float u, float v, float epxn, float epyn,
+template <bool UNI, bool Q8>
+__device__ float line_stereo(const ObsCtx<Q8>& o, const lsdg_params& P, float u, float v, float epxn, float epyn,
                              float min_idepth, float prior_idepth, float max_idepth, const StereoRef& ref,
                              float& r_idepth, float& r_var, float& r_epl) {
   const int width = o.g.w, height = o.g.h;
-  const float* kfImg = o.kfImg;
-  const float* refImg = ref.img;
+  using Q = typename TexImg<Q8>::Q;
+  const TexImg<Q8> refImg = ref_tex<Q8>(ref);
   float KinvP[3] = {o.g.fxi * u + o.g.cxi, o.g.fyi * v + o.g.cyi, 1.0f};
   float pInf[3];
 #pragma unroll
@@ -298,11 +354,12 @@ __device__ float line_stereo(const ObsCtx& o, const lsdg_params& P, float u, flo
       lastX <= 0.0f || lastX >= (float)(width - 2) || lastY <= 0.0f || lastY >= (float)(height - 2))
     return -1.0f;
   if (!(rescale > 0.7f && rescale < 1.4f)) return -1.0f;
-  float rv_p1 = dinterp(kfImg, u + epxn * rescale, v + epyn * rescale, width);
-  float rv_m1 = dinterp(kfImg, u - epxn * rescale, v - epyn * rescale, width);
-  float rv = dinterp(kfImg, u, v, width);
-  float rv_m2 = dinterp(kfImg, u - 2.0f * epxn * rescale, v - 2.0f * epyn * rescale, width);
-  float rv_p2 = dinterp(kfImg, u + 2.0f * epxn * rescale, v + 2.0f * epyn * rescale, width);
+  const auto kf_at = [&](float x, float y) { return blend_quad(fetch_quad(o.kf, x, y, width, height), x, y); };
+  const float rv_p1 = kf_at(u + epxn * rescale, v + epyn * rescale);
+  const float rv_m1 = kf_at(u - epxn * rescale, v - epyn * rescale);
+  const float rv = kf_at(u, v);
+  const float rv_m2 = kf_at(firstX, firstY);
+  const float rv_p2 = kf_at(lastX, lastY);
 
   float pClose[3], pFar[3];
 #pragma unroll
@@ -385,10 +442,11 @@ __device__ float line_stereo(const ObsCtx& o, const lsdg_params& P, float u, flo
   // additions gives again (walk), so they equal what the reference's loop
   // records when it meets the best.
   const float cp0x = pFar[0], cp0y = pFar[1];
-  const float init_m2 = dinterp(refImg, cp0x - 2.0f * incx, cp0y - 2.0f * incy, width);
-  const float init_m1 = dinterp(refImg, cp0x - incx, cp0y - incy, width);
-  const float init_0 = dinterp(refImg, cp0x, cp0y, width);
-  const float init_p1 = dinterp(refImg, cp0x + incx, cp0y + incy, width);
+  const auto ref_at = [&](float x, float y) { return blend_quad(fetch_quad(refImg, x, y, width, height), x, y); };
+  const float init_m2 = ref_at(cp0x - 2.0f * incx, cp0y - 2.0f * incy);
+  const float init_m1 = ref_at(cp0x - incx, cp0y - incy);
+  const float init_0 = ref_at(cp0x, cp0y);
+  const float init_p1 = ref_at(cp0x + incx, cp0y + incy);
   const int maxSteps = P.stereo_max_steps;
   const bool negx = incx < 0.0f, negy = incy < 0.0f;
   const float closeX = pClose[0], closeY = pClose[1];
@@ -413,16 +471,16 @@ __device__ float line_stereo(const ObsCtx& o, const lsdg_params& P, float u, flo
   asm("v_mov_b32 %0, %1" : "=v"(stepLimit) : "s"(maxSteps));
   {
     float lx = cpx, ly = cpy;
-    const TexBuf tb = tex_buf(refImg, width, height);
-    const auto ring_fetch = [&](float fx, float fy) {
-      if constexpr (UNI) return fetch_quad(tb, fx, fy, width);
+    const TexBuf tb = tex_buf<Q8>(refImg, width, height);
+    const auto ring_fetch = [&](float fx, float fy) -> Q {
+      if constexpr (UNI) return fetch_quad_buf<Q8>(tb, fx, fy, width);
       else return fetch_quad(refImg, fx, fy, width, height);
     };
     // The texels of the next STEREO_AHEAD steps' samples are in flight
     // while a step is evaluated: a lead copy of the position chain fetches
     // each sample STEREO_AHEAD steps early.  Lead fetches past the line's
     // end are clamped to the image and never used.
-    Quad ring[STEREO_AHEAD];
+    Q ring[STEREO_AHEAD];
 #pragma unroll
     for (int k = 0; k < STEREO_AHEAD; ++k) {
       ring[k] = ring_fetch(lx + 2.0f * incx, ly + 2.0f * incy);
@@ -584,6 +642,7 @@ struct ObsArgs {
   HypBuf cur;
   uint8_t* obs;
   const float* kfImg;
+  const uint32_t* kfQuad;  // its packed form, when every frame of the update has one
   const float* kfMaxg;
   const float4* kfGrad;
   const StereoRef* refs;  // device copies when not inline
@@ -786,7 +845,13 @@ constexpr int STEREO_MIN_BLOCKS = LSDG_STEREO_MIN_BLOCKS;
 
 // observeDepthCreate item `i` of segment `seg`; creates search the whole
 // inverse-depth range, so their lines are long.
-template <bool INL>
+template <bool Q8>
+__device__ inline ObsCtx<Q8> obs_ctx(const ObsArgs& a) {
+  if constexpr (Q8) return ObsCtx<Q8>{a.g, TexImg<true>{a.kfQuad}, a.kfGrad};
+  else return ObsCtx<Q8>{a.g, TexImg<false>{a.kfImg}, a.kfGrad};
+}
+
+template <bool INL, bool Q8>
 __device__ inline void observe_create(const ObsArgs& a, const lsdg_params& P, const int4* __restrict__ work,
                                       int segcap, int seg, int i) {
   const int4 item = work[(size_t)seg * segcap + i];
@@ -796,10 +861,10 @@ __device__ inline void observe_create(const ObsArgs& a, const lsdg_params& P, co
   // every create searches the same frame (item.y holds this index): read
   // as a launch-uniform value its image pointer and products stay scalar
   const StereoRef& ref = obs_ref<INL>(a, a.kfReactivated ? a.newestIdx : a.oldestIdx);
-  ObsCtx o{a.g, a.kfImg, a.kfGrad};
+  const ObsCtx<Q8> o = obs_ctx<Q8>(a);
   float rid, rvar, repl;
   float err =
-      line_stereo<true>(o, P, (float)x, (float)y, epx, epy, 0.0f, 1.0f, 1.0f / P.min_depth, ref, rid, rvar, repl);
+      line_stereo<true, Q8>(o, P, (float)x, (float)y, epx, epy, 0.0f, 1.0f, 1.0f / P.min_depth, ref, rid, rvar, repl);
   uint8_t code;
   if (err == -3.0f || err == -2.0f) a.cur.bl[idx] = a.cur.bl[idx] - 1;
   if (err < 0.0f) {
@@ -816,7 +881,7 @@ __device__ inline void observe_create(const ObsArgs& a, const lsdg_params& P, co
 
 // observeDepthUpdate item `i` of segment `seg` (slot segcap - 1 - i), one
 // lane (short lines around the prior).
-template <bool INL>
+template <bool INL, bool Q8>
 __device__ inline void observe_update(const ObsArgs& a, const lsdg_params& P, const int4* __restrict__ work,
                                       int segcap, int seg, int i) {
   const int4 item = work[(size_t)seg * segcap + segcap - 1 - i];
@@ -824,7 +889,7 @@ __device__ inline void observe_update(const ObsArgs& a, const lsdg_params& P, co
   const int idx = item.x, x = idx % w, y = idx / w;
   const float epx = __int_as_float(item.z), epy = __int_as_float(item.w);
   const StereoRef& ref = obs_ref<INL>(a, item.y);
-  ObsCtx o{a.g, a.kfImg, a.kfGrad};
+  const ObsCtx<Q8> o = obs_ctx<Q8>(a);
   uint8_t code;
   // observeDepthUpdate
   Hyp t = load_hyp(a.cur, idx);
@@ -834,7 +899,7 @@ __device__ inline void observe_update(const ObsArgs& a, const lsdg_params& P, co
   if (min_id < 0.0f) min_id = 0.0f;
   if (max_id > 1.0f / P.min_depth) max_id = 1.0f / P.min_depth;
   float rid = 0.0f, rvar = 0.0f, repl = 0.0f;
-  float err = line_stereo<false>(o, P, (float)x, (float)y, epx, epy, min_id, t.dv.z, max_id, ref, rid, rvar, repl);
+  float err = line_stereo<false, Q8>(o, P, (float)x, (float)y, epx, epy, min_id, t.dv.z, max_id, ref, rid, rvar, repl);
   float diff = rid - t.dv.z;
   if (err == -1.0f) {
     code = LSDG_OBS_STEREO_FAIL_BASE + 1;
@@ -895,7 +960,7 @@ __device__ inline void observe_update(const ObsArgs& a, const lsdg_params& P, co
 // first create chunks, round 1 the rest of the creates and then updates, and
 // round 2 updates only on the CUs whose round-1 block took none of the
 // creates.  Later chunks go to every wave in turn.
-template <bool INL>
+template <bool INL, bool Q8>
 __global__ __launch_bounds__(256, STEREO_MIN_BLOCKS) void k_observe_stereo(ObsArgs a, lsdg_params P, const int4* __restrict__ work,
                                                         const int* __restrict__ count, int segcap, int simds) {
   const int lane = (int)(threadIdx.x & 63);
@@ -940,7 +1005,7 @@ __global__ __launch_bounds__(256, STEREO_MIN_BLOCKS) void k_observe_stereo(ObsAr
           seg += below ? 1 : 0;
           base = below ? cpre[t] : base;
         }
-        observe_create<INL>(a, P, work, segcap, seg, vi - base);
+        observe_create<INL, Q8>(a, P, work, segcap, seg, vi - base);
       }
     } else {
       const int u = c - nCreateChunks;
@@ -951,7 +1016,7 @@ __global__ __launch_bounds__(256, STEREO_MIN_BLOCKS) void k_observe_stereo(ObsAr
       const int q = u - (seg > 0 ? __shfl(pre, OBS_SEGS + seg - 1, 64) : 0);
       const int n = __shfl(nItems, OBS_SEGS + seg, 64);
       const int i = q * 64 + lane;
-      if (i < n) observe_update<INL>(a, P, work, segcap, seg, i);
+      if (i < n) observe_update<INL, Q8>(a, P, work, segcap, seg, i);
     }
   }
 }
@@ -1595,6 +1660,9 @@ hipError_t launch_observe(lsdg_depthmap dm, const lsdg_params& P, const StereoRe
   a.obs = dm->d_obs;
   lsdg_frame kf = dm->kf;
   a.kfImg = kf->d_image[0];
+  bool q8 = kf->u8Level0;
+  for (int i = 0; i < nRefs; ++i) q8 = q8 && h_refs[i].quad != nullptr;
+  a.kfQuad = q8 ? kf->d_quad : nullptr;
   a.kfMaxg = kf->d_maxg[0];
   a.kfGrad = kf->d_grad[0];
   a.nRefById = nRefById;
@@ -1630,11 +1698,12 @@ hipError_t launch_observe(lsdg_depthmap dm, const lsdg_params& P, const StereoRe
   dm->obsParity ^= 1;
   // stereo grid: the blocks the device holds at once, at most one wave per
   // chunk the lists can hold
-  int& resident = dm->stereoBlocks[inl ? 0 : 1];
+  auto stereo = inl ? (q8 ? k_observe_stereo<true, true> : k_observe_stereo<true, false>)
+                    : (q8 ? k_observe_stereo<false, true> : k_observe_stereo<false, false>);
+  int& resident = dm->stereoBlocks[(inl ? 0 : 1) + (q8 ? 2 : 0)];
   if (resident == 0) {
     int perCU = 0;
-    e = inl ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, k_observe_stereo<true>, 256, 0)
-            : hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, k_observe_stereo<false>, 256, 0);
+    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, stereo, 256, 0);
     if (e != hipSuccess) return e;
     resident = perCU > 0 ? perCU * dm->ctx->num_cus : 1;
   }
@@ -1643,11 +1712,10 @@ hipError_t launch_observe(lsdg_depthmap dm, const lsdg_params& P, const StereoRe
   const dim3 gs((unsigned)std::min<long long>(resident, (maxChunks + 3) / 4));
   if (inl) {
     k_observe_gate<true><<<gg, dim3(256), 0, s>>>(a, P, dm->d_work, count, other, segcap);
-    k_observe_stereo<true><<<gs, dim3(256), 0, s>>>(a, P, dm->d_work, count, segcap, simds);
   } else {
     k_observe_gate<false><<<gg, dim3(256), 0, s>>>(a, P, dm->d_work, count, other, segcap);
-    k_observe_stereo<false><<<gs, dim3(256), 0, s>>>(a, P, dm->d_work, count, segcap, simds);
   }
+  stereo<<<gs, dim3(256), 0, s>>>(a, P, dm->d_work, count, segcap, simds);
   return hipGetLastError();
 }
 

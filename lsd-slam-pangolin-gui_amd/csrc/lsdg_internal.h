@@ -84,6 +84,7 @@ struct HypBuf {
 // Frame::prepareForStereoWith products of one reference frame, FP32.
 struct StereoRef {
   const float* img;
+  const uint32_t* quad;    // packed 8-bit form, null when the image is not 8-bit
   const uint8_t* wasGood;  // refPixelWasGood gate, null when not tracked on the keyframe
   float KR[9];             // K_otherToThis_R
   float Kt[3];             // K_otherToThis_t
@@ -284,7 +285,8 @@ struct lsdg_frame_s {
   float* d_idepth[lsdg::PYR];
   float* d_ivar[lsdg::PYR];
   uint8_t* d_input_u8 = nullptr;  // staging for u8 uploads (w*h)
-  bool u8Level0 = false;          // d_input_u8 holds level 0 (every level-0 writer keeps it so)
+  uint32_t* d_quad = nullptr;     // per pixel, the four bytes of the 2x2 pixels to its right and below
+  bool u8Level0 = false;          // d_input_u8 and d_quad hold level 0 (every level-0 writer keeps it so)
   uint8_t* d_wasGood = nullptr;   // refPixelWasGood (level 1)
   unsigned valid = 0;             // built pyramid data (fd_bit flags)
   bool wasGoodAllocated = false;
@@ -335,7 +337,7 @@ struct lsdg_depthmap_s {
   int4* d_work = nullptr;    // epipolar-search work items, one slot per pixel
   int* d_work_count = nullptr;  // two sets of per-segment (create, update) item counters
   int obsParity = 0;            // counter set of the next observe pass
-  int stereoBlocks[2] = {0, 0};  // resident blocks of the stereo pass (refs inline, in memory), 0 = not yet queried
+  int stereoBlocks[4] = {0, 0, 0, 0};  // resident blocks of the stereo pass (refs inline or not, then packed), 0 = not yet queried
   lsdg::StereoRef* h_refs = nullptr;  // pinned staging
   int* h_refById = nullptr;
   // propagation scratch
@@ -356,13 +358,15 @@ struct lsdg_depthmap_s {
 namespace lsdg {
 
 // pyramid.hip
-// image pyramid of f: with fromU8, level 0 converted from the 8-bit staging
-// and levels 1-4; otherwise levels 1-4 from level 0 (read from the 8-bit
-// copy when it still holds level 0)
-hipError_t launch_pyr_images(lsdg_frame f, bool fromU8, hipStream_t s);
+// levels 1-4 of f's image from level 0 (read from the 8-bit copy when it
+// holds level 0)
+hipError_t launch_pyr_images(lsdg_frame f, hipStream_t s);
+// level 0 and its packed form from the 8-bit image uploaded to d_input_u8,
+// and levels 1-4
+hipError_t launch_pyr_images_u8(lsdg_frame f, hipStream_t s);
 // undistorts the 8-bit image d_src (row length inW) through the table d_map
 // (one source position per level-0 pixel) into f's level 0, builds levels
-// 1-4, and writes the 8-bit undistorted image to d_undist unless it is null
+// 1-4, and writes the 8-bit undistorted image to d_undist
 hipError_t launch_ingest(lsdg_frame f, const uint8_t* d_src, int inW, const float2* d_map, uint8_t* d_undist,
                          hipStream_t s);
 // Gradients / packed copies / max-gradients of the levels named in `need`
