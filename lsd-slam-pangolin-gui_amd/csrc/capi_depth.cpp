@@ -48,7 +48,6 @@ extern "C" lsdg_status lsdg_depthmap_create(lsdg_ctx c, const lsdg_camera* cam, 
   g.cxi = -g.cx / g.fx;
   g.cyi = -g.cy / g.fy;
   const size_t n = (size_t)g.w * g.h;
-  const size_t nb = (n + 255) / 256;
   size_t total = 0;
   auto take = [&](size_t bytes) {
     size_t o = total;
@@ -63,9 +62,8 @@ extern "C" lsdg_status lsdg_depthmap_create(lsdg_ctx c, const lsdg_camera* cam, 
     ob[k][3] = take(n * 4);
     ob[k][4] = take(n * 16);
   }
-  size_t o_obs = take(n), o_dest = take(n * 4), o_iv = take(n * 8), o_cnt = take((n + 1) * 4),
-         o_fill = take(n * 4), o_bucket = take(n * 4), o_blk = take((nb + 1) * 4), o_red = take(2 * 1024 * 8),
-         o_rc = take(64), o_work = take(obs_work_slots(g.w, g.h) * 16),
+  size_t o_obs = take(n), o_iv = take(n * 8), o_head = take(n * 4), o_next = take(n * 4),
+         o_mean = take(mean_rows(g.w, g.h) * sizeof(double2)), o_work = take(obs_work_slots(g.w, g.h) * 16),
          o_wc = take(OBS_COUNT_BYTES);
   hipError_t e = hipMalloc(&dm->d_pool, total);
   if (e != hipSuccess) {
@@ -81,14 +79,10 @@ extern "C" lsdg_status lsdg_depthmap_create(lsdg_ctx c, const lsdg_camera* cam, 
     dm->buf[k].dv = (float4*)(b + ob[k][4]);
   }
   dm->d_obs = (uint8_t*)(b + o_obs);
-  dm->d_dest = (int*)(b + o_dest);
   dm->d_newIV = (float2*)(b + o_iv);
-  dm->d_count = (int*)(b + o_cnt);
-  dm->d_fill = (int*)(b + o_fill);
-  dm->d_bucket = (int*)(b + o_bucket);
-  dm->d_scanblk = (int*)(b + o_blk);
-  dm->d_red = (double*)(b + o_red);
-  dm->d_red_counter = (unsigned*)(b + o_rc);
+  dm->d_head = (int*)(b + o_head);
+  dm->d_next = (int*)(b + o_next);
+  dm->d_mean = (double2*)(b + o_mean);
   dm->d_work = (int4*)(b + o_work);
   dm->d_work_count = (int*)(b + o_wc);
   if ((e = hipMemsetAsync(dm->d_pool, 0, total, c->stream)) != hipSuccess ||
@@ -134,8 +128,9 @@ static lsdg_status check_frame(lsdg_depthmap dm, lsdg_frame f) {
 // its depth pyramid.
 static lsdg_status set_depth(lsdg_depthmap dm, lsdg_frame f) {
   lsdg_ctx c = dm->ctx;
-  CK(c, launch_set_depth(dm, f, c->stream));
-  return frame_depth_from_level0(f);
+  CK(c, launch_set_depth(dm, f, false, c->stream));
+  frame_depth_written(f);
+  return LSDG_OK;
 }
 
 extern "C" lsdg_status lsdg_depth_initialize_from_gt(lsdg_depthmap dm, lsdg_frame kf) {
@@ -282,7 +277,7 @@ extern "C" lsdg_status lsdg_depth_update(lsdg_depthmap dm, const lsdg_frame* ref
   ProfMark pm = prof_begin(c, LSDG_KERNEL_DEPTH);
   CK(c, launch_observe(dm, P, dm->h_refs, n, dm->h_refById, (int)byId.size(), offset, 0, n - 1,
                        (float)kf->numFramesTrackedOnThis, (float)kf->numMappedOnThis, c->stream));
-  CK(c, launch_fill_regularize(dm, P, P.val_sum_min_for_keep, kf, c->stream));
+  CK(c, launch_fill_regularize(dm, P, P.val_sum_min_for_keep, kf, false, c->stream));
   frame_depth_written(kf);
   // algorithmic bytes of one update (181 B per pixel: observe 70, fill holes 66,
   // regularize 37, setDepth 8)
@@ -311,19 +306,14 @@ extern "C" lsdg_status lsdg_depth_create_keyframe(lsdg_depthmap dm, lsdg_frame n
   dm->kf = nkf;
   dm->kfReactivated = false;
   CK(c, launch_regularize(dm, P, true, P.val_sum_min_for_keep, c->stream));
-  CK(c, launch_fill_regularize(dm, P, P.val_sum_min_for_keep, nullptr, c->stream));
-  CK(c, launch_mean_idepth(dm, c->stream));
-  CK(c, hipStreamSynchronize(c->stream));
-  double cnt = dm->h_red[0], sum = dm->h_red[1];
-  float rescale = (float)(cnt / sum);
-  CK(c, launch_rescale(dm, rescale, c->stream));
-  Pose tp = pose_inv(oldToNew);
-  tp.s = (double)rescale;
-  nkf->thisToParent = tp;
-  st = set_depth(dm, nkf);
-  if (st != LSDG_OK) return st;
+  CK(c, launch_fill_regularize(dm, P, P.val_sum_min_for_keep, nullptr, true, c->stream));
+  CK(c, launch_set_depth(dm, nkf, true, c->stream));
+  frame_depth_written(nkf);
   prof_end(c, pm, 0.0);
   CK(c, hipStreamSynchronize(c->stream));
+  Pose tp = pose_inv(oldToNew);
+  tp.s = (double)(float)(dm->h_red[0] / dm->h_red[1]);
+  nkf->thisToParent = tp;
   return LSDG_OK;
 }
 
@@ -333,7 +323,7 @@ extern "C" lsdg_status lsdg_depth_finalize_keyframe(lsdg_depthmap dm) {
   if (!dm->valid || !dm->kf) return fail(c, LSDG_ESTATE, "depth map has no active keyframe");
   lsdg_status st0 = frame_require(dm->kf, KF_DATA);
   if (st0 != LSDG_OK) return st0;
-  CK(c, launch_fill_regularize(dm, c->P, c->P.val_sum_min_for_keep, dm->kf, c->stream));
+  CK(c, launch_fill_regularize(dm, c->P, c->P.val_sum_min_for_keep, dm->kf, false, c->stream));
   frame_depth_written(dm->kf);
   CK(c, hipStreamSynchronize(c->stream));
   return LSDG_OK;

@@ -11,12 +11,14 @@
 //                  and optionally Frame::setDepth in one pass over a 4-pixel
 //                  halo; the reference's integral image of validity is
 //                  replaced by the equal integer 5x5 box sum.
-//   k_set_depth    Frame::setDepth (level 0; the pyramid follows).
+//   k_set_depth    Frame::setDepth and the keyframe's depth pyramid, after
+//                  createKeyFrame's rescale where it is due.
 //   k_prop_*       propagateDepth as a deterministic scatter: project every
-//                  source, count per destination, scan, bucket, then one
-//                  thread per destination folds its sources in raster order,
-//                  which is the order the reference's sequential loop uses.
-//   k_mean_idepth  createKeyFrame's mean inverse depth (FP64, deterministic).
+//                  source onto its destination's list, then one thread per
+//                  destination folds its sources in raster order, which is
+//                  the order the reference's sequential loop uses.
+//   k_mean_merge   createKeyFrame's mean inverse depth (FP64, deterministic)
+//                  from k_fill_regularize's per-tile sums.
 //
 // The hypothesis maps rotate through three buffers: `cur` and `oth` hold what
 // the reference's current and other maps hold, the third is spare.  A pass
@@ -1251,10 +1253,48 @@ __device__ inline int2 xcd_tile(int gx, int gy) {
   return make_int2(t % gx, t / gx);
 }
 
+// A keyframe's inverse-depth levels 1-4 from a 16x16 tile's setDepth values
+// d0 (one per thread): each level-l pixel fuses the 2^l x 2^l level-0 pixels
+// below it, which lie in this tile, so the levels follow in shared memory
+// (level by level, in place: a level's reads end at a barrier before its
+// writes).
 static_assert(PYR == 5, "a 16x16 tile holds whole 2^(PYR-1) blocks of level-0 pixels");
+__device__ __forceinline__ void depth_levels_of_tile(float2 d0, int2 tile, const PyrDepthArgs& kf) {
+  __shared__ float pid[16][17], pvar[16][17];
+  pid[threadIdx.x >> 4][threadIdx.x & 15] = d0.x;
+  pvar[threadIdx.x >> 4][threadIdx.x & 15] = d0.y;
+  __syncthreads();
+#pragma unroll
+  for (int l = 1, n = 8; l < PYR; ++l, n >>= 1) {
+    const int tx = threadIdx.x % n, ty = threadIdx.x / n;
+    float oi = -1.0f, ov = -1.0f;
+    if ((int)threadIdx.x < n * n) {
+      const int px = tile.x * n + tx, py = tile.y * n + ty;
+      if (px < kf.w[l] && py < kf.h[l]) {
+        const float ia[4] = {pid[2 * ty][2 * tx], pid[2 * ty][2 * tx + 1], pid[2 * ty + 1][2 * tx],
+                             pid[2 * ty + 1][2 * tx + 1]};
+        const float va[4] = {pvar[2 * ty][2 * tx], pvar[2 * ty][2 * tx + 1], pvar[2 * ty + 1][2 * tx],
+                             pvar[2 * ty + 1][2 * tx + 1]};
+        fuse4(ia, va, oi, ov);
+        kf.id[l][px + py * kf.w[l]] = oi;
+        kf.var[l][px + py * kf.w[l]] = ov;
+      }
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < n * n) {
+      pid[ty][tx] = oi;
+      pvar[ty][tx] = ov;
+    }
+    __syncthreads();
+  }
+}
+
+// meanRows, when set, receives per block the count and the FP64 sum of the
+// regularized idepths (createKeyFrame's mean; summed by k_mean_merge).
 __global__ __launch_bounds__(TILE_THREADS) void k_fill_regularize(DepthGeom g, HypBuf in, HypBuf filled, HypBuf out,
                                                                   const float* __restrict__ maxg, lsdg_params P,
-                                                                  int validityTH, PyrDepthArgs kf) {
+                                                                  int validityTH, PyrDepthArgs kf,
+                                                                  double2* __restrict__ meanRows) {
   __shared__ FillTile<24> a;  // input, pixels and a 4-pixel halo
   __shared__ RegTile<20> f;   // filled, pixels and a 2-pixel halo
   constexpr int AITER = (24 * 24 + TILE_THREADS - 1) / TILE_THREADS;
@@ -1322,6 +1362,8 @@ __global__ __launch_bounds__(TILE_THREADS) void k_fill_regularize(DepthGeom g, H
   }
   __syncthreads();
   float2 d0 = make_float2(-1.0f, -1.0f);
+  double mean = 0.0;
+  bool counted = false;
   if (inside) {
     const int cx = lx + 2, cy = ly + 2;
     // the filled hypothesis: DepthMapPixelHypothesis(obs, VAR_RANDOM_INIT_INITIAL, 0) where created
@@ -1334,46 +1376,78 @@ __global__ __launch_bounds__(TILE_THREADS) void k_fill_regularize(DepthGeom g, H
     const Hyp r = regularize_pixel(f, cx, cy, x, y, w, h, d, P, 0, validityTH);
     store_hyp(out, idx, r);
     if (kf.id[0]) d0 = set_depth_pixel(r, idx, kf.id[0], kf.var[0]);
+    counted = r.valid;
+    if (counted) mean = (double)r.dv.z;
   }
-  if (!kf.id[0]) return;  // (uniform)
-  // The keyframe's depth pyramid: each level-l pixel fuses the 2^l x 2^l
-  // level-0 pixels below it, which lie in this tile, so levels 1-4 follow
-  // from the tile's setDepth values in shared memory (level by level, in
-  // place: a level's reads end at a barrier before its writes).
-  __shared__ float pid[16][17], pvar[16][17];
-  pid[ly][lx] = d0.x;
-  pvar[ly][lx] = d0.y;
-  __syncthreads();
+  if (kf.id[0]) depth_levels_of_tile(d0, tile, kf);  // (uniform)
+  if (meanRows) {                                    // (uniform)
+    __shared__ double rows[TILE_THREADS / 64];
+    const int cnt = __syncthreads_count(counted);
 #pragma unroll
-  for (int l = 1, n = 8; l < PYR; ++l, n >>= 1) {
-    const int tx = threadIdx.x % n, ty = threadIdx.x / n;
-    float oi = -1.0f, ov = -1.0f;
-    if ((int)threadIdx.x < n * n) {
-      const int px = tile.x * n + tx, py = tile.y * n + ty;
-      if (px < kf.w[l] && py < kf.h[l]) {
-        const float ia[4] = {pid[2 * ty][2 * tx], pid[2 * ty][2 * tx + 1], pid[2 * ty + 1][2 * tx],
-                             pid[2 * ty + 1][2 * tx + 1]};
-        const float va[4] = {pvar[2 * ty][2 * tx], pvar[2 * ty][2 * tx + 1], pvar[2 * ty + 1][2 * tx],
-                             pvar[2 * ty + 1][2 * tx + 1]};
-        fuse4(ia, va, oi, ov);
-        kf.id[l][px + py * kf.w[l]] = oi;
-        kf.var[l][px + py * kf.w[l]] = ov;
-      }
-    }
+    for (int o = 32; o > 0; o >>= 1) mean += __shfl_xor(mean, o);
+    if (__lane_id() == 0) rows[threadIdx.x >> 6] = mean;
     __syncthreads();
-    if ((int)threadIdx.x < n * n) {
-      pid[ty][tx] = oi;
-      pvar[ty][tx] = ov;
-    }
-    __syncthreads();
+    if (threadIdx.x == 0)
+      meanRows[blockIdx.x + blockIdx.y * gridDim.x] = make_double2((double)cnt, (rows[0] + rows[1]) + (rows[2] + rows[3]));
   }
 }
 
+// ---------------------------------------------------- mean inverse depth
+// Sums the tiles' (count, sum) rows, each thread its rows in order and the
+// threads in a fixed tree, into *total (device) and *host.
+__global__ __launch_bounds__(1024) void k_mean_merge(const double2* __restrict__ rows, int n, double2* __restrict__ total,
+                                                     double* __restrict__ host) {
+  __shared__ double2 sh[16];
+  double c = 0.0, v = 0.0;
+  for (int i = threadIdx.x; i < n; i += 1024) {
+    const double2 r = rows[i];
+    c += r.x;
+    v += r.y;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    c += __shfl_xor(c, o);
+    v += __shfl_xor(v, o);
+  }
+  if (__lane_id() == 0) sh[threadIdx.x >> 6] = make_double2(c, v);
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  for (int k = 1; k < 16; ++k) {
+    c += sh[k].x;
+    v += sh[k].y;
+  }
+  *total = make_double2(c, v);
+  host[0] = c;
+  host[1] = v;
+}
+
 // -------------------------------------------------------- Frame::setDepth
-__global__ void k_set_depth(HypBuf cur, int n, float* __restrict__ idepth, float* __restrict__ var) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  set_depth_pixel(load_hyp(cur, i), i, idepth, var);
+// setDepth of the whole map and the keyframe's levels 1-4, in one launch; with
+// `mean` set (count, sum of the idepths) the map is first rescaled to mean
+// inverse depth 1, as createKeyFrame does.  The factor is computed here from
+// the sums, so no wait for them on the host comes before (count, merge, wait,
+// rescale, setDepth and levels took five launches and about 55 us at 640x480,
+// 18 of them a single-counter reduction; now this and k_mean_merge).
+__global__ __launch_bounds__(TILE_THREADS) void k_set_depth(DepthGeom g, HypBuf cur, PyrDepthArgs kf,
+                                                            const double2* __restrict__ mean) {
+  const int2 tile = xcd_tile(gridDim.x, gridDim.y);
+  const int x = tile.x * 16 + (threadIdx.x & 15), y = tile.y * 16 + (threadIdx.x >> 4);
+  float2 d0 = make_float2(-1.0f, -1.0f);
+  if (x < g.w && y < g.h) {
+    const int i = x + y * g.w;
+    Hyp d = load_hyp(cur, i);
+    if (mean && d.valid) {
+      const double2 m = *mean;
+      const float f = (float)(m.x / m.y), f2 = f * f;
+      d.dv.x *= f;
+      d.dv.z *= f;
+      d.dv.y *= f2;
+      d.dv.w *= f2;
+      cur.dv[i] = d.dv;
+    }
+    d0 = set_depth_pixel(d, i, kf.id[0], kf.var[0]);
+  }
+  depth_levels_of_tile(d0, tile, kf);
 }
 
 // ------------------------------------------------------------ propagate
@@ -1385,16 +1459,15 @@ struct PropArgs {
   const float* kfImg;        // old keyframe image
   const float* newMaxg;
   const float* newImg;
-  int* dest;
   float2* newIV;
-  int* count;
+  int* head;  // per destination: 1 + the source listed last, 0 for none
+  int* next;  // per source: 1 + the one listed before it at its destination, 0 for none
 };
 
 __global__ __launch_bounds__(256) void k_prop_project(PropArgs a, lsdg_params P) {
   const int W = a.g.w, H = a.g.h;
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= W * H) return;
-  a.dest[i] = -1;
   if (!a.src.valid[i]) return;
   int y = i / W, x = i - y * W;
   float4 s = a.src.dv[i];
@@ -1423,175 +1496,83 @@ __global__ __launch_bounds__(256) void k_prop_project(PropArgs a, lsdg_params P)
   r4 *= r4;
   r4 *= r4;
   float new_var = r4 * s.y;
-  a.dest[i] = nidx;
   a.newIV[i] = make_float2(new_id, new_var);
-  atomicAdd(&a.count[nidx], 1);
-}
-
-__global__ __launch_bounds__(256) void k_prop_bucket(const int* __restrict__ dest, const int* __restrict__ offsets,
-                                                     int* __restrict__ fill, int* __restrict__ bucket, int n) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  int d = dest[i];
-  if (d < 0) return;
-  int pos = atomicAdd(&fill[d], 1);
-  bucket[offsets[d] + pos] = i;
+  a.next[i] = atomicExch(&a.head[nidx], i + 1);
 }
 
 // One thread per destination: sources in ascending (raster) order, the
 // reference's occlusion / create / merge rules.  Empty destinations only get
-// the wipe (isValid = false, blacklisted = 0).
+// the wipe (isValid = false, blacklisted = 0).  k_prop_project lists a
+// destination's sources in any order (mostly one or two); each walk of the
+// list takes the PROP_SORT smallest not yet folded, sorted in registers, so
+// the fold's order is the raster's whatever order they were listed in.  The
+// list is emptied for the next propagation.  (A count, a three-launch scan, two
+// clears and a bucket pass in the place of the list took 30 us at 640x480.)
+constexpr int PROP_SORT = 8;
 __global__ __launch_bounds__(256) void k_prop_fold(HypBuf src, HypBuf out, const float2* __restrict__ newIV,
-                                                   const int* __restrict__ offsets, const int* __restrict__ bucket,
-                                                   int n, lsdg_params P) {
-  int d = blockIdx.x * blockDim.x + threadIdx.x;
+                                                   int* __restrict__ head, const int* __restrict__ next, int n,
+                                                   lsdg_params P) {
+  const int d = blockIdx.x * blockDim.x + threadIdx.x;
   if (d >= n) return;
-  int b0 = offsets[d], b1 = offsets[d + 1];
-  if (b0 == b1) {
+  const int first = head[d];
+  if (first == 0) {
     out.valid[d] = 0;
     out.bl[d] = 0;
     return;
   }
+  head[d] = 0;
   Hyp t;
   t.valid = false;
   t.bl = 0;
   t.nsid = out.nsid[d];
   t.val = out.val[d];
   t.dv = out.dv[d];
-  int last = -1;
-  for (int k = b0; k < b1; ++k) {
-    // next source in raster order
-    int si = 0x7fffffff;
-    for (int j = b0; j < b1; ++j) {
-      int c = bucket[j];
-      if (c > last && c < si) si = c;
-    }
-    last = si;
-    float2 iv = newIV[si];
-    float new_id = iv.x, new_var = iv.y;
-    int sval = src.val[si];
-    if (t.valid) {
-      float diff = t.dv.x - new_id;
-      if (P.diff_fac_prop_merge * diff * diff > new_var + t.dv.y) {
-        if (new_id < t.dv.x) continue;
-        t.valid = false;
+  int last = 0;  // sources are kept as 1 + their pixel
+  bool more = true;
+  while (more) {
+    int s[PROP_SORT];
+#pragma unroll
+    for (int k = 0; k < PROP_SORT; ++k) s[k] = INT_MAX;
+    more = false;
+    for (int c = first; c != 0; c = next[c - 1]) {
+      int v = c > last ? c : INT_MAX;
+#pragma unroll
+      for (int k = 0; k < PROP_SORT; ++k) {
+        const int lo = min(s[k], v);
+        v = max(s[k], v);
+        s[k] = lo;
       }
+      more |= v != INT_MAX;
     }
-    if (!t.valid) {
-      t = make_hyp(new_id, new_var, min(P.validity_counter_max_variable, sval));
-    } else {
-      float wgt = new_var / (t.dv.y + new_var);
-      float merged = wgt * t.dv.x + (1.0f - wgt) * new_id;
-      int mv = sval + t.val;
-      int cap = P.validity_counter_max + P.validity_counter_max_variable;
-      if (mv > cap) mv = cap;
-      t = make_hyp(merged, 1.0f / (1.0f / t.dv.y + 1.0f / new_var), mv);
+    while (s[0] != INT_MAX) {
+      const int si = s[0] - 1;
+      last = s[0];
+#pragma unroll
+      for (int k = 0; k + 1 < PROP_SORT; ++k) s[k] = s[k + 1];
+      s[PROP_SORT - 1] = INT_MAX;
+      const float2 iv = newIV[si];
+      const float new_id = iv.x, new_var = iv.y;
+      const int sval = src.val[si];
+      if (t.valid) {
+        const float diff = t.dv.x - new_id;
+        if (P.diff_fac_prop_merge * diff * diff > new_var + t.dv.y) {
+          if (new_id < t.dv.x) continue;
+          t.valid = false;
+        }
+      }
+      if (!t.valid) {
+        t = make_hyp(new_id, new_var, min(P.validity_counter_max_variable, sval));
+      } else {
+        const float wgt = new_var / (t.dv.y + new_var);
+        const float merged = wgt * t.dv.x + (1.0f - wgt) * new_id;
+        int mv = sval + t.val;
+        const int cap = P.validity_counter_max + P.validity_counter_max_variable;
+        if (mv > cap) mv = cap;
+        t = make_hyp(merged, 1.0f / (1.0f / t.dv.y + 1.0f / new_var), mv);
+      }
     }
   }
   store_hyp(out, d, t);
-}
-
-// Exclusive scan of count[0..n) into offsets (in place), offsets[n] = total.
-// Three kernels: per-block sums, a one-block scan of block sums, per-block scan.
-__global__ __launch_bounds__(256) void k_scan_blocksum(const int* __restrict__ a, int n, int* __restrict__ blk) {
-  __shared__ int sh[256];
-  int i = blockIdx.x * 256 + threadIdx.x;
-  sh[threadIdx.x] = i < n ? a[i] : 0;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (threadIdx.x < s) sh[threadIdx.x] += sh[threadIdx.x + s];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) blk[blockIdx.x] = sh[0];
-}
-
-__global__ __launch_bounds__(1024) void k_scan_top(int* blk, int nb) {
-  __shared__ int sh[1024];
-  __shared__ int carry;
-  if (threadIdx.x == 0) carry = 0;
-  __syncthreads();
-  for (int base = 0; base < nb; base += 1024) {
-    int i = base + threadIdx.x;
-    int v = i < nb ? blk[i] : 0;
-    sh[threadIdx.x] = v;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-      int t = threadIdx.x >= off ? sh[threadIdx.x - off] : 0;
-      __syncthreads();
-      sh[threadIdx.x] += t;
-      __syncthreads();
-    }
-    if (i < nb) blk[i] = carry + sh[threadIdx.x] - v;
-    __syncthreads();
-    if (threadIdx.x == 1023) carry += sh[1023];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) blk[nb] = carry;
-}
-
-__global__ __launch_bounds__(256) void k_scan_apply(int* a, int n, const int* __restrict__ blk) {
-  __shared__ int sh[256];
-  int i = blockIdx.x * 256 + threadIdx.x;
-  int v = i < n ? a[i] : 0;
-  sh[threadIdx.x] = v;
-  __syncthreads();
-  for (int off = 1; off < 256; off <<= 1) {
-    int t = threadIdx.x >= off ? sh[threadIdx.x - off] : 0;
-    __syncthreads();
-    sh[threadIdx.x] += t;
-    __syncthreads();
-  }
-  if (i < n) a[i] = blk[blockIdx.x] + sh[threadIdx.x] - v;
-  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) a[n] = blk[gridDim.x];
-}
-
-// ---------------------------------------------------- mean inverse depth
-// Count and FP64 sum of idepth_smoothed over valid pixels; the last block
-// merges the per-block rows in block order and writes (count, sum).
-__global__ __launch_bounds__(256) void k_mean_idepth(HypBuf cur, int n, double* __restrict__ partials,
-                                                     unsigned* counter, double* __restrict__ out) {
-  __shared__ double shc[256], shs[256];
-  __shared__ bool amLast;
-  double c = 0.0, s = 0.0;
-  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256)
-    if (cur.valid[i]) {
-      c += 1.0;
-      s += (double)cur.dv[i].z;
-    }
-  shc[threadIdx.x] = c;
-  shs[threadIdx.x] = s;
-  __syncthreads();
-  for (int k = 128; k > 0; k >>= 1) {
-    if (threadIdx.x < k) {
-      shc[threadIdx.x] += shc[threadIdx.x + k];
-      shs[threadIdx.x] += shs[threadIdx.x + k];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    partials[2 * blockIdx.x] = shc[0];
-    partials[2 * blockIdx.x + 1] = shs[0];
-  }
-  __threadfence();
-  __syncthreads();
-  if (threadIdx.x == 0) amLast = atomicAdd(counter, 1u) == gridDim.x - 1;
-  __syncthreads();
-  if (!amLast) return;
-  __threadfence();
-  merge_rows<2, 256>(partials, gridDim.x, out);
-  if (threadIdx.x == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__global__ void k_rescale(HypBuf cur, int n, float f) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n || !cur.valid[i]) return;
-  float f2 = f * f;
-  float4 d = cur.dv[i];
-  d.x *= f;
-  d.z *= f;
-  d.y *= f2;
-  d.w *= f2;
-  cur.dv[i] = d;
 }
 
 // Hypotheses from (idepth, var) arrays: valid where var > 0 and idepth is
@@ -1726,28 +1707,42 @@ hipError_t launch_regularize(lsdg_depthmap dm, const lsdg_params& P, bool remove
   return hipGetLastError();
 }
 
-hipError_t launch_fill_regularize(lsdg_depthmap dm, const lsdg_params& P, int th, lsdg_frame setDepth,
+static PyrDepthArgs pyr_depth_args(lsdg_frame f) {
+  PyrDepthArgs a;
+  for (int l = 0; l < PYR; ++l) {
+    a.id[l] = f->d_idepth[l];
+    a.var[l] = f->d_ivar[l];
+    a.w[l] = f->w[l];
+    a.h[l] = f->h[l];
+  }
+  return a;
+}
+
+size_t mean_rows(int w, int h) {
+  const dim3 g = grid16(w, h);
+  return (size_t)g.x * g.y + 1;  // and the total
+}
+
+hipError_t launch_fill_regularize(lsdg_depthmap dm, const lsdg_params& P, int th, lsdg_frame setDepth, bool mean,
                                   hipStream_t s) {
   const int in = dm->cur, fill = dm->oth, reg = 3 - dm->cur - dm->oth;
-  PyrDepthArgs kf{};
-  if (setDepth) {
-    for (int l = 0; l < PYR; ++l) {
-      kf.id[l] = setDepth->d_idepth[l];
-      kf.var[l] = setDepth->d_ivar[l];
-      kf.w[l] = setDepth->w[l];
-      kf.h[l] = setDepth->h[l];
-    }
-  }
-  k_fill_regularize<<<grid16(dm->g.w, dm->g.h), dim3(TILE_THREADS), 0, s>>>(
-      dm->g, dm->buf[in], dm->buf[fill], dm->buf[reg], dm->kf->d_maxg[0], P, th, kf);
+  const PyrDepthArgs kf = setDepth ? pyr_depth_args(setDepth) : PyrDepthArgs{};
+  const dim3 grid = grid16(dm->g.w, dm->g.h);
+  k_fill_regularize<<<grid, dim3(TILE_THREADS), 0, s>>>(dm->g, dm->buf[in], dm->buf[fill], dm->buf[reg],
+                                                        dm->kf->d_maxg[0], P, th, kf, mean ? dm->d_mean : nullptr);
   dm->oth = fill;
   dm->cur = reg;
+  if (mean) {
+    const int n = (int)(grid.x * grid.y);
+    k_mean_merge<<<dim3(1), dim3(1024), 0, s>>>(dm->d_mean, n, dm->d_mean + n, dm->d_red_out);
+  }
   return hipGetLastError();
 }
 
-hipError_t launch_set_depth(lsdg_depthmap dm, lsdg_frame f, hipStream_t s) {
-  int n = dm->g.w * dm->g.h;
-  k_set_depth<<<dim3((n + 255) / 256), dim3(256), 0, s>>>(dm->buf[dm->cur], n, f->d_idepth[0], f->d_ivar[0]);
+hipError_t launch_set_depth(lsdg_depthmap dm, lsdg_frame f, bool rescale, hipStream_t s) {
+  const dim3 grid = grid16(dm->g.w, dm->g.h);
+  k_set_depth<<<grid, dim3(TILE_THREADS), 0, s>>>(dm->g, dm->buf[dm->cur], pyr_depth_args(f),
+                                                  rescale ? dm->d_mean + grid.x * grid.y : nullptr);
   return hipGetLastError();
 }
 
@@ -1755,9 +1750,6 @@ hipError_t launch_propagate(lsdg_depthmap dm, const lsdg_params& P, lsdg_frame n
                             const uint8_t* d_wasGood, hipStream_t s) {
   const int n = dm->g.w * dm->g.h;
   const int nb = (n + 255) / 256;
-  hipError_t e;
-  if ((e = hipMemsetAsync(dm->d_count, 0, sizeof(int) * (n + 1), s)) != hipSuccess) return e;
-  if ((e = hipMemsetAsync(dm->d_fill, 0, sizeof(int) * n, s)) != hipSuccess) return e;
   PropArgs a;
   a.g = dm->g;
   a.src = dm->buf[dm->cur];
@@ -1766,32 +1758,13 @@ hipError_t launch_propagate(lsdg_depthmap dm, const lsdg_params& P, lsdg_frame n
   a.kfImg = dm->kf->d_image[0];
   a.newMaxg = nkf->d_maxg[0];
   a.newImg = nkf->d_image[0];
-  a.dest = dm->d_dest;
   a.newIV = dm->d_newIV;
-  a.count = dm->d_count;
+  a.head = dm->d_head;
+  a.next = dm->d_next;
   k_prop_project<<<dim3(nb), dim3(256), 0, s>>>(a, P);
-  k_scan_blocksum<<<dim3(nb), dim3(256), 0, s>>>(dm->d_count, n, dm->d_scanblk);
-  k_scan_top<<<dim3(1), dim3(1024), 0, s>>>(dm->d_scanblk, nb);
-  k_scan_apply<<<dim3(nb), dim3(256), 0, s>>>(dm->d_count, n, dm->d_scanblk);
-  k_prop_bucket<<<dim3(nb), dim3(256), 0, s>>>(dm->d_dest, dm->d_count, dm->d_fill, dm->d_bucket, n);
-  k_prop_fold<<<dim3(nb), dim3(256), 0, s>>>(dm->buf[dm->cur], dm->buf[dm->oth], dm->d_newIV, dm->d_count,
-                                             dm->d_bucket, n, P);
+  k_prop_fold<<<dim3(nb), dim3(256), 0, s>>>(dm->buf[dm->cur], dm->buf[dm->oth], dm->d_newIV, dm->d_head, dm->d_next,
+                                             n, P);
   std::swap(dm->cur, dm->oth);
-  return hipGetLastError();
-}
-
-hipError_t launch_mean_idepth(lsdg_depthmap dm, hipStream_t s) {
-  int n = dm->g.w * dm->g.h;
-  int nb = (n + 255 * 8) / (256 * 8);
-  if (nb > 1024) nb = 1024;
-  if (nb < 1) nb = 1;
-  k_mean_idepth<<<dim3(nb), dim3(256), 0, s>>>(dm->buf[dm->cur], n, dm->d_red, dm->d_red_counter, dm->d_red_out);
-  return hipGetLastError();
-}
-
-hipError_t launch_rescale(lsdg_depthmap dm, float f, hipStream_t s) {
-  int n = dm->g.w * dm->g.h;
-  k_rescale<<<dim3((n + 255) / 256), dim3(256), 0, s>>>(dm->buf[dm->cur], n, f);
   return hipGetLastError();
 }
 

@@ -341,16 +341,12 @@ struct lsdg_depthmap_s {
   lsdg::StereoRef* h_refs = nullptr;  // pinned staging
   int* h_refById = nullptr;
   // propagation scratch
-  int* d_dest = nullptr;
   float2* d_newIV = nullptr;
-  int* d_count = nullptr;   // P + 1
-  int* d_fill = nullptr;    // P
-  int* d_bucket = nullptr;  // P
-  int* d_scanblk = nullptr;
+  int* d_head = nullptr;  // per destination, its sources' list (0: empty, between propagations too)
+  int* d_next = nullptr;
   // rescale reduction
-  double* d_red = nullptr;  // partial rows
-  unsigned* d_red_counter = nullptr;
-  double* h_red = nullptr;  // pinned, host-mapped (count, sum)
+  double2* d_mean = nullptr;  // (count, sum) per tile, then the total
+  double* h_red = nullptr;    // pinned, host-mapped (count, sum)
   double* d_red_out = nullptr;
 };
 
@@ -425,17 +421,19 @@ hipError_t launch_regularize(lsdg_depthmap dm, const lsdg_params& P, bool remove
                              hipStream_t s);  // swaps buffers
 // regularizeDepthMapFillHoles then regularizeDepthMap(false, th) in one pass,
 // leaving the current and other maps as the two passes would; with setDepth
-// non-null, also launch_set_depth(setDepth) and the frame's inverse-depth
-// levels 1-4 (what launch_pyr_depth would write after it)
-hipError_t launch_fill_regularize(lsdg_depthmap dm, const lsdg_params& P, int th, lsdg_frame setDepth,
+// non-null, also what launch_set_depth(setDepth) would write after it; with
+// mean, the count and sum of the new map's idepths to dm->d_mean's last entry
+// and h_red
+hipError_t launch_fill_regularize(lsdg_depthmap dm, const lsdg_params& P, int th, lsdg_frame setDepth, bool mean,
                                   hipStream_t s);
-hipError_t launch_set_depth(lsdg_depthmap dm, lsdg_frame f, hipStream_t s);
+size_t mean_rows(int w, int h);  // entries of dm->d_mean
+// Frame::setDepth (levels 0-4) of f from the current map, which rescale first
+// scales by count / sum of the last mean
+hipError_t launch_set_depth(lsdg_depthmap dm, lsdg_frame f, bool rescale, hipStream_t s);
 // DepthMap::initializeRandomly on dm->kf's level-0 max-gradients
 hipError_t launch_random_init(lsdg_depthmap dm, const lsdg_params& P, unsigned long long seed, hipStream_t s);
 hipError_t launch_propagate(lsdg_depthmap dm, const lsdg_params& P, lsdg_frame nkf, const Xf& oldToNew,
                             const uint8_t* d_wasGood, hipStream_t s);  // swaps buffers
-hipError_t launch_mean_idepth(lsdg_depthmap dm, hipStream_t s);  // h_red[0] = count, h_red[1] = sum
-hipError_t launch_rescale(lsdg_depthmap dm, float f, hipStream_t s);
 hipError_t launch_hyp_prior(lsdg_depthmap dm, const float* d_id, const float* d_var, int validity, int gt,
                             float gtVar, hipStream_t s);
 
