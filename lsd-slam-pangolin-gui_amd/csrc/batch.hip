@@ -32,6 +32,16 @@ constexpr int BATCH_WAVES = BATCH_BS / 64;
 #endif
 constexpr int BATCH_U = LSDG_BATCH_U;  // points per thread with loads in flight together
 constexpr int BATCH_SOLVE_BS = 256;
+constexpr int COOP_MAX_BS = 512;
+// Waves per SIMD the cooperative kernel is compiled for (168 registers).  With
+// two (215 registers) the loop over the points waited for memory and for the
+// one wave of a block that runs the LM step: 64 Sim3 jobs of 1920x1080 1322 us,
+// with three 1150.  The job's level and pose in scalar registers, counts in one
+// register each, affine statistics only where they are estimated and the LM
+// step's coefficients out of the loop's registers make room for it.  With four
+// (128 registers, one point per thread in flight) 64 SE3 jobs of 640x480 gain
+// 3%, 24 of 752x478 lose 5%, and Sim3 jobs stay where they are.
+constexpr int COOP_WAVES_PER_SIMD = 3;
 
 // ------------------------------------------------------------- kernels
 // Start state of every job: T = (frameToRef_init)^-1, first level, counters
@@ -113,8 +123,8 @@ __global__ __launch_bounds__(BATCH_BS) void k_batch_eval(BatchArgs a, int parity
     const JobDesc& jd = a.jobs[j];
     const JobState* st = a.st + j;
     const int lvl = st->level;
-    const JobLevel& L = jd.lv[lvl];
-    const Xf x = st->xf;
+    const JobLevel L = uniform(jd.lv[lvl]);
+    const Xf x = uniform(st->xf);
     TrackKParams kp = a.kp;
     kp.aff_a = st->affA;
     kp.aff_b = st->affB;
@@ -125,10 +135,10 @@ __global__ __launch_bounds__(BATCH_BS) void k_batch_eval(BatchArgs a, int parity
     const int i1 = min(i0 + tileSize, L.pts.n);
     if (KIND == LSDG_JOB_SIM3) {
       kp.roll[0] = st->roll[0]; kp.roll[1] = st->roll[1]; kp.roll[2] = st->roll[2]; kp.roll[3] = st->roll[3];
-      sim3_points<PREC, BATCH_U>(L.pts, i0 + tid, BATCH_BS, i1, L.img, L.fid, L.fvar, L.g, x, kp, acc);
+      sim3_points<PREC, BATCH_U, SUMS_LM_AFFINE>(L.pts, i0 + tid, BATCH_BS, i1, L.img, L.fid, L.fvar, L.g, x, kp, acc);
     } else {
-      uint8_t* mask = lvl == 1 ? jd.isGood : nullptr;
-      se3_points<PREC, BATCH_U>(L.pts, i0 + tid, BATCH_BS, i1, L.img, L.g, x, kp, mask, acc);
+      uint8_t* mask = lvl == 1 ? uniform(jd.isGood) : nullptr;
+      se3_points<PREC, BATCH_U, SUMS_LM_AFFINE>(L.pts, i0 + tid, BATCH_BS, i1, L.img, L.g, x, kp, mask, acc);
     }
     const double wsum = acc.wave_slot();
     if (lane < NS) sh[wave][lane] = wsum;
@@ -225,22 +235,22 @@ __global__ __launch_bounds__(BATCH_JOB_BS) void k_batch_job(BatchArgs a) {
   for (int it = 0; it < BATCH_JOB_MAX_EVALS; ++it) {
     // s and jd are read after a barrier: the exit test is uniform over the block
     if (s.status != 0) break;
-    const int lvl = s.level;
-    const JobLevel& L = jd.lv[lvl];
+    const int lvl = uniform(s.level);
+    const JobLevel L = uniform(jd.lv[lvl]);
     if (L.pts.n > a.jobMaxPoints) break;
-    const Xf x = s.xf;
+    const Xf x = uniform(s.xf);
     TrackKParams kp = a.kp;
-    kp.aff_a = s.affA;
-    kp.aff_b = s.affB;
+    kp.aff_a = uniform(s.affA);
+    kp.aff_b = uniform(s.affB);
     Accum<ACC, NS> acc;
     acc.zero();
     const int n = L.pts.n;
     if (KIND == LSDG_JOB_SIM3) {
-      kp.roll[0] = s.roll[0]; kp.roll[1] = s.roll[1]; kp.roll[2] = s.roll[2]; kp.roll[3] = s.roll[3];
-      sim3_points<PREC, BATCH_U>(L.pts, tid, BATCH_JOB_BS, n, L.img, L.fid, L.fvar, L.g, x, kp, acc);
+      for (int k = 0; k < 4; ++k) kp.roll[k] = uniform(s.roll[k]);
+      sim3_points<PREC, BATCH_U, SUMS_LM_AFFINE>(L.pts, tid, BATCH_JOB_BS, n, L.img, L.fid, L.fvar, L.g, x, kp, acc);
     } else {
-      uint8_t* mask = lvl == 1 ? jd.isGood : nullptr;
-      se3_points<PREC, BATCH_U>(L.pts, tid, BATCH_JOB_BS, n, L.img, L.g, x, kp, mask, acc);
+      uint8_t* mask = lvl == 1 ? uniform(jd.isGood) : nullptr;
+      se3_points<PREC, BATCH_U, SUMS_LM_AFFINE>(L.pts, tid, BATCH_JOB_BS, n, L.img, L.g, x, kp, mask, acc);
     }
     const double wsum = acc.wave_slot();
     if (lane < NS) sh[wave][lane] = wsum;
@@ -276,15 +286,16 @@ __global__ __launch_bounds__(BATCH_JOB_BS) void k_batch_job(BatchArgs a) {
 // K blocks of a job cannot all be resident (the grid is sized from the
 // occupancy, so this does not happen on an idle device), the blocks stop and
 // set *remaining negative, which the host reports as an error.  The block
-// size BS (256 or 512 threads) is one of the shapes the plan's tuner picks.
+// size (256 or 512 threads) is the launch's.
 #ifndef LSDG_SPIN_SLEEP
 #define LSDG_SPIN_SLEEP 2
 #endif
 
-template <int KIND, int PREC, int ACC, int COOP_BS>
-__global__ __launch_bounds__(COOP_BS) void k_batch_coop(BatchArgs a) {
+template <int KIND, int PREC, int ACC, int SUMS>
+__global__ __launch_bounds__(COOP_MAX_BS, COOP_WAVES_PER_SIMD) void k_batch_coop(BatchArgs a) {
   constexpr int NS = KIND == LSDG_JOB_SIM3 ? NS_SIM3 : NS_SE3;
-  constexpr int WAVES = COOP_BS / 64;
+  constexpr int WAVES = COOP_MAX_BS / 64;  // rows of sh; those of absent waves stay zero
+  const int bs = (int)blockDim.x, waves = bs / 64;
   __shared__ JobState s;
   __shared__ JobDesc jd;
   __shared__ LmParams sP;
@@ -309,33 +320,42 @@ __global__ __launch_bounds__(COOP_BS) void k_batch_coop(BatchArgs a) {
   int* remaining = part == 0 ? a.remaining : nullptr;
   unsigned long long* rows = a.coopRows + (size_t)j * 2 * K * NS * 2;
   const unsigned epochTag = (*a.epoch & 0xFFFFu) << 16;
-  block_copy(&s, a.st + j, COOP_BS);
-  block_copy(&jd, a.jobs + j, COOP_BS);
-  block_copy(&sP, &a.P, COOP_BS);
+  block_copy(&s, a.st + j, bs);
+  block_copy(&jd, a.jobs + j, bs);
+  block_copy(&sP, &a.P, bs);
   if (tid == 0) failed = 0;
+  for (int i = tid; i < WAVES * NS; i += bs) (&sh[0][0])[i] = 0.0;
   __syncthreads();
+  // of level cur, in scalar registers: the job's level, whether it is split,
+  // and this block's points of it
+  JobLevel L{};
+  int cur = -1, i0 = 0, i1 = 0;
+  bool split = false;
   unsigned gen = 0;  // synchronised iterations of this job so far
   for (int it = 0; it < BATCH_JOB_MAX_EVALS; ++it) {
     // s is read after a barrier: the exit test is uniform over the block
     if (s.status != 0) break;
-    const int lvl = s.level;
-    const JobLevel& L = jd.lv[lvl];
-    const int n = L.pts.n;
-    const bool split = K > 1 && n > a.soloMax;
-    const int i0 = split ? (int)((long long)n * part / K) : 0;
-    const int i1 = split ? (int)((long long)n * (part + 1) / K) : n;
-    const Xf x = s.xf;
+    const int lvl = uniform(s.level);
+    if (lvl != cur) {
+      cur = lvl;
+      L = uniform(jd.lv[lvl]);
+      split = K > 1 && L.pts.n > a.soloMax;
+      const PartRange r = split ? part_range(L.pts.n, part, K) : PartRange{0, L.pts.n};
+      i0 = r.begin;
+      i1 = r.end;
+    }
+    const Xf x = uniform(s.xf);
     TrackKParams kp = a.kp;
-    kp.aff_a = s.affA;
-    kp.aff_b = s.affB;
+    kp.aff_a = uniform(s.affA);
+    kp.aff_b = uniform(s.affB);
     Accum<ACC, NS> acc;
     acc.zero();
     if (KIND == LSDG_JOB_SIM3) {
-      kp.roll[0] = s.roll[0]; kp.roll[1] = s.roll[1]; kp.roll[2] = s.roll[2]; kp.roll[3] = s.roll[3];
-      sim3_points<PREC, BATCH_U>(L.pts, i0 + tid, COOP_BS, i1, L.img, L.fid, L.fvar, L.g, x, kp, acc);
+      for (int k = 0; k < 4; ++k) kp.roll[k] = uniform(s.roll[k]);
+      sim3_points<PREC, BATCH_U, SUMS>(L.pts, i0 + tid, bs, i1, L.img, L.fid, L.fvar, L.g, x, kp, acc);
     } else {
-      uint8_t* mask = lvl == 1 ? jd.isGood : nullptr;
-      se3_points<PREC, BATCH_U>(L.pts, i0 + tid, COOP_BS, i1, L.img, L.g, x, kp, mask, acc);
+      uint8_t* mask = lvl == 1 ? uniform(jd.isGood) : nullptr;
+      se3_points<PREC, BATCH_U, SUMS>(L.pts, i0 + tid, bs, i1, L.img, L.g, x, kp, mask, acc);
     }
     const double wsum = acc.wave_slot();
     if (lane < NS) sh[wave][lane] = wsum;
@@ -363,7 +383,7 @@ __global__ __launch_bounds__(COOP_BS) void k_batch_coop(BatchArgs a) {
       __syncthreads();  // sh is read above and written below
       // at most spinMax polls after the first look; a wave's rows are added
       // in part order, the waves' sums in wave order
-      const int q0 = K * wave / WAVES, q1 = K * (wave + 1) / WAVES;
+      const int q0 = K * wave / waves, q1 = K * (wave + 1) / waves;
       double v = 0.0;
       for (unsigned spins = 0;; ++spins) {
         bool mine = true;
@@ -395,6 +415,7 @@ __global__ __launch_bounds__(COOP_BS) void k_batch_coop(BatchArgs a) {
       }
       if (tid < NS) {
         double t = sh[0][tid];
+#pragma unroll
         for (int w = 1; w < WAVES; ++w) t += sh[w][tid];
         S[tid] = t;
       }
@@ -402,14 +423,16 @@ __global__ __launch_bounds__(COOP_BS) void k_batch_coop(BatchArgs a) {
     }
     __syncthreads();
     if (tid < 64) {
+      __builtin_amdgcn_s_setprio(3);
       int next = 0;
       if (KIND == LSDG_JOB_SIM3) lm_step_sim3(s, jd, S, sP, &next, remaining);
       else lm_step_se3(s, jd, S, sP, &next, remaining);
+      __builtin_amdgcn_s_setprio(0);
     }
     __syncthreads();
   }
   if (part == 0) {
-    block_copy(a.st + j, &s, COOP_BS);
+    block_copy(a.st + j, &s, bs);
     if (tid == 0) a.ntiles[j] = s.status == 0 ? jd.lv[s.level].ntiles : 0;
   }
 }
@@ -430,38 +453,38 @@ hipError_t launch_batch_job(const BatchArgs& a, int kind, int prec, int acc, hip
   return launch_k(k, dim3(a.njobs), dim3(BATCH_JOB_BS), s, t, a);
 }
 
-template <int ACC, int BS>
-static void (*coop_kernel_bs(int kind, int prec))(BatchArgs) {
+template <int ACC, int SUMS>
+static void (*coop_kernel_of(int kind, int prec))(BatchArgs) {
   if (kind == LSDG_JOB_SIM3)
-    return prec == LSDG_FP16 ? k_batch_coop<LSDG_JOB_SIM3, LSDG_FP16, ACC, BS>
-           : prec == LSDG_BF16 ? k_batch_coop<LSDG_JOB_SIM3, LSDG_BF16, ACC, BS>
-                               : k_batch_coop<LSDG_JOB_SIM3, LSDG_FP32, ACC, BS>;
-  return prec == LSDG_FP16 ? k_batch_coop<LSDG_JOB_SE3, LSDG_FP16, ACC, BS>
-         : prec == LSDG_BF16 ? k_batch_coop<LSDG_JOB_SE3, LSDG_BF16, ACC, BS>
-                             : k_batch_coop<LSDG_JOB_SE3, LSDG_FP32, ACC, BS>;
+    return prec == LSDG_FP16 ? k_batch_coop<LSDG_JOB_SIM3, LSDG_FP16, ACC, SUMS>
+           : prec == LSDG_BF16 ? k_batch_coop<LSDG_JOB_SIM3, LSDG_BF16, ACC, SUMS>
+                               : k_batch_coop<LSDG_JOB_SIM3, LSDG_FP32, ACC, SUMS>;
+  return prec == LSDG_FP16 ? k_batch_coop<LSDG_JOB_SE3, LSDG_FP16, ACC, SUMS>
+         : prec == LSDG_BF16 ? k_batch_coop<LSDG_JOB_SE3, LSDG_BF16, ACC, SUMS>
+                             : k_batch_coop<LSDG_JOB_SE3, LSDG_FP32, ACC, SUMS>;
 }
 
-static void (*coop_kernel(int kind, int prec, int acc, int bs))(BatchArgs) {
+static void (*coop_kernel(int kind, int prec, int acc, bool affine))(BatchArgs) {
   if (acc == BATCH_ACC_KAHAN)
-    return bs == 256 ? coop_kernel_bs<ACC_KAHAN, 256>(kind, prec) : coop_kernel_bs<ACC_KAHAN, 512>(kind, prec);
-  return bs == 256 ? coop_kernel_bs<ACC_F64, 256>(kind, prec) : coop_kernel_bs<ACC_F64, 512>(kind, prec);
+    return affine ? coop_kernel_of<ACC_KAHAN, SUMS_LM_AFFINE>(kind, prec) : coop_kernel_of<ACC_KAHAN, SUMS_LM>(kind, prec);
+  return affine ? coop_kernel_of<ACC_F64, SUMS_LM_AFFINE>(kind, prec) : coop_kernel_of<ACC_F64, SUMS_LM>(kind, prec);
 }
 
-bool batch_coop_block_size_ok(int bs) { return bs == 256 || bs == 512; }
+bool batch_coop_block_size_ok(int bs) { return bs == 256 || bs == COOP_MAX_BS; }
 
 int batch_coop_grid(int njobs, int K, int xcds) {
   if (xcds <= 1) return njobs * K;
   return ((njobs + xcds - 1) / xcds) * xcds * K;
 }
 
-hipError_t batch_coop_capacity(int kind, int prec, int acc, int bs, int* blocks) {
+hipError_t batch_coop_capacity(int kind, int prec, int acc, bool affine, int bs, int* blocks) {
   *blocks = 0;
   if (!batch_coop_block_size_ok(bs)) return hipErrorInvalidValue;
   int dev = 0, perCU = 0, cus = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   if (e == hipSuccess)
-    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, coop_kernel(kind, prec, acc, bs), bs, 0);
+    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, coop_kernel(kind, prec, acc, affine), bs, 0);
   *blocks = e == hipSuccess ? perCU * cus : 0;
   return e;
 }
@@ -469,7 +492,7 @@ hipError_t batch_coop_capacity(int kind, int prec, int acc, int bs, int* blocks)
 hipError_t launch_batch_coop(const BatchArgs& a, int kind, int prec, int acc, int bs, hipStream_t s,
                              const KTimer* t) {
   if (!batch_coop_block_size_ok(bs)) return hipErrorInvalidValue;
-  return launch_k(coop_kernel(kind, prec, acc, bs), dim3(batch_coop_grid(a.njobs, a.coopK, a.xcds)), dim3(bs), s,
+  return launch_k(coop_kernel(kind, prec, acc, a.kp.aff_stats != 0), dim3(batch_coop_grid(a.njobs, a.coopK, a.xcds)), dim3(bs), s,
                   t, a);
 }
 

@@ -275,17 +275,31 @@ static lsdg_status validate_jobs(lsdg_ctx c, const lsdg_job* jobs, int32_t n) {
   return LSDG_OK;
 }
 
-// The default shape: the cooperative kernel with 512-thread blocks, as many
-// blocks per job as the device holds at once (at most 16), levels above 2048
-// points split; when the device cannot hold two blocks per job, the
+// The default shape: the cooperative kernel with as many blocks per job as the
+// device holds at once (at most 16); when it cannot hold two per job, the
 // whole-job kernel for levels up to 6144 points and multi-block steps above,
 // in two chains from 16 jobs on.
-lsdg_batch_config lsdg::batch_default_shape(int n) {
+//   Threads per block.  A CU holds one block of 512 threads or three of 256
+// (168 registers), so the small blocks give a job half as many threads again,
+// unless the limit of 16 blocks binds, but more rows to exchange.  Few jobs are
+// bound by the exchange: 512 (24 SE3 jobs of 752x478: 265 us against 286 with
+// 256; 32 Sim3 jobs of 640x480: 386 against 412).  Many are bound by issue: 256
+// (128 SE3 jobs of 640x480: 686 us against 790 with 512; 64 Sim3 jobs of
+// 1920x1080: 1150 against 1396, of 640x480: 511 against 542).  Between them the
+// line follows what a point costs: 64 SE3 jobs of 640x480 take 425 us with 512
+// and 434 with 256.
+//   Levels of up to two points per thread are not split: evaluating them whole
+// costs no more than an exchange (24 SE3 jobs of 752x478, 512 threads: 265 us,
+// with a limit of 512 points 277; 64 Sim3 jobs of 640x480, 256 threads: 456,
+// with a limit of 1024 points 492).
+lsdg_batch_config lsdg::batch_default_shape(lsdg_ctx c, int kind, int n) {
+  const int perJob = c->num_cus / n;  // blocks of 512 threads
+  const bool small = kind == LSDG_JOB_SIM3 ? perJob <= 4 : perJob < 4;
   lsdg_batch_config s{};
   s.schedule = LSDG_SCHEDULE_COOP;
-  s.coop_block = 512;
+  s.coop_block = small ? 256 : 512;
   s.coop_k = 16;
-  s.solo_max = 2048;
+  s.solo_max = 2 * s.coop_block;
   s.job_max_points = 12 * BATCH_JOB_BS;
   s.chains = n >= 16 ? 2 : 1;
   s.points_per_thread = 4;
@@ -339,7 +353,7 @@ lsdg_status lsdg::batch_create_shaped(lsdg_ctx c, const lsdg_job* jobs, int32_t 
   // blocks per job the plan falls back to the whole-job kernel and steps.
   if (shape.schedule == LSDG_SCHEDULE_COOP) {
     int cap = 0;
-    if (batch_coop_capacity(kind, prec, b->acc, shape.coop_block, &cap) == hipSuccess) {
+    if (batch_coop_capacity(kind, prec, b->acc, P.use_affine_lightning_estimation != 0, shape.coop_block, &cap) == hipSuccess) {
       // with dispatch groups the jobs are padded to a multiple of the groups
       const int xcds = std::max(1, std::min(64, shape.xcd_groups));
       const int nPad = xcds > 1 ? ((n + xcds - 1) / xcds) * xcds : n;
@@ -458,7 +472,7 @@ extern "C" lsdg_status lsdg_batch_create(lsdg_ctx c, const lsdg_job* jobs, int32
   lsdg_status st = validate_jobs(c, jobs, n);
   if (st != LSDG_OK) return st;
   // the tuned shape of this class of batch when the table has one
-  lsdg_batch_config shape = batch_default_shape(n);
+  lsdg_batch_config shape = batch_default_shape(c, jobs[0].kind, n);
   char key[LSDG_TUNE_KEY_BYTES];
   if (lsdg_batch_tune_key(c, jobs, n, key) == LSDG_OK) tune_table_lookup(key, &shape);
   env_shape(shape, n);

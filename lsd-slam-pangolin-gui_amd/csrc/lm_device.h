@@ -9,7 +9,8 @@
 // host form in lsdg_lie.h (used by the launch-per-evaluation tracker):
 //   - the normal equations are solved unnormalised (a common factor of A and b
 //     drops out), with one reciprocal per pivot;
-//   - exp of a step is its power series in th^2 up to |w| = 0.5 rad;
+//   - exp of a step is its power series in th^2 up to |w| = 0.5 rad, and the
+//     square of half the step's beyond;
 //   - products of unit quaternions are renormalised with one Newton step;
 //   - the divisions by counts that only feed the result are left to the host.
 //   - the values a step's decision needs are read from LDS together.
@@ -75,38 +76,61 @@ __device__ inline Pose lm_pose_mul(const Pose& a, const Pose& b) {
   return r;
 }
 
-// Power series in x2 = th^2 <= 1/4, to 2^-53:
-//   sin(th / 2) / th, cos(th / 2), (1 - cos th) / th^2, (th - sin th) / th^3.
-__device__ inline double horner(double x, double c6, double c5, double c4, double c3, double c2, double c1, double c0) {
-  double r = __builtin_fma(x, c6, c5);
-  r = __builtin_fma(x, r, c4);
-  r = __builtin_fma(x, r, c3);
-  r = __builtin_fma(x, r, c2);
-  r = __builtin_fma(x, r, c1);
-  return __builtin_fma(x, r, c0);
+// Coefficients of the power series in th^2 <= 1/4, to 2^-53, highest power
+// first: sin(th) / th, cos(th), (1 - cos th) / th^2, (th - sin th) / th^3; then
+// 1 / k for k = 1 ... 17 and 1 / k! for k = 15 ... 2.  They are read through a
+// pointer that the compiler cannot follow: as literals it moves them out of
+// the iteration into registers, where they cost the loop over the points its
+// occupancy.
+constexpr int LM_SIN = 0, LM_COS = 7, LM_B = 14, LM_C = 21, LM_RECIP = 28, LM_FACT = 45, LM_COEFS = 59;
+static __constant__ double lm_coef_table[LM_COEFS] = {
+    1.0 / 6227020800.0, -1.0 / 39916800.0, 1.0 / 362880.0, -1.0 / 5040.0, 1.0 / 120.0, -1.0 / 6.0, 1.0,
+    1.0 / 479001600.0, -1.0 / 3628800.0, 1.0 / 40320.0, -1.0 / 720.0, 1.0 / 24.0, -0.5, 1.0,
+    1.0 / 87178291200.0, -1.0 / 479001600.0, 1.0 / 3628800.0, -1.0 / 40320.0, 1.0 / 720.0, -1.0 / 24.0, 0.5,
+    1.0 / 1307674368000.0, -1.0 / 6227020800.0, 1.0 / 39916800.0, -1.0 / 362880.0, 1.0 / 5040.0, -1.0 / 120.0,
+    1.0 / 6.0,
+    1.0, 1.0 / 2, 1.0 / 3, 1.0 / 4, 1.0 / 5, 1.0 / 6, 1.0 / 7, 1.0 / 8, 1.0 / 9, 1.0 / 10, 1.0 / 11, 1.0 / 12,
+    1.0 / 13, 1.0 / 14, 1.0 / 15, 1.0 / 16, 1.0 / 17,
+    1.0 / 1307674368000.0, 1.0 / 87178291200.0, 1.0 / 6227020800.0, 1.0 / 479001600.0, 1.0 / 39916800.0,
+    1.0 / 3628800.0, 1.0 / 362880.0, 1.0 / 40320.0, 1.0 / 5040.0, 1.0 / 720.0, 1.0 / 120.0, 1.0 / 24.0, 1.0 / 6.0,
+    0.5};
+typedef const __attribute__((address_space(4))) double* LmCoef;
+__device__ inline LmCoef lm_coef() {
+  LmCoef c = (LmCoef)lm_coef_table;
+  asm volatile("" : "+s"(c));
+  return c;
+}
+
+__device__ inline double horner7(double x, LmCoef c) {
+  double r = c[0];
+#pragma unroll
+  for (int k = 1; k < 7; ++k) r = __builtin_fma(x, r, c[k]);
+  return r;
 }
 constexpr double LM_SERIES_TH2 = 0.25;
-__device__ inline void exp_q_series(const double* w, double th2, double* q) {
+__device__ inline void exp_q_series(const double* w, double th2, double* q, LmCoef c) {
   const double h = 0.25 * th2;  // (th / 2)^2
-  const double k = 0.5 * horner(h, 1.0 / 6227020800.0, -1.0 / 39916800.0, 1.0 / 362880.0, -1.0 / 5040.0, 1.0 / 120.0,
-                                -1.0 / 6.0, 1.0);
+  const double k = 0.5 * horner7(h, c + LM_SIN);
   q[0] = k * w[0]; q[1] = k * w[1]; q[2] = k * w[2];
-  q[3] = horner(h, 1.0 / 479001600.0, -1.0 / 3628800.0, 1.0 / 40320.0, -1.0 / 720.0, 1.0 / 24.0, -0.5, 1.0);
+  q[3] = horner7(h, c + LM_COS);
   quat_renormalize(q);
 }
 
+// exp of twists outside the series' range: exp(xi) = exp(xi / 2^k)^(2^k).
+constexpr int LM_MAX_HALVINGS = 64;
+
 __device__ inline Pose lm_se3_exp(const double* xi) {
-  const double* w = xi + 3;
-  const double th2 = w[0] * w[0] + w[1] * w[1] + w[2] * w[2];
-  if (!(th2 <= LM_SERIES_TH2)) return se3_exp(xi);
+  const LmCoef cf = lm_coef();
+  double v[3] = {xi[0], xi[1], xi[2]}, w[3] = {xi[3], xi[4], xi[5]};
+  double th2 = w[0] * w[0] + w[1] * w[1] + w[2] * w[2];
+  int halvings = 0;
+  for (; th2 > LM_SERIES_TH2 && halvings < LM_MAX_HALVINGS; ++halvings, th2 *= 0.25)
+    for (int k = 0; k < 3; ++k) v[k] *= 0.5, w[k] *= 0.5;
   Pose r;
-  exp_q_series(w, th2, r.q);
-  const double b = horner(th2, 1.0 / 87178291200.0, -1.0 / 479001600.0, 1.0 / 3628800.0, -1.0 / 40320.0, 1.0 / 720.0,
-                          -1.0 / 24.0, 0.5);
-  const double c = horner(th2, 1.0 / 1307674368000.0, -1.0 / 6227020800.0, 1.0 / 39916800.0, -1.0 / 362880.0,
-                          1.0 / 5040.0, -1.0 / 120.0, 1.0 / 6.0);
-  apply_abc(1.0, b, c, w, xi, r.t);
+  exp_q_series(w, th2, r.q, cf);
+  apply_abc(1.0, horner7(th2, cf + LM_B), horner7(th2, cf + LM_C), w, v, r.t);
   r.s = 1.0;
+  for (; halvings > 0; --halvings) r = lm_pose_mul(r, r);
   return r;
 }
 
@@ -116,23 +140,32 @@ __device__ inline Pose lm_se3_exp(const double* xi) {
 // I_{k-1} = (e^sg - sg I_k) / k is stable and forgets its start
 // (I_16 ~ e^sg / 17) by sg^16 / 16!.
 __device__ inline Pose lm_sim3_exp(const double* xi) {
-  const double* w = xi + 3;
-  const double sg = xi[6];
-  const double th2 = w[0] * w[0] + w[1] * w[1] + w[2] * w[2];
-  if (!(th2 <= LM_SERIES_TH2 && fabs(sg) <= 0.5)) return sim3_exp(xi);
+  const LmCoef cf = lm_coef();
+  double v[3] = {xi[0], xi[1], xi[2]}, w[3] = {xi[3], xi[4], xi[5]};
+  double sg = xi[6];
+  double th2 = w[0] * w[0] + w[1] * w[1] + w[2] * w[2];
+  int halvings = 0;
+  for (; (th2 > LM_SERIES_TH2 || fabs(sg) > 0.5) && halvings < LM_MAX_HALVINGS; ++halvings, th2 *= 0.25, sg *= 0.5)
+    for (int k = 0; k < 3; ++k) v[k] *= 0.5, w[k] *= 0.5;
   Pose r;
-  exp_q_series(w, th2, r.q);
-  const double es = exp(sg);
-  double I[17];
-  I[16] = es * (1.0 / 17.0);
+  exp_q_series(w, th2, r.q, cf);
+  double es = cf[LM_FACT];
 #pragma unroll
-  for (int k = 16; k >= 1; --k) I[k - 1] = __builtin_fma(-sg, I[k], es) * (1.0 / k);
-  const double b = horner(th2, I[13] * (1.0 / 6227020800.0), I[11] * (-1.0 / 39916800.0), I[9] * (1.0 / 362880.0),
-                          I[7] * (-1.0 / 5040.0), I[5] * (1.0 / 120.0), I[3] * (-1.0 / 6.0), I[1]);
-  const double c = horner(th2, I[14] * (1.0 / 87178291200.0), I[12] * (-1.0 / 479001600.0), I[10] * (1.0 / 3628800.0),
-                          I[8] * (-1.0 / 40320.0), I[6] * (1.0 / 720.0), I[4] * (-1.0 / 24.0), I[2] * 0.5);
-  apply_abc(I[0], b, c, w, xi, r.t);
+  for (int k = 1; k < 14; ++k) es = __builtin_fma(sg, es, cf[LM_FACT + k]);
+  es = __builtin_fma(sg, __builtin_fma(sg, es, 1.0), 1.0);
+  // b and c take I_1 ... I_14 one at a time, downwards
+  double I = es * cf[LM_RECIP + 16], b = 0.0, c = 0.0;
+#pragma unroll
+  for (int k = 16; k >= 1; --k) {
+    I = __builtin_fma(-sg, I, es) * cf[LM_RECIP + k - 1];  // I_{k-1}
+    if (k - 1 >= 1 && k - 1 <= 14) {
+      if ((k - 1) & 1) b = __builtin_fma(th2, b, I * cf[LM_SIN + 6 - (k - 2) / 2]);
+      else c = __builtin_fma(th2, c, I * cf[LM_B + 6 - (k - 3) / 2]);
+    }
+  }
+  apply_abc(I, b, c, w, v, r.t);
   r.s = es;
+  for (; halvings > 0; --halvings) r = lm_pose_mul(r, r);
   return r;
 }
 
@@ -425,6 +458,17 @@ __device__ inline void lm_begin(JobState& s, const JobDesc& jd, const LmParams& 
   s.affB = 0.0f;
   if (jd.kind == LSDG_JOB_SIM3) begin_level<LSDG_JOB_SIM3>(s, jd, P, jd.startLevel, ntNext, remaining);
   else begin_level<LSDG_JOB_SE3>(s, jd, P, jd.startLevel, ntNext, remaining);
+}
+
+// The points [begin, end) of part `part` of `parts`: contiguous, whole and
+// within one of each other.
+struct PartRange {
+  int begin, end;
+};
+__device__ inline PartRange part_range(int n, int part, int parts) {
+  const int q = n / parts, r = n - q * parts;
+  const int b = part * q + min(part, r);
+  return {b, b + q + (part < r ? 1 : 0)};
 }
 
 // Copies a trivially copyable object between global memory and LDS with the

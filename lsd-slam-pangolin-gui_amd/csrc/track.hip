@@ -124,7 +124,7 @@ __global__ __launch_bounds__(EVAL_BS) void k_se3_eval(PointsLevel pts, const voi
                                                       double* __restrict__ out) {
   Accum<ACC, NS_SE3> acc;
   acc.zero();
-  se3_points<PREC, EVAL_U>(pts, blockIdx.x * EVAL_BS + threadIdx.x, gridDim.x * EVAL_BS, pts.n, img, g, x, kp, isGood,
+  se3_points<PREC, EVAL_U, SUMS_ALL>(pts, blockIdx.x * EVAL_BS + threadIdx.x, gridDim.x * EVAL_BS, pts.n, img, g, x, kp, isGood,
                            acc);
   reduce_and_merge(acc, partials, counter, out);
 }
@@ -138,7 +138,7 @@ __global__ __launch_bounds__(EVAL_BS) void k_sim3_eval(PointsLevel pts, const vo
                                                        double* __restrict__ out) {
   Accum<ACC, NS_SIM3> acc;
   acc.zero();
-  sim3_points<PREC, EVAL_U>(pts, blockIdx.x * EVAL_BS + threadIdx.x, gridDim.x * EVAL_BS, pts.n, img, fid, fvar, g, x,
+  sim3_points<PREC, EVAL_U, SUMS_ALL>(pts, blockIdx.x * EVAL_BS + threadIdx.x, gridDim.x * EVAL_BS, pts.n, img, fid, fvar, g, x,
                             kp, acc);
   reduce_and_merge(acc, partials, counter, out);
 }

@@ -68,6 +68,19 @@ __device__ inline Taps interp3(const void* img, float x, float y, int w) {
   return o;
 }
 
+// Loads and stores of device memory through a pointer that the compiler only
+// knows as a generic one (read from a job's descriptor): global accesses need
+// no wait for the LDS queue and return in order, flat ones do neither.
+template <class T>
+__device__ inline T gload(const T* p) {
+  static_assert(sizeof(T) % 4 == 0, "loaded as 32-bit words");
+  constexpr int N = sizeof(T) / 4;
+  typedef unsigned V __attribute__((ext_vector_type(N)));
+  const V v = *(const __attribute__((address_space(1))) V*)p;
+  return __builtin_bit_cast(T, v);
+}
+__device__ inline void gstore(uint8_t* p, uint8_t v) { *(__attribute__((address_space(1))) uint8_t*)p = v; }
+
 // The four raw taps of one bilinear sample, fetched ahead of their use so a
 // thread can keep several points' loads in flight.
 template <int PREC>
@@ -98,11 +111,12 @@ __device__ inline void fetch_taps(const void* img, float x, float y, int w, TapR
   int ix = (int)x, iy = (int)y;
   t.dx = x - (float)ix;
   t.dy = y - (float)iy;
-  int b = ix + iy * w;
-  t.a11 = im[b + 1 + w];
-  t.a01 = im[b + w];
-  t.a10 = im[b + 1];
-  t.a00 = im[b];
+  const T* r0 = im + (unsigned)(ix + iy * w);
+  const T* r1 = r0 + (unsigned)w;
+  t.a11 = gload(r1 + 1);
+  t.a01 = gload(r1);
+  t.a10 = gload(r0 + 1);
+  t.a00 = gload(r0);
 }
 
 // interp3's weighted sum of fetched taps (same operations, same order).
@@ -342,11 +356,42 @@ __device__ inline double swap_sum(double lo, double up, int offset) {
   return nl + nu;
 }
 
+// A value from the lane that offset h of the reduce-scatters below pairs with
+// this one, by data parallel primitives (no LDS round trip): h = 8 is a
+// rotation of the row of 16 by 8 (lane ^ 8), 4 the mirror of half a row
+// (lane ^ 7), 2 and 1 quad permutations (lane ^ 2, lane ^ 1).  lane ^ 7
+// differs from the lane in bit 2, as lane ^ 4 does, which is all the halving
+// needs; the pairings span the row all the same.
+template <int H>
+__device__ inline unsigned dpp_partner(unsigned x) {
+  constexpr int CTRL = H == 8 ? 0x128 : H == 4 ? 0x141 : H == 2 ? 0x4E : 0xB1;
+  return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xF, 0xF, false);
+}
+template <int H>
+__device__ inline double dpp_partner(double x) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(x);
+  const unsigned lo = dpp_partner<H>((unsigned)b), hi = dpp_partner<H>((unsigned)(b >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+template <int H>
+__device__ inline void halve_f64(double* a, int lane) {
+  const bool hi = (lane & H) != 0;
+#pragma unroll
+  for (int i = 0; i < H; ++i) {
+    const double send = hi ? a[i] : a[i + H];
+    const double keep = hi ? a[i + H] : a[i];
+    a[i] = keep + dpp_partner<H>(send);
+  }
+}
+
 // Reduce-scatter over the wave (NS <= 64): afterwards lane l holds the wave
-// total of value l (0 for l >= NS).  Halving butterfly: at offset o each lane
-// keeps one half of its values and receives the other half from lane ^ o.
+// total of value l (0 for l >= NS).  Halving butterfly: at each offset a lane
+// keeps one half of its values and receives the other half from its partner.
 // Offsets 32 and 16 use the permlane swaps (the sum of the swapped pair is
-// already the kept half: no lane selects); offsets 8..1 shuffle.
+// already the kept half: no lane selects), offsets 8..1 DPP moves.  Every
+// evaluation of an alignment ends in one, on its critical path; as shuffles
+// through the LDS the last four offsets waited for it four times.
 template <int NS>
 __device__ inline double wave_reduce_scatter_f64(const double* v) {
   static_assert(NS <= 64, "reduce-scatter holds one value per lane");
@@ -356,16 +401,10 @@ __device__ inline double wave_reduce_scatter_f64(const double* v) {
   for (int i = 0; i < 32; ++i) a[i] = i < NS ? swap_sum(v[i], (i + 32 < NS) ? v[i + 32] : 0.0, 32) : 0.0;
 #pragma unroll
   for (int i = 0; i < 16; ++i) a[i] = swap_sum(a[i], a[i + 16], 16);
-#pragma unroll
-  for (int h = 8; h >= 1; h >>= 1) {
-    const bool hi = (lane & h) != 0;
-#pragma unroll
-    for (int i = 0; i < h; ++i) {
-      double send = hi ? a[i] : a[i + h];
-      double keep = hi ? a[i + h] : a[i];
-      a[i] = keep + __shfl_xor(send, h);
-    }
-  }
+  halve_f64<8>(a, lane);
+  halve_f64<4>(a, lane);
+  halve_f64<2>(a, lane);
+  halve_f64<1>(a, lane);
   return a[0];
 }
 
@@ -375,11 +414,14 @@ struct Accum;
 template <int NS>
 struct Accum<ACC_F64, NS> {
   double v[NS];
+  int n[2];  // counts, one register each until set_count
   __device__ inline void zero() {
 #pragma unroll
     for (int k = 0; k < NS; ++k) v[k] = 0.0;
+    n[0] = n[1] = 0;
   }
   __device__ inline void add(int k, float x) { v[k] += (double)x; }
+  __device__ inline void set_count(int k, int c) { v[k] = (double)c; }
   __device__ inline void wave_reduce() {
 #pragma unroll
     for (int k = 0; k < NS; ++k) {
@@ -428,6 +470,19 @@ __device__ inline void unpack_pair(double cell, float& s, float& c) {
 
 // The reduce-scatter of wave_reduce_scatter_f64 over (sum, correction) pairs:
 // afterwards lane l holds the wave's pair of value l ((0, 0) for l >= NS).
+template <int H>
+__device__ inline void halve_pair(float* s, float* c, int lane) {
+  const bool hi = (lane & H) != 0;
+#pragma unroll
+  for (int i = 0; i < H; ++i) {
+    const float ss = hi ? s[i] : s[i + H], sc = hi ? c[i] : c[i + H];
+    float ks = hi ? s[i + H] : s[i], kc = hi ? c[i + H] : c[i];
+    pair_merge(ks, kc, __uint_as_float(dpp_partner<H>(__float_as_uint(ss))),
+               __uint_as_float(dpp_partner<H>(__float_as_uint(sc))));
+    s[i] = ks;
+    c[i] = kc;
+  }
+}
 template <int NS>
 __device__ inline void wave_reduce_scatter_pair(const float* vs, const float* vc, float& rs, float& rc) {
   static_assert(NS <= 64, "reduce-scatter holds one value per lane");
@@ -451,18 +506,10 @@ __device__ inline void wave_reduce_scatter_pair(const float* vs, const float* vc
     c[i] = __uint_as_float(b[0]);
     pair_merge(s[i], c[i], __uint_as_float(a[1]), __uint_as_float(b[1]));
   }
-#pragma unroll
-  for (int h = 8; h >= 1; h >>= 1) {
-    const bool hi = (lane & h) != 0;
-#pragma unroll
-    for (int i = 0; i < h; ++i) {
-      const float ss = hi ? s[i] : s[i + h], sc = hi ? c[i] : c[i + h];
-      float ks = hi ? s[i + h] : s[i], kc = hi ? c[i + h] : c[i];
-      pair_merge(ks, kc, __shfl_xor(ss, h), __shfl_xor(sc, h));
-      s[i] = ks;
-      c[i] = kc;
-    }
-  }
+  halve_pair<8>(s, c, lane);
+  halve_pair<4>(s, c, lane);
+  halve_pair<2>(s, c, lane);
+  halve_pair<1>(s, c, lane);
   rs = s[0];
   rc = c[0];
 }
@@ -470,11 +517,15 @@ __device__ inline void wave_reduce_scatter_pair(const float* vs, const float* vc
 template <int NS>
 struct Accum<ACC_KAHAN, NS> {
   float s[NS], c[NS];
+  int n[2];
   __device__ inline void zero() {
 #pragma unroll
     for (int k = 0; k < NS; ++k) s[k] = c[k] = 0.f;
+    n[0] = n[1] = 0;
   }
   __device__ inline void add(int k, float x) { kahan_add(s[k], c[k], x); }
+  // (a thread's count is far below 2^24, so the float holds it)
+  __device__ inline void set_count(int k, int c_) { s[k] = (float)c_; c[k] = 0.f; }
   // The LDS cell lane l of each wave writes for value l.
   __device__ inline double wave_slot() const {
     float rs, rc;
@@ -495,26 +546,50 @@ struct Accum<ACC_KAHAN, NS> {
   }
 };
 
+// Which of a point's sums the caller reads.  An LM step reads neither the
+// unweighted residuals nor, unless the affine brightness is estimated, the
+// affine statistics; leaving them out frees 12 of the loop's registers.
+constexpr int SUMS_LM = 0;         // the LM step's, no affine statistics
+constexpr int SUMS_LM_AFFINE = 1;  // the LM step's, affine statistics where kp.aff_stats asks for them
+constexpr int SUMS_ALL = 2;        // every slot (affine statistics where kp.aff_stats asks for them)
+
+// Values of LDS or memory that every lane of the wave reads alike, moved to
+// scalar registers: a loop over points then holds none of them in vector
+// registers.
+template <class T>
+__device__ inline T uniform(const T& x) {
+  static_assert(sizeof(T) % 4 == 0, "moved as 32-bit words");
+  constexpr int N = sizeof(T) / 4;
+  union {
+    T t;
+    unsigned w[N];
+  } u;
+  u.t = x;
+#pragma unroll
+  for (int k = 0; k < N; ++k) u.w[k] = __builtin_amdgcn_readfirstlane(u.w[k]);
+  return u.t;
+}
+
 // Index of (i, j), i <= j, in the row-major upper triangle of a 7x7 matrix.
 __host__ __device__ constexpr int tri7(int i, int j) { return i * 7 - i * (i - 1) / 2 + (j - i); }
 
 // One reference point of an SE3 evaluation: warp, bounds, taps, residual,
 // isGood, affine statistics, weights, Jacobian and normal-equation terms.
 // Rest of one SE3 point once its projection and taps are in hand.
-template <int PREC, class ACC>
+template <int PREC, int SUMS, class ACC>
 __device__ inline void se3_finish(const float4& p, float pvar, int pidx, const Proj& w, const TapRaw<PREC>& t,
                                   const Xf& x, const LevelGeom& g, const TrackKParams& kp,
                                   uint8_t* __restrict__ isGood, ACC& acc) {
   const float Wx = w.Wx, Wy = w.Wy;
   if (!w.in) {
-    if (isGood) isGood[pidx] = 0;
+    if (isGood) gstore(isGood + (unsigned)pidx, 0);
     return;
   }
   Taps ri = blend_taps<PREC>(t);
   float c1 = kp.aff_a * p.w + kp.aff_b;
   float c2 = ri.I;
   float r = c1 - c2;
-  if (kp.aff_stats) {  // affine-brightness statistics (read only when that estimation is on)
+  if (SUMS != SUMS_LM && kp.aff_stats) {  // affine-brightness statistics (read only when that estimation is on)
     float wgt = fabsf(r) < 5.0f ? 1.0f : fdiv<PREC>(5.0f, fabsf(r));
     acc.add(S3_SXX, c1 * c1 * wgt);
     acc.add(S3_SYY, c2 * c2 * wgt);
@@ -523,18 +598,16 @@ __device__ inline void se3_finish(const float4& p, float pvar, int pidx, const P
     acc.add(S3_SW, wgt);
   }
   bool good = ratio_below_one(r * r, kp.max_diff_constant + kp.max_diff_grad_mult * (ri.gx * ri.gx + ri.gy * ri.gy));
-  if (isGood) isGood[pidx] = good ? 1 : 0;
+  if (isGood) gstore(isGood + (unsigned)pidx, good ? 1 : 0);
   float gx = g.fx * ri.gx, gy = g.fy * ri.gy;
   const PointGeom q = point_geom<PREC, false>(p.z, w, x);
   if (good) {
-    acc.add(S3_RESUNW, r * r);
+    if (SUMS == SUMS_ALL) acc.add(S3_RESUNW, r * r);
     acc.add(S3_SIGNED, r);
-    acc.add(S3_GOOD, 1.0f);
-  } else {
-    acc.add(S3_BAD, 1.0f);
   }
+  acc.n[0] += good ? 1 : 0;
+  acc.n[1] += 1;
   acc.add(S3_USAGE, q.dc < 1.0f ? q.dc : 1.0f);
-  acc.add(S3_WARPED, 1.0f);
   // calcWeightsAndResidual
   float s = kp.var_weight * pvar;
   float drpdd = gx * q.g0 + gy * q.g1;
@@ -561,7 +634,7 @@ __device__ inline void se3_finish(const float4& p, float pvar, int pidx, const P
 // at a time: the U points' loads are issued, then their projections' taps,
 // then the U points are finished in index order (the per-thread summation
 // order of a one-point-at-a-time loop).
-template <int PREC, int U, class ACC>
+template <int PREC, int U, int SUMS, class ACC>
 __device__ inline void se3_points(const PointsLevel& pts, int i, int stride, int end, const void* __restrict__ img,
                                   const LevelGeom& g, const Xf& x, const TrackKParams& kp,
                                   uint8_t* __restrict__ isGood, ACC& acc) {
@@ -573,9 +646,9 @@ __device__ inline void se3_points(const PointsLevel& pts, int i, int stride, int
     for (int u = 0; u < U; ++u) {
       const int k = i + u * stride;
       if (k < end) {
-        p[u] = pts.posI[k];
-        pv[u] = pts.var[k];
-        pi[u] = isGood ? pts.idx[k] : 0;
+        p[u] = gload(pts.posI + (unsigned)k);
+        pv[u] = gload(pts.var + (unsigned)k);
+        pi[u] = isGood ? gload(pts.idx + (unsigned)k) : 0;
       }
     }
     Proj w[U];
@@ -589,13 +662,16 @@ __device__ inline void se3_points(const PointsLevel& pts, int i, int stride, int
     }
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (i + u * stride < end) se3_finish<PREC>(p[u], pv[u], pi[u], w[u], t[u], x, g, kp, isGood, acc);
+      if (i + u * stride < end) se3_finish<PREC, SUMS>(p[u], pv[u], pi[u], w[u], t[u], x, g, kp, isGood, acc);
   }
+  acc.set_count(S3_GOOD, acc.n[0]);
+  acc.set_count(S3_BAD, acc.n[1] - acc.n[0]);
+  acc.set_count(S3_WARPED, acc.n[1]);
 }
 
 // Rest of one Sim3 point (photometric + depth residual) once its
 // projection, taps and the frame's depth at the rounded pixel are in hand.
-template <int PREC, class ACC>
+template <int PREC, int SUMS, class ACC>
 __device__ inline void sim3_finish(const float4& p, float pvar, float2 rg, const Proj& w, const TapRaw<PREC>& t,
                                    float fidR, float varF, const Xf& x, const LevelGeom& g, const TrackKParams& kp,
                                    ACC& acc) {
@@ -615,7 +691,7 @@ __device__ inline void sim3_finish(const float4& p, float pvar, float2 rg, const
   float c1 = kp.aff_a * p.w + kp.aff_b;
   float c2 = ri.I;
   float rp = c1 - c2;
-  if (kp.aff_stats) {
+  if (SUMS != SUMS_LM && kp.aff_stats) {
     float wgt = fabsf(rp) < 2.0f ? 1.0f : fdiv<PREC>(2.0f, fabsf(rp));
     acc.add(SM_SXX, c1 * c1 * wgt);
     acc.add(SM_SYY, c2 * c2 * wgt);
@@ -633,7 +709,7 @@ __device__ inline void sim3_finish(const float4& p, float pvar, float2 rg, const
     vard = -1.0f;
   }
   acc.add(SM_USAGE, q.dc < 1.0f ? q.dc : 1.0f);
-  acc.add(SM_WARPED, 1.0f);
+  acc.n[1] += 1;
   // calcSim3WeightsAndResidual
   float s = kp.var_weight * pvar;
   float sv = kp.var_weight * vard;
@@ -647,7 +723,7 @@ __device__ inline void sim3_finish(const float4& p, float pvar, float2 rg, const
   float wh = huber_weight<PREC>(wabs, kp.huber);
   if (sv > 0.0f) {
     acc.add(SM_RESD, wh * w_d * rd * rd);
-    acc.add(SM_NTD, 1.0f);
+    acc.n[0] += 1;
   }
   acc.add(SM_RESP, wh * w_p * rp * rp);
   float wp = wh * w_p;
@@ -679,7 +755,7 @@ __device__ inline void sim3_finish(const float4& p, float pvar, float2 rg, const
 // Sim3 evaluation of points i, i + stride, ... < end of one thread, U points
 // at a time (loads first, then taps and the frame depth at the rounded
 // projection, then the points in index order).
-template <int PREC, int U, class ACC>
+template <int PREC, int U, int SUMS, class ACC>
 __device__ inline void sim3_points(const PointsLevel& pts, int i, int stride, int end, const void* __restrict__ img,
                                    const float* __restrict__ fid, const float* __restrict__ fvar, const LevelGeom& g,
                                    const Xf& x, const TrackKParams& kp, ACC& acc) {
@@ -691,9 +767,9 @@ __device__ inline void sim3_points(const PointsLevel& pts, int i, int stride, in
     for (int u = 0; u < U; ++u) {
       const int k = i + u * stride;
       if (k < end) {
-        p[u] = pts.posI[k];
-        pv[u] = pts.var[k];
-        rg[u] = kp.use_esm ? pts.grad[k] : make_float2(0.f, 0.f);
+        p[u] = gload(pts.posI + (unsigned)k);
+        pv[u] = gload(pts.var + (unsigned)k);
+        rg[u] = kp.use_esm ? gload(pts.grad + (unsigned)k) : make_float2(0.f, 0.f);
       }
     }
     Proj w[U];
@@ -706,15 +782,17 @@ __device__ inline void sim3_points(const PointsLevel& pts, int i, int stride, in
         if (w[u].in) {
           fetch_taps<PREC>(img, w[u].u, w[u].v, g.w, t[u]);
           int ir = (int)(w[u].u + 0.5f) + g.w * (int)(w[u].v + 0.5f);
-          fv[u] = fvar[ir];
-          fd[u] = fid[ir];
+          fv[u] = gload(fvar + (unsigned)ir);
+          fd[u] = gload(fid + (unsigned)ir);
         }
       }
     }
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (i + u * stride < end) sim3_finish<PREC>(p[u], pv[u], rg[u], w[u], t[u], fd[u], fv[u], x, g, kp, acc);
+      if (i + u * stride < end) sim3_finish<PREC, SUMS>(p[u], pv[u], rg[u], w[u], t[u], fd[u], fv[u], x, g, kp, acc);
   }
+  acc.set_count(SM_NTD, acc.n[0]);
+  acc.set_count(SM_WARPED, acc.n[1]);
 }
 
 // One reference point of the adjoint: dE/dxi into acc[0..6), E into acc[6],

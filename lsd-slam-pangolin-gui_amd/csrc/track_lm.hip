@@ -61,31 +61,37 @@ __global__ __launch_bounds__(TRACK_LM_BS) void k_track_lm(TrackLmArgs a) {
     if (tid < PYR) s.npts[tid] = jd.lv[tid].pts.n;
   }
   __syncthreads();
+  // every block takes part in every exchange: one that only read could be
+  // overtaken by the others' next rows
+  const int parts = a.blocks;
+  JobLevel L{};  // of level cur, as are split, i0 and i1 (in scalar registers)
+  int cur = -1, i0 = 0, i1 = 0;
+  bool split = false;
   unsigned gen = 0;  // exchanges so far
   for (int it = 0; it < BATCH_JOB_MAX_EVALS; ++it) {
     // s is read after a barrier: the exit test is uniform over the block
     if (s.status != 0) break;
-    const int lvl = s.level;
-    const JobLevel& L = jd.lv[lvl];
-    const int n = L.pts.n;
-    // every block takes part in every exchange: one that only read could be
-    // overtaken by the others' next rows
-    const int parts = a.blocks;
-    const bool split = parts > 1 && n > TRACK_LM_SOLO;
-    const int i0 = split ? (int)((long long)n * part / parts) : 0;
-    const int i1 = split ? (int)((long long)n * (part + 1) / parts) : n;
-    const Xf x = s.xf;
+    const int lvl = uniform(s.level);
+    if (lvl != cur) {
+      cur = lvl;
+      L = uniform(jd.lv[lvl]);
+      split = parts > 1 && L.pts.n > TRACK_LM_SOLO;
+      const PartRange r = split ? part_range(L.pts.n, part, parts) : PartRange{0, L.pts.n};
+      i0 = r.begin;
+      i1 = r.end;
+    }
+    const Xf x = uniform(s.xf);
     TrackKParams kp = a.kp;
-    kp.aff_a = s.affA;
-    kp.aff_b = s.affB;
+    kp.aff_a = uniform(s.affA);
+    kp.aff_b = uniform(s.affB);
     Accum<ACC, NS> acc;
     acc.zero();
     if (KIND == LSDG_JOB_SIM3) {
-      kp.roll[0] = s.roll[0]; kp.roll[1] = s.roll[1]; kp.roll[2] = s.roll[2]; kp.roll[3] = s.roll[3];
-      sim3_points<PREC, EVAL_U>(L.pts, i0 + tid, TRACK_LM_BS, i1, L.img, L.fid, L.fvar, L.g, x, kp, acc);
+      for (int k = 0; k < 4; ++k) kp.roll[k] = uniform(s.roll[k]);
+      sim3_points<PREC, EVAL_U, SUMS_LM_AFFINE>(L.pts, i0 + tid, TRACK_LM_BS, i1, L.img, L.fid, L.fvar, L.g, x, kp, acc);
     } else {
-      uint8_t* mask = lvl == 1 ? jd.isGood : nullptr;
-      se3_points<PREC, EVAL_U>(L.pts, i0 + tid, TRACK_LM_BS, i1, L.img, L.g, x, kp, mask, acc);
+      uint8_t* mask = lvl == 1 ? uniform(jd.isGood) : nullptr;
+      se3_points<PREC, EVAL_U, SUMS_LM_AFFINE>(L.pts, i0 + tid, TRACK_LM_BS, i1, L.img, L.g, x, kp, mask, acc);
     }
     const double wsum = acc.wave_slot();
     if (lane < NS) sh[wave][lane] = wsum;
