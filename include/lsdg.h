@@ -204,7 +204,9 @@ typedef struct lsdg_hypotheses {
 void lsdg_params_default(lsdg_params* p);
 
 /* One context per host thread: device, stream and the parameters that
- * settings.h / Conf() hold globally in the reference (tools/LSD.cpp:97-100). */
+ * settings.h / Conf() hold globally in the reference (tools/LSD.cpp:97-100).
+ * A context keeps up to 256 MiB of device and 16 MiB of pinned memory that its
+ * destroyed objects gave back, for the next ones; it ends with the context. */
 lsdg_status lsdg_ctx_create(int32_t device, const lsdg_params* params, lsdg_ctx* out);
 lsdg_status lsdg_ctx_destroy(lsdg_ctx ctx);
 lsdg_status lsdg_ctx_set_params(lsdg_ctx ctx, const lsdg_params* params);

@@ -51,9 +51,9 @@ __global__ __launch_bounds__(256) void k_batch_init(BatchArgs a) {
   if (threadIdx.x == 0) {
     *a.remaining = 0;
     // the run's epoch tags the cooperative row exchange; its low 16 bits
-    // never take the value 0, which the rows are cleared to on the first run
-    // and whenever the low bits wrap, so no word left by an earlier run can
-    // carry a tag of this one
+    // never take the value 0, which the plan's rows are cleared to when it is
+    // made (its epochs start behind 1) and here whenever the low bits wrap, so
+    // no word left by an earlier run can carry a tag of this one
     unsigned e = *a.epoch + 1;
     if ((e & 0xFFFFu) == 0) ++e;
     *a.epoch = e;

@@ -122,8 +122,8 @@ constexpr size_t TRACK_LM_WORDS = (size_t)2 * TRACK_LM_MAX_BLOCKS * NS_MAX * 2;
 // Blocks of a launch for alignments whose finest level has `pixels` pixels.
 int track_lm_blocks(lsdg_ctx c, int pixels);
 hipError_t launch_track_lm(const TrackLmArgs& a, int prec, int acc, hipStream_t s, const KTimer* t = nullptr);
-// Zeroes n tagged words (a fill kernel).
-hipError_t launch_track_lm_clear(unsigned long long* rows, size_t n, hipStream_t s);
+// Sets n 64-bit words (a fill kernel).
+hipError_t launch_fill_words(void* words, size_t n, unsigned long long value, hipStream_t s);
 
 hipError_t launch_batch_init(const BatchArgs& a, hipStream_t s);
 // Cooperative whole-LM kernel (a.coopK blocks of `bs` threads per job, all
@@ -148,7 +148,7 @@ hipError_t launch_batch_step(const BatchArgs& a, int kind, int prec, int acc, in
 // Plan shapes (capi_batch.cpp) and the tuning table (capi_tune.cpp).
 lsdg_batch_config batch_default_shape(lsdg_ctx c, int kind, int n);
 lsdg_status batch_create_shaped(lsdg_ctx c, const lsdg_job* jobs, int32_t n, const lsdg_batch_config& shape,
-                                lsdg_batch* out);
+                                bool oneRun, lsdg_batch* out);
 // The table's entry for key into *out; false when there is none.
 bool tune_table_lookup(const char* key, lsdg_batch_config* out);
 

@@ -245,7 +245,7 @@ lsdg_status lsdg::frame_alloc(lsdg_ctx c, int32_t id, const lsdg_camera* cam, in
   size_t off_u8 = take((size_t)f->w[0] * f->h[0]);
   size_t off_quad = take((size_t)f->w[0] * f->h[0] * 4);
   size_t off_wg = take((size_t)f->w[1] * f->h[1]);
-  hipError_t e = hipMalloc(&f->d_pool, total);
+  hipError_t e = c->blocks.get(&f->d_pool, total);
   if (e != hipSuccess) {
     delete f;
     return fail(c, LSDG_ENOMEM, "hipMalloc(frame)", e);
@@ -269,7 +269,7 @@ lsdg_status lsdg::frame_alloc(lsdg_ctx c, int32_t id, const lsdg_camera* cam, in
 extern "C" lsdg_status lsdg_frame_destroy(lsdg_frame f) {
   if (!f) return LSDG_EINVAL;
   (void)hipStreamSynchronize(f->ctx->stream);
-  if (f->d_pool) (void)hipFree(f->d_pool);
+  f->ctx->blocks.put(f->d_pool);
   delete f;
   return LSDG_OK;
 }
@@ -529,9 +529,8 @@ extern "C" lsdg_status lsdg_ref_create(lsdg_ctx c, lsdg_frame kf, lsdg_ref* out)
 extern "C" lsdg_status lsdg_ref_destroy(lsdg_ref r) {
   if (!r) return LSDG_EINVAL;
   (void)hipStreamSynchronize(r->ctx->stream);
-  for (int l = 0; l < PYR; ++l)
-    if (r->d_pool[l]) (void)hipFree(r->d_pool[l]);
-  if (r->d_counts) (void)hipFree(r->d_counts);
+  for (int l = 0; l < PYR; ++l) r->ctx->blocks.put(r->d_pool[l]);
+  r->ctx->blocks.put(r->d_counts);
   delete r;
   return LSDG_OK;
 }
@@ -743,7 +742,7 @@ static lsdg_status track_lm(lsdg_ctx c, lsdg_ref r, lsdg_frame f, int kind, cons
   // carries it
   c->track_epoch = (c->track_epoch + 1) & 0xFFFFu;
   if (c->track_epoch == 0) c->track_epoch = 1;
-  if (c->track_epoch == 1) CK(c, launch_track_lm_clear(c->d_track_rows, TRACK_LM_WORDS, c->stream));
+  if (c->track_epoch == 1) CK(c, launch_fill_words(c->d_track_rows, TRACK_LM_WORDS, 0ull, c->stream));
   a.epochTag = c->track_epoch << 16;
   KTimer kt = prof_timer(c);
   CK(c, launch_track_lm(a, f->precision, c->sums == LSDG_SUMS_KAHAN ? BATCH_ACC_KAHAN : BATCH_ACC_F64, c->stream, &kt));

@@ -54,7 +54,7 @@ struct lsdg_batch_s {
   unsigned* d_epoch = nullptr;           // per-chain run counters
   std::vector<lsdg_job> jobs;
   std::vector<int> depthVersion;
-  std::vector<JobDesc> h_jobs;
+  JobDesc* h_jobs = nullptr;  // pinned
   JobDesc* d_jobs = nullptr;
   JobState* d_st = nullptr;
   int* d_ntiles = nullptr;
@@ -75,30 +75,29 @@ struct lsdg_batch_s {
   void* d_pyr = nullptr;
   void* h_pyr = nullptr;
   PyrBatch pyr{};
+  // A plan that runs once is launched in stream order: its graphs' capture and
+  // instantiation would cost more than the launches (a search of eight
+  // candidates, three plans of 16 jobs: 1207 -> 614 us with the
+  // blocks kept).
+  bool graphs = true;
   hipGraphExec_t first = nullptr, cont = nullptr;
   hipGraph_t g_first = nullptr, g_cont = nullptr;
   JobState* h_st = nullptr;  // pinned: every graph ends by copying the control blocks here
 };
 
 static void batch_free(lsdg_batch b) {
+  (void)hipStreamSynchronize(b->ctx->stream);  // its pinned blocks may be read by queued copies
   if (b->first) (void)hipGraphExecDestroy(b->first);
   if (b->cont) (void)hipGraphExecDestroy(b->cont);
   if (b->g_first) (void)hipGraphDestroy(b->g_first);
   if (b->g_cont) (void)hipGraphDestroy(b->g_cont);
-  if (b->d_jobs) (void)hipFree(b->d_jobs);
-  if (b->d_st) (void)hipFree(b->d_st);
-  if (b->d_ntiles) (void)hipFree(b->d_ntiles);
-  if (b->d_counters) (void)hipFree(b->d_counters);
+  lsdg_ctx c = b->ctx;
+  for (void* p : {(void*)b->d_jobs, (void*)b->d_st, (void*)b->d_ntiles, (void*)b->d_counters, (void*)b->d_remaining,
+                  (void*)b->d_partials, (void*)b->d_coop, (void*)b->d_epoch, b->d_pyr})
+    c->blocks.put(p);
+  for (void* p : {(void*)b->h_jobs, (void*)b->h_remaining, (void*)b->h_st, b->h_pyr}) c->pinned.put(p);
   for (hipStream_t st : b->side) (void)hipStreamDestroy(st);
   for (hipEvent_t ev : b->forkJoin) (void)hipEventDestroy(ev);
-  if (b->d_remaining) (void)hipFree(b->d_remaining);
-  if (b->h_remaining) (void)hipHostFree(b->h_remaining);
-  if (b->h_st) (void)hipHostFree(b->h_st);
-  if (b->d_partials) (void)hipFree(b->d_partials);
-  if (b->d_coop) (void)hipFree(b->d_coop);
-  if (b->d_epoch) (void)hipFree(b->d_epoch);
-  if (b->d_pyr) (void)hipFree(b->d_pyr);
-  if (b->h_pyr) (void)hipHostFree(b->h_pyr);
   delete b;
 }
 
@@ -107,7 +106,7 @@ static void batch_free(lsdg_batch b) {
 static lsdg_status build_job_table(lsdg_batch b) {
   lsdg_ctx c = b->ctx;
   const int tile = 256 * b->ppt;
-  b->h_jobs.assign(b->n, JobDesc{});
+  for (int j = 0; j < b->n; ++j) b->h_jobs[j] = JobDesc{};
   size_t slot = 0;
   // queue every keyframe's point clouds before the first wait for a count
   for (const lsdg_job& J : b->jobs) {
@@ -148,13 +147,12 @@ static lsdg_status build_job_table(lsdg_batch b) {
   }
   const int NS = b->kind == LSDG_JOB_SIM3 ? NS_SIM3 : NS_SE3;
   if (slot > b->rows) {
-    if (b->d_partials) (void)hipFree(b->d_partials);
-    b->d_partials = nullptr;
-    CK(c, hipMalloc(&b->d_partials, sizeof(double) * NS * slot));
+    c->blocks.put(b->d_partials);
+    b->rows = 0;
+    CK(c, c->blocks.get(&b->d_partials, sizeof(double) * NS * slot));
     b->rows = slot;
   }
-  CK(c, hipMemcpyAsync(b->d_jobs, b->h_jobs.data(), sizeof(JobDesc) * b->n, hipMemcpyHostToDevice, c->stream));
-  CK(c, hipStreamSynchronize(c->stream));
+  CK(c, hipMemcpyAsync(b->d_jobs, b->h_jobs, sizeof(JobDesc) * b->n, hipMemcpyHostToDevice, c->stream));
   return LSDG_OK;
 }
 
@@ -321,7 +319,7 @@ static void env_shape(lsdg_batch_config& s, int n) {
 }
 
 lsdg_status lsdg::batch_create_shaped(lsdg_ctx c, const lsdg_job* jobs, int32_t n, const lsdg_batch_config& shape,
-                                      lsdg_batch* out) {
+                                      bool oneRun, lsdg_batch* out) {
   if (!out) return LSDG_EINVAL;
   lsdg_status vst = validate_jobs(c, jobs, n);
   if (vst != LSDG_OK) return vst;
@@ -379,16 +377,19 @@ lsdg_status lsdg::batch_create_shaped(lsdg_ctx c, const lsdg_job* jobs, int32_t 
   b->depthVersion.assign(n, -1);
   lsdg_status st = LSDG_OK;
   hipError_t e;
-  if ((e = hipMalloc(&b->d_jobs, sizeof(JobDesc) * n)) != hipSuccess ||
-      (e = hipMalloc(&b->d_st, sizeof(JobState) * n)) != hipSuccess ||
-      (e = hipMalloc(&b->d_ntiles, sizeof(int) * 2 * n)) != hipSuccess ||
-      (e = hipMalloc(&b->d_counters, sizeof(unsigned) * n)) != hipSuccess ||
-      (e = hipMalloc(&b->d_remaining, 64)) != hipSuccess ||
-      (b->coopK > 0 && (e = hipMalloc(&b->d_coop, sizeof(unsigned long long) * 2 * b->coopK * NS_SIM3 * 2 * (size_t)n)) !=
-                           hipSuccess) ||
-      (e = hipMalloc(&b->d_epoch, 64)) != hipSuccess || (e = hipMemset(b->d_epoch, 0, 64)) != hipSuccess ||
-      (e = hipHostMalloc(&b->h_remaining, 64, hipHostMallocDefault)) != hipSuccess ||
-      (e = hipHostMalloc(&b->h_st, sizeof(JobState) * n, hipHostMallocDefault)) != hipSuccess) {
+  const size_t coopWords = (size_t)2 * b->coopK * NS_SIM3 * 2 * (size_t)n;
+  if ((e = c->blocks.get(&b->d_jobs, sizeof(JobDesc) * n)) != hipSuccess ||
+      (e = c->blocks.get(&b->d_st, sizeof(JobState) * n)) != hipSuccess ||
+      (e = c->blocks.get(&b->d_ntiles, sizeof(int) * 2 * n)) != hipSuccess ||
+      (e = c->blocks.get(&b->d_counters, sizeof(unsigned) * n)) != hipSuccess ||
+      (e = c->blocks.get(&b->d_remaining, 64)) != hipSuccess ||
+      (b->coopK > 0 && (e = c->blocks.get(&b->d_coop, sizeof(unsigned long long) * coopWords)) != hipSuccess) ||
+      (b->coopK > 0 && (e = launch_fill_words(b->d_coop, coopWords, 0ull, c->stream)) != hipSuccess) ||
+      (e = c->blocks.get(&b->d_epoch, 64)) != hipSuccess ||
+      (e = launch_fill_words(b->d_epoch, 8, 0x100000001ull, c->stream)) != hipSuccess ||
+      (e = c->pinned.get(&b->h_jobs, sizeof(JobDesc) * n)) != hipSuccess ||
+      (e = c->pinned.get(&b->h_remaining, 64)) != hipSuccess ||
+      (e = c->pinned.get(&b->h_st, sizeof(JobState) * n)) != hipSuccess) {
     batch_free(b);
     return fail(c, LSDG_ENOMEM, "batch allocation", e);
   }
@@ -433,12 +434,12 @@ lsdg_status lsdg::batch_create_shaped(lsdg_ctx c, const lsdg_job* jobs, int32_t 
     b->rebuilt.push_back(std::find(b->pyrFrames.begin(), b->pyrFrames.end(), f) != b->pyrFrames.end());
   if (!b->pyrFrames.empty()) {
     size_t bytes = pyr_batch_bytes((int)b->pyrFrames.size());
-    if ((e = hipMalloc(&b->d_pyr, bytes)) != hipSuccess || (e = hipHostMalloc(&b->h_pyr, bytes)) != hipSuccess) {
+    if ((e = c->blocks.get(&b->d_pyr, bytes)) != hipSuccess || (e = c->pinned.get(&b->h_pyr, bytes)) != hipSuccess) {
       batch_free(b);
       return fail(c, LSDG_ENOMEM, "batch pyramid tables", e);
     }
     pyr_batch_tables(b->pyrFrames.data(), b->pyrNeed.data(), (int)b->pyrFrames.size(), b->h_pyr, b->d_pyr, &b->pyr);
-    if ((e = hipMemcpy(b->d_pyr, b->h_pyr, bytes, hipMemcpyHostToDevice)) != hipSuccess) {
+    if ((e = hipMemcpyAsync(b->d_pyr, b->h_pyr, bytes, hipMemcpyHostToDevice, c->stream)) != hipSuccess) {
       batch_free(b);
       return fail(c, LSDG_EDEVICE, "batch pyramid tables", e);
     }
@@ -455,11 +456,13 @@ lsdg_status lsdg::batch_create_shaped(lsdg_ctx c, const lsdg_job* jobs, int32_t 
   if (!std::getenv("LSDG_BATCH_STEPS")) {
     // no multi-block steps in the first graph when every level runs in k_batch_job
     int maxPts = 0;
-    for (const JobDesc& d : b->h_jobs)
-      for (int l = 0; l < PYR; ++l) maxPts = std::max(maxPts, d.lv[l].pts.n);
+    for (int j = 0; j < n; ++j)
+      for (int l = 0; l < PYR; ++l) maxPts = std::max(maxPts, b->h_jobs[j].lv[l].pts.n);
     if (maxPts <= b->jobMaxPoints) b->steps = 0;
   }
-  if ((st = batch_graphs(b)) != LSDG_OK) {
+  // the step schedule's chains run side by side only as graph branches
+  b->graphs = !oneRun || b->coopK == 0;
+  if (b->graphs && (st = batch_graphs(b)) != LSDG_OK) {
     batch_free(b);
     return st;
   }
@@ -467,7 +470,7 @@ lsdg_status lsdg::batch_create_shaped(lsdg_ctx c, const lsdg_job* jobs, int32_t 
   return LSDG_OK;
 }
 
-extern "C" lsdg_status lsdg_batch_create(lsdg_ctx c, const lsdg_job* jobs, int32_t n, lsdg_batch* out) {
+static lsdg_status batch_create(lsdg_ctx c, const lsdg_job* jobs, int32_t n, bool oneRun, lsdg_batch* out) {
   if (!c || !jobs || !out || n < 1) return LSDG_EINVAL;
   lsdg_status st = validate_jobs(c, jobs, n);
   if (st != LSDG_OK) return st;
@@ -476,7 +479,11 @@ extern "C" lsdg_status lsdg_batch_create(lsdg_ctx c, const lsdg_job* jobs, int32
   char key[LSDG_TUNE_KEY_BYTES];
   if (lsdg_batch_tune_key(c, jobs, n, key) == LSDG_OK) tune_table_lookup(key, &shape);
   env_shape(shape, n);
-  return batch_create_shaped(c, jobs, n, shape, out);
+  return batch_create_shaped(c, jobs, n, shape, oneRun, out);
+}
+
+extern "C" lsdg_status lsdg_batch_create(lsdg_ctx c, const lsdg_job* jobs, int32_t n, lsdg_batch* out) {
+  return batch_create(c, jobs, n, false, out);
 }
 
 extern "C" lsdg_status lsdg_batch_create_with_config(lsdg_ctx c, const lsdg_job* jobs, int32_t n,
@@ -484,7 +491,7 @@ extern "C" lsdg_status lsdg_batch_create_with_config(lsdg_ctx c, const lsdg_job*
   if (!c || !jobs || !config || !out || n < 1) return LSDG_EINVAL;
   if (config->schedule != LSDG_SCHEDULE_COOP && config->schedule != LSDG_SCHEDULE_STEPS)
     return fail(c, LSDG_EINVAL, "unknown schedule");
-  return batch_create_shaped(c, jobs, n, *config, out);
+  return batch_create_shaped(c, jobs, n, *config, false, out);
 }
 
 extern "C" lsdg_status lsdg_batch_get_config(lsdg_batch b, lsdg_batch_config* out) {
@@ -503,7 +510,6 @@ extern "C" lsdg_status lsdg_batch_get_config(lsdg_batch b, lsdg_batch_config* ou
 
 extern "C" lsdg_status lsdg_batch_destroy(lsdg_batch b) {
   if (!b) return LSDG_EINVAL;
-  (void)hipStreamSynchronize(b->ctx->stream);
   batch_free(b);
   return LSDG_OK;
 }
@@ -566,9 +572,10 @@ static void fill_result(lsdg_batch b, int j, const JobState& s, lsdg_job_result*
   r->status = LSDG_OK;
 }
 
-// The same work as the graphs, launched in stream order with an event pair
-// around every LM-step kernel (and the pyramid rebuild) for lsdg_ctx_profile.
-static lsdg_status batch_run_profiled(lsdg_batch b) {
+// The same work as the graphs, launched in stream order: for a plan without
+// graphs, and for lsdg_ctx_profile with an event pair around every LM-step
+// kernel (and the pyramid rebuild).
+static lsdg_status batch_run_launched(lsdg_batch b) {
   lsdg_ctx c = b->ctx;
   if (b->pyr.nf > 0) {
     double pb = 0.0;
@@ -602,13 +609,15 @@ static lsdg_status batch_run_profiled(lsdg_batch b) {
         prof_timer_done(c, LSDG_KERNEL_BATCH_SOLVE, ks, 0.0);
       }
       CK(c, hipMemcpyAsync(b->h_remaining + k, b->d_remaining + k, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+      CK(c, hipMemcpyAsync(b->h_st + chain_begin(b, k), b->d_st + chain_begin(b, k), sizeof(JobState) * a.njobs,
+                           hipMemcpyDeviceToHost, c->stream));
       CK(c, hipStreamSynchronize(c->stream));
       if (b->h_remaining[k] < 0) return fail(c, LSDG_EDEVICE, "batched LM: cooperative blocks not co-resident");
       done = b->h_remaining[k] <= 0;
     }
     if (!done) return fail(c, LSDG_ESTATE, "batched LM did not finish");
   }
-  return prof_resolve(c);
+  return c->prof_on ? prof_resolve(c) : LSDG_OK;
 }
 
 static int remaining_jobs(lsdg_batch b) {
@@ -653,11 +662,11 @@ extern "C" lsdg_status lsdg_batch_run(lsdg_batch b, lsdg_job_result* results) {
   for (int j = 0; j < b->n; ++j) stale |= b->jobs[j].ref->kf->depthVersion != b->depthVersion[j];
   if (stale) {
     lsdg_status st = build_job_table(b);
-    if (st == LSDG_OK) st = batch_graphs(b);
+    if (st == LSDG_OK && b->graphs) st = batch_graphs(b);
     if (st != LSDG_OK) return st;
   }
-  if (c->prof_on) {
-    lsdg_status st = batch_run_profiled(b);
+  if (c->prof_on || !b->graphs) {
+    lsdg_status st = batch_run_launched(b);
     if (st != LSDG_OK) return st;
   } else {
     CK(c, hipGraphLaunch(b->first, c->stream));
@@ -691,7 +700,6 @@ extern "C" lsdg_status lsdg_batch_run(lsdg_batch b, lsdg_job_result* results) {
   // the graph rebuilt these frames' levels
   for (size_t k = 0; k < b->pyrFrames.size(); ++k) b->pyrFrames[k]->valid |= b->pyrNeed[k];
   if (results || c->prof_on) {
-    if (c->prof_on) CK(c, hipMemcpy(b->h_st, b->d_st, sizeof(JobState) * b->n, hipMemcpyDeviceToHost));
     if (results)
       for (int j = 0; j < b->n; ++j) fill_result(b, j, b->h_st[j], &results[j]);
     if (c->prof_on) {
@@ -717,7 +725,7 @@ extern "C" lsdg_status lsdg_batch_run(lsdg_batch b, lsdg_job_result* results) {
 
 extern "C" lsdg_status lsdg_batch_track(lsdg_ctx c, const lsdg_job* jobs, int32_t n, lsdg_job_result* results) {
   lsdg_batch b = nullptr;
-  lsdg_status st = lsdg_batch_create(c, jobs, n, &b);
+  lsdg_status st = batch_create(c, jobs, n, true, &b);
   if (st != LSDG_OK) return st;
   st = lsdg_batch_run(b, results);
   lsdg_batch_destroy(b);

@@ -18,12 +18,9 @@ using namespace lsdg;
 static constexpr unsigned KF_DATA = fd_bit(FD_GRAD, 0) | fd_bit(FD_MAXG, 0);
 
 static void free_dm(lsdg_depthmap dm) {
-  if (dm->d_pool) (void)hipFree(dm->d_pool);
-  if (dm->d_refs) (void)hipFree(dm->d_refs);
-  if (dm->d_refById) (void)hipFree(dm->d_refById);
-  if (dm->h_refs) (void)hipHostFree(dm->h_refs);
-  if (dm->h_refById) (void)hipHostFree(dm->h_refById);
-  if (dm->h_red) (void)hipHostFree(dm->h_red);
+  lsdg_ctx c = dm->ctx;
+  for (void* p : {(void*)dm->d_pool, (void*)dm->d_refs, (void*)dm->d_refById}) c->blocks.put(p);
+  for (void* p : {(void*)dm->h_refs, (void*)dm->h_refById, (void*)dm->h_red}) c->pinned.put(p);
   delete dm;
 }
 
@@ -65,7 +62,7 @@ extern "C" lsdg_status lsdg_depthmap_create(lsdg_ctx c, const lsdg_camera* cam, 
   size_t o_obs = take(n), o_iv = take(n * 8), o_head = take(n * 4), o_next = take(n * 4),
          o_mean = take(mean_rows(g.w, g.h) * sizeof(double2)), o_work = take(obs_work_slots(g.w, g.h) * 16),
          o_wc = take(OBS_COUNT_BYTES);
-  hipError_t e = hipMalloc(&dm->d_pool, total);
+  hipError_t e = c->blocks.get(&dm->d_pool, total);
   if (e != hipSuccess) {
     free_dm(dm);
     return fail(c, LSDG_ENOMEM, "hipMalloc(depth map)", e);
@@ -86,7 +83,7 @@ extern "C" lsdg_status lsdg_depthmap_create(lsdg_ctx c, const lsdg_camera* cam, 
   dm->d_work = (int4*)(b + o_work);
   dm->d_work_count = (int*)(b + o_wc);
   if ((e = hipMemsetAsync(dm->d_pool, 0, total, c->stream)) != hipSuccess ||
-      (e = hipHostMalloc(&dm->h_red, 64, hipHostMallocMapped)) != hipSuccess ||
+      (e = c->pinned.get(&dm->h_red, 64)) != hipSuccess ||
       (e = hipHostGetDevicePointer((void**)&dm->d_red_out, dm->h_red, 0)) != hipSuccess ||
       (e = hipStreamSynchronize(c->stream)) != hipSuccess) {
     free_dm(dm);
@@ -214,23 +211,25 @@ static void prepare_stereo(const DepthGeom& g, const Pose& thisToOther, StereoRe
 static lsdg_status ensure_ref_storage(lsdg_depthmap dm, int nrefs, int nbyid) {
   lsdg_ctx c = dm->ctx;
   if (nrefs > dm->refs_cap) {
-    if (dm->d_refs) (void)hipFree(dm->d_refs);
-    if (dm->h_refs) (void)hipHostFree(dm->h_refs);
+    CK(c, hipStreamSynchronize(c->stream));
+    c->blocks.put(dm->d_refs);
+    c->pinned.put(dm->h_refs);
     dm->d_refs = nullptr;
     dm->h_refs = nullptr;
     dm->refs_cap = 0;
-    CK(c, hipMalloc(&dm->d_refs, sizeof(StereoRef) * nrefs));
-    CK(c, hipHostMalloc(&dm->h_refs, sizeof(StereoRef) * nrefs, hipHostMallocDefault));
+    CK(c, c->blocks.get(&dm->d_refs, sizeof(StereoRef) * nrefs));
+    CK(c, c->pinned.get(&dm->h_refs, sizeof(StereoRef) * nrefs));
     dm->refs_cap = nrefs;
   }
   if (nbyid > dm->refById_cap) {
-    if (dm->d_refById) (void)hipFree(dm->d_refById);
-    if (dm->h_refById) (void)hipHostFree(dm->h_refById);
+    CK(c, hipStreamSynchronize(c->stream));
+    c->blocks.put(dm->d_refById);
+    c->pinned.put(dm->h_refById);
     dm->d_refById = nullptr;
     dm->h_refById = nullptr;
     dm->refById_cap = 0;
-    CK(c, hipMalloc(&dm->d_refById, sizeof(int) * nbyid));
-    CK(c, hipHostMalloc(&dm->h_refById, sizeof(int) * nbyid, hipHostMallocDefault));
+    CK(c, c->blocks.get(&dm->d_refById, sizeof(int) * nbyid));
+    CK(c, c->pinned.get(&dm->h_refById, sizeof(int) * nbyid));
     dm->refById_cap = nbyid;
   }
   return LSDG_OK;

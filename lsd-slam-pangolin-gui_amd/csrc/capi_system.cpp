@@ -7,6 +7,7 @@
 // relocaliser (upstream's Relocalizer, fed by trackFrame while tracking is
 // lost) over one batched SE3 plan per image.  Single-threaded and
 // deterministic; the pose graph and loop closures are not part of it.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <deque>
@@ -135,38 +136,47 @@ extern "C" lsdg_status lsdg_system_init_random(lsdg_system s, int32_t id, const 
 
 // Frame::meanIdepth of frame k: the float mean, in raster order, of the
 // level-0 idepth setDepth wrote (pixels without depth hold -1).
+// The sum is one chain of additions, so the values are first gathered without
+// a branch (every third pixel or so has depth, in no order that a branch
+// predictor finds), from pinned memory where the image is of a usual size.
+constexpr size_t MEAN_PINNED_BYTES = (size_t)8 << 20;
 static lsdg_status frame_mean_idepth(lsdg_system s, lsdg_frame k, float* out) {
   const size_t n = (size_t)s->cam.w * s->cam.h;
-  std::vector<float> d(n);
-  lsdg_status st = lsdg_frame_read(k, LSDG_WHAT_IDEPTH, 0, d.data(), n * sizeof(float));
-  if (st != LSDG_OK) return st;
-  float sum = 0.0f;
-  int num = 0;
-  for (size_t i = 0; i < n; ++i)
-    if (d[i] != -1.0f) {
-      sum += d[i];
-      ++num;
+  lsdg_ctx c = s->ctx;
+  float* d = nullptr;
+  const bool pinned = n * sizeof(float) <= MEAN_PINNED_BYTES && c->pinned.get(&d, n * sizeof(float)) == hipSuccess;
+  if (!pinned) {
+    s->scratch.resize(n);
+    d = s->scratch.data();
+  }
+  lsdg_status st = lsdg_frame_read(k, LSDG_WHAT_IDEPTH, 0, d, n * sizeof(float));
+  if (st == LSDG_OK) {
+    float sum = 0.0f, got[1024];
+    int num = 0;
+    for (size_t i = 0; i < n;) {
+      const size_t end = std::min(n, i + 1024);
+      int m = 0;
+      for (; i < end; ++i) {
+        got[m] = d[i];
+        m += d[i] != -1.0f ? 1 : 0;
+      }
+      for (int j = 0; j < m; ++j) sum += got[j];
+      num += m;
     }
-  *out = sum / (float)num;
-  return LSDG_OK;
+    *out = sum / (float)num;
+  } else {
+    (void)hipStreamSynchronize(c->stream);  // a copy into d may be queued
+  }
+  if (pinned) c->pinned.put(d);
+  return st;
 }
 
 // meanIdepth of the current keyframe, cached per depth version.
 static lsdg_status mean_idepth(lsdg_system s, float* out) {
   lsdg_frame k = s->kf.get();
   if (s->meanFor != k || s->meanVersion != k->depthVersion) {
-    const size_t n = (size_t)s->cam.w * s->cam.h;
-    s->scratch.resize(n);
-    lsdg_status st = lsdg_frame_read(k, LSDG_WHAT_IDEPTH, 0, s->scratch.data(), n * sizeof(float));
+    lsdg_status st = frame_mean_idepth(s, k, &s->meanIdepth);
     if (st != LSDG_OK) return st;
-    float sum = 0.0f;
-    int num = 0;
-    for (size_t i = 0; i < n; ++i)
-      if (s->scratch[i] != -1.0f) {
-        sum += s->scratch[i];
-        ++num;
-      }
-    s->meanIdepth = sum / (float)num;
     s->meanFor = k;
     s->meanVersion = k->depthVersion;
   }
@@ -254,10 +264,7 @@ static lsdg_status reloc_checks(lsdg_system s, lsdg_frame f, const std::vector<i
   lsdg_status st = lsdg_ctx_set_params(c, &q);
   if (st != LSDG_OK) return st;
   std::vector<lsdg_job_result> res(n);
-  lsdg_batch b = nullptr;
-  st = lsdg_batch_create(c, jobs.data(), n, &b);
-  if (st == LSDG_OK) st = lsdg_batch_run(b, res.data());
-  if (b) lsdg_batch_destroy(b);
+  st = lsdg_batch_track(c, jobs.data(), n, res.data());
   lsdg_ctx_set_params(c, &saved);
   if (st != LSDG_OK) return st;
   const double thr = 1.0 - 0.75 * (1.0 - (double)saved.min_goodpergoodbad_pixel);

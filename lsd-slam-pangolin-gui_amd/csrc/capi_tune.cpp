@@ -326,7 +326,7 @@ struct Search {
   // (which also sizes the plan's step graphs); *taken = the plan's shape.
   lsdg_status measure(const lsdg_batch_config& want, lsdg_batch_config* taken, double* ms) {
     lsdg_batch b = nullptr;
-    lsdg_status st = batch_create_shaped(c, jobs, n, want, &b);
+    lsdg_status st = batch_create_shaped(c, jobs, n, want, false, &b);
     if (st != LSDG_OK) return st;
     lsdg_batch_get_config(b, taken);
     for (auto& s : seen)

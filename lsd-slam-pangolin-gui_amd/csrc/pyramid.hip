@@ -702,10 +702,10 @@ constexpr size_t PC_ROOM_MAX = (size_t)1 << 22;
 
 static hipError_t pc_storage(lsdg_ref r, int l, size_t points) {
   if (points <= (size_t)r->cap[l] && r->d_pool[l]) return hipSuccess;
-  if (r->d_pool[l]) (void)hipFree(r->d_pool[l]);
+  r->ctx->blocks.put(r->d_pool[l]);  // its last readers are queued on the context's stream, as its next users will be
   r->d_pool[l] = nullptr;
   r->cap[l] = 0;
-  hipError_t e = hipMalloc(&r->d_pool[l], points * (sizeof(float4) + sizeof(float) + sizeof(float2) + sizeof(int)) + 256);
+  hipError_t e = r->ctx->blocks.get(&r->d_pool[l], points * (sizeof(float4) + sizeof(float) + sizeof(float2) + sizeof(int)) + 256);
   if (e == hipSuccess) r->cap[l] = (int)points;
   return e;
 }
@@ -716,7 +716,7 @@ hipError_t launch_point_clouds(lsdg_ref r, unsigned levels, hipStream_t s) {
   int tile0[PYR + 1] = {0};
   for (int l = 0; l < PYR; ++l) tile0[l + 1] = tile0[l] + (f->w[l] * f->h[l] + PC_TILE - 1) / PC_TILE;
   if (!r->d_counts) {
-    e = hipMalloc(&r->d_counts, sizeof(int) * (PYR + tile0[PYR]));
+    e = r->ctx->blocks.get(&r->d_counts, sizeof(int) * (PYR + tile0[PYR]));
     if (e != hipSuccess) return e;
   }
   PcArgs a;

@@ -158,8 +158,8 @@ __global__ __launch_bounds__(TRACK_LM_BS) void k_track_lm(TrackLmArgs a) {
   }
 }
 
-__global__ __launch_bounds__(256) void k_track_lm_clear(unsigned long long* rows, size_t n) {
-  for (size_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) rows[i] = 0ull;
+__global__ __launch_bounds__(256) void k_fill_words(unsigned long long* words, size_t n, unsigned long long value) {
+  for (size_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) words[i] = value;
 }
 
 int track_lm_blocks(lsdg_ctx c, int pixels) {
@@ -188,8 +188,9 @@ hipError_t launch_track_lm(const TrackLmArgs& a, int prec, int acc, hipStream_t 
   return launch_k(k, dim3(a.blocks), dim3(TRACK_LM_BS), s, t, a);
 }
 
-hipError_t launch_track_lm_clear(unsigned long long* rows, size_t n, hipStream_t s) {
-  k_track_lm_clear<<<dim3((unsigned)std::min<size_t>((n + 255) / 256, 256)), dim3(256), 0, s>>>(rows, n);
+hipError_t launch_fill_words(void* words, size_t n, unsigned long long value, hipStream_t s) {
+  k_fill_words<<<dim3((unsigned)std::min<size_t>((n + 255) / 256, 256)), dim3(256), 0, s>>>(
+      (unsigned long long*)words, n, value);
   return hipGetLastError();
 }
 
