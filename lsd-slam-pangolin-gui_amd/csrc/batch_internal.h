@@ -122,8 +122,6 @@ constexpr size_t TRACK_LM_WORDS = (size_t)2 * TRACK_LM_MAX_BLOCKS * NS_MAX * 2;
 // Blocks of a launch for alignments whose finest level has `pixels` pixels.
 int track_lm_blocks(lsdg_ctx c, int pixels);
 hipError_t launch_track_lm(const TrackLmArgs& a, int prec, int acc, hipStream_t s, const KTimer* t = nullptr);
-// Sets n 64-bit words (a fill kernel).
-hipError_t launch_fill_words(void* words, size_t n, unsigned long long value, hipStream_t s);
 
 hipError_t launch_batch_init(const BatchArgs& a, hipStream_t s);
 // Cooperative whole-LM kernel (a.coopK blocks of `bs` threads per job, all

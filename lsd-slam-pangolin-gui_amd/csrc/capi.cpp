@@ -123,7 +123,7 @@ extern "C" lsdg_status lsdg_ctx_create(int32_t device, const lsdg_params* params
   c->partials_blocks = 4096;
   if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
       hipMalloc(&c->d_partials, sizeof(double) * NS_MAX * c->partials_blocks) != hipSuccess ||
-      hipMalloc(&c->d_counter, 64) != hipSuccess || hipMemset(c->d_counter, 0, 64) != hipSuccess ||
+      hipMalloc(&c->d_eval_rows, sizeof(unsigned long long) * EVAL_ROW_WORDS) != hipSuccess ||
       hipHostMalloc(&c->h_result, sizeof(double) * 64, hipHostMallocMapped) != hipSuccess ||
       hipHostGetDevicePointer((void**)&c->d_result, c->h_result, 0) != hipSuccess ||
       hipMalloc(&c->d_track_rows, sizeof(unsigned long long) * TRACK_LM_WORDS) != hipSuccess ||
@@ -146,7 +146,7 @@ extern "C" lsdg_status lsdg_ctx_destroy(lsdg_ctx c) {
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   if (c->d_partials) (void)hipFree(c->d_partials);
-  if (c->d_counter) (void)hipFree(c->d_counter);
+  if (c->d_eval_rows) (void)hipFree(c->d_eval_rows);
   if (c->h_result) (void)hipHostFree(c->h_result);
   if (c->d_track_rows) (void)hipFree(c->d_track_rows);
   if (c->h_track) (void)hipHostFree(c->h_track);

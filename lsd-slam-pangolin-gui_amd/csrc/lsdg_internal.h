@@ -31,6 +31,8 @@ constexpr int PYR = LSDG_PYRAMID_LEVELS;
 constexpr int NS_SE3 = 40;
 constexpr int NS_SIM3 = 48;
 constexpr int NS_MAX = 48;
+constexpr int EVAL_MAX_BLOCKS = 128;  // blocks of one evaluation (track.hip)
+constexpr size_t EVAL_ROW_WORDS = (size_t)EVAL_MAX_BLOCKS * NS_MAX * 2;
 
 // Pyramid data of a frame, one validity bit per (kind, level): the
 // reference's Frame::require() flags (IMAGE, GRADIENTS, MAX_GRADIENTS), built
@@ -138,55 +140,6 @@ __device__ inline void fuse4(const float* ida, const float* va, float& oid, floa
   }
 }
 
-// The merge by the last block of a launch: out[k] = the sum over b of
-// rows[b * NS + k], in block order (k < NS; BS threads).  The rows are staged
-// through LDS a chunk at a time, every thread issuing its agent-scope atomic
-// loads back to back (the rows were written with agent-scope stores; no L2
-// invalidation needed), so a chunk costs one memory round trip rather than
-// one per row; NS lanes then add their column in block order, as a
-// sequential loop over the rows would.
-constexpr int MERGE_CHUNK = 2048;  // doubles staged per round (16 KB of LDS)
-template <int NS, int BS>
-__device__ inline void merge_rows(const double* __restrict__ rows, unsigned nrows, double* __restrict__ out) {
-  static_assert(MERGE_CHUNK % BS == 0 && NS <= BS, "merge layout");
-  constexpr int LOADS = MERGE_CHUNK / BS;
-  __shared__ double stage[MERGE_CHUNK];
-  const unsigned total = nrows * NS;
-  double s = 0.0;
-  for (unsigned base = 0; base < total; base += MERGE_CHUNK) {
-    const unsigned m = min((unsigned)MERGE_CHUNK, total - base);
-    unsigned long long v[LOADS];
-#pragma unroll
-    for (int u = 0; u < LOADS; ++u) {
-      const unsigned i = threadIdx.x + u * BS;
-      v[u] = i < m ? __hip_atomic_load((const unsigned long long*)&rows[base + i], __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT)
-                   : 0ull;
-    }
-#pragma unroll
-    for (int u = 0; u < LOADS; ++u) {
-      const unsigned i = threadIdx.x + u * BS;
-      if (i < m) stage[i] = __longlong_as_double((long long)v[u]);
-    }
-    __syncthreads();
-    if (threadIdx.x < NS) {
-      // this column's entries of the chunk, added in row order; eight LDS
-      // reads are in flight ahead of the additions
-      unsigned i = (threadIdx.x + NS - base % NS) % NS;
-      for (; i + 7 * NS < m; i += 8 * NS) {
-        double r[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) r[u] = stage[i + u * NS];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) s += r[u];
-      }
-      for (; i < m; i += NS) s += stage[i];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x < NS) out[threadIdx.x] = s;
-}
-
 struct PyrBatch {
   const void* img_args;
   const void* grad_args;
@@ -284,7 +237,8 @@ struct lsdg_ctx_s {
   // reduction scratch for the plain (one-alignment-at-a-time) path
   double* d_partials = nullptr;
   int partials_blocks = 0;
-  unsigned* d_counter = nullptr;
+  unsigned long long* d_eval_rows = nullptr;  // tagged rows of one evaluation, and the launch that tags them
+  unsigned eval_epoch = 0;
   double* h_result = nullptr;  // pinned, host-mapped
   double* d_result = nullptr;  // device view of h_result
   int num_cus = 256;
@@ -431,6 +385,8 @@ size_t vbo_block_count(int w, int h);
 hipError_t launch_vbo(const lsdg_point_dense* in, const VboArgs& a, int* blk, lsdg_vertex* out, hipStream_t s);
 
 // track.hip
+// Sets n 64-bit words (a fill kernel).
+hipError_t launch_fill_words(void* words, size_t n, unsigned long long value, hipStream_t s);
 hipError_t launch_se3_eval(lsdg_ctx c, const PointsLevel& pts, lsdg_frame f, int level, const Xf& x,
                            const TrackKParams& kp, uint8_t* d_isgood, double* d_out, const KTimer* t = nullptr);
 hipError_t launch_sim3_eval(lsdg_ctx c, const PointsLevel& pts, lsdg_frame f, int level, const Xf& x,

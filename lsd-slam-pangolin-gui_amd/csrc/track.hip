@@ -11,9 +11,9 @@
 //   per thread  FP64 accumulation of the FP32 per-point terms over a
 //               grid-stride slice of points (or, with LSDG_SUMS_KAHAN,
 //               Kahan-compensated FP32 pairs),
-//   per wave    butterfly (__shfl_xor; pairs: TwoSum reduce-scatter),
+//   per wave    reduce-scatter (pairs: by TwoSum),
 //   per block   sum of the wave results in LDS -> one FP64 partial row,
-//   last block  FP64 sum of all partial rows in block order (deterministic),
+//   block 0     FP64 sum of all partial rows in a fixed order (deterministic),
 //               written straight to the caller's (possibly host-mapped) buffer.
 // The per-point float expressions keep the reference's operation order so the
 // isGood mask and counts match the CPU restatement bit for bit.
@@ -23,63 +23,84 @@
 
 namespace lsdg {
 
-// Block-wide reduction of the per-thread accumulators into one FP64 partial
-// row, then the last block to finish merges all rows in block order.
+// This block's FP64 row in sh[0][0 .. NS): the wave results added in wave order.
 template <int MODE, int NS>
-__device__ inline void reduce_and_merge(Accum<MODE, NS>& acc, double* __restrict__ partials, unsigned* counter,
-                                        double* __restrict__ out) {
-  __shared__ double sh[EVAL_WAVES][NS];
-  __shared__ bool amLast;
+__device__ inline double block_row(const Accum<MODE, NS>& acc, double (&sh)[EVAL_WAVES][NS]) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if constexpr (MODE == ACC_F64) {
-    acc.wave_reduce();
-    if (lane == 0) {
+  const double cell = acc.wave_slot();
+  if (lane < NS) sh[wave][lane] = cell;
+  __syncthreads();
+  return threadIdx.x < NS ? Accum<MODE, NS>::merge_waves(&sh[0][threadIdx.x], NS, EVAL_WAVES) : 0.0;
+}
+
+// Block-wide reduction of the per-thread accumulators into one FP64 row, then
+// block 0 adds the rows of all blocks: the waves take a quarter of the rows
+// each, in block order, and their sums are added in wave order.  A row is
+// published as tagged words (k_track_lm's exchange: half a value and the
+// launch's tag in each), so block 0 sees by the words themselves which rows
+// are there: a store and a load on the critical path, where a completion
+// counter takes a store, a wait for it, an atomic and a load.  No block waits
+// for block 0, so its wait ends.
+template <int MODE, int NS>
+__device__ inline void reduce_and_merge(const Accum<MODE, NS>& acc, unsigned long long* __restrict__ rows,
+                                        unsigned tag, double* __restrict__ out) {
+  __shared__ double sh[EVAL_WAVES][NS];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nb = gridDim.x;
+  const double v = block_row(acc, sh);
+  if (nb == 1) {
+    if (tid < NS) out[tid] = v;
+    return;
+  }
+  if (tid < NS) {
+    const unsigned long long bits = (unsigned long long)__double_as_longlong(v), t64 = (unsigned long long)tag << 32;
+    unsigned long long* w = rows + ((size_t)blockIdx.x * NS + tid) * 2;
+    __hip_atomic_store(w, t64 | (bits & 0xFFFFFFFFull), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(w + 1, t64 | (bits >> 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (blockIdx.x != 0) return;
+  __syncthreads();  // sh is read above and written below
+  const int q1 = nb * (wave + 1) / EVAL_WAVES;
+  double sum = 0.0;
+  constexpr int AHEAD = 8;
+  for (int q = nb * wave / EVAL_WAVES; q < q1;) {
+    // the rows' loads go out together; the ones that are there in order are
+    // added, the rest are looked at again
+    unsigned long long lo[AHEAD], hi[AHEAD];
 #pragma unroll
-      for (int k = 0; k < NS; ++k) sh[wave][k] = acc.value(k);
+    for (int u = 0; u < AHEAD; ++u) {
+      const unsigned long long* w = rows + ((size_t)min(q + u, q1 - 1) * NS + (lane < NS ? lane : 0)) * 2;
+      lo[u] = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      hi[u] = __hip_atomic_load(w + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-  } else {
-    const double cell = acc.wave_slot();
-    if (lane < NS) sh[wave][lane] = cell;
+    int got = 0;
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      const bool there = __all((unsigned)(lo[u] >> 32) == tag && (unsigned)(hi[u] >> 32) == tag);
+      if (got == u && q + u < q1 && there) {
+        sum += __longlong_as_double((long long)((hi[u] << 32) | (lo[u] & 0xFFFFFFFFull)));
+        got = u + 1;
+      }
+    }
+    q += got;
+    if (got == 0) __builtin_amdgcn_s_sleep(1);
   }
+  if (lane < NS) sh[wave][lane] = sum;
   __syncthreads();
-  if (threadIdx.x < NS) {
-    const double s = Accum<MODE, NS>::merge_waves(&sh[0][threadIdx.x], NS, EVAL_WAVES);
-    __hip_atomic_store((unsigned long long*)&partials[(size_t)blockIdx.x * NS + threadIdx.x],
-                       (unsigned long long)__double_as_longlong(s), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (tid < NS) {
+    double t = sh[0][tid];
+    for (int w = 1; w < EVAL_WAVES; ++w) t += sh[w][tid];
+    out[tid] = t;
   }
-  wait_own_stores();
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned prev = atomicAdd(counter, 1u);
-    amLast = (prev == gridDim.x - 1);
-  }
-  __syncthreads();
-  if (!amLast) return;
-  merge_rows<NS, EVAL_BS>(partials, gridDim.x, out);
-  if (threadIdx.x == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Block-wide reduction of the per-thread accumulators into this block's FP64
-// row (the merge is a second launch, k_merge_rows: no completion counter, so
-// no same-address atomics, which serialise once the grid has more than a
-// few hundred blocks).
+// row (the merge is a second launch, k_merge_rows: the adjoint's grid has up
+// to a few hundred blocks more than one block should add).
 template <int MODE, int NS>
-__device__ inline void reduce_to_row(Accum<MODE, NS>& acc, double* __restrict__ rows) {
+__device__ inline void reduce_to_row(const Accum<MODE, NS>& acc, double* __restrict__ rows) {
   __shared__ double sh[EVAL_WAVES][NS];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if constexpr (MODE == ACC_F64) {
-    acc.wave_reduce();
-    if (lane == 0) {
-#pragma unroll
-      for (int k = 0; k < NS; ++k) sh[wave][k] = acc.value(k);
-    }
-  } else {
-    const double cell = acc.wave_slot();
-    if (lane < NS) sh[wave][lane] = cell;
-  }
-  __syncthreads();
-  if (threadIdx.x < NS)
-    rows[(size_t)blockIdx.x * NS + threadIdx.x] = Accum<MODE, NS>::merge_waves(&sh[0][threadIdx.x], NS, EVAL_WAVES);
+  const double v = block_row(acc, sh);
+  if (threadIdx.x < NS) rows[(size_t)blockIdx.x * NS + threadIdx.x] = v;
 }
 
 // out[k] = the sum of rows[b * NS + k] over the nrows blocks, in a fixed
@@ -120,13 +141,13 @@ __global__ __launch_bounds__(EVAL_BS) void k_merge_rows(const double* __restrict
 template <int PREC, int ACC>
 __global__ __launch_bounds__(EVAL_BS) void k_se3_eval(PointsLevel pts, const void* __restrict__ img, LevelGeom g,
                                                       Xf x, TrackKParams kp, uint8_t* __restrict__ isGood,
-                                                      double* __restrict__ partials, unsigned* counter,
+                                                      unsigned long long* __restrict__ rows, unsigned tag,
                                                       double* __restrict__ out) {
   Accum<ACC, NS_SE3> acc;
   acc.zero();
   se3_points<PREC, EVAL_U, SUMS_ALL>(pts, blockIdx.x * EVAL_BS + threadIdx.x, gridDim.x * EVAL_BS, pts.n, img, g, x, kp, isGood,
                            acc);
-  reduce_and_merge(acc, partials, counter, out);
+  reduce_and_merge(acc, rows, tag, out);
 }
 
 // ------------------------------------------------------------------ Sim3
@@ -134,13 +155,13 @@ template <int PREC, int ACC>
 __global__ __launch_bounds__(EVAL_BS) void k_sim3_eval(PointsLevel pts, const void* __restrict__ img,
                                                        const float* __restrict__ fid, const float* __restrict__ fvar,
                                                        LevelGeom g, Xf x, TrackKParams kp,
-                                                       double* __restrict__ partials, unsigned* counter,
+                                                       unsigned long long* __restrict__ rows, unsigned tag,
                                                        double* __restrict__ out) {
   Accum<ACC, NS_SIM3> acc;
   acc.zero();
   sim3_points<PREC, EVAL_U, SUMS_ALL>(pts, blockIdx.x * EVAL_BS + threadIdx.x, gridDim.x * EVAL_BS, pts.n, img, fid, fvar, g, x,
                             kp, acc);
-  reduce_and_merge(acc, partials, counter, out);
+  reduce_and_merge(acc, rows, tag, out);
 }
 
 // --------------------------------------------------------------- adjoint
@@ -174,17 +195,25 @@ __global__ __launch_bounds__(EVAL_BS) void k_energy_grad_sim3(PointsLevel pts, c
 
 // ------------------------------------------------------------ launchers
 // Plain-path evaluation grid: one point per thread (the shortest dependency
-// chain per thread; 1.74k frames/s on the 64 headline instances against 1.61k
-// at four points per thread), at most EVAL_MAX_BLOCKS blocks: every block
-// adds once to the launch's completion counter, and same-address atomics
-// serialise, so larger levels take more points per thread instead.
-constexpr int EVAL_MAX_BLOCKS = 256;
-static inline int eval_blocks(lsdg_ctx c, int n) {
+// chain per thread), at most EVAL_MAX_BLOCKS blocks: block 0 reads a row of
+// each.  Eight evaluations (levels 1-4, SE3 and Sim3) with at most 32, 64, 128
+// and 256 blocks: 640x480 180, 175, 176, 176 us; 1280x960 (FP16) 194, 184, 182,
+// 186.  With a completion counter, shuffles through the LDS in the wave
+// reduction and one column of additions in the last block's merge they took
+// 216 and 240 us (the kernel 12 us on average, now 6.8; the rest of a call is
+// its launch and wait).
+static inline int eval_blocks(int n) {
   int nb = (n + EVAL_BS - 1) / EVAL_BS;
   if (nb < 1) nb = 1;
   if (nb > EVAL_MAX_BLOCKS) nb = EVAL_MAX_BLOCKS;
-  if (nb > c->partials_blocks) nb = c->partials_blocks;
   return nb;
+}
+
+// The next launch's tag: never 0, which the rows are cleared to at the first
+// launch and whenever the tags start over.
+static hipError_t next_eval(lsdg_ctx c) {
+  if (++c->eval_epoch == 0) c->eval_epoch = 1;
+  return c->eval_epoch == 1 ? launch_fill_words(c->d_eval_rows, EVAL_ROW_WORDS, 0ull, c->stream) : hipSuccess;
 }
 
 static inline const void* level_image(lsdg_frame f, int level) {
@@ -207,20 +236,24 @@ static auto kern_sim3_eval(int prec) {
 hipError_t launch_se3_eval(lsdg_ctx c, const PointsLevel& pts, lsdg_frame f, int level, const Xf& x,
                            const TrackKParams& kp, uint8_t* d_isgood, double* d_out, const KTimer* t) {
   LevelGeom g{f->w[level], f->h[level], f->fx[level], f->fy[level], f->cx[level], f->cy[level]};
-  const dim3 grid(eval_blocks(c, pts.n)), block(EVAL_BS);
+  const dim3 grid(eval_blocks(pts.n)), block(EVAL_BS);
   const void* img = level_image(f, level);
+  hipError_t e = next_eval(c);
+  if (e != hipSuccess) return e;
   auto k = c->sums == LSDG_SUMS_KAHAN ? kern_se3_eval<ACC_KAHAN>(f->precision) : kern_se3_eval<ACC_F64>(f->precision);
-  return launch_k(k, grid, block, c->stream, t, pts, img, g, x, kp, d_isgood, c->d_partials, c->d_counter, d_out);
+  return launch_k(k, grid, block, c->stream, t, pts, img, g, x, kp, d_isgood, c->d_eval_rows, c->eval_epoch, d_out);
 }
 
 hipError_t launch_sim3_eval(lsdg_ctx c, const PointsLevel& pts, lsdg_frame f, int level, const Xf& x,
                             const TrackKParams& kp, double* d_out, const KTimer* t) {
   LevelGeom g{f->w[level], f->h[level], f->fx[level], f->fy[level], f->cx[level], f->cy[level]};
-  const dim3 grid(eval_blocks(c, pts.n)), block(EVAL_BS);
+  const dim3 grid(eval_blocks(pts.n)), block(EVAL_BS);
   const void* img = level_image(f, level);
+  hipError_t e = next_eval(c);
+  if (e != hipSuccess) return e;
   auto k = c->sums == LSDG_SUMS_KAHAN ? kern_sim3_eval<ACC_KAHAN>(f->precision) : kern_sim3_eval<ACC_F64>(f->precision);
   return launch_k(k, grid, block, c->stream, t, pts, img, (const float*)f->d_idepth[level],
-                  (const float*)f->d_ivar[level], g, x, kp, c->d_partials, c->d_counter, d_out);
+                  (const float*)f->d_ivar[level], g, x, kp, c->d_eval_rows, c->eval_epoch, d_out);
 }
 
 // Adjoint grid: two points per thread (one, two and four measure within 10%

@@ -12,17 +12,6 @@
 
 namespace lsdg {
 
-// Waits until this wave's earlier memory operations have completed.  Stores
-// made as agent-scope atomics (sc1) are coherent at agent scope once complete,
-// so a wait orders them before a later counter update with no write-back of
-// the XCD's L2 (which an agent-scope release adds for ordinary stores).  The
-// signal fences keep the compiler from moving memory operations across it.
-__device__ inline void wait_own_stores() {
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
-  __builtin_amdgcn_s_waitcnt(0);
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
-}
-
 constexpr int EVAL_BS = 256;
 constexpr int EVAL_WAVES = EVAL_BS / 64;
 constexpr int EVAL_U = 2;  // points per thread with loads in flight together (plain kernels)
@@ -422,16 +411,6 @@ struct Accum<ACC_F64, NS> {
   }
   __device__ inline void add(int k, float x) { v[k] += (double)x; }
   __device__ inline void set_count(int k, int c) { v[k] = (double)c; }
-  __device__ inline void wave_reduce() {
-#pragma unroll
-    for (int k = 0; k < NS; ++k) {
-      double a = v[k];
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) a += __shfl_xor(a, off);
-      v[k] = a;
-    }
-  }
-  __device__ inline double value(int k) const { return v[k]; }
   __device__ inline double wave_slot() const { return wave_reduce_scatter_f64<NS>(v); }
   __device__ static inline double merge_waves(const double* cells, int stride, int waves) {
     double t = 0.0;
