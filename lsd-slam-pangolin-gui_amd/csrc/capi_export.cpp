@@ -16,17 +16,17 @@ extern "C" void lsdg_vbo_params_default(lsdg_vbo_params* p) {
   p->min_near_support = 9;
 }
 
-// Scratch for n pixels: records | block offsets | vertices.
+// Scratch for n pixels: records | the filter's masks and counts | vertices.
 struct ExportScratch {
   lsdg_point_dense* rec;
-  int* blk;
+  void* vbo;
   lsdg_vertex* vtx;
 };
 
 static lsdg_status export_scratch(lsdg_ctx c, int w, int h, ExportScratch* out) {
   const size_t n = (size_t)w * h;
   auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
-  const size_t oRec = 0, oBlk = up(n * sizeof(lsdg_point_dense)), oVtx = oBlk + up((vbo_block_count(w, h) + 1) * 4);
+  const size_t oRec = 0, oBlk = up(n * sizeof(lsdg_point_dense)), oVtx = oBlk + up(vbo_scratch_bytes(w, h));
   const size_t total = oVtx + up(n * sizeof(lsdg_vertex));
   if (total > c->exportCap) {
     CK(c, hipStreamSynchronize(c->stream));
@@ -38,7 +38,7 @@ static lsdg_status export_scratch(lsdg_ctx c, int w, int h, ExportScratch* out) 
   }
   char* b = (char*)c->d_export;
   out->rec = (lsdg_point_dense*)(b + oRec);
-  out->blk = (int*)(b + oBlk);
+  out->vbo = b + oBlk;
   out->vtx = (lsdg_vertex*)(b + oVtx);
   return LSDG_OK;
 }
@@ -59,27 +59,42 @@ static VboArgs vbo_args(int w, int h, float fx, float fy, float cx, float cy, co
   return a;
 }
 
+// Depth and image of frame f at `level` are there.
+static lsdg_status exportable(lsdg_frame f, int level) {
+  if (!f->hasDepth) return fail(f->ctx, LSDG_ESTATE, "keyframe has no depth");
+  return frame_require(f, fd_bit(FD_IMAGE, level));
+}
+
 // Records of frame f at `level` into s.rec (device).
 static lsdg_status dense_records(lsdg_frame f, int level, const ExportScratch& s) {
   lsdg_ctx c = f->ctx;
-  if (!f->hasDepth) return fail(c, LSDG_ESTATE, "keyframe has no depth");
-  lsdg_status st = frame_require(f, fd_bit(FD_IMAGE, level));
+  lsdg_status st = exportable(f, level);
   if (st != LSDG_OK) return st;
   CK(c, launch_kf_dense(f->d_idepth[level], f->d_ivar[level], f->d_image[level], f->w[level] * f->h[level], s.rec,
                         c->stream));
   return LSDG_OK;
 }
 
-// Runs the filter on s.rec and copies the kept vertices to host `out`.
-static lsdg_status run_vbo(lsdg_ctx c, const VboArgs& a, const ExportScratch& s, lsdg_vertex* out, int32_t* count) {
-  const int nb = (int)vbo_block_count(a.w, a.h);
-  int total = 0;
-  if (nb > 0) {
-    CK(c, launch_vbo(s.rec, a, s.blk, s.vtx, c->stream));
-    CK(c, hipMemcpyAsync(&total, s.blk + nb, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    CK(c, hipStreamSynchronize(c->stream));
+// The device's view of host memory that it can write (pinned), or null.
+static void* device_view(void* host) {
+  hipPointerAttribute_t at{};
+  if (hipPointerGetAttributes(&at, host) != hipSuccess) {
+    (void)hipGetLastError();  // ordinary host memory
+    return nullptr;
   }
-  if (total > 0) {
+  return at.type == hipMemoryTypeHost ? at.devicePointer : nullptr;
+}
+
+// Runs the filter (`launch` is given where the count and the vertices go) and
+// brings the kept vertices to host `out`: written there by the kernel when the
+// buffer is pinned, copied after the count is known otherwise.
+template <class F>
+static lsdg_status run_vbo(lsdg_ctx c, const ExportScratch& s, lsdg_vertex* out, int32_t* count, F&& launch) {
+  lsdg_vertex* pinned = (lsdg_vertex*)device_view(out);
+  CK(c, launch((int*)c->d_result, pinned ? pinned : s.vtx));
+  CK(c, hipStreamSynchronize(c->stream));
+  const int total = *(const volatile int*)c->h_result;
+  if (total > 0 && !pinned) {
     CK(c, hipMemcpyAsync(out, s.vtx, sizeof(lsdg_vertex) * (size_t)total, hipMemcpyDeviceToHost, c->stream));
     CK(c, hipStreamSynchronize(c->stream));
   }
@@ -108,7 +123,9 @@ extern "C" lsdg_status lsdg_points_vbo(lsdg_ctx c, const lsdg_point_dense* in, i
   lsdg_status st = export_scratch(c, w, h, &s);
   if (st != LSDG_OK) return st;
   CK(c, hipMemcpyAsync(s.rec, in, sizeof(lsdg_point_dense) * (size_t)w * h, hipMemcpyHostToDevice, c->stream));
-  return run_vbo(c, vbo_args(w, h, fx, fy, cx, cy, *p), s, out, count);
+  const VboArgs a = vbo_args(w, h, fx, fy, cx, cy, *p);
+  return run_vbo(c, s, out, count,
+                 [&](int* total, lsdg_vertex* v) { return launch_vbo(s.rec, a, s.vbo, total, v, c->stream); });
 }
 
 extern "C" lsdg_status lsdg_keyframe_vbo(lsdg_frame kf, int32_t level, const lsdg_vbo_params* p, lsdg_vertex* out,
@@ -118,7 +135,10 @@ extern "C" lsdg_status lsdg_keyframe_vbo(lsdg_frame kf, int32_t level, const lsd
   const int w = kf->w[level], h = kf->h[level];
   ExportScratch s;
   lsdg_status st = export_scratch(c, w, h, &s);
-  if (st == LSDG_OK) st = dense_records(kf, level, s);
+  if (st == LSDG_OK) st = exportable(kf, level);
   if (st != LSDG_OK) return st;
-  return run_vbo(c, vbo_args(w, h, kf->fx[level], kf->fy[level], kf->cx[level], kf->cy[level], *p), s, out, count);
+  const VboArgs a = vbo_args(w, h, kf->fx[level], kf->fy[level], kf->cx[level], kf->cy[level], *p);
+  return run_vbo(c, s, out, count, [&](int* total, lsdg_vertex* v) {
+    return launch_vbo(kf->d_idepth[level], kf->d_ivar[level], kf->d_image[level], a, s.vbo, total, v, c->stream);
+  });
 }

@@ -6,10 +6,10 @@
 //                  (lib/Pangolin_IOWrapper/PangolinOutputIOWrapper.cpp:81-89):
 //                  idepth, idepth variance and the image as four color bytes.
 //   k_vbo_count,   Keyframe::computeVbo (lib/Pangolin_IOWrapper/Keyframe.h:
-//   k_vbo_scan,    91-142) as a stream compaction that keeps the viewer's
-//   k_vbo_write    raster order: per-block counts of the kept pixels, one
-//                  scan, then each block writes its kept pixels at its offset
-//                  in lane order.  Every float expression keeps the
+//   k_vbo_write    91-142) as a stream compaction that keeps the viewer's
+//                  raster order: a mask of kept pixels and their count per
+//                  tile, then each tile adds up the counts before it and
+//                  writes its kept pixels.  Every float expression keeps the
 //                  reference's operation order (no contraction), so the
 //                  vertices match a sequential loop bit for bit.
 #include "lsdg_internal.h"
@@ -37,25 +37,43 @@ __global__ __launch_bounds__(256) void k_kf_dense(const float* __restrict__ id, 
   out[i] = p;
 }
 
-__device__ inline bool vbo_keep(const lsdg_point_dense* __restrict__ in, int x, int y, const VboArgs& a,
-                                float& depth) {
+// Where the filter's input comes from: the point records, or the arrays of the
+// keyframe that k_kf_dense would make them from.
+struct VboRecords {
+  const lsdg_point_dense* in;
+  __device__ float idepth(int i) const { return in[i].idepth; }
+  __device__ float var(int i) const { return in[i].idepth_var; }
+  __device__ void color(int i, uint8_t* c) const {
+    for (int k = 0; k < 3; ++k) c[k] = in[i].color[k];
+  }
+};
+struct VboFrame {
+  const float *id, *iv, *img;
+  __device__ float idepth(int i) const { return id[i]; }
+  __device__ float var(int i) const { return iv[i]; }
+  __device__ void color(int i, uint8_t* c) const { c[0] = c[1] = c[2] = color_byte(img[i]); }
+};
+
+template <class SRC>
+__device__ inline bool vbo_keep(const SRC& in, int x, int y, const VboArgs& a) {
   const int w = a.w;
   if (x < 1 || x >= w - 1 || y < 1 || y >= a.h - 1) return false;
-  const lsdg_point_dense c = in[x + y * w];
-  if (c.idepth <= 0) return false;
-  depth = 1 / c.idepth;
+  const float idepth = in.idepth(x + y * w);
+  if (idepth <= 0) return false;
+  const float var = in.var(x + y * w);
+  const float depth = 1 / idepth;
   float depth4 = depth * depth;
   depth4 *= depth4;
-  if (c.idepth_var * depth4 > a.scaledTH) return false;
-  if (c.idepth_var * depth4 * a.scale * a.scale > a.absTH) return false;
+  if (var * depth4 > a.scaledTH) return false;
+  if (var * depth4 * a.scale * a.scale > a.absTH) return false;
   if (a.minNear > 1) {
     int near = 0;
     for (int dx = -1; dx < 2; dx++)
       for (int dy = -1; dy < 2; dy++) {
-        const float nid = in[x + dx + (y + dy) * w].idepth;
+        const float nid = in.idepth(x + dx + (y + dy) * w);
         if (nid > 0) {
           const float diff = nid - 1.0f / depth;
-          if (diff * diff < 2 * c.idepth_var) near++;
+          if (diff * diff < 2 * var) near++;
         }
       }
     if (near < a.minNear) return false;
@@ -63,17 +81,27 @@ __device__ inline bool vbo_keep(const lsdg_point_dense* __restrict__ in, int x, 
   return true;
 }
 
-// Kept pixels of block b (pixels 256 b .. 256 b + 255 in raster order).
-__global__ __launch_bounds__(256) void k_vbo_count(const lsdg_point_dense* __restrict__ in, VboArgs a,
-                                                   int* __restrict__ blk) {
+// A tile is VBO_TILE pixels in raster order, VBO_PX rounds of a block.
+// mask[16 tile + 4 i + v] holds the kept pixels of wave v in round i.
+constexpr int VBO_PX = 4;
+constexpr int VBO_TILE = 256 * VBO_PX;
+
+template <class SRC>
+__global__ __launch_bounds__(256) void k_vbo_count(SRC in, VboArgs a, unsigned long long* __restrict__ mask,
+                                                   int* __restrict__ tiles) {
   __shared__ int wc[4];
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  float depth;
-  const bool keep = i < a.w * a.h && vbo_keep(in, i % a.w, i / a.w, a, depth);
-  const unsigned long long m = __ballot(keep);
-  if (__lane_id() == 0) wc[threadIdx.x >> 6] = __popcll(m);
+  const int wave = threadIdx.x >> 6;
+  int c = 0;
+#pragma unroll
+  for (int r = 0; r < VBO_PX; ++r) {
+    const int i = blockIdx.x * VBO_TILE + r * 256 + (int)threadIdx.x;
+    const unsigned long long m = __ballot(i < a.w * a.h && vbo_keep(in, i % a.w, i / a.w, a));
+    if (__lane_id() == 0) mask[(size_t)blockIdx.x * 16 + r * 4 + wave] = m;
+    c += __popcll(m);
+  }
+  if (__lane_id() == 0) wc[wave] = c;
   __syncthreads();
-  if (threadIdx.x == 0) blk[blockIdx.x] = wc[0] + wc[1] + wc[2] + wc[3];
+  if (threadIdx.x == 0) tiles[blockIdx.x] = wc[0] + wc[1] + wc[2] + wc[3];
 }
 
 // Exclusive scan of blk[0, nb) in place, blk[nb] = total; one block.
@@ -101,31 +129,54 @@ __global__ __launch_bounds__(1024) void k_vbo_scan(int* blk, int nb) {
   if (threadIdx.x == 0) blk[nb] = carry;
 }
 
-__global__ __launch_bounds__(256) void k_vbo_write(const lsdg_point_dense* __restrict__ in, VboArgs a,
-                                                   const int* __restrict__ blk, lsdg_vertex* __restrict__ out) {
-  __shared__ int wc[4];
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  const int x = i % a.w, y = i / a.w;
-  float depth = 0.0f;
-  const bool keep = i < a.w * a.h && vbo_keep(in, x, y, a, depth);
-  const unsigned long long m = __ballot(keep);
-  const int wave = threadIdx.x >> 6;
-  if (__lane_id() == 0) wc[wave] = __popcll(m);
+// The kept pixels of a tile, behind those of the tiles before it (whose counts
+// the block adds up itself, or with `scanned` finds added up).  They are
+// gathered in LDS and leave in whole lines: `out` may be host memory, where a
+// few vertices per store would be a bus transaction each.  A record per pixel,
+// a count, a scan, a write and a copy behind a wait for the count took 51 us for
+// a keyframe of 640x480; two launches and one wait take 27.
+template <class SRC>
+__global__ __launch_bounds__(256) void k_vbo_write(SRC in, VboArgs a, const unsigned long long* __restrict__ mask,
+                                                   const int* __restrict__ tiles, int scanned, int* __restrict__ total,
+                                                   lsdg_vertex* __restrict__ out) {
+  static_assert(sizeof(lsdg_vertex) == sizeof(uint4), "vertices move as 16-byte words");
+  __shared__ uint4 stage[VBO_TILE];
+  __shared__ int before[4];
+  const int tile = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (!scanned) {
+    int part = 0;
+    for (int t = threadIdx.x; t < tile; t += 256) part += tiles[t];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) part += __shfl_xor(part, o);
+    if (lane == 0) before[wave] = part;
+  }
+  int n = 0;  // kept pixels of the tile's earlier waves and rounds, then of all
+#pragma unroll
+  for (int r = 0; r < VBO_PX; ++r)
+    for (int v = 0; v < 4; ++v) {
+      const unsigned long long m = mask[(size_t)tile * 16 + r * 4 + v];
+      if (v == wave && (m >> lane & 1ull)) {
+        const int i = tile * VBO_TILE + r * 256 + (int)threadIdx.x;
+        const int x = i % a.w, y = i / a.w;
+        const float depth = 1 / in.idepth(i);
+        uint8_t c[3];
+        in.color(i, c);
+        lsdg_vertex o;
+        o.point[0] = ((float)x * a.fxi + a.cxi) * depth;
+        o.point[1] = ((float)y * a.fyi + a.cyi) * depth;
+        o.point[2] = depth;
+        o.color[3] = 100;
+        o.color[2] = c[0];
+        o.color[1] = c[1];
+        o.color[0] = c[2];
+        stage[n + __popcll(m & ((1ull << lane) - 1ull))] = __builtin_bit_cast(uint4, o);
+      }
+      n += __popcll(m);
+    }
   __syncthreads();
-  if (!keep) return;
-  int r = blk[blockIdx.x] +
-          (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-  for (int v = 0; v < wave; ++v) r += wc[v];
-  const lsdg_point_dense c = in[i];
-  lsdg_vertex o;
-  o.point[0] = ((float)x * a.fxi + a.cxi) * depth;
-  o.point[1] = ((float)y * a.fyi + a.cyi) * depth;
-  o.point[2] = depth;
-  o.color[3] = 100;
-  o.color[2] = c.color[0];
-  o.color[1] = c.color[1];
-  o.color[0] = c.color[2];
-  out[r] = o;
+  const int base = scanned ? tiles[tile] : before[0] + before[1] + before[2] + before[3];
+  for (int k = threadIdx.x; k < n; k += 256) ((uint4*)out)[(size_t)base + k] = stage[k];
+  if (tile == (int)gridDim.x - 1 && threadIdx.x == 0) *total = base + n;
 }
 
 // ------------------------------------------------------------ launchers
@@ -136,15 +187,33 @@ hipError_t launch_kf_dense(const float* id, const float* var, const float* img, 
   return hipGetLastError();
 }
 
-size_t vbo_block_count(int w, int h) { return ((size_t)w * h + 255) / 256; }
+// Up to this many tiles (4 Mpixel) every tile adds up the counts before it
+// itself: at most 16 integers per thread, less than the scan's launch.
+constexpr size_t VBO_SELF_SCAN_TILES = 4096;
 
-hipError_t launch_vbo(const lsdg_point_dense* in, const VboArgs& a, int* blk, lsdg_vertex* out, hipStream_t s) {
-  const int nb = (int)vbo_block_count(a.w, a.h);
-  if (nb == 0) return hipSuccess;
-  k_vbo_count<<<dim3(nb), dim3(256), 0, s>>>(in, a, blk);
-  k_vbo_scan<<<dim3(1), dim3(1024), 0, s>>>(blk, nb);
-  k_vbo_write<<<dim3(nb), dim3(256), 0, s>>>(in, a, blk, out);
+static size_t vbo_tiles(int w, int h) { return ((size_t)w * h + VBO_TILE - 1) / VBO_TILE; }
+size_t vbo_scratch_bytes(int w, int h) { return vbo_tiles(w, h) * (16 * sizeof(unsigned long long) + sizeof(int)) + 64; }
+
+template <class SRC>
+static hipError_t launch_vbo_of(const SRC& in, const VboArgs& a, void* scratch, int* total, lsdg_vertex* out,
+                                hipStream_t s) {
+  const size_t nt = vbo_tiles(a.w, a.h);
+  unsigned long long* mask = (unsigned long long*)scratch;
+  int* tiles = (int*)(mask + nt * 16);
+  const int scan = nt > VBO_SELF_SCAN_TILES ? 1 : 0;
+  k_vbo_count<<<dim3((unsigned)nt), dim3(256), 0, s>>>(in, a, mask, tiles);
+  if (scan) k_vbo_scan<<<dim3(1), dim3(1024), 0, s>>>(tiles, (int)nt);
+  k_vbo_write<<<dim3((unsigned)nt), dim3(256), 0, s>>>(in, a, mask, tiles, scan, total, out);
   return hipGetLastError();
+}
+
+hipError_t launch_vbo(const lsdg_point_dense* in, const VboArgs& a, void* scratch, int* total, lsdg_vertex* out,
+                      hipStream_t s) {
+  return launch_vbo_of(VboRecords{in}, a, scratch, total, out, s);
+}
+hipError_t launch_vbo(const float* id, const float* var, const float* img, const VboArgs& a, void* scratch, int* total,
+                      lsdg_vertex* out, hipStream_t s) {
+  return launch_vbo_of(VboFrame{id, var, img}, a, scratch, total, out, s);
 }
 
 }  // namespace lsdg

@@ -380,9 +380,14 @@ hipError_t launch_pyr_batch(const PyrBatch& b, hipStream_t s);
 // keyframe.hip
 hipError_t launch_kf_dense(const float* id, const float* var, const float* img, int n, lsdg_point_dense* out,
                            hipStream_t s);
-size_t vbo_block_count(int w, int h);
-// blk: vbo_block_count + 1 ints; out: capacity (w - 2) * (h - 2)
-hipError_t launch_vbo(const lsdg_point_dense* in, const VboArgs& a, int* blk, lsdg_vertex* out, hipStream_t s);
+size_t vbo_scratch_bytes(int w, int h);
+// The viewer's filter over point records, or over a keyframe's arrays: kept
+// vertices to out (capacity (w - 2) * (h - 2); device or host-mapped memory),
+// their number to *total.
+hipError_t launch_vbo(const lsdg_point_dense* in, const VboArgs& a, void* scratch, int* total, lsdg_vertex* out,
+                      hipStream_t s);
+hipError_t launch_vbo(const float* id, const float* var, const float* img, const VboArgs& a, void* scratch, int* total,
+                      lsdg_vertex* out, hipStream_t s);
 
 // track.hip
 // Sets n 64-bit words (a fill kernel).

@@ -80,3 +80,35 @@ def test_no_depth_is_an_error(ctx):
     f = ctx.frame(0, cam, np.zeros((96, 128), np.uint8))
     with pytest.raises(RuntimeError):
         f.keyframe_points(0)
+
+
+def _host_memory(n, pinned):
+    """n bytes of host memory, pinned by the runtime the library is linked to
+    or ordinary, and what frees it."""
+    if not pinned:
+        return np.zeros(n, np.uint8), lambda: None
+    path = next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line)
+    hip, p = lsdg.C.CDLL(path), lsdg.C.c_void_p()
+    assert hip.hipHostMalloc(lsdg.C.byref(p), lsdg.C.c_size_t(n), 0) == 0
+    return np.ctypeslib.as_array((lsdg.C.c_uint8 * n).from_address(p.value)), lambda: hip.hipHostFree(p)
+
+
+# tiles of 1024 pixels: one, a whole number of them, one pixel into the next
+# wave, round and tile, and more than the kernels add up by themselves
+@pytest.mark.parametrize("w,h", [(3, 3), (32, 32), (64, 16), (65, 16), (43, 31), (205, 5), (4100, 1030)])
+@pytest.mark.parametrize("pinned", [False, True])
+def test_points_vbo_tiles(ctx, w, h, pinned):
+    rng = np.random.default_rng(w * h)
+    rec = np.zeros(w * h, lsdg.POINT_DENSE_DTYPE)
+    rec["idepth"] = np.where(rng.random(w * h) < 0.7, rng.uniform(0.5, 2.0, w * h), -1).astype(np.float32)
+    rec["idepth_var"] = 1e-6
+    rec["color"] = rng.integers(0, 256, (w * h, 4), dtype=np.uint8)
+    cam4, p = (300.0, 280.0, 18.0, 14.0), lsdg.vbo_params(1.0, min_near_support=1)
+    out, free = _host_memory(16 * w * h, pinned)
+    n = lsdg.C.c_int32()
+    ctx.check(ctx.L.lsdg_points_vbo(ctx.h, rec.ctypes.data, w, h, *cam4, lsdg.C.byref(p), out.ctypes.data,
+                                    lsdg.C.byref(n)), "lsdg_points_vbo")
+    want = pyoracle.Oracle(0).compute_vbo(rec, w, h, cam4, p)
+    assert n.value == len(want)
+    assert out[:16 * n.value].tobytes() == np.ascontiguousarray(want).tobytes()
+    free()
