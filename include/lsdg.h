@@ -398,7 +398,8 @@ lsdg_status lsdg_depth_active_keyframe(lsdg_depthmap dm, int32_t* id);
  * for FP32 and 6 for FP16/BF16 pyramids; Sim3 adds N_l * 9 + P_l * 8).
  * No counterpart in the reference, whose core only keeps gettimeofday
  * averages (msTrackFrame, msObserve, ...).  Off by default. */
-#define LSDG_KERNEL_EVAL 0        /* fused SE3 / Sim3 evaluation (plain path) */
+#define LSDG_KERNEL_EVAL 0        /* plain path: one alignment's launch, or one evaluation's (single
+                                     passes, alignments whose blocks could not all run at once) */
 #define LSDG_KERNEL_PYRAMID 1     /* frame pyramid build */
 #define LSDG_KERNEL_DEPTH 2       /* depth-map kernels of one update */
 #define LSDG_KERNEL_BATCH_EVAL 3  /* batched evaluation sweep */
