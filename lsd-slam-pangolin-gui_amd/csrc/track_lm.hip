@@ -12,8 +12,8 @@
 // repeats the same LM step on its own copy of the control block, so an
 // iteration is one evaluation, one exchange and one LM step.
 //
-// 320x240 camera image to pose: 685 -> 228 us; 640x480 through the
-// undistorter: 635 -> 260 us (the launch itself about 170 us for 28
+// 320x240 camera image to pose: 725 -> 206 us; 640x480 through the
+// undistorter: 638 -> 259 us (the launch itself about 170 us for 28
 // evaluations: 1.4-2 us of points, 2-2.5 us of exchange and 1.3 us of LM step
 // each).
 //
