@@ -880,6 +880,7 @@ extern "C" lsdg_status lsdg_se3_track(lsdg_ctx c, lsdg_ref r, lsdg_frame f, cons
   if (f->w[0] != r->kf->w[0] || f->h[0] != r->kf->h[0]) return fail(c, LSDG_EINVAL, "frame / keyframe size mismatch");
   const lsdg_params& P = c->P;
   uint8_t* mask = nullptr;
+  const bool hadMask = f->wasGoodAllocated;
   if (P.se3_min_level == 1) {  // refPixelWasGood is a level-1 mask
     lsdg_status s0 = frame_ensure_was_good(f);
     if (s0 != LSDG_OK) return s0;
@@ -888,6 +889,10 @@ extern "C" lsdg_status lsdg_se3_track(lsdg_ctx c, lsdg_ref r, lsdg_frame f, cons
   const JobState* s = nullptr;
   bool ran = false;
   lsdg_status s0 = track_lm(c, r, f, LSDG_JOB_SE3, pose_from7(init), P.se3_max_level - 1, P.se3_min_level, mask, &s, &ran);
+  // a frame has a mask from its first evaluation at level 1 on: an alignment
+  // that ended before it leaves the frame without (propagation then tests the
+  // residuals instead)
+  if (!hadMask && (s0 != LSDG_OK || !ran || s->evalsAt[1] == 0)) f->wasGoodAllocated = false;
   if (s0 != LSDG_OK) return s0;
   if (!ran) return se3_track_steps(c, r, f, init, out, stats);
   lsdg_track_stats st;
