@@ -1110,6 +1110,7 @@ static lsdg_status sim3_track_steps(lsdg_ctx c, lsdg_ref r, lsdg_frame f, const 
     lsdg_status s0 = sim3_eval_sync(c, r, f, finalLevel, T, affA, affB, S);
     if (s0 != LSDG_OK) return s0;
     finalRes = sim3_res(S);
+    pointUsage = S[SM_USAGE] / (double)r->lv[finalLevel].n;
     std::memcpy(Sacc, S, sizeof(double) * NS_SIM3);
   }
   {

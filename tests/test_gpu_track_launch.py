@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 import lsdg
+import pyoracle
 import synth
 from helpers import twist
 
@@ -65,6 +66,41 @@ def test_one_launch_equals_launch_per_evaluation(ctx, monkeypatch, w, h, prec):
         H, H2 = np.array(st3.hessian[:]), np.array(st32.hessian[:])
         assert np.abs(H - H2).max() <= 1e-9 * max(np.abs(H2).max(), 1e-30)
     other.close()
+
+
+@pytest.mark.parametrize("steps", [False, True])
+def test_sim3_final_level_without_iterations(ctx, monkeypatch, steps):
+    """The final evaluation, at a level that has no iterations, is the last
+    one whose point usage counts, in both forms as in the oracle."""
+    cam = synth.camera(322, 242)
+    p = pyoracle.default_params()
+    p.max_its_per_lvl[1] = 0
+    p.convergence_eps[2] = 0.0  # level 2 ends on an accepted step, so a final evaluation follows
+    c = _steps_context(monkeypatch) if steps else ctx
+    c.set_params(p)
+    try:
+        a, b, ref = _pair(c, cam, 43, lsdg.FP32)
+        c.profile(True)
+        q, st, status = c.sim3_track(ref, b, [*synth.IDENTITY7, 1.0], 4, 1)
+        launches = c.kernel_stats(lsdg.KERNEL_EVAL)["launches"]
+    finally:
+        c.profile(False)
+        c.set_params(lsdg.default_params())
+    o = pyoracle.Oracle(2, params=p)
+    d = synth.sim3_instance(43, cam=cam, max_trans=0.03, max_rot_deg=1.0, scale_range=(0.98, 1.02))
+    oa, ob = o.frame(0, cam, d["a_img"].astype(np.float32)), o.frame(1, cam, d["b_img"].astype(np.float32))
+    oa.set_depth(d["a_idepth"], d["a_var"])
+    ob.set_depth(d["b_idepth"], d["b_var"])
+    oq, ost, ostatus = o.sim3_track(o.ref(oa), ob, [*synth.IDENTITY7, 1.0], 4, 1)
+    assert status == ostatus == lsdg.OK and st.num_residual_calls[1] == 0
+    assert launches > 1 if steps else launches == 1  # the form that ran
+    assert twist(q[:7], oq[:7]) <= 1e-9 and abs(q[7] - oq[7]) <= 1e-9
+    # one FP64 sum of FP32 terms in another order, rounded to float
+    assert np.isclose(st.point_usage, ost.point_usage, rtol=2.0 ** -22)
+    for x in (ref, b, a):
+        x.destroy()
+    if steps:
+        c.close()
 
 
 def test_contexts_align_at_the_same_time():
