@@ -703,8 +703,10 @@ static void se3_pass_stats(const double* S, int N, Se3Out& o) {
 
 // ------------------------------------------------- one-launch alignments
 // Runs one alignment's LM loop in one launch (track_lm.hip).  *ran is false
-// when the blocks could not all run at once: nothing is written then, and the
-// caller takes the launch-per-evaluation path.
+// when the blocks could not all run at once, or when the alignment needs more
+// evaluations than a launch makes (BATCH_JOB_MAX_EVALS): the caller then takes
+// the launch-per-evaluation path, which starts over (the mask may be partly
+// written; its evaluations write it again).
 static lsdg_status track_lm(lsdg_ctx c, lsdg_ref r, lsdg_frame f, int kind, const Pose& init, int startLevel,
                             int finalLevel, uint8_t* mask, const JobState** out, bool* ran) {
   TrackLmArgs a;
@@ -754,7 +756,7 @@ static lsdg_status track_lm(lsdg_ctx c, lsdg_ref r, lsdg_frame f, int kind, cons
     bytes += s->evalsAt[l] * eval_bytes(r->lv[l].n, f, l, kind == LSDG_JOB_SIM3);
   prof_timer_done(c, LSDG_KERNEL_EVAL, kt, bytes);
   *out = s;
-  *ran = s->status >= 0;
+  *ran = s->status > 0;
   return LSDG_OK;
 }
 

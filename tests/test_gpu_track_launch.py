@@ -103,6 +103,37 @@ def test_sim3_final_level_without_iterations(ctx, monkeypatch, steps):
         c.close()
 
 
+def test_more_evaluations_than_one_launch_makes(ctx):
+    """An alignment of 70001 evaluations (heavily damped steps towards a smooth
+    minimum), where a launch ends after 65536: it is finished launch by launch,
+    not reported as done where it stood."""
+    cam = synth.camera(64, 64)
+    y, x = np.mgrid[0:64, 0:64].astype(np.float64)
+    image = lambda u, v: (128 + 50 * np.sin(u / 7.0) + 50 * np.cos(v / 9.0 + u / 31.0)).astype(np.float32)
+    idepth = np.full((64, 64), -1, np.float32)
+    idepth[16:48, 16:48] = 1.0  # away from the border: no point enters or leaves the image
+    var = np.full((64, 64), 0.01, np.float32)
+    p = pyoracle.default_params()
+    p.se3_min_level, p.se3_max_level = 1, 2
+    p.max_its_per_lvl[1], p.lambda_initial[1], p.lambda_success_fac[1] = 70000, 3e4, 1.0
+    p.convergence_eps[1], p.step_size_min[1] = 1.0, 0.0
+
+    def align(c):
+        kf, fr = c.frame(0, cam, image(x, y)), c.frame(1, cam, image(x - 4.0, y))
+        kf.set_depth(idepth, var)
+        return c.se3_track(c.ref(kf), fr, synth.IDENTITY7)
+
+    ctx.set_params(p)
+    try:
+        pose, st, status = align(ctx)
+    finally:
+        ctx.set_params(lsdg.default_params())
+    opose, ost, ostatus = align(pyoracle.Oracle(2, params=p))
+    assert ost.num_residual_calls[1] == 70001
+    assert status == ostatus and _fields(st) == _fields(ost)
+    assert twist(pose, opose) <= 1e-9 and np.isclose(st.last_residual, ost.last_residual, rtol=1e-6)
+
+
 def test_contexts_align_at_the_same_time():
     """Six threads, each with its own context, aligning at once: every result
     equals the single-threaded one."""
