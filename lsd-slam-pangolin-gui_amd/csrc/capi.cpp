@@ -707,8 +707,16 @@ static void se3_pass_stats(const double* S, int N, Se3Out& o) {
 // evaluations than a launch makes (BATCH_JOB_MAX_EVALS): the caller then takes
 // the launch-per-evaluation path, which starts over (the mask may be partly
 // written; its evaluations write it again).
+// Blocks that gave up have polled for up to 16 ms: what keeps them out (other
+// work on the device) is likely still there for the next image, so the
+// context's next TRACK_LM_PAUSE alignments don't try.
 static lsdg_status track_lm(lsdg_ctx c, lsdg_ref r, lsdg_frame f, int kind, const Pose& init, int startLevel,
                             int finalLevel, uint8_t* mask, const JobState** out, bool* ran) {
+  *ran = false;
+  if (c->track_pause > 0) {
+    --c->track_pause;
+    return LSDG_OK;
+  }
   TrackLmArgs a;
   std::memset(&a, 0, sizeof a);
   a.jd.kind = kind;
@@ -754,7 +762,8 @@ static lsdg_status track_lm(lsdg_ctx c, lsdg_ref r, lsdg_frame f, int kind, cons
   double bytes = 0.0;
   for (int l = finalLevel; l <= startLevel; ++l)
     bytes += s->evalsAt[l] * eval_bytes(r->lv[l].n, f, l, kind == LSDG_JOB_SIM3);
-  prof_timer_done(c, LSDG_KERNEL_EVAL, kt, bytes);
+  prof_timer_done(c, LSDG_KERNEL_EVAL, kt, s->status < 0 ? 0.0 : bytes);
+  if (s->status < 0) c->track_pause = TRACK_LM_PAUSE;
   *out = s;
   *ran = s->status > 0;
   return LSDG_OK;

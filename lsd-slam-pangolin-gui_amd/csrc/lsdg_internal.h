@@ -249,6 +249,7 @@ struct lsdg_ctx_s {
   void* h_track = nullptr;
   void* d_track = nullptr;
   unsigned track_spin_max = 0;
+  int track_pause = 0;  // alignments left that go launch by launch
   // per-kernel timing (lsdg_ctx_profile)
   struct ProfRec {
     int kind;

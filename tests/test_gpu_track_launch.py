@@ -32,6 +32,17 @@ def _pair(ctx, cam, seed, prec):
     return a, b, ctx.ref(a)
 
 
+def _launches(c, align):
+    """align()'s result and the launches it took: one of the one-launch form,
+    one per evaluation otherwise."""
+    c.profile(True)
+    try:
+        out = align()
+        return out, c.kernel_stats(lsdg.KERNEL_EVAL)["launches"]
+    finally:
+        c.profile(False)
+
+
 def _fields(st):
     return [st.last_good_count, st.last_bad_count, st.diverged, st.tracking_was_good, *st.num_residual_calls,
             *st.num_warp_update_calls]
@@ -47,9 +58,17 @@ def test_one_launch_equals_launch_per_evaluation(ctx, monkeypatch, w, h, prec):
         res = []
         for c in (ctx, other):
             a, b, ref = _pair(c, cam, seed, prec)
-            p, st, status = c.se3_track(ref, b, synth.IDENTITY7)
+            (p, st, status), n = _launches(c, lambda: c.se3_track(ref, b, synth.IDENTITY7))
             mask = b.read(lsdg.WHAT_REF_PIXEL_WAS_GOOD)
-            q, st3, status3 = c.sim3_track(ref, b, [*synth.IDENTITY7, 1.0], 4, 1)
+            (q, st3, status3), n3 = _launches(c, lambda: c.sim3_track(ref, b, [*synth.IDENTITY7, 1.0], 4, 1))
+            # the form that ran: at 64x64 no level is split, so nothing waits;
+            # elsewhere the other context's first alignment gives up, and the
+            # ones after it go launch by launch without a try
+            if c is ctx or w == 64:
+                assert n == 1 and n3 == 1
+            else:
+                assert n == sum(st.num_residual_calls) + (1 if seed == 41 else 0)
+                assert n3 - sum(st3.num_residual_calls) in (0, 1)  # 1: the evaluation for the information matrix
             res.append((p, st, status, mask, q, st3, status3))
             for x in (ref, b, a):
                 x.destroy()
@@ -101,6 +120,20 @@ def test_sim3_final_level_without_iterations(ctx, monkeypatch, steps):
         x.destroy()
     if steps:
         c.close()
+
+
+def test_a_context_that_gave_up_tries_again_after_a_while(monkeypatch):
+    cam = synth.camera(130, 98)
+    c = _steps_context(monkeypatch)
+    a, b, ref = _pair(c, cam, 41, lsdg.FP32)
+    vain = []
+    for _ in range(203):
+        (_, st, _), n = _launches(c, lambda: c.se3_track(ref, b, synth.IDENTITY7))
+        vain.append(n - sum(st.num_residual_calls))
+    assert vain == [1] + [0] * 100 + [1] + [0] * 100 + [1]
+    for x in (ref, b, a):
+        x.destroy()
+    c.close()
 
 
 def test_more_evaluations_than_one_launch_makes(ctx):
