@@ -104,31 +104,6 @@ __global__ __launch_bounds__(256) void k_vbo_count(SRC in, VboArgs a, unsigned l
   if (threadIdx.x == 0) tiles[blockIdx.x] = wc[0] + wc[1] + wc[2] + wc[3];
 }
 
-// Exclusive scan of blk[0, nb) in place, blk[nb] = total; one block.
-__global__ __launch_bounds__(1024) void k_vbo_scan(int* blk, int nb) {
-  __shared__ int sh[1024];
-  __shared__ int carry;
-  if (threadIdx.x == 0) carry = 0;
-  __syncthreads();
-  for (int base = 0; base < nb; base += 1024) {
-    const int i = base + threadIdx.x;
-    const int v = i < nb ? blk[i] : 0;
-    sh[threadIdx.x] = v;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-      const int t = threadIdx.x >= off ? sh[threadIdx.x - off] : 0;
-      __syncthreads();
-      sh[threadIdx.x] += t;
-      __syncthreads();
-    }
-    if (i < nb) blk[i] = carry + sh[threadIdx.x] - v;
-    __syncthreads();
-    if (threadIdx.x == 0) carry += sh[1023];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) blk[nb] = carry;
-}
-
 // The kept pixels of a tile, behind those of the tiles before it (whose counts
 // the block adds up itself, or with `scanned` finds added up).  They are
 // gathered in LDS and leave in whole lines: `out` may be host memory, where a
@@ -187,10 +162,6 @@ hipError_t launch_kf_dense(const float* id, const float* var, const float* img, 
   return hipGetLastError();
 }
 
-// Up to this many tiles (4 Mpixel) every tile adds up the counts before it
-// itself: at most 16 integers per thread, less than the scan's launch.
-constexpr size_t VBO_SELF_SCAN_TILES = 4096;
-
 static size_t vbo_tiles(int w, int h) { return ((size_t)w * h + VBO_TILE - 1) / VBO_TILE; }
 size_t vbo_scratch_bytes(int w, int h) { return vbo_tiles(w, h) * (16 * sizeof(unsigned long long) + sizeof(int)) + 64; }
 
@@ -200,9 +171,12 @@ static hipError_t launch_vbo_of(const SRC& in, const VboArgs& a, void* scratch, 
   const size_t nt = vbo_tiles(a.w, a.h);
   unsigned long long* mask = (unsigned long long*)scratch;
   int* tiles = (int*)(mask + nt * 16);
-  const int scan = nt > VBO_SELF_SCAN_TILES ? 1 : 0;
+  const int scan = nt > (size_t)TILE_SCAN_MIN ? 1 : 0;
   k_vbo_count<<<dim3((unsigned)nt), dim3(256), 0, s>>>(in, a, mask, tiles);
-  if (scan) k_vbo_scan<<<dim3(1), dim3(1024), 0, s>>>(tiles, (int)nt);
+  if (scan) {
+    hipError_t e = launch_tile_scan(tiles, (int)nt, total, s);
+    if (e != hipSuccess) return e;
+  }
   k_vbo_write<<<dim3((unsigned)nt), dim3(256), 0, s>>>(in, a, mask, tiles, scan, total, out);
   return hipGetLastError();
 }

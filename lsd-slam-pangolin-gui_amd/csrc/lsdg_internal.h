@@ -374,6 +374,14 @@ hipError_t launch_depth_normalize(float* idepth, float* ivar, int n, hipStream_t
 // Queues the point clouds of the levels with a bit in `levels`: sets r->lv
 // (n left 0) and writes the counts to r->d_counts[level].
 hipError_t launch_point_clouds(lsdg_ref r, unsigned levels, hipStream_t s);
+// Compactions by tiles (point clouds, vertices): up to this many tiles (4
+// Mpixel) every tile adds up the counts before it itself, at most 16 integers
+// per thread; more are scanned by a launch in between, as that work grows with
+// the square of the size.  Points of one level, added up by the tiles / by a
+// scan: 1024^2 41 / 43 us, 2048^2 (4096 tiles) 69 / 67, 4096^2 255 / 198, 8192^2
+// 1687 / 698.
+constexpr int TILE_SCAN_MIN = 4096;
+hipError_t launch_tile_scan(int* tiles, int n, int* total, hipStream_t s);
 size_t pyr_batch_bytes(int nf);
 void pyr_batch_tables(lsdg_frame const* fs, const unsigned* need, int nf, void* h, void* d, PyrBatch* out);
 hipError_t launch_pyr_batch(const PyrBatch& b, hipStream_t s);

@@ -470,8 +470,9 @@ __device__ inline bool pc_valid(const float* id, const float* var, int idx, int 
 // The point clouds of several levels in two launches.  A tile is PC_TILE
 // consecutive pixels of one level, PC_PX per thread (pixel i of thread t at
 // t + 256 i, so loads coalesce).  k_pc_count counts each tile's points;
-// k_pc_write adds up the counts of the level's earlier tiles (a few hundred
-// integers, read by the whole block) and writes its points behind them in
+// k_pc_write adds up the counts of the level's earlier tiles (300 integers at
+// most for 640x480, read by the whole block), or on a level of more tiles
+// finds them added up (TILE_SCAN_MIN), and writes its points behind them in
 // row-major order.  Nothing returns to the host: the counts of points stay
 // on the device beside the points, and an alignment reads them there.  (One
 // count, scan and write launch and one wait for the count per level took 45 us
@@ -492,6 +493,7 @@ struct PcLevel {
   int* tiles;  // points of each tile
   int* total;  // points of the level
   int ntiles;
+  int scanned;  // tiles holds the points before each tile
 };
 struct PcArgs {
   PcLevel lv[PYR];
@@ -526,7 +528,11 @@ __global__ __launch_bounds__(256) void k_pc_write(PcArgs a) {
   const PcLevel& L = a.lv[k];
   const int n = L.w * L.h, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   int part = 0;
-  for (int t = threadIdx.x; t < tile; t += 256) part += L.tiles[t];
+  if (L.scanned) {
+    if (threadIdx.x == 0) part = L.tiles[tile];
+  } else {
+    for (int t = threadIdx.x; t < tile; t += 256) part += L.tiles[t];
+  }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) part += __shfl_xor(part, o);
   bool v[PC_PX];
@@ -565,7 +571,50 @@ __global__ __launch_bounds__(256) void k_pc_write(PcArgs a) {
   if (tile == L.ntiles - 1 && threadIdx.x == 0) *L.total = base;
 }
 
+// Exclusive scan of tiles[0, n) in place, their sum to *total; one block, four
+// counts per thread and round.
+__global__ __launch_bounds__(1024) void k_tile_scan(int* __restrict__ tiles, int n, int* __restrict__ total) {
+  __shared__ int wsum[16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int carry = 0;
+  for (int base = 0; base < n; base += 4096) {
+    const int i = base + 4 * (int)threadIdx.x;
+    int v[4], own = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      v[k] = i + k < n ? tiles[i + k] : 0;
+      own += v[k];
+    }
+    int upTo = own;  // of the wave, this lane's included
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int t = __shfl_up(upTo, o);
+      if (lane >= o) upTo += t;
+    }
+    if (lane == 63) wsum[wave] = upTo;
+    __syncthreads();
+    int before = carry + upTo - own;
+    for (int k = 0; k < 16; ++k) {
+      if (k < wave) before += wsum[k];
+      carry += wsum[k];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (i + k < n) {
+        tiles[i + k] = before;
+        before += v[k];
+      }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) *total = carry;
+}
+
 // ------------------------------------------------------------ launchers
+hipError_t launch_tile_scan(int* tiles, int n, int* total, hipStream_t s) {
+  k_tile_scan<<<dim3(1), dim3(1024), 0, s>>>(tiles, n, total);
+  return hipGetLastError();
+}
+
 static PyrImgArgs pyr_img_args(lsdg_frame f) {
   PyrImgArgs p;
   for (int l = 0; l < PYR; ++l) {
@@ -699,6 +748,7 @@ hipError_t launch_depth_normalize(float* id, float* var, int n, hipStream_t s) {
 // Levels whose interior has more pixels than this get exactly sized point
 // storage (after a wait for the count) instead of room for every pixel.
 constexpr size_t PC_ROOM_MAX = (size_t)1 << 22;
+static_assert(PC_ROOM_MAX >= (size_t)TILE_SCAN_MIN * PC_TILE, "levels above PC_ROOM_MAX are scanned");
 
 static hipError_t pc_storage(lsdg_ref r, int l, size_t points) {
   if (points <= (size_t)r->cap[l] && r->d_pool[l]) return hipSuccess;
@@ -737,6 +787,7 @@ hipError_t launch_point_clouds(lsdg_ref r, unsigned levels, hipStream_t s) {
     L.tiles = r->d_counts + PYR + tile0[l];
     L.total = r->d_counts + l;
     L.ntiles = tile0[l + 1] - tile0[l];
+    L.scanned = L.ntiles > TILE_SCAN_MIN ? 1 : 0;
     const size_t room = (size_t)(f->w[l] - 2) * (f->h[l] - 2);
     if (room <= PC_ROOM_MAX) {
       if ((e = pc_storage(r, l, room)) != hipSuccess) return e;
@@ -751,16 +802,17 @@ hipError_t launch_point_clouds(lsdg_ref r, unsigned levels, hipStream_t s) {
   if (nl == 0) return hipSuccess;
   k_pc_count<<<dim3(blocks), dim3(256), 0, s>>>(a);
   if ((e = hipGetLastError()) != hipSuccess) return e;
+  for (int k = 0; k < nl; ++k)
+    if (a.lv[k].scanned && (e = launch_tile_scan(a.lv[k].tiles, a.lv[k].ntiles, a.lv[k].total, s)) != hipSuccess) return e;
   if (exact) {
-    std::vector<int> t(tile0[PYR]);
-    e = hipMemcpyAsync(t.data(), r->d_counts + PYR, sizeof(int) * t.size(), hipMemcpyDeviceToHost, s);
+    // a level without room for every pixel has more than TILE_SCAN_MIN tiles:
+    // its count of points is there now
+    int n[PYR];
+    e = hipMemcpyAsync(n, r->d_counts, sizeof n, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     for (int k = 0; k < nl && e == hipSuccess; ++k) {
       const int l = lvl[k];
-      if ((size_t)(f->w[l] - 2) * (f->h[l] - 2) <= PC_ROOM_MAX) continue;
-      size_t n = 0;
-      for (int i = tile0[l]; i < tile0[l + 1]; ++i) n += (size_t)t[i];
-      e = pc_storage(r, l, std::max<size_t>(n, 1));
+      if ((size_t)(f->w[l] - 2) * (f->h[l] - 2) > PC_ROOM_MAX) e = pc_storage(r, l, (size_t)std::max(n[l], 1));
     }
     if (e != hipSuccess) return e;
   }

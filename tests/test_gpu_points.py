@@ -1,7 +1,8 @@
 """Point clouds of several levels at once: every level's points in row-major
 order with the pixel's depth, variance and gradient, at sizes around a tile,
-without points, with every interior pixel, and past the size up to which
-storage is taken for every pixel; after a depth change, and when an alignment
+without points, with every interior pixel, and past the sizes up to which
+storage is taken for every pixel and tiles add up the counts before them
+themselves (4228 tiles, and 8409: three rounds of the scan); after a depth change, and when an alignment
 builds them before the host knows their counts."""
 import numpy as np
 import pytest
@@ -20,7 +21,7 @@ def _expect(kf, level, img):
 
 
 @pytest.mark.parametrize("w,h,density", [(64, 64, 0.3), (66, 98, 1.0), (130, 94, 0.0), (642, 482, 0.25),
-                                         (2402, 1802, 0.02)])
+                                         (2402, 1802, 0.02), (4100, 2100, 0.05)])
 def test_levels_are_compacted_in_order(ctx, w, h, density):
     rng = np.random.default_rng(w)
     cam = synth.camera(w, h)
