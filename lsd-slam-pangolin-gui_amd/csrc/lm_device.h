@@ -23,11 +23,13 @@
 
 namespace lsdg {
 
-// f^n by repeated multiplication (exact for the default factor 2).
+// f^n as std::pow of floats gives it: the product in FP64, rounded once.
+// (Rounded to float at every factor, a factor that is not a power of two gave
+// another damping after a few rejections, and poses up to 5e-8 apart.)
 __host__ __device__ inline float pow_int(float f, int n) {
-  float r = 1.0f;
-  for (int i = 0; i < n; ++i) r *= f;
-  return r;
+  double r = 1.0;
+  for (int i = 0; i < n; ++i) r *= (double)f;
+  return (float)r;
 }
 
 __device__ inline int lm_lane() { return (int)(threadIdx.x & 63); }

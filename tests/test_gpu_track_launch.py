@@ -122,6 +122,40 @@ def test_sim3_final_level_without_iterations(ctx, monkeypatch, steps):
         c.close()
 
 
+@pytest.mark.parametrize("fail_fac", [2.0, 1.7, 3.1])
+def test_damping_after_rejections(ctx, monkeypatch, fail_fac):
+    """Steps rejected several times in a row multiply the damping by a power of
+    the factor: the same power in the one-launch form, the batch and the host's
+    LM step (std::pow), also where the factor's powers round."""
+    cam = synth.camera(642, 482)
+    p = lsdg.default_params()
+    for l in range(5):
+        p.lambda_fail_fac[l], p.convergence_eps[l], p.step_size_min[l] = fail_fac, 0.9999, 1e-14
+    steps = _steps_context(monkeypatch)
+    for c in (ctx, steps):
+        c.set_params(p)
+    try:
+        for seed in range(41, 49):
+            out = []
+            for c in (ctx, steps):
+                a, b, ref = _pair(c, cam, seed, lsdg.FP32)
+                pose, st, status = c.se3_track(ref, b, synth.IDENTITY7)
+                assert sum(st.num_residual_calls) > sum(st.num_warp_update_calls) + 8  # rejections
+                out.append((pose, _fields(st), status))
+                if c is ctx:
+                    plan = c.batch([lsdg.Job(ref.h, b.h, lsdg.pose8([*synth.IDENTITY7, 1.0]), lsdg.JOB_SE3, 4, 1, 1)])
+                    res = plan.run()[0]
+                    out.append((np.array(res.frame_to_ref[:7]), _fields(res.stats), res.status))
+                    plan.destroy()
+                for x in (ref, b, a):
+                    x.destroy()
+            # the sums' order differs, by FP64 rounding
+            assert all(twist(o[0], out[0][0]) <= 1e-12 and o[1:] == out[0][1:] for o in out)
+    finally:
+        ctx.set_params(lsdg.default_params())
+        steps.close()
+
+
 def test_a_context_that_gave_up_tries_again_after_a_while(monkeypatch):
     cam = synth.camera(130, 98)
     c = _steps_context(monkeypatch)
