@@ -110,11 +110,16 @@ __global__ __launch_bounds__(256) void k_vbo_count(SRC in, VboArgs a, unsigned l
 // few vertices per store would be a bus transaction each.  A record per pixel,
 // a count, a scan, a write and a copy behind a wait for the count took 51 us for
 // a keyframe of 640x480; two launches and one wait take 27.
+// A vertex as it is stored: 16 bytes of which only 4-byte alignment is known
+// (the caller's buffer may begin anywhere in its pinned block).
+typedef unsigned VertexWords __attribute__((ext_vector_type(4), aligned(4)));
 template <class SRC>
 __global__ __launch_bounds__(256) void k_vbo_write(SRC in, VboArgs a, const unsigned long long* __restrict__ mask,
                                                    const int* __restrict__ tiles, int scanned, int* __restrict__ total,
                                                    lsdg_vertex* __restrict__ out) {
-  static_assert(sizeof(lsdg_vertex) == sizeof(uint4), "vertices move as 16-byte words");
+  static_assert(sizeof(lsdg_vertex) == sizeof(uint4) && sizeof(lsdg_vertex) == sizeof(VertexWords) &&
+                    alignof(lsdg_vertex) == alignof(VertexWords),
+                "vertices move as 16-byte words");
   __shared__ uint4 stage[VBO_TILE];
   __shared__ int before[4];
   const int tile = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -150,7 +155,8 @@ __global__ __launch_bounds__(256) void k_vbo_write(SRC in, VboArgs a, const unsi
     }
   __syncthreads();
   const int base = scanned ? tiles[tile] : before[0] + before[1] + before[2] + before[3];
-  for (int k = threadIdx.x; k < n; k += 256) ((uint4*)out)[(size_t)base + k] = stage[k];
+  for (int k = threadIdx.x; k < n; k += 256)
+    ((VertexWords*)out)[(size_t)base + k] = __builtin_bit_cast(VertexWords, stage[k]);
   if (tile == (int)gridDim.x - 1 && threadIdx.x == 0) *total = base + n;
 }
 

@@ -93,6 +93,24 @@ def _host_memory(n, pinned):
     return np.ctypeslib.as_array((lsdg.C.c_uint8 * n).from_address(p.value)), lambda: hip.hipHostFree(p)
 
 
+@pytest.mark.parametrize("offset", [0, 4, 8, 12, 16, 4100])
+def test_vertices_into_the_middle_of_a_pinned_block(keyframes, offset):
+    """The buffer begins anywhere in its block, aligned as a vertex is (4
+    bytes); what is beside the vertices stays as it was."""
+    g, of, o = keyframes
+    p = lsdg.vbo_params(1.0)
+    w, h = of.size(0)
+    want = np.ascontiguousarray(o.compute_vbo(of.keyframe_points(0), w, h, of.camera(0), p)).tobytes()
+    out, free = _host_memory(16 * w * h + offset + 64, True)
+    out[:] = 0xA5
+    n = lsdg.C.c_int32()
+    g.ctx.check(g.ctx.L.lsdg_keyframe_vbo(g.h, 0, lsdg.C.byref(p), out.ctypes.data + offset, lsdg.C.byref(n)),
+                "lsdg_keyframe_vbo")
+    assert out[offset:offset + len(want)].tobytes() == want and 16 * n.value == len(want)
+    assert (out[:offset] == 0xA5).all() and (out[offset + len(want):] == 0xA5).all()
+    free()
+
+
 # tiles of 1024 pixels: one, a whole number of them, one pixel into the next
 # wave, round and tile, and more than the kernels add up by themselves
 @pytest.mark.parametrize("w,h", [(3, 3), (32, 32), (64, 16), (65, 16), (43, 31), (205, 5), (4100, 1030)])
