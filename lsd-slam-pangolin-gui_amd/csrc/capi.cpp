@@ -122,12 +122,12 @@ extern "C" lsdg_status lsdg_ctx_create(int32_t device, const lsdg_params* params
   if (hipGetDeviceProperties(&prop, device) == hipSuccess) c->num_cus = prop.multiProcessorCount;
   c->partials_blocks = 4096;
   if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
-      hipMalloc(&c->d_partials, sizeof(double) * NS_MAX * c->partials_blocks) != hipSuccess ||
-      hipMalloc(&c->d_eval_rows, sizeof(unsigned long long) * EVAL_ROW_WORDS) != hipSuccess ||
-      hipHostMalloc(&c->h_result, sizeof(double) * 64, hipHostMallocMapped) != hipSuccess ||
+      alloc_device((void**)&c->d_partials, sizeof(double) * NS_MAX * c->partials_blocks) != hipSuccess ||
+      alloc_device((void**)&c->d_eval_rows, sizeof(unsigned long long) * EVAL_ROW_WORDS) != hipSuccess ||
+      alloc_pinned((void**)&c->h_result, sizeof(double) * 64) != hipSuccess ||
       hipHostGetDevicePointer((void**)&c->d_result, c->h_result, 0) != hipSuccess ||
-      hipMalloc(&c->d_track_rows, sizeof(unsigned long long) * TRACK_LM_WORDS) != hipSuccess ||
-      hipHostMalloc(&c->h_track, sizeof(JobState), hipHostMallocMapped) != hipSuccess ||
+      alloc_device((void**)&c->d_track_rows, sizeof(unsigned long long) * TRACK_LM_WORDS) != hipSuccess ||
+      alloc_pinned(&c->h_track, sizeof(JobState)) != hipSuccess ||
       hipHostGetDevicePointer(&c->d_track, c->h_track, 0) != hipSuccess ||
       noalloc_scratch_init(device) != hipSuccess) {  // the allocation-free entry point's device array
     lsdg_ctx_destroy(c);
@@ -962,7 +962,7 @@ extern "C" lsdg_status lsdg_se3_evaluate(lsdg_ctx c, lsdg_ref r, lsdg_frame f, i
   uint8_t* d_mask = nullptr;
   size_t mbytes = (size_t)r->kf->w[1] * r->kf->h[1];
   if (is_good && level == 1) {  // refPixelWasGood is a level-1 mask
-    CK(c, hipMalloc(&d_mask, mbytes));
+    CK(c, alloc_device((void**)&d_mask, mbytes));
     hipError_t e = hipMemcpyAsync(d_mask, is_good, mbytes, hipMemcpyHostToDevice, c->stream);
     if (e != hipSuccess) {
       (void)hipFree(d_mask);
@@ -1211,7 +1211,7 @@ static lsdg_status adjoint_buffer(lsdg_ctx c, int n, float** out) {
     if (c->d_adj) (void)hipFree(c->d_adj);
     c->d_adj = nullptr;
     c->adjCap = 0;
-    CK(c, hipMalloc(&c->d_adj, sizeof(float) * (size_t)n));
+    CK(c, alloc_device((void**)&c->d_adj, sizeof(float) * (size_t)n));
     c->adjCap = n;
   }
   *out = c->d_adj;

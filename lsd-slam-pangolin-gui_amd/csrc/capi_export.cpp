@@ -33,7 +33,7 @@ static lsdg_status export_scratch(lsdg_ctx c, int w, int h, ExportScratch* out) 
     if (c->d_export) (void)hipFree(c->d_export);
     c->d_export = nullptr;
     c->exportCap = 0;
-    CK(c, hipMalloc(&c->d_export, total));
+    CK(c, alloc_device(&c->d_export, total));
     c->exportCap = total;
   }
   char* b = (char*)c->d_export;

@@ -39,9 +39,9 @@ extern "C" lsdg_status lsdg_undistorter_create(lsdg_ctx c, int32_t inW, int32_t 
   u->inH = inH;
   u->outW = outW;
   u->outH = outH;
-  hipError_t e = hipMalloc(&u->d_map, n * sizeof(float2));
-  if (e == hipSuccess) e = hipMalloc(&u->d_src, (size_t)inW * inH);
-  if (e == hipSuccess) e = hipHostMalloc(&u->h_src, (size_t)inW * inH, hipHostMallocDefault);
+  hipError_t e = alloc_device((void**)&u->d_map, n * sizeof(float2));
+  if (e == hipSuccess) e = alloc_device((void**)&u->d_src, (size_t)inW * inH);
+  if (e == hipSuccess) e = alloc_pinned((void**)&u->h_src, (size_t)inW * inH);
   if (e == hipSuccess) e = hipMemcpyAsync(u->d_map, map, n * sizeof(float2), hipMemcpyHostToDevice, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   if (e != hipSuccess) {

@@ -7,15 +7,13 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
-#include <map>
-#include <mutex>
 #include <string>
-#include <unordered_map>
 #include <utility>
 #include <vector>
 
 #include "../../include/lsdg.h"
 #include "lsdg_lie.h"
+#include "pool.h"
 
 namespace lsdg {
 
@@ -185,47 +183,6 @@ struct VboArgs {
   float scaledTH, absTH, scale;
   int minNear;
 };
-}  // namespace lsdg
-
-namespace lsdg {
-// Device or pinned host blocks that a context's objects give back, kept for
-// the next ones: allocating and freeing a frame's arrays cost 38 of the 63 us
-// that making and destroying a 320x240 frame took, and a batch plan has eight
-// device and three pinned blocks.  An idle block serves a request of at least
-// four fifths of its size.  At most `limit` bytes stay idle (a block that does
-// not fit is freed at once); all of it is given back when an allocation fails
-// and with the context.  A block is given back only when no queued work of
-// another stream than the context's touches it, and a pinned one when nothing
-// queued does.
-class BlockPool {
- public:
-  BlockPool(bool host, size_t limit) : host_(host), limit_(limit) {}
-  BlockPool(const BlockPool&) = delete;
-  BlockPool& operator=(const BlockPool&) = delete;
-  ~BlockPool() { trim(); }
-  template <class T>
-  hipError_t get(T** p, size_t bytes) {
-    void* q = nullptr;
-    hipError_t e = take(&q, bytes);
-    *p = static_cast<T*>(q);
-    return e;
-  }
-  void put(void* p);  // null: nothing
-  void trim();        // frees every idle block
-
- private:
-  hipError_t take(void** p, size_t bytes);
-  hipError_t allocate(void** p, size_t bytes);
-  void release(void* p);
-  const bool host_;
-  const size_t limit_;
-  std::mutex m_;
-  std::unordered_map<void*, size_t> live_;
-  std::multimap<size_t, void*> idle_;
-  size_t idleBytes_ = 0;
-};
-constexpr size_t POOL_DEVICE_BYTES = (size_t)256 << 20;
-constexpr size_t POOL_HOST_BYTES = (size_t)16 << 20;
 }  // namespace lsdg
 
 struct lsdg_ctx_s {

@@ -1,13 +1,49 @@
-// BlockPool: a context's device and pinned blocks between the objects that use
-// them (lsdg_internal.h).
-#include "lsdg_internal.h"
+// Allocation and BlockPool (pool.h).  Locks: the list of pools before a pool's
+// own; allocations run under neither, as a failed one trims every pool.
+#include "pool.h"
 
 namespace lsdg {
 
+static std::mutex g_poolsMutex;
+static BlockPool* g_pools = nullptr;
+
 static size_t rounded(size_t bytes) { return (bytes + 4095) & ~(size_t)4095; }
 
-hipError_t BlockPool::allocate(void** p, size_t bytes) {
-  return host_ ? hipHostMalloc(p, bytes, hipHostMallocMapped) : hipMalloc(p, bytes);
+static hipError_t allocate(bool host, void** p, size_t bytes) {
+  const auto once = [&] { return host ? hipHostMalloc(p, bytes, hipHostMallocMapped) : hipMalloc(p, bytes); };
+  hipError_t e = once();
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    BlockPool::trim_all(host);
+    e = once();
+  }
+  if (e != hipSuccess) *p = nullptr;
+  return e;
+}
+
+hipError_t alloc_device(void** p, size_t bytes) { return allocate(false, p, bytes); }
+hipError_t alloc_pinned(void** p, size_t bytes) { return allocate(true, p, bytes); }
+
+BlockPool::BlockPool(bool host, size_t limit) : host_(host), limit_(limit) {
+  std::lock_guard<std::mutex> lock(g_poolsMutex);
+  next_ = g_pools;
+  if (next_) next_->prev_ = this;
+  g_pools = this;
+}
+
+BlockPool::~BlockPool() {
+  {
+    std::lock_guard<std::mutex> lock(g_poolsMutex);
+    (prev_ ? prev_->next_ : g_pools) = next_;
+    if (next_) next_->prev_ = prev_;
+  }
+  trim();
+}
+
+void BlockPool::trim_all(bool host) {
+  std::lock_guard<std::mutex> lock(g_poolsMutex);
+  for (BlockPool* q = g_pools; q; q = q->next_)
+    if (q->host_ == host) q->trim();
 }
 
 void BlockPool::release(void* p) {
@@ -18,28 +54,21 @@ void BlockPool::release(void* p) {
 hipError_t BlockPool::take(void** p, size_t bytes) {
   *p = nullptr;
   bytes = rounded(bytes ? bytes : 1);
+  {
+    std::lock_guard<std::mutex> lock(m_);
+    auto it = idle_.lower_bound(bytes);
+    if (it != idle_.end() && it->first - bytes <= bytes / 4) {
+      live_.emplace(it->second, it->first);
+      *p = it->second;
+      idleBytes_ -= it->first;
+      idle_.erase(it);
+      return hipSuccess;
+    }
+  }
+  hipError_t e = allocate(host_, p, bytes);
+  if (e != hipSuccess) return e;
   std::lock_guard<std::mutex> lock(m_);
-  auto it = idle_.lower_bound(bytes);
-  if (it != idle_.end() && it->first - bytes <= bytes / 4) {
-    *p = it->second;
-    idleBytes_ -= it->first;
-    live_[*p] = it->first;
-    idle_.erase(it);
-    return hipSuccess;
-  }
-  hipError_t e = allocate(p, bytes);
-  if (e != hipSuccess && !idle_.empty()) {
-    (void)hipGetLastError();
-    for (auto& b : idle_) release(b.second);
-    idle_.clear();
-    idleBytes_ = 0;
-    e = allocate(p, bytes);
-  }
-  if (e != hipSuccess) {
-    *p = nullptr;
-    return e;
-  }
-  live_[*p] = bytes;
+  live_.emplace(*p, bytes);
   return hipSuccess;
 }
 
@@ -50,12 +79,12 @@ void BlockPool::put(void* p) {
   if (it == live_.end()) return;
   const size_t bytes = it->second;
   live_.erase(it);
-  if (idleBytes_ + bytes > limit_) {
-    release(p);
+  if (idleBytes_ + bytes <= limit_) {
+    idle_.emplace(bytes, p);
+    idleBytes_ += bytes;
     return;
   }
-  idle_.emplace(bytes, p);
-  idleBytes_ += bytes;
+  release(p);
 }
 
 void BlockPool::trim() {

@@ -1,6 +1,7 @@
 """Objects made in memory that earlier objects of the context gave back: they
 read nothing of what those left there, whatever the order of sizes, kinds and
 destruction, and a batch that runs once gives what a kept plan gives."""
+import queue
 import threading
 
 import numpy as np
@@ -71,3 +72,47 @@ def test_reused_memory_changes_nothing():
     for t in threads:
         t.join()
     assert not bad
+
+
+def test_another_thread_destroys_while_the_owner_creates(ctx):
+    """Frames and references of one context, given back by a second thread
+    while the owner makes the next ones in their memory: none is handed out
+    while the other still holds it."""
+    cam = synth.camera(160, 120)
+    rng = np.random.default_rng(9)
+    images = [rng.integers(0, 256, (120, 160)).astype(np.uint8) for _ in range(4)]
+    depth, var = np.full((120, 160), 1.0, np.float32), np.full((120, 160), 0.01, np.float32)
+    q = queue.Queue()
+    errors = []
+
+    def destroy():
+        try:
+            for x in iter(q.get, None):
+                x.destroy()
+        except Exception as e:  # reported below
+            errors.append(e)
+
+    t = threading.Thread(target=destroy)
+    t.start()
+    held = []
+    try:
+        for k in range(200):
+            f = ctx.frame(k, cam, images[k % 4])
+            f.set_depth(depth, var)
+            r = ctx.ref(f)
+            n = r.num_points(1)
+            held.append((k, f, r, n))
+            if len(held) > 3:
+                j, f, r, n = held.pop(0)
+                assert np.array_equal(f.read(lsdg.WHAT_IMAGE, 0), images[j % 4].astype(np.float32))
+                p = r.points(1)
+                assert len(p) == n and (p[:, 2] == 1.0).all()
+                q.put(r)
+                q.put(f)
+        for _, f, r, _ in held:
+            q.put(r)
+            q.put(f)
+    finally:
+        q.put(None)
+        t.join()
+    assert not errors
