@@ -2,6 +2,8 @@
 // own; allocations run under neither, as a failed one trims every pool.
 #include "pool.h"
 
+#include <exception>
+
 namespace lsdg {
 
 static std::mutex g_poolsMutex;
@@ -54,7 +56,7 @@ void BlockPool::release(void* p) {
 hipError_t BlockPool::take(void** p, size_t bytes) {
   *p = nullptr;
   bytes = rounded(bytes ? bytes : 1);
-  {
+  try {
     std::lock_guard<std::mutex> lock(m_);
     auto it = idle_.lower_bound(bytes);
     if (it != idle_.end() && it->first - bytes <= bytes / 4) {
@@ -64,11 +66,19 @@ hipError_t BlockPool::take(void** p, size_t bytes) {
       idle_.erase(it);
       return hipSuccess;
     }
+  } catch (const std::exception&) {
+    return hipErrorOutOfMemory;  // of the host, for the pool's own record
   }
   hipError_t e = allocate(host_, p, bytes);
   if (e != hipSuccess) return e;
-  std::lock_guard<std::mutex> lock(m_);
-  live_.emplace(*p, bytes);
+  try {
+    std::lock_guard<std::mutex> lock(m_);
+    live_.emplace(*p, bytes);
+  } catch (const std::exception&) {
+    release(*p);
+    *p = nullptr;
+    return hipErrorOutOfMemory;
+  }
   return hipSuccess;
 }
 
@@ -80,9 +90,12 @@ void BlockPool::put(void* p) {
   const size_t bytes = it->second;
   live_.erase(it);
   if (idleBytes_ + bytes <= limit_) {
-    idle_.emplace(bytes, p);
-    idleBytes_ += bytes;
-    return;
+    try {
+      idle_.emplace(bytes, p);
+      idleBytes_ += bytes;
+      return;
+    } catch (const std::exception&) {  // no record of it: freed
+    }
   }
   release(p);
 }

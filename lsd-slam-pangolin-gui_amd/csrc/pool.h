@@ -23,7 +23,7 @@ hipError_t alloc_pinned(void** p, size_t bytes);
 // not fit is freed at once); all of it is given back when an allocation of the
 // process fails and with the context.  A block is given back only when no
 // queued work of another stream than the context's touches it, and a pinned
-// one when nothing queued does.
+// one when nothing queued does.  Nothing throws.
 class BlockPool {
  public:
   BlockPool(bool host, size_t limit);

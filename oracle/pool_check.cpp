@@ -1,12 +1,13 @@
 // The library's block pool (csrc/pool.cpp) over an allocator that counts and
 // can run out: reuse, its bound, giving idle blocks back to other pools and to
-// plain allocations, and blocks given back by other threads.  Host code only;
-// prints "ok" per check.
+// plain allocations, failing allocations of the host's own memory, and blocks
+// given back by other threads.  Host code only; prints "ok" per check.
 #include "../lsd-slam-pangolin-gui_amd/csrc/pool.h"
 
 #include <atomic>
 #include <cstdio>
 #include <cstdlib>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -14,6 +15,7 @@ namespace {
 std::mutex g_m;
 std::map<void*, size_t>* g_blocks;
 size_t g_used = 0, g_capacity = (size_t)-1;
+thread_local long g_failNewIn = -1;  // >= 0: the operator new after this many throws
 
 hipError_t take(void** p, size_t n) {
   std::lock_guard<std::mutex> lock(g_m);
@@ -46,12 +48,26 @@ void expect(bool ok, const char* what) {
 }  // namespace
 
 extern "C" {
-hipError_t hipMalloc(void** p, size_t n) { return take(p, n); }
+hipError_t hipMalloc(void** p, size_t n) {
+  const long f = g_failNewIn;
+  g_failNewIn = -1;  // the counted failures are the pool's own records
+  hipError_t e = take(p, n);
+  g_failNewIn = f;
+  return e;
+}
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return hipMalloc(p, n); }
 hipError_t hipFree(void* p) { return give(p); }
 hipError_t hipHostFree(void* p) { return give(p); }
 hipError_t hipGetLastError() { return hipSuccess; }
 }
+
+void* operator new(size_t n) {
+  if (g_failNewIn >= 0 && g_failNewIn-- == 0) throw std::bad_alloc();
+  if (void* p = std::malloc(n)) return p;
+  throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
 
 using lsdg::BlockPool;
 constexpr size_t KB = 1024;
@@ -97,6 +113,27 @@ int main() {
     (void)hipFree(p);
     (void)hipHostFree(q);
     g_capacity = (size_t)-1;
+  }
+  expect(g_used == 0, "nothing is left");
+  std::printf("ok\n");
+  {  // the host's memory runs out for the pool's records: an error or a free, no exception, no leak
+    BlockPool a(false, 1000 * KB);
+    for (long k = 0; k < 3; ++k) {
+      void *p, *q = nullptr;
+      g_failNewIn = k;
+      hipError_t e = a.get(&p, 16 * KB);
+      g_failNewIn = -1;
+      expect(e == hipSuccess ? p != nullptr : e == hipErrorOutOfMemory && p == nullptr, "get without a record");
+      if (e != hipSuccess) expect(a.get(&p, 16 * KB) == hipSuccess, "get");
+      g_failNewIn = k;
+      a.put(p);
+      g_failNewIn = -1;
+      g_failNewIn = k;
+      e = a.get(&q, 16 * KB);
+      g_failNewIn = -1;
+      expect((e == hipSuccess) == (q != nullptr), "get of an idle block without a record");
+      a.put(q);
+    }
   }
   expect(g_used == 0, "nothing is left");
   std::printf("ok\n");
