@@ -5,7 +5,7 @@
 //
 // Whole-job kernel (k_batch_job).  While a job's level is small, one block
 // runs the job's LM loop by itself: evaluation over the level's points,
-// deterministic block reduction, LM step in lane 0, repeat.  No launch and no
+// deterministic block reduction, LM step on wave 0, repeat.  No launch and no
 // inter-block communication per iteration.
 //
 // Multi-block steps (k_batch_eval + k_batch_solve).  For larger levels each
@@ -15,7 +15,7 @@
 // double-buffered per step so every block sees the same list) and writes each
 // tile's FP64 partial sums to a fixed slot.  k_batch_solve then merges each
 // job's slots in a fixed order (deterministic) and runs the job's LM step in
-// one lane: the reference's accept / reject / lambda / convergence logic
+// one wave: the reference's accept / reject / lambda / convergence logic
 // (SE3Tracker::trackFrame, Sim3Tracker::trackFrameSim3), an FP64 LDL^T solve
 // and exp(d) * T, and writes the pose the job's next evaluation uses.  The
 // kernel boundary between the two orders the partial sums, so no block waits
@@ -69,7 +69,6 @@ __global__ __launch_bounds__(256) void k_batch_init(BatchArgs a) {
     a.st[j] = s;
     a.ntiles[j] = nt;  // parity 0
     a.ntiles[a.njobs + j] = 0;
-    a.counters[j] = 0u;
     if (nt > 0) atomicAdd(a.remaining, 1);
   }
 }
@@ -151,7 +150,7 @@ __global__ __launch_bounds__(BATCH_BS) void k_batch_eval(BatchArgs a, int parity
 
 // Merge and LM step of one LM iteration: one block per job.  Wave w sums the
 // job's tile rows w, w + 4, ... (row order within a wave), the four wave sums
-// are added in wave order, and lane 0 runs the LM step on the job's
+// are added in wave order, and wave 0 runs the LM step on the job's
 // descriptor and control block staged in LDS (their loads are issued
 // alongside the row loads).  Also zeroes the next step's tile count of jobs
 // that are already finished.
@@ -213,7 +212,7 @@ __global__ __launch_bounds__(BATCH_SOLVE_BS) void k_batch_solve(BatchArgs a, int
 // Whole LM of one job in one block, for as long as the job's current level
 // has at most a.jobMaxPoints points: the level's evaluation over the block,
 // the block's deterministic reduction (wave reduce-scatter, then waves in
-// order) and the LM step in lane 0, repeated with no launch and no
+// order) and the LM step on wave 0, repeated with no launch and no
 // inter-block communication in between.  The job's descriptor and control
 // block live in LDS meanwhile.  On exit the job is finished or stands at a
 // larger level, whose tile count goes to the parity-0 slot for the

@@ -81,7 +81,6 @@ struct BatchArgs {
   JobState* st;
   int njobs;
   int* ntiles;        // [2][njobs] tile counts of this / next step
-  unsigned* counters; // [njobs] finished tiles of this step
   double* partials;   // rows of NS doubles
   int* remaining;     // jobs still running
   int ppt;            // points per thread per tile

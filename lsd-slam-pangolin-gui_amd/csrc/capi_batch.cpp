@@ -58,7 +58,6 @@ struct lsdg_batch_s {
   JobDesc* d_jobs = nullptr;
   JobState* d_st = nullptr;
   int* d_ntiles = nullptr;
-  unsigned* d_counters = nullptr;
   int* d_remaining = nullptr;
   int* h_remaining = nullptr;  // pinned
   double* d_partials = nullptr;
@@ -92,7 +91,7 @@ static void batch_free(lsdg_batch b) {
   if (b->g_first) (void)hipGraphDestroy(b->g_first);
   if (b->g_cont) (void)hipGraphDestroy(b->g_cont);
   lsdg_ctx c = b->ctx;
-  for (void* p : {(void*)b->d_jobs, (void*)b->d_st, (void*)b->d_ntiles, (void*)b->d_counters, (void*)b->d_remaining,
+  for (void* p : {(void*)b->d_jobs, (void*)b->d_st, (void*)b->d_ntiles, (void*)b->d_remaining,
                   (void*)b->d_partials, (void*)b->d_coop, (void*)b->d_epoch, b->d_pyr})
     c->blocks.put(p);
   for (void* p : {(void*)b->h_jobs, (void*)b->h_remaining, (void*)b->h_st, b->h_pyr}) c->pinned.put(p);
@@ -168,7 +167,6 @@ static BatchArgs batch_args(lsdg_batch b, int c) {
   a.st = b->d_st + j0;
   a.njobs = j1 - j0;
   a.ntiles = b->d_ntiles + 2 * j0;
-  a.counters = b->d_counters + j0;
   a.partials = b->d_partials;
   a.remaining = b->d_remaining + c;
   a.ppt = b->ppt;
@@ -381,7 +379,6 @@ lsdg_status lsdg::batch_create_shaped(lsdg_ctx c, const lsdg_job* jobs, int32_t 
   if ((e = c->blocks.get(&b->d_jobs, sizeof(JobDesc) * n)) != hipSuccess ||
       (e = c->blocks.get(&b->d_st, sizeof(JobState) * n)) != hipSuccess ||
       (e = c->blocks.get(&b->d_ntiles, sizeof(int) * 2 * n)) != hipSuccess ||
-      (e = c->blocks.get(&b->d_counters, sizeof(unsigned) * n)) != hipSuccess ||
       (e = c->blocks.get(&b->d_remaining, 64)) != hipSuccess ||
       (b->coopK > 0 && (e = c->blocks.get(&b->d_coop, sizeof(unsigned long long) * coopWords)) != hipSuccess) ||
       (b->coopK > 0 && (e = launch_fill_words(b->d_coop, coopWords, 0ull, c->stream)) != hipSuccess) ||

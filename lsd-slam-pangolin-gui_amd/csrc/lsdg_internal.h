@@ -103,7 +103,6 @@ struct DepthGeom {
   float fx, fy, cx, cy, fxi, fyi, cxi, cyi;
 };
 
-// Device tables of a batched pyramid rebuild.
 // A frame's inverse-depth pyramid (levels 0 .. PYR - 1, each half the one
 // above, rounded down).
 struct PyrDepthArgs {
@@ -138,6 +137,7 @@ __device__ inline void fuse4(const float* ida, const float* va, float& oid, floa
   }
 }
 
+// Device tables of a batched pyramid rebuild.
 struct PyrBatch {
   const void* img_args;
   const void* grad_args;

@@ -18,7 +18,7 @@ hipError_t alloc_pinned(void** p, size_t bytes);
 // Device or pinned host blocks that a context's objects give back, kept for
 // the next ones: allocating and freeing a frame's arrays cost 38 of the 63 us
 // that making and destroying a 320x240 frame took, and a batch plan has eight
-// device and three pinned blocks.  An idle block serves a request of at least
+// device and four pinned blocks.  An idle block serves a request of at least
 // four fifths of its size.  At most `limit` bytes stay idle (a block that does
 // not fit is freed at once); all of it is given back when an allocation of the
 // process fails and with the context.  A block is given back only when no
