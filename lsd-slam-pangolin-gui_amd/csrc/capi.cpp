@@ -207,8 +207,8 @@ static void frame_intrinsics(lsdg_frame f, const lsdg_camera* cam) {
   }
 }
 
-lsdg_status lsdg::frame_alloc(lsdg_ctx c, int32_t id, const lsdg_camera* cam, int32_t precision,
-                                lsdg_frame* out) {
+lsdg_status lsdg::frame_alloc(lsdg_ctx c, int32_t id, const lsdg_camera* cam, int32_t precision, bool quad,
+                              lsdg_frame* out) {
   if (!c || !cam || !out) return LSDG_EINVAL;
   if (cam->w < 32 || cam->h < 32 || cam->w > 16384 || cam->h > 16384 || (cam->w >> (PYR - 1)) < 4 ||
       (cam->h >> (PYR - 1)) < 4)
@@ -225,7 +225,7 @@ lsdg_status lsdg::frame_alloc(lsdg_ctx c, int32_t id, const lsdg_camera* cam, in
   f->id = id;
   f->precision = precision;
   frame_intrinsics(f, cam);
-  // one pool: per level image, grad4, [gradh], maxg, idepth, ivar; then u8 staging and the level-1 mask
+  // one pool: per level image, grad4, [gradh], maxg, idepth, ivar; then u8 staging, [quad] and the level-1 mask
   size_t off[PYR][6];
   size_t total = 0;
   auto take = [&](size_t bytes) {
@@ -243,7 +243,7 @@ lsdg_status lsdg::frame_alloc(lsdg_ctx c, int32_t id, const lsdg_camera* cam, in
     off[l][5] = take(n * 4);
   }
   size_t off_u8 = take((size_t)f->w[0] * f->h[0]);
-  size_t off_quad = take((size_t)f->w[0] * f->h[0] * 4);
+  size_t off_quad = quad ? take((size_t)f->w[0] * f->h[0] * 4) : 0;
   size_t off_wg = take((size_t)f->w[1] * f->h[1]);
   hipError_t e = c->blocks.get(&f->d_pool, total);
   if (e != hipSuccess) {
@@ -260,9 +260,16 @@ lsdg_status lsdg::frame_alloc(lsdg_ctx c, int32_t id, const lsdg_camera* cam, in
     f->d_ivar[l] = (float*)(b + off[l][5]);
   }
   f->d_input_u8 = (uint8_t*)(b + off_u8);
-  f->d_quad = (uint32_t*)(b + off_quad);
+  f->d_quad = quad ? (uint32_t*)(b + off_quad) : nullptr;
   f->d_wasGood = (uint8_t*)(b + off_wg);
   *out = f;
+  return LSDG_OK;
+}
+
+lsdg_status lsdg::frame_ensure_quad(lsdg_frame f) {
+  if (f->d_quad) return LSDG_OK;
+  CK(f->ctx, f->ctx->blocks.get(&f->d_quadBlock, (size_t)f->w[0] * f->h[0] * 4));
+  f->d_quad = (uint32_t*)f->d_quadBlock;
   return LSDG_OK;
 }
 
@@ -270,6 +277,7 @@ extern "C" lsdg_status lsdg_frame_destroy(lsdg_frame f) {
   if (!f) return LSDG_EINVAL;
   (void)hipStreamSynchronize(f->ctx->stream);
   f->ctx->blocks.put(f->d_pool);
+  f->ctx->blocks.put(f->d_quadBlock);
   delete f;
   return LSDG_OK;
 }
@@ -328,7 +336,7 @@ extern "C" lsdg_status lsdg_frame_create(lsdg_ctx c, int32_t id, const lsdg_came
                                          int32_t precision, lsdg_frame* out) {
   if (!image) return LSDG_EINVAL;
   lsdg_frame f;
-  lsdg_status st = frame_alloc(c, id, cam, precision, &f);
+  lsdg_status st = frame_alloc(c, id, cam, precision, false, &f);
   if (st != LSDG_OK) return st;
   size_t n = (size_t)cam->w * cam->h;
   hipError_t e = hipMemcpyAsync(f->d_image[0], image, n * 4, hipMemcpyHostToDevice, c->stream);
@@ -350,7 +358,7 @@ extern "C" lsdg_status lsdg_frame_create_u8(lsdg_ctx c, int32_t id, const lsdg_c
                                             int32_t stride, int32_t precision, lsdg_frame* out) {
   if (!image || !cam || stride < cam->w) return LSDG_EINVAL;
   lsdg_frame f;
-  lsdg_status st = frame_alloc(c, id, cam, precision, &f);
+  lsdg_status st = frame_alloc(c, id, cam, precision, true, &f);
   if (st != LSDG_OK) return st;
   // a 2D copy from pageable memory goes row by row: pack padded rows first
   std::vector<uint8_t> packed;

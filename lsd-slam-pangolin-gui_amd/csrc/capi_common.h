@@ -11,7 +11,10 @@ lsdg_status frame_depth_from_level0(lsdg_frame f);
 // queued, e.g. launch_fill_regularize with the frame as setDepth.
 void frame_depth_written(lsdg_frame f);
 // A frame of camera cam with every array allocated and nothing valid yet.
-lsdg_status frame_alloc(lsdg_ctx c, int32_t id, const lsdg_camera* cam, int32_t precision, lsdg_frame* out);
+// quad: with the array of the packed 8-bit level 0 (frame_ensure_quad adds it
+// to a frame made without).
+lsdg_status frame_alloc(lsdg_ctx c, int32_t id, const lsdg_camera* cam, int32_t precision, bool quad, lsdg_frame* out);
+lsdg_status frame_ensure_quad(lsdg_frame f);
 // Builds the pyramid data in `need` (fd_bit flags) that the frame does not
 // hold yet, on the context stream (Frame::require).
 lsdg_status frame_require(lsdg_frame f, unsigned need);

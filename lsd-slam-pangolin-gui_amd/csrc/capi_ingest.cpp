@@ -124,7 +124,7 @@ extern "C" lsdg_status lsdg_frame_create_undistorted(lsdg_ctx c, int32_t id, con
   lsdg_status st = check_ingest(c, cam->w, cam->h, u, image, stride);
   if (st != LSDG_OK) return st;
   lsdg_frame f;
-  st = frame_alloc(c, id, cam, precision, &f);
+  st = frame_alloc(c, id, cam, precision, true, &f);
   if (st != LSDG_OK) return st;
   st = ingest_into(f, u, image, stride, undistorted);
   if (st != LSDG_OK) {
@@ -140,6 +140,8 @@ extern "C" lsdg_status lsdg_frame_ingest(lsdg_frame f, int32_t id, lsdg_undistor
   if (!f) return LSDG_EINVAL;
   lsdg_ctx c = f->ctx;
   lsdg_status st = check_ingest(c, f->w[0], f->h[0], u, image, stride);
+  if (st != LSDG_OK) return st;
+  st = frame_ensure_quad(f);
   if (st != LSDG_OK) return st;
   // every field as in a new frame; the arrays and the camera stay, and the
   // depth version moves on so point clouds built from the old content are
@@ -170,6 +172,7 @@ extern "C" lsdg_status lsdg_frame_ingest(lsdg_frame f, int32_t id, lsdg_undistor
   }
   fresh.d_input_u8 = f->d_input_u8;
   fresh.d_quad = f->d_quad;
+  fresh.d_quadBlock = f->d_quadBlock;
   fresh.d_wasGood = f->d_wasGood;
   fresh.depthVersion = f->depthVersion + 1;
   *f = fresh;

@@ -243,7 +243,8 @@ struct lsdg_frame_s {
   float* d_idepth[lsdg::PYR];
   float* d_ivar[lsdg::PYR];
   uint8_t* d_input_u8 = nullptr;  // staging for u8 uploads (w*h)
-  uint32_t* d_quad = nullptr;     // per pixel, the four bytes of the 2x2 pixels to its right and below
+  uint32_t* d_quad = nullptr;     // per pixel, the four bytes of the 2x2 pixels to its right and below; null: never 8-bit
+  void* d_quadBlock = nullptr;    // its own block where the frame was made without it
   bool u8Level0 = false;          // d_input_u8 and d_quad hold level 0 (every level-0 writer keeps it so)
   uint8_t* d_wasGood = nullptr;   // refPixelWasGood (level 1)
   unsigned valid = 0;             // built pyramid data (fd_bit flags)
