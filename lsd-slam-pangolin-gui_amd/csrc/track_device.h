@@ -150,7 +150,9 @@ __device__ inline float fsqrt(float x) {
 // correctly rounded reciprocal serves every division by the same value.
 //
 // recip_rn: v_rcp_f32 is within 1 ulp; one Newton step in fma arithmetic gives
-// 1 / b correctly rounded (checked for every significand).
+// 1 / b correctly rounded (oracle/rounding_check.hip compares all three on the
+// device: reciprocals and roots of every float of the range, quotients for
+// every significand of the denominator).
 // div_rn: a / b from y = RN(1 / b).  q0 = RN(a y) is within two ulps; the
 // remainder a - b q0 is exact up to 2^-24 of itself, so q1 is within one ulp
 // of a / b, its remainder is exact, and the last fma rounds correctly

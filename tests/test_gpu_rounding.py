@@ -1,7 +1,11 @@
 """The FP32 evaluation's unscaled divisions (shared correctly rounded
 reciprocals) and the scaled ones they fall back to at the ends of the exponent
 range: both give the oracle's terms, so the sums agree as in the plain parity
-tests wherever the depths' unit puts the denominators."""
+tests wherever the depths' unit puts the denominators.  The operations
+themselves are compared with correctly rounded ones over every significand."""
+import ctypes as C
+import os
+
 import numpy as np
 import pytest
 
@@ -63,3 +67,18 @@ def test_evaluations_at_the_ends_of_the_range(ctx, k, mixed, trans):
             _close([a.usage], [b.usage], n)
     for x in (ref, fr, kf):
         x.destroy()
+
+
+@pytest.mark.parametrize("what,least", [("reciprocals", 2 * 121 << 23), ("square roots", 121 << 23),
+                                        ("quotients", 50 << 23)])
+def test_unscaled_operations_round_correctly(what, least):
+    """oracle/rounding_check.hip: reciprocals and square roots of every float
+    from 2^-60 to 2^61, quotients for every significand of the denominator."""
+    path = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "oracle", "librounding_check.so")
+    if not os.path.exists(path):
+        pytest.fail(f"{path} is not built; run `make -C oracle`")
+    L = C.CDLL(path)
+    out, example = (C.c_ulonglong * 2)(), (C.c_uint * 4)()
+    assert L.rounding_check(["reciprocals", "square roots", "quotients"].index(what), out, example) == 0
+    assert out[1] == 0, [hex(v) for v in example]
+    assert out[0] >= least
