@@ -29,7 +29,7 @@ constexpr int PYR = LSDG_PYRAMID_LEVELS;
 constexpr int NS_SE3 = 40;
 constexpr int NS_SIM3 = 48;
 constexpr int NS_MAX = 48;
-constexpr int EVAL_MAX_BLOCKS = 128;  // blocks of one evaluation (track.hip)
+constexpr int EVAL_MAX_BLOCKS = 512;  // blocks of one evaluation (track.hip)
 constexpr size_t EVAL_ROW_WORDS = (size_t)EVAL_MAX_BLOCKS * NS_MAX * 2;
 
 // Pyramid data of a frame, one validity bit per (kind, level): the

@@ -17,6 +17,7 @@
 //               written straight to the caller's (possibly host-mapped) buffer.
 // The per-point float expressions keep the reference's operation order so the
 // isGood mask and counts match the CPU restatement bit for bit.
+#include <algorithm>
 #include <mutex>
 
 #include "track_device.h"
@@ -195,18 +196,20 @@ __global__ __launch_bounds__(EVAL_BS) void k_energy_grad_sim3(PointsLevel pts, c
 
 // ------------------------------------------------------------ launchers
 // Plain-path evaluation grid: one point per thread (the shortest dependency
-// chain per thread), at most EVAL_MAX_BLOCKS blocks: block 0 reads a row of
-// each.  Eight evaluations (levels 1-4, SE3 and Sim3) with at most 32, 64, 128
-// and 256 blocks: 640x480 180, 175, 176, 176 us; 1280x960 (FP16) 194, 184, 182,
-// 186.  With a completion counter, shuffles through the LDS in the wave
-// reduction and one column of additions in the last block's merge they took
-// 216 and 240 us (the kernel 12 us on average, now 6.8; the rest of a call is
-// its launch and wait).
+// chain per thread) up to 128 blocks, as block 0 reads a row of each: 256 of
+// them cost 1 us more than they save up to about 100 thousand points.  From
+// five points per thread of 128 blocks on there are 256, from 16 per thread of
+// those 512.  One SE3 evaluation with 128 / 256 / 512 blocks: 75 thousand points
+// 22.2 / 23.6 / 24.4 us, 169 thousand 25.0 / 24.9 / 29.9, 291 thousand 31.4 /
+// 28.9 / 32.8, 882 thousand 57 / 43 / 43, 2.3 million 114 / 73 / 61.
+//   (Behind the rows: with a completion counter, shuffles through the LDS in the
+// wave reduction and one column of additions in the last block's merge, eight
+// evaluations of 640x480, levels 1-4, took 216 us, 1280x960 FP16 240; now 175
+// and 182, the kernel 6.8 us on average where it took 12: the rest of a call is
+// its launch and wait.)
 static inline int eval_blocks(int n) {
-  int nb = (n + EVAL_BS - 1) / EVAL_BS;
-  if (nb < 1) nb = 1;
-  if (nb > EVAL_MAX_BLOCKS) nb = EVAL_MAX_BLOCKS;
-  return nb;
+  const int most = n < 128 * EVAL_BS * 5 ? 128 : n < 256 * EVAL_BS * 16 ? 256 : EVAL_MAX_BLOCKS;
+  return std::max(1, std::min((n + EVAL_BS - 1) / EVAL_BS, most));
 }
 
 // The next launch's tag: never 0, which the rows are cleared to at the first
