@@ -437,7 +437,8 @@ extern "C" lsdg_status lsdg_frame_set_depth(lsdg_frame f, const float* idepth, c
 
 lsdg_status lsdg::frame_ensure_was_good(lsdg_frame f) {
   if (f->wasGoodAllocated) return LSDG_OK;
-  CK(f->ctx, hipMemsetAsync(f->d_wasGood, 1, (size_t)f->w[1] * f->h[1], f->ctx->stream));
+  if (!f->wasGoodOnes) CK(f->ctx, hipMemsetAsync(f->d_wasGood, 1, (size_t)f->w[1] * f->h[1], f->ctx->stream));
+  f->wasGoodOnes = false;
   f->wasGoodAllocated = true;
   return LSDG_OK;
 }
@@ -900,7 +901,7 @@ extern "C" lsdg_status lsdg_se3_track(lsdg_ctx c, lsdg_ref r, lsdg_frame f, cons
   const lsdg_params& P = c->P;
   uint8_t* mask = nullptr;
   const bool hadMask = f->wasGoodAllocated;
-  if (P.se3_min_level == 1) {  // refPixelWasGood is a level-1 mask
+  if (P.se3_min_level == 1 && c->track_pause == 0) {  // refPixelWasGood is a level-1 mask
     lsdg_status s0 = frame_ensure_was_good(f);
     if (s0 != LSDG_OK) return s0;
     mask = f->d_wasGood;
@@ -911,7 +912,10 @@ extern "C" lsdg_status lsdg_se3_track(lsdg_ctx c, lsdg_ref r, lsdg_frame f, cons
   // a frame has a mask from its first evaluation at level 1 on: an alignment
   // that ended before it leaves the frame without (propagation then tests the
   // residuals instead)
-  if (!hadMask && (s0 != LSDG_OK || !ran || s->evalsAt[1] == 0)) f->wasGoodAllocated = false;
+  if (!hadMask && (s0 != LSDG_OK || !ran || s->evalsAt[1] == 0)) {
+    f->wasGoodAllocated = false;
+    f->wasGoodOnes = mask && s0 == LSDG_OK && ran;
+  }
   if (s0 != LSDG_OK) return s0;
   if (!ran) return se3_track_steps(c, r, f, init, out, stats);
   lsdg_track_stats st;

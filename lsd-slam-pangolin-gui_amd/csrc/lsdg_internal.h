@@ -249,6 +249,7 @@ struct lsdg_frame_s {
   uint8_t* d_wasGood = nullptr;   // refPixelWasGood (level 1)
   unsigned valid = 0;             // built pyramid data (fd_bit flags)
   bool wasGoodAllocated = false;
+  bool wasGoodOnes = false;       // not allocated, but all ones since an alignment that never wrote it
   bool hasDepth = false;
   // pose fields
   int parentId = -1;

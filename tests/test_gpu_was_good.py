@@ -59,3 +59,29 @@ def test_failed_alignment_leaves_no_mask(ctx, how):
     assert plain["is_valid"].any() and not np.array_equal(plain["is_valid"], masked["is_valid"])
     for k in plain:
         assert np.array_equal(plain[k].view(np.uint8), failed[k].view(np.uint8)), k
+
+
+def test_mask_after_alignments_that_wrote_none(ctx):
+    """The first alignment that reaches level 1 starts from an all-ones mask,
+    however many failed before it."""
+    cam = synth.camera(200, 152)
+    d = synth.sim3_instance(41, cam=cam, max_trans=0.02, max_rot_deg=0.5, scale_range=(1.0, 1.0))
+    kf = ctx.frame(0, cam, d["a_img"])
+    kf.set_depth(d["a_idepth"], d["a_var"])
+    ref = ctx.ref(kf)
+    masks = []
+    for failures in ([], ["no depth"], ["few points", "few points"], ["few points", "no depth", "few points"]):
+        fr = ctx.frame(1, cam, d["b_img"])
+        for how in failures:
+            _fail(ctx, how, cam, d["a_img"], kf, fr)
+        assert (fr.read(lsdg.WHAT_REF_PIXEL_WAS_GOOD) == 1).all()
+        _, _, status = ctx.se3_track(ref, fr, synth.IDENTITY7)
+        assert status == lsdg.OK
+        masks.append(fr.read(lsdg.WHAT_REF_PIXEL_WAS_GOOD))
+        # and a failure afterwards leaves it
+        _fail(ctx, "few points", cam, d["a_img"], kf, fr)
+        assert np.array_equal(fr.read(lsdg.WHAT_REF_PIXEL_WAS_GOOD), masks[-1])
+        fr.destroy()
+    assert (masks[0] == 0).any() and all(np.array_equal(m, masks[0]) for m in masks)
+    ref.destroy()
+    kf.destroy()
