@@ -119,7 +119,7 @@ constexpr unsigned TRACK_LM_SPIN_MAX = 1u << 14;  // polls of about a microsecon
 // Alignments without a try after blocks gave up: the 16 ms of a vain one come
 // to 0.16 ms of each, beside the 0.6 ms that an alignment takes launch by launch.
 constexpr int TRACK_LM_PAUSE = 100;
-constexpr int TRACK_LM_MAX_BLOCKS = 64;
+constexpr int TRACK_LM_MAX_BLOCKS = 256;
 constexpr size_t TRACK_LM_WORDS = (size_t)2 * TRACK_LM_MAX_BLOCKS * NS_MAX * 2;
 // Blocks of a launch for alignments whose finest level has `pixels` pixels.
 int track_lm_blocks(lsdg_ctx c, int pixels);

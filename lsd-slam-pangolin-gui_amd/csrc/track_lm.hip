@@ -167,10 +167,16 @@ int track_lm_blocks(lsdg_ctx c, int pixels) {
   // best number goes with the square root of the points.  Measured per
   // alignment (FP32): 320x240 162 us with 16 blocks, 168 with 32, 187 with 64;
   // 640x480 175, 171, 187; 1280x960 224, 179, 172; 1920x1080 (FP16) 292, 210,
-  // 189.  The size alone decides, so that an image's result does not depend on
-  // whether the host knows the count of points yet.
-  const int nb = ((int)(std::sqrt((double)pixels) / 9.0) + 4) / 8 * 8;
-  return std::max(1, std::min(std::max(nb, 8), std::min(TRACK_LM_MAX_BLOCKS, c->num_cus)));
+  // 189.  Alignments down to a level of up to 1.5 Mpixel keep to 64 (the finest
+  // level 1280x960, SE3: 274 us, with 123 blocks 296); past it the finest level
+  // outweighs the exchanges of the coarser ones (finest level 1920x1080, SE3 /
+  // Sim3: 324 / 598 us with 64, 288 / 473 with 128, 299 / 472 with 160;
+  // 2048x1536: 286 / 478, 218 / 328, with 200 227 / 309; 4096x3072: 648 / 1742,
+  // 410 / 989, with 256 348 / 670).  The size alone decides, so that an image's
+  // result does not depend on whether the host knows the count of points yet.
+  const bool large = pixels > 3 << 19;
+  const int nb = ((int)(std::sqrt((double)pixels) / (large ? 11.0 : 9.0)) + 4) / 8 * 8;
+  return std::max(1, std::min(std::max(nb, 8), std::min(large ? TRACK_LM_MAX_BLOCKS : 64, c->num_cus)));
 }
 
 template <int KIND, int PREC>

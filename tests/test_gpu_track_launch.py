@@ -48,7 +48,7 @@ def _fields(st):
             *st.num_warp_update_calls]
 
 
-# 64x64: every level is small; 130x98: the split threshold; 322x242: ragged; 1282x962: the most blocks
+# 64x64: every level is small; 130x98: the split threshold; 322x242: ragged; 1282x962: 64 blocks
 @pytest.mark.parametrize("w,h", [(64, 64), (130, 98), (322, 242), (1282, 962)])
 @pytest.mark.parametrize("prec", [lsdg.FP32, lsdg.FP16])
 def test_one_launch_equals_launch_per_evaluation(ctx, monkeypatch, w, h, prec):
@@ -85,6 +85,32 @@ def test_one_launch_equals_launch_per_evaluation(ctx, monkeypatch, w, h, prec):
         H, H2 = np.array(st3.hessian[:]), np.array(st32.hessian[:])
         assert np.abs(H - H2).max() <= 1e-9 * max(np.abs(H2).max(), 1e-30)
     other.close()
+
+
+@pytest.mark.parametrize("prec", [lsdg.FP32, lsdg.BF16])
+def test_large_finest_level(ctx, monkeypatch, prec):
+    """Down to a level of more than 1.5 Mpixel, which takes more blocks."""
+    cam = synth.camera(1402, 1202)
+    p = lsdg.default_params()
+    p.se3_min_level = 0
+    steps = _steps_context(monkeypatch)
+    res = []
+    try:
+        for c in (ctx, steps):
+            c.set_params(p)
+            a, b, ref = _pair(c, cam, 41, prec)
+            (pose, st, status), n = _launches(c, lambda: c.se3_track(ref, b, synth.IDENTITY7))
+            (q, st3, status3), n3 = _launches(c, lambda: c.sim3_track(ref, b, [*synth.IDENTITY7, 1.0], 4, 0))
+            assert (n == 1 and n3 == 1) if c is ctx else (n > 2 and n3 > 2)
+            res.append((pose, q, _fields(st) + [status], _fields(st3) + [status3]))
+            for x in (ref, b, a):
+                x.destroy()
+    finally:
+        ctx.set_params(lsdg.default_params())
+        steps.close()
+    (pose, q, f, f3), (pose2, q2, g, g3) = res
+    assert f == g and f3 == g3
+    assert twist(pose, pose2) <= 1e-9 and twist(q[:7], q2[:7]) <= 1e-9 and abs(q[7] - q2[7]) <= 1e-9
 
 
 @pytest.mark.parametrize("steps", [False, True])
