@@ -60,8 +60,8 @@ hipError_t BlockPool::take(void** p, size_t bytes) {
     std::lock_guard<std::mutex> lock(m_);
     auto it = idle_.lower_bound(bytes);
     if (it != idle_.end() && it->first - bytes <= bytes / 4) {
-      live_.emplace(it->second, it->first);
-      *p = it->second;
+      live_.emplace(it->second.p, it->first);
+      *p = it->second.p;
       idleBytes_ -= it->first;
       idle_.erase(it);
       return hipSuccess;
@@ -89,20 +89,28 @@ void BlockPool::put(void* p) {
   if (it == live_.end()) return;
   const size_t bytes = it->second;
   live_.erase(it);
-  if (idleBytes_ + bytes <= limit_) {
+  if (bytes <= limit_) {
     try {
-      idle_.emplace(bytes, p);
+      idle_.emplace(bytes, Idle{p, puts_++});
       idleBytes_ += bytes;
-      return;
+      p = nullptr;
     } catch (const std::exception&) {  // no record of it: freed
     }
   }
-  release(p);
+  if (p) release(p);
+  while (idleBytes_ > limit_) {
+    auto oldest = idle_.begin();
+    for (auto b = idle_.begin(); b != idle_.end(); ++b)
+      if (b->second.since < oldest->second.since) oldest = b;
+    release(oldest->second.p);
+    idleBytes_ -= oldest->first;
+    idle_.erase(oldest);
+  }
 }
 
 void BlockPool::trim() {
   std::lock_guard<std::mutex> lock(m_);
-  for (auto& b : idle_) release(b.second);
+  for (auto& b : idle_) release(b.second.p);
   idle_.clear();
   idleBytes_ = 0;
 }

@@ -1,7 +1,8 @@
 // The library's block pool (csrc/pool.cpp) over an allocator that counts and
-// can run out: reuse, its bound, giving idle blocks back to other pools and to
-// plain allocations, failing allocations of the host's own memory, and blocks
-// given back by other threads.  Host code only; prints "ok" per check.
+// can run out: reuse, its bound and what it keeps, giving idle blocks back to
+// other pools and to plain allocations, failing allocations of the host's own
+// memory, and blocks given back by other threads.  Host code only; prints "ok"
+// per check.
 #include "../lsd-slam-pangolin-gui_amd/csrc/pool.h"
 
 #include <atomic>
@@ -14,7 +15,7 @@
 namespace {
 std::mutex g_m;
 std::map<void*, size_t>* g_blocks;
-size_t g_used = 0, g_capacity = (size_t)-1;
+size_t g_used = 0, g_capacity = (size_t)-1, g_allocations = 0;
 thread_local long g_failNewIn = -1;  // >= 0: the operator new after this many throws
 
 hipError_t take(void** p, size_t n) {
@@ -26,6 +27,7 @@ hipError_t take(void** p, size_t n) {
   *p = std::malloc(n);
   (*g_blocks)[*p] = n;
   g_used += n;
+  ++g_allocations;
   return hipSuccess;
 }
 hipError_t give(void* p) {
@@ -95,6 +97,20 @@ int main() {
     for (void*& p : v) expect(a.get(&p, 16 * KB) == hipSuccess, "get");
     for (void* p : v) a.put(p);
     expect(g_used == 64 * KB, "idle bytes are bounded");
+    // the blocks in use now replace the ones idle longest, and are found again
+    void* p;
+    for (int k = 0; k < 5; ++k) {
+      const size_t before = g_allocations;
+      expect(a.get(&p, 40 * KB) == hipSuccess, "get");
+      a.put(p);
+      expect(g_allocations == before + (k == 0 ? 1 : 0), "a size in use is kept beside older blocks");
+      expect(g_used <= 64 * KB, "idle bytes are bounded");
+    }
+    expect(a.get(&p, 16 * KB) == hipSuccess && g_used == 56 * KB, "the newest of the older blocks stayed");
+    a.put(p);
+    expect(a.get(&p, 100 * KB) == hipSuccess, "get");
+    a.put(p);
+    expect(g_used == 56 * KB, "a block over the limit is freed, and no other");
   }
   std::printf("ok\n");
   {  // idle blocks go back where another pool, or a plain allocation, finds no memory
