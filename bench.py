@@ -767,7 +767,7 @@ def main():
                  "max_twist_vs_fp64_sums": max(posemath.twist_error(a, b) for a, b in zip(posesk, poses32))}
         if not args.no_plain:
             _, k_ks = kernel_roofline(ctx, tk.plain_step, lsdg.KERNEL_EVAL)
-            kahan["plain_eval_avg_launch_us"] = round(1e3 * k_ks["ms"] / max(k_ks["launches"], 1), 3)
+            kahan["plain_alignment_avg_launch_us"] = round(1e3 * k_ks["ms"] / max(k_ks["launches"], 1), 3)
     finally:
         ctx.set_sums(lsdg.SUMS_FP64)
 
@@ -779,8 +779,8 @@ def main():
         out_plain = {"plain_fp32_frames_per_s": round(plain_fps, 2),
                      "batched_fp32_vs_plain_speedup": round(batched32_fps / plain_fps, 1),
                      "batched_fp16_vs_plain_speedup": round(batched16_fps / plain_fps, 1),
-                     "plain_eval_kernel_gbs": round(plain_ach, 2),
-                     "plain_eval_avg_launch_us": round(1e3 * plain_ks["ms"] / max(plain_ks["launches"], 1), 3),
+                     "plain_alignment_kernel_gbs": round(plain_ach, 2),
+                     "plain_alignment_avg_launch_us": round(1e3 * plain_ks["ms"] / max(plain_ks["launches"], 1), 3),
                      "max_twist_batched_fp32_vs_plain": max(posemath.twist_error(a, b)
                                                             for a, b in zip(poses32, t32.poses))}
 
