@@ -146,7 +146,7 @@ hipError_t launch_batch_solve(const BatchArgs& a, int kind, int parity, hipStrea
 hipError_t launch_batch_step(const BatchArgs& a, int kind, int prec, int acc, int parity, int grid, hipStream_t s);
 
 // Plan shapes (capi_batch.cpp) and the tuning table (capi_tune.cpp).
-lsdg_batch_config batch_default_shape(lsdg_ctx c, int kind, int n);
+lsdg_batch_config batch_default_shape(lsdg_ctx c, int n);
 lsdg_status batch_create_shaped(lsdg_ctx c, const lsdg_job* jobs, int32_t n, const lsdg_batch_config& shape,
                                 bool oneRun, lsdg_batch* out);
 // The table's entry for key into *out; false when there is none.

@@ -278,19 +278,23 @@ static lsdg_status validate_jobs(lsdg_ctx c, const lsdg_job* jobs, int32_t n) {
 //   Threads per block.  A CU holds one block of 512 threads or three of 256
 // (168 registers), so the small blocks give a job half as many threads again,
 // unless the limit of 16 blocks binds, but more rows to exchange.  Few jobs are
-// bound by the exchange: 512 (24 SE3 jobs of 752x478: 265 us against 286 with
-// 256; 32 Sim3 jobs of 640x480: 386 against 412).  Many are bound by issue: 256
-// (128 SE3 jobs of 640x480: 686 us against 790 with 512; 64 Sim3 jobs of
-// 1920x1080: 1150 against 1396, of 640x480: 511 against 542).  Between them the
-// line follows what a point costs: 64 SE3 jobs of 640x480 take 425 us with 512
-// and 434 with 256.
+// bound by the exchange: 512 (a run of 24 SE3 jobs of 640x480 331 us against 396
+// with 256; 8 Sim3 jobs 544 against 597, 32 659 against 720).  Many are bound by
+// issue: 256, from the number on where four blocks of 512 or fewer fit per job
+// (64 SE3 jobs of 640x480 475 us against 482 with 512, FP16 425 against 428, of
+// 320x240 to 1280x960 in one plan 715 against 809; 64 Sim3 jobs of 640x480 776
+// against 876, FP32 933 against 1044, of 1920x1080 4321 against 6033).
 //   Levels of up to two points per thread are not split: evaluating them whole
-// costs no more than an exchange (24 SE3 jobs of 752x478, 512 threads: 265 us,
-// with a limit of 512 points 277; 64 Sim3 jobs of 640x480, 256 threads: 456,
-// with a limit of 1024 points 492).
-lsdg_batch_config lsdg::batch_default_shape(lsdg_ctx c, int kind, int n) {
+// costs no more than an exchange where a job has many rows to read (launches of
+// 24 SE3 jobs of 752x478, 512 threads: 265 us, with a limit of 512 points 277).
+// For 64 jobs of 640x480 splitting every level is 1% faster, for 24 the same.
+//   No dispatch groups: eight of them gain 1% for the SE3 plans above, but a
+// plan in whose order every eighth job is alike has all its long jobs on one
+// XCD then (64 Sim3 jobs over eight pairs of 640x480 780 -> 1019 us, of
+// 1920x1080 4363 -> 6927).  The tuner measures the jobs at hand and may take them.
+lsdg_batch_config lsdg::batch_default_shape(lsdg_ctx c, int n) {
   const int perJob = c->num_cus / n;  // blocks of 512 threads
-  const bool small = kind == LSDG_JOB_SIM3 ? perJob <= 4 : perJob < 4;
+  const bool small = perJob <= 4;
   lsdg_batch_config s{};
   s.schedule = LSDG_SCHEDULE_COOP;
   s.coop_block = small ? 256 : 512;
@@ -472,7 +476,7 @@ static lsdg_status batch_create(lsdg_ctx c, const lsdg_job* jobs, int32_t n, boo
   lsdg_status st = validate_jobs(c, jobs, n);
   if (st != LSDG_OK) return st;
   // the tuned shape of this class of batch when the table has one
-  lsdg_batch_config shape = batch_default_shape(c, jobs[0].kind, n);
+  lsdg_batch_config shape = batch_default_shape(c, n);
   char key[LSDG_TUNE_KEY_BYTES];
   if (lsdg_batch_tune_key(c, jobs, n, key) == LSDG_OK) tune_table_lookup(key, &shape);
   env_shape(shape, n);

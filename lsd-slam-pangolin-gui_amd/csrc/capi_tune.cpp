@@ -368,7 +368,7 @@ extern "C" lsdg_status lsdg_batch_tune(lsdg_ctx c, const lsdg_job* jobs, int32_t
     c->prof_on = prof;
     return s;
   };
-  const lsdg_batch_config def = batch_default_shape(c, jobs[0].kind, n);
+  const lsdg_batch_config def = batch_default_shape(c, n);
   if ((st = S.measure(def, &cur, &curMs)) != LSDG_OK) return done(st);
   if (default_ms) *default_ms = curMs;
   auto consider = [&](const lsdg_batch_config& want) -> lsdg_status {

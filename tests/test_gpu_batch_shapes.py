@@ -1,5 +1,5 @@
 """The default shape of a batch plan: blocks of 512 threads while jobs are few,
-of 256 when they are many, with and without the affine brightness estimate
+of 256 when they are many (either side of the line on 256 CUs), with and without the affine brightness estimate
 (whose sums the kernels leave out otherwise).  Every job takes the LM path of
 the same alignment run by itself."""
 import pytest
@@ -11,7 +11,7 @@ from helpers import twist
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n,block", [(3, 512), (96, 256)])
+@pytest.mark.parametrize("n,block", [(3, 512), (51, 512), (52, 256), (96, 256)])
 @pytest.mark.parametrize("affine", [0, 1])
 @pytest.mark.parametrize("kind", [lsdg.JOB_SE3, lsdg.JOB_SIM3])
 def test_default_shape_takes_the_single_alignments_path(kind, affine, n, block):
