@@ -41,6 +41,14 @@ constexpr int COOP_MAX_BS = 512;
 // step's coefficients out of the loop's registers make room for it.  With four
 // (128 registers, one point per thread in flight) 64 SE3 jobs of 640x480 gain
 // 3%, 24 of 752x478 lose 5%, and Sim3 jobs stay where they are.
+//   What the limit costs: SE3 forms take 150 to 168 registers and spill none to
+// memory (two with FP32, the affine sums and compensated sums together); Sim3
+// forms take all 168, and FP32 spills two (nine with the affine sums, twelve
+// with compensated sums as well), FP16 and BF16 one in that last form only.
+// 13 to 48 scalars sit in vector lanes.  With two waves per SIMD none spilled,
+// and 64 Sim3 FP32 jobs of 640x480 took 609 us where they take 512 (affine 616
+// and 516, affine and compensated 736 and 629).  Blocks of 512 threads, of which
+// a CU holds one, are two waves per SIMD under the same limit.
 constexpr int COOP_WAVES_PER_SIMD = 3;
 
 // ------------------------------------------------------------- kernels
