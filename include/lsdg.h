@@ -216,10 +216,13 @@ lsdg_status lsdg_ctx_synchronize(lsdg_ctx ctx);
  *   LSDG_SUMS_FP64  (default) each term is widened to FP64 and summed in FP64
  *                   per thread and through every tree: the CPU restatement's
  *                   sums to ~1e-16, so the GPU takes its LM path.
- *   LSDG_SUMS_KAHAN compensated FP32: Kahan per-thread sums, TwoSum-merged
- *                   wave and block trees, FP64 only in the cross-block merge
- *                   and the solve.  Sums within ~1e-7 relative of the FP64
- *                   ones, which can flip a borderline LM accept.
+ *   LSDG_SUMS_KAHAN compensated FP32: per-thread (sum, correction) pairs (batch
+ *                   plans by Kahan's update, single evaluations and alignments
+ *                   by TwoSum), TwoSum-merged wave and block trees, FP64 only in
+ *                   the cross-block merge and the solve.  A batch's sums are
+ *                   within ~1e-7 relative of the FP64 ones, which can flip a
+ *                   borderline LM accept; a single call's within ~1e-13 of their
+ *                   terms' magnitudes.
  * Applies to the SE3 and Sim3 evaluations (lsdg_se3_*, lsdg_sim3_*) and to
  * batch plans created afterwards; the adjoint kernels always sum in FP64.
  * No counterpart in the reference, whose LGS6/LGS7 accumulations (upstream

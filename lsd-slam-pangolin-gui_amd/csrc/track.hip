@@ -10,7 +10,7 @@
 // the Jacobian row and its normal-equation terms, and reduces them:
 //   per thread  FP64 accumulation of the FP32 per-point terms over a
 //               grid-stride slice of points (or, with LSDG_SUMS_KAHAN,
-//               Kahan-compensated FP32 pairs),
+//               compensated FP32 pairs),
 //   per wave    reduce-scatter (pairs: by TwoSum),
 //   per block   sum of the wave results in LDS -> one FP64 partial row,
 //   block 0     FP64 sum of all partial rows in a fixed order (deterministic),
@@ -243,7 +243,7 @@ hipError_t launch_se3_eval(lsdg_ctx c, const PointsLevel& pts, lsdg_frame f, int
   const void* img = level_image(f, level);
   hipError_t e = next_eval(c);
   if (e != hipSuccess) return e;
-  auto k = c->sums == LSDG_SUMS_KAHAN ? kern_se3_eval<ACC_KAHAN>(f->precision) : kern_se3_eval<ACC_F64>(f->precision);
+  auto k = c->sums == LSDG_SUMS_KAHAN ? kern_se3_eval<ACC_TWOSUM>(f->precision) : kern_se3_eval<ACC_F64>(f->precision);
   return launch_k(k, grid, block, c->stream, t, pts, img, g, x, kp, d_isgood, c->d_eval_rows, c->eval_epoch, d_out);
 }
 
@@ -254,7 +254,7 @@ hipError_t launch_sim3_eval(lsdg_ctx c, const PointsLevel& pts, lsdg_frame f, in
   const void* img = level_image(f, level);
   hipError_t e = next_eval(c);
   if (e != hipSuccess) return e;
-  auto k = c->sums == LSDG_SUMS_KAHAN ? kern_sim3_eval<ACC_KAHAN>(f->precision) : kern_sim3_eval<ACC_F64>(f->precision);
+  auto k = c->sums == LSDG_SUMS_KAHAN ? kern_sim3_eval<ACC_TWOSUM>(f->precision) : kern_sim3_eval<ACC_F64>(f->precision);
   return launch_k(k, grid, block, c->stream, t, pts, img, (const float*)f->d_idepth[level],
                   (const float*)f->d_ivar[level], g, x, kp, c->d_eval_rows, c->eval_epoch, d_out);
 }

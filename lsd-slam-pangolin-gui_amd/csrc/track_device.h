@@ -323,8 +323,18 @@ __device__ inline bool ratio_below_one(float a, float b) { return a < b || (b < 
 //             once, and only the cross-block merge runs in FP64.  The error
 //             of a block total is ~2 * 2^-24 * sum |term|, independent of the
 //             point count.
+//  ACC_TWOSUM: the same pairs, but each term's rounding error is recovered
+//             exactly (TwoSum, 7 FP32 operations) and only the corrections'
+//             sum rounds: about 2^-48 * sum |term| per term of a thread.  The
+//             single evaluations and alignments sum this way: their grids give
+//             a thread several points, where Kahan's update, which rounds the
+//             correction into the next term, loses what one point per thread
+//             keeps (SE3 poses of 60 pairs up to 1280x960 came out 2e-8 on
+//             average from the FP64 mode's, 6e-7 at most; now 4e-16 and 5e-15).
+//             An alignment takes 4% longer for it (640x480 207 -> 215 us).
 constexpr int ACC_F64 = 0;
 constexpr int ACC_KAHAN = 1;
+constexpr int ACC_TWOSUM = 2;
 
 // lo + up after swapping lo's upper half-wave (offset 32) or odd rows
 // (offset 16) with up's lower half-wave / even rows, 32 bits at a time
@@ -429,6 +439,14 @@ __device__ inline void kahan_add(float& s, float& c, float x) {
   s = t;
 }
 
+// (s, c) += x, the sum's rounding error recovered exactly.
+__device__ inline void two_sum_add(float& s, float& c, float x) {
+  const float t = s + x;
+  const float bp = t - s;
+  c += (s - (t - bp)) + (x - bp);
+  s = t;
+}
+
 // (s, c) += (s2, c2): the sums' rounding error is recovered exactly with
 // TwoSum and folded into the correction.
 __device__ inline void pair_merge(float& s, float& c, float s2, float c2) {
@@ -525,6 +543,11 @@ struct Accum<ACC_KAHAN, NS> {
     }
     return (double)ts + (double)tc;
   }
+};
+
+template <int NS>
+struct Accum<ACC_TWOSUM, NS> : Accum<ACC_KAHAN, NS> {
+  __device__ inline void add(int k, float x) { two_sum_add(this->s[k], this->c[k], x); }
 };
 
 // Which of a point's sums the caller reads.  An LM step reads neither the

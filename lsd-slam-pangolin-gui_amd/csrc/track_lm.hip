@@ -181,7 +181,7 @@ int track_lm_blocks(lsdg_ctx c, int pixels) {
 
 template <int KIND, int PREC>
 static void (*track_kernel(int acc))(TrackLmArgs) {
-  return acc == BATCH_ACC_KAHAN ? k_track_lm<KIND, PREC, ACC_KAHAN> : k_track_lm<KIND, PREC, ACC_F64>;
+  return acc == BATCH_ACC_KAHAN ? k_track_lm<KIND, PREC, ACC_TWOSUM> : k_track_lm<KIND, PREC, ACC_F64>;
 }
 
 hipError_t launch_track_lm(const TrackLmArgs& a, int prec, int acc, hipStream_t s, const KTimer* t) {

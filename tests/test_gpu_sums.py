@@ -14,8 +14,9 @@ sum |x_i| that the outputs themselves give (Cauchy-Schwarz with w >= 0):
 A dropped correction term (plain FP32 sums) misses these bars by orders of
 magnitude at the larger levels; an error in the pair merges shows in A.
 
-Tracking: Kahan sums differ from FP64 ones by ~1e-10 of the bound above
-(measured), which can still flip a borderline LM accept; the bar is 1e-5
+Tracking: a batch's Kahan sums differ from FP64 ones by up to ~1e-10 of the
+bound above (measured; single calls, which recover each term's error exactly,
+by ~1e-15), which can still flip a borderline LM accept; the bar is 1e-5
 twist against the twin on the 12 seeded 640x480 instances and a
 mixed-resolution batch, and for Sim3 1e-5 plus the FP32-sum restatement's own
 spread."""
@@ -87,6 +88,59 @@ def test_kahan_se3_evaluate(kahan, level):
         rel0 = np.max(np.abs(A0 - e2.A7()[:6, :6]) / np.outer(d, d))
         print(f"level 1: Kahan max |dA|/bound {rel:.2e}, plain FP32 sums {rel0:.2e}")
         assert rel < rel0
+
+
+@pytest.mark.parametrize("w,h,density", [(642, 482, 0.25), (1282, 962, 0.5), (1282, 962, 1.0)])
+def test_single_evaluations_keep_each_terms_error(ctx, w, h, density):
+    """Single evaluations recover each term's rounding error exactly, however
+    many points a thread has (one to seven here): against the FP64 mode's sums
+    of the same terms only the corrections round, 2^-24 of 2^-24 of the
+    magnitudes for each of a thread's points and of the ten merges."""
+    cam = synth.camera(w, h)
+    d = synth.sim3_instance(71, cam=cam, max_trans=0.03, max_rot_deg=1.0, scale_range=(0.98, 1.02))
+    rng = np.random.default_rng(3)
+    idepth = np.where(rng.random((h, w)) < density, rng.uniform(0.4, 1.0, (h, w)), -1).astype(np.float32)
+    a, b = ctx.frame(0, cam, d["a_img"]), ctx.frame(1, cam, d["b_img"])
+    a.set_depth(idepth, np.where(idepth > 0, 0.01, -1).astype(np.float32))
+    b.set_depth(d["b_idepth"], d["b_var"])
+    ref = ctx.ref(a)
+    pose = [*synth.sample_pose(77, 0.01, 0.5), 1.02]
+    out = []
+    for mode in (lsdg.SUMS_FP64, lsdg.SUMS_KAHAN):
+        ctx.set_sums(mode)
+        out.append((ctx.se3_evaluate(ref, b, 1, pose[:7])[0], ctx.sim3_evaluate(ref, b, 1, pose)))
+    ctx.set_sums(lsdg.SUMS_FP64)
+    bar = (7 + 10) * 2.0 ** -48
+    for n, e2, ev in ((6, out[0][0], out[1][0]), (7, out[0][1], out[1][1])):
+        A, A2 = ev.A7()[:n, :n], e2.A7()[:n, :n]
+        diag = np.sqrt(np.diag(A2))
+        assert np.all(np.abs(A - A2) <= bar * np.outer(diag, diag))
+        assert np.all(np.abs(np.array(ev.b[:n]) - e2.b[:n]) <= bar * np.sqrt(2.0 * np.diag(A2) * e2.error))
+        assert abs(ev.error - e2.error) <= bar * e2.error and abs(ev.usage - e2.usage) <= bar * e2.usage
+    for x in (ref, b, a):
+        x.destroy()
+
+
+@pytest.mark.parametrize("w,h", [(322, 242), (642, 482), (1282, 962)])
+def test_single_alignments_match_the_fp64_mode(ctx, w, h):
+    """With sums to 1e-13 of their magnitudes, an SE3 alignment in the
+    compensated mode ends where the FP64 mode's does."""
+    cam = synth.camera(w, h)
+    for seed in (41, 42, 43):
+        d = synth.sim3_instance(seed, cam=cam, max_trans=0.03, max_rot_deg=1.0, scale_range=(0.98, 1.02))
+        a, b = ctx.frame(0, cam, d["a_img"]), ctx.frame(1, cam, d["b_img"])
+        a.set_depth(d["a_idepth"], d["a_var"])
+        ref = ctx.ref(a)
+        out = []
+        for mode in (lsdg.SUMS_FP64, lsdg.SUMS_KAHAN):
+            ctx.set_sums(mode)
+            out.append(ctx.se3_track(ref, b, synth.IDENTITY7))
+        ctx.set_sums(lsdg.SUMS_FP64)
+        (p, st, status), (q, st2, status2) = out
+        assert status == status2 and list(st.num_residual_calls) == list(st2.num_residual_calls)
+        assert twist(p, q) <= 1e-11
+        for x in (ref, b, a):
+            x.destroy()
 
 
 @pytest.mark.parametrize("level", [1, 2, 3])
