@@ -268,7 +268,8 @@ lsdg_status lsdg::frame_alloc(lsdg_ctx c, int32_t id, const lsdg_camera* cam, in
 
 lsdg_status lsdg::frame_ensure_quad(lsdg_frame f) {
   if (f->d_quad) return LSDG_OK;
-  CK(f->ctx, f->ctx->blocks.get(&f->d_quadBlock, (size_t)f->w[0] * f->h[0] * 4));
+  hipError_t e = f->ctx->blocks.get(&f->d_quadBlock, (size_t)f->w[0] * f->h[0] * 4);
+  if (e != hipSuccess) return fail(f->ctx, LSDG_ENOMEM, "hipMalloc(packed image)", e);
   f->d_quad = (uint32_t*)f->d_quadBlock;
   return LSDG_OK;
 }
